@@ -631,14 +631,17 @@ __device__ inline void rbgs_cell(const Dims &d, const SysCoef<T> &S, const uint8
                                  int color, int zero_in, uint3 bk) {
     const int j = bk.y * 4 + threadIdx.y, k = bk.z;
     const int i = 2 * (bk.x * 64 + threadIdx.x) + ((j + k + color) & 1);
-    if (i >= d.nx || j >= d.ny) return;
-    const long q = cidx(d, i, j, k);
+    if (j >= d.ny) return;
     if (zero_in) {
         // the initial x is zero: this lane also clears the other cell of its
-        // pair (2t, 2t + 1), so every interior cell is written once
+        // pair (2t, 2t + 1), so every interior cell is written once; in a row
+        // of odd length that other cell may be the row's last one while the
+        // lane's own cell lies past the row's end
         const int ip = i ^ 1;
         if (ip < d.nx) x[cidx(d, ip, j, k)] = T(0);
     }
+    if (i >= d.nx) return;
+    const long q = cidx(d, i, j, k);
     const uint8_t f = flag[q];
     const T bv = b[q];
     const T xo = zero_in ? T(0) : x[q];
