@@ -95,6 +95,7 @@ void IBMSolver_destroy(IBMSolver *s) {
     if (s->ev_rhs) (void)hipEventDestroy(s->ev_rhs);
     (void)hipHostFree(s->sums_h);
     (void)hipHostFree(s->gm_h);
+    if (s->io_h) (void)hipHostFree(s->io_h);
     (void)hipStreamDestroy(s->stream);
     delete s;  // device buffers are released by their owners' destructors
 }
@@ -670,6 +671,8 @@ static void init_device(IBMSolver *s) {
     s->sums_h_epoch = reinterpret_cast<unsigned *>(s->sums_h + kSumSlots);
     s->sums_d_epoch = reinterpret_cast<unsigned *>(s->sums_d + kSumSlots);
     HIP_CHECK(hipHostMalloc((void **)&s->gm_h, 64 * sizeof(double), hipHostMallocDefault));
+    HIP_CHECK(hipHostMalloc((void **)&s->io_h, kIoDoubles * sizeof(double), hipHostMallocMapped));
+    HIP_CHECK(hipHostGetDevicePointer((void **)&s->io_d, s->io_h, 0));
     s->ks.alloc(1);
     s->sums.alloc(kSumSlots);
 }
@@ -789,12 +792,25 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
 // ---------------------------------------------------------------------------
 // initialisation  <- src/ibm3d_init.c:15-37, 237-262
 // ---------------------------------------------------------------------------
+// Device address of scratch for a field of cnt values in the host layout:
+// mapped host memory for small fields (one launch and a host copy; 64 KiB
+// fields: four reads cost the 1.6 ms step-and-look call 3% more through a
+// device scratch and a copy), else a Krylov vector that no kernel carries
+// from one solve to the next and no stencil reads (the padded cells fit its
+// allocation).
+static double *host_layout_scratch(IBMSolver *s, size_t cnt) {
+    return cnt <= kIoDoubles ? s->io_d : s->kry.v64[7].p;
+}
+
 static void upload_cell_field(IBMSolver *s, DBuf<double> &dst, const double *ref) {
-    std::vector<double> h(s->d.ncell, 0.0);
-    for (int i = -2; i < s->Nx + 2; i++)
-        for (int j = -2; j < s->Ny + 2; j++)
-            for (int k = -2; k < s->Nz + 2; k++) h[cidx(s->d, i, j, k)] = ref[host_ref_index(s, i, j, k)];
-    dst.upload(h);
+    const int X = s->Nx + 4, Y = s->Ny + 4, Z = s->Nz + 4;
+    const size_t cnt = (size_t)X * Y * Z;
+    double *scr = host_layout_scratch(s, cnt);
+    if (scr == s->io_d) std::copy(ref, ref + cnt, s->io_h);
+    else HIP_CHECK(hipMemcpyAsync(scr, ref, cnt * sizeof(double), hipMemcpyHostToDevice, s->stream));
+    launch_ref_layout(s->stream, s->d, dst.p, scr, X, Y, Z, -2, -2, -2, false);
+    // the caller's array is its own again when this returns
+    HIP_CHECK(hipStreamSynchronize(s->stream));
 }
 
 extern "C" void IBMSolver_init_flow_const(IBMSolver *s, const double u1, const double u2, const double u3,
@@ -805,11 +821,7 @@ extern "C" void IBMSolver_init_flow_const(IBMSolver *s, const double u1, const d
     s->conv_ready = false;
     const double v[4] = {u1, u2, u3, p};
     DBuf<double> *dst[4] = {&s->u[0], &s->u[1], &s->u[2], &s->p};
-    std::vector<double> h(s->d.ncell);
-    for (int a = 0; a < 4; a++) {
-        std::fill(h.begin(), h.end(), v[a]);
-        dst[a]->upload(h);
-    }
+    for (int a = 0; a < 4; a++) launch_fill(s->stream, dst[a]->p, s->d.ncell, v[a]);
 }
 
 extern "C" void IBMSolver_init_flow_func(IBMSolver *s, IBMSolverInitFunc f1, IBMSolverInitFunc f2,
@@ -856,51 +868,35 @@ static DBuf<double> *cell_field(IBMSolver *s, int field) {
 
 extern "C" void IBMSolver_get_field(IBMSolver *s, int field, double *out) {
     if (!s->assembled) fatal("IBMSolver_get_field before IBMSolver_assemble");
-    HIP_CHECK(hipStreamSynchronize(s->stream));
-    const Dims &d = s->d;
-    const int Nx = s->Nx, Ny = s->Ny, Nz = s->Nz;
-    std::vector<double> h(d.ncell);
+    int n[3] = {s->Nx + 4, s->Ny + 4, s->Nz + 4}, o[3] = {-2, -2, -2};
+    DBuf<double> *src;
     if (field >= IBM3D_FIELD_FACE_U1 && field <= IBM3D_FIELD_FACE_U3) {
+        // N + 1 faces along the field's own axis, padded along the others
         const int a = field - IBM3D_FIELD_FACE_U1;
-        HIP_CHECK(hipMemcpyAsync(h.data(), s->F[a].p, d.ncell * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-        HIP_CHECK(hipStreamSynchronize(s->stream));
-        if (a == 0) {
-            for (int i = 0; i <= Nx; i++)
-                for (int j = -2; j < Ny + 2; j++)
-                    for (int k = -2; k < Nz + 2; k++)
-                        out[((long)i * (Ny + 4) + j + 2) * (Nz + 4) + k + 2] = h[cidx(d, i, j, k)];
-        } else if (a == 1) {
-            for (int i = -2; i < Nx + 2; i++)
-                for (int j = 0; j <= Ny; j++)
-                    for (int k = -2; k < Nz + 2; k++)
-                        out[((long)(i + 2) * (Ny + 1) + j) * (Nz + 4) + k + 2] = h[cidx(d, i, j, k)];
-        } else {
-            for (int i = -2; i < Nx + 2; i++)
-                for (int j = -2; j < Ny + 2; j++)
-                    for (int k = 0; k <= Nz; k++)
-                        out[((long)(i + 2) * (Ny + 4) + j + 2) * (Nz + 1) + k] = h[cidx(d, i, j, k)];
-        }
-        return;
+        src = &s->F[a];
+        n[a] -= 3;
+        o[a] = 0;
+    } else {
+        src = cell_field(s, field);
+        if (!src) fatal("unknown field");
     }
-    DBuf<double> *src = cell_field(s, field);
-    if (!src) fatal("unknown field");
+    const size_t cnt = (size_t)n[0] * n[1] * n[2];
     if (!src->p) {
-        const long P = (long)(Nx + 4) * (Ny + 4) * (Nz + 4);
-        for (long q = 0; q < P; q++) out[q] = 0;
+        std::fill(out, out + cnt, 0.0);
         return;
     }
-    HIP_CHECK(hipMemcpyAsync(h.data(), src->p, d.ncell * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    double *scr = host_layout_scratch(s, cnt);
+    launch_ref_layout(s->stream, s->d, src->p, scr, n[0], n[1], n[2], o[0], o[1], o[2], true);
+    if (scr != s->io_d)
+        HIP_CHECK(hipMemcpyAsync(out, scr, cnt * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     HIP_CHECK(hipStreamSynchronize(s->stream));
-    for (int i = -2; i < Nx + 2; i++)
-        for (int j = -2; j < Ny + 2; j++)
-            for (int k = -2; k < Nz + 2; k++) out[host_ref_index(s, i, j, k)] = h[cidx(d, i, j, k)];
+    if (scr == s->io_d) std::copy(s->io_h, s->io_h + cnt, out);
 }
 
 extern "C" void IBMSolver_set_field(IBMSolver *s, int field, const double *in) {
     if (!s->assembled) fatal("IBMSolver_set_field before IBMSolver_assemble");
     if (field != IBM3D_FIELD_U1 && field != IBM3D_FIELD_U2 && field != IBM3D_FIELD_U3 && field != IBM3D_FIELD_P)
         fatal("set_field supports u1, u2, u3, p");
-    HIP_CHECK(hipStreamSynchronize(s->stream));
     upload_cell_field(s, *cell_field(s, field), in);
     s->conv_ready = false;
 }

@@ -267,6 +267,7 @@ struct _ibm_solver {
     bool mom_lanes = false;
     double *sums_h = nullptr;        // pinned
     double *gm_h = nullptr;          // pinned, 64 scalars of the GMRES / PCG solvers
+    double *io_h = nullptr, *io_d = nullptr;  // device-mapped host memory, kIoDoubles: small fields in the host layout
 
     // ghost cells
     int ng = 0;
@@ -309,6 +310,9 @@ namespace ibm {
 // convective outflow faces' BC-row norms (3 per face, bc[] order)
 constexpr int kSumSlots = 32;
 constexpr int kConvNormSlot = 12;
+// fields of up to this many values (1 MiB) cross between host and device
+// through mapped memory that the layout kernel itself reads or writes
+constexpr size_t kIoDoubles = 1u << 17;
 constexpr int kConvSpeedSlot = 31;  // convection speed of the face being advanced
 
 // Errors of one case (rejected input, a non-finite residual, a lost Krylov

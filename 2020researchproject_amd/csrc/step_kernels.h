@@ -97,4 +97,12 @@ void launch_body_force(hipStream_t st, const Geo &g, const uint8_t *flag, const 
 void launch_maxdiv(hipStream_t st, const Geo &g, const uint8_t *flag, long pin, const double *const U[3],
                    double *partial);
 
+// Host (reference) layout <-> device layout: the ni x nj x nk array with k
+// fastest whose element (a, b, c) is cell (i0 + a, j0 + b, k0 + c) of the
+// device field f. to_host: ref <- f, else f <- ref.
+void launch_ref_layout(hipStream_t st, const Dims &d, double *f, double *ref, int ni, int nj, int nk, int i0, int j0,
+                       int k0, bool to_host);
+// a[0 .. n) = v
+void launch_fill(hipStream_t st, double *a, long n, double v);
+
 }  // namespace ibm

@@ -25,3 +25,28 @@ def test_pressure_cycle_of_odd_rows_converges_as_of_even_rows(new_gpu, cases, sh
         s.iterate(4)
         its.append(int(s.last_iters()[3]))
     assert abs(its[0] - its[1]) <= 2, its
+
+
+@pytest.mark.parametrize("shape", [(33, 31, 35), (64, 5, 7), (6, 40, 66), (128, 32, 33)])
+def test_fields_cross_the_host_boundary_unchanged(new_gpu, I, cases, shape):
+    """set / get of a cell field move every padded cell to its place (tile
+    remainders on both transposed axes, small and large fields), and a face
+    field is the interpolation of the cells it lies between."""
+    s = new_gpu()
+    cases.setup_cavity(s, shape=shape, tol=1e-10)
+    rng = np.random.default_rng(3)
+    a = {n: rng.standard_normal(s.shape) for n in ("U1", "U2", "U3", "P")}
+    for n, v in a.items():
+        s.set(n, v)
+    for n, v in a.items():
+        np.testing.assert_array_equal(s.get(n), v)
+    s.iterate(0)  # outer layers and face velocities from the cell fields
+    for ax, n in enumerate(("U1", "U2", "U3")):
+        u = s.get(n)
+        sl = [slice(2, -2)] * 3
+        lo, hi = list(sl), list(sl)
+        lo[ax], hi[ax] = slice(1, -2), slice(2, -1)
+        f = s.get("FACE_" + n)
+        inner = list(sl)
+        inner[ax] = slice(None)
+        np.testing.assert_allclose(f[tuple(inner)], 0.5 * (u[tuple(lo)] + u[tuple(hi)]), rtol=1e-13, atol=1e-13)
