@@ -784,6 +784,7 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
                 if (s->bc[face_bc(a, hi)].type == BC_CONVECTIVE_OUTFLOW) s->conv_g[face_bc(a, hi)].alloc(4 * ext[a]);
         s->conv_ready = false;
     }
+    if (s->precision != IBM3D_PREC_MIXED) build_momentum_tables(s);
     build_mg(s);
     s->assembled = true;
     HIP_CHECK(hipStreamSynchronize(s->stream));

@@ -228,6 +228,10 @@ struct _ibm_solver {
     double mg_omega = 1.3;       // over-relaxation factor of the pressure multigrid smoother
     int mom_solver = 0;          // IBMSolver_set_momentum_solver: 0 automatic, 1 BiCGSTAB
     int mom_sweeps = -1;         // FP32 sweeps per refinement round of the momentum solves (0: not used; -1: unset)
+    ibm::DBuf<ibm::MomTable<double>> mt64;  // operands of the batched momentum launches
+    ibm::DBuf<ibm::MomTable<float>> mt32;   // mixed-Krylov mode: the FP32 corrections
+    ibm::DBuf<double> mgv64;     // ghost values of the three components (two buffers each)
+    ibm::DBuf<float> mgv32;
     double mom_rate = 0;         // estimated red-black sweep contraction of the momentum operators
 
     // ---- host mirrors ----
@@ -343,6 +347,7 @@ void build_system(const IBMSolver *s, const std::vector<double> *D[3], const std
 // step.cpp
 void iterate_impl(IBMSolver *s, int steps, bool verbose);
 void build_mg(IBMSolver *s);
+void build_momentum_tables(IBMSolver *s);
 double max_div_impl(IBMSolver *s);
 void body_force_impl(IBMSolver *s, double *dst);
 void body_force_read(IBMSolver *s, double out[3]);

@@ -32,6 +32,17 @@ struct KScal {
     int pad;
 };
 
+// Operands of the three momentum systems, in device memory: right-hand sides
+// b (brw: the same, where a kernel writes them), solutions x, residuals r and
+// the ghost rows' two value buffers per component.
+template <typename T>
+struct MomTable {
+    SysCoef<T> S[3];
+    const T *b[3];
+    T *brw[3], *x[3], *r[3];
+    T *gv[3][2];
+};
+
 // Which per-row scale the normalised residual uses: none, or 1 / sum K on
 // fluid rows (the reference's diagonal-normalised pressure rows).
 struct NormSpec {
@@ -108,6 +119,28 @@ template <typename T>
 int launch_rbgs_color_ghost(hipStream_t st, const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const T *b,
                             T *x, int color, const GhostRows<T> &G, int prev);
 
+// The three momentum systems of the table *M (device memory) in one launch
+// each; components outside `mask` are left alone.
+// One colour; prev: where the ghost values are (launch_ghost_relax), returned
+// anew. zero_in: from a zero start, without the ghost rows.
+template <typename T>
+int launch_mom_colour(hipStream_t st, const Dims &d, const MomTable<T> *M, unsigned mask, const uint8_t *flag,
+                      int color, int zero_in, const GhostRows<T> &G, int prev);
+// ghost rows of colour `only` after a zero start: values left in buffer 0
+template <typename T>
+void launch_mom_ghost(hipStream_t st, const Dims &d, const MomTable<T> *M, unsigned mask, const GhostRows<T> &G,
+                      int only);
+// residuals (written to M->r when store) with partial[3 blk + c] = the block's
+// share of ||b_c - A_c x_c||^2, apply_partials blocks
+void launch_mom_residual(hipStream_t st, const Dims &d, const MomTable<double> *M, unsigned mask,
+                         const GhostRows<double> &G, const uint8_t *flag, bool store, double *partial);
+// FP32 right-hand sides M32->b from M->b or M->r, and the first colour in M32->x
+void launch_mom_d2f_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
+                          unsigned mask, const uint8_t *flag, bool from_b);
+// M->x = M32->x, or (add) M->x += M32->x
+void launch_mom_add(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
+                    unsigned mask, bool add);
+
 // BiCGSTAB pieces
 template <typename T>
 // x = 0, r = rh = b, p = v = 0 (p and v left alone when p is null: the
@@ -174,6 +207,10 @@ void launch_finalize(hipStream_t st, int op, const double *partial, long nblk, i
 void launch_publish(hipStream_t st, const double *in, int nv, double *out, unsigned *epoch_out, unsigned epoch);
 // out[a] = sum (or max) over blocks of partial[b * nv + a]
 void launch_sum_partials(hipStream_t st, const double *partial, long nblk, int nv, double *out, int reduce_max);
+
+// launch_sum_partials into device-mapped host memory, followed by the epoch
+void launch_sum_publish(hipStream_t st, const double *partial, long nblk, int nv, double *out, int reduce_max,
+                        unsigned *epoch_out, unsigned epoch);
 
 // precision conversion / accumulation over interior cells
 void launch_d2f(hipStream_t st, const Dims &d, const double *a, float *b);

@@ -353,25 +353,26 @@ __device__ inline double nscale(const NormSpec &ns, const Dims &d, int i, int j,
     return 1.0 / (ns.ksx[i] + ns.ksy[j] + ns.ksz[k]);
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRows<T> G,
-                                                  const uint8_t *__restrict__ flag, const T *__restrict__ b,
-                                                  const T *__restrict__ x, T *__restrict__ r, NormSpec ns,
-                                                  double *partial, unsigned ngb, unsigned gx, unsigned gy) {
+// One block of the residual r = b - A x (blocks below ngb: ghost rows, the
+// others cell pairs, XCD-contiguous of `nb` blocks in all): acc gets the
+// block's lanes' shares of ||r||^2 and ||D^-1 r||^2. STORE: r is written.
+template <bool STORE, typename T>
+__device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const GhostRows<T> &G,
+                                      const uint8_t *__restrict__ flag, const T *__restrict__ b,
+                                      const T *__restrict__ x, T *__restrict__ r, const NormSpec &ns, unsigned wb,
+                                      unsigned nb, unsigned ngb, unsigned gx, unsigned gy, double (&acc)[2]) {
     using T2 = typename Vec2<T>::type;
-    const unsigned wb = blockIdx.x;
-    double acc[2] = {0, 0};
     if (wb < ngb) {
         const int s = (int)wb * 64 + threadIdx.x;
         if (threadIdx.y == 0 && s < G.ng) {
             long c;
             const T yv = ghost_row_apply<T>(G, S.is_p, x, s, c);
             const T rv = b[c] - yv;
-            r[c] = rv;
+            if (STORE) r[c] = rv;
             acc[0] = acc[1] = (double)rv * (double)rv;
         }
     } else {
-        const uint3 bk = xcd_map(wb - ngb, gridDim.x - ngb, gx, gy);
+        const uint3 bk = xcd_map(wb - ngb, nb - ngb, gx, gy);
         const int i0 = 2 * (bk.x * 64 + threadIdx.x), j = bk.y * 4 + threadIdx.y;
         const int k0 = bk.z * kRedZP, k1 = min(k0 + kRedZP, d.nz);
         if (i0 < d.nx && j < d.ny) {
@@ -402,7 +403,7 @@ __global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRow
                     gh[o] = !ident && f == F_GHOST;  // written by the ghost blocks
                     on[o] = i0 + o < d.nx && (ident || f == F_FLUID);
                 }
-                store_pair_skip(d, i0, q0, r, v[0], v[1], gh[0], gh[1]);
+                if (STORE) store_pair_skip(d, i0, q0, r, v[0], v[1], gh[0], gh[1]);
 #pragma unroll
                 for (int o = 0; o < 2; o++) {
                     if (!on[o]) continue;
@@ -414,7 +415,16 @@ __global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRow
             }
         }
     }
-    bsum<2>(acc, partial, wb);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRows<T> G,
+                                                  const uint8_t *__restrict__ flag, const T *__restrict__ b,
+                                                  const T *__restrict__ x, T *__restrict__ r, NormSpec ns,
+                                                  double *partial, unsigned ngb, unsigned gx, unsigned gy) {
+    double acc[2] = {0, 0};
+    residual_block<true>(d, S, G, flag, b, x, r, ns, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    bsum<2>(acc, partial, blockIdx.x);
 }
 
 template <typename T>
@@ -930,8 +940,8 @@ void launch_rbgs_fused(hipStream_t st, const Dims &d, const SysCoef<T> &S, const
 // order in which waves run. Eight lanes per row, one per source; the row's
 // sum is formed in source order from the values exchanged within the wave.
 template <typename T>
-__global__ void __launch_bounds__(256) k_ghost_relax(GhostRows<T> G, int is_p, const T *b, T *x, const T *prev,
-                                                     T *next, Dims d, int only) {
+__device__ inline void ghost_relax_rows(const GhostRows<T> &G, int is_p, const T *b, T *x, const T *prev, T *next,
+                                        const Dims &d, int only) {
     const int s = ghost_row_of_lane(blockIdx.x), t = threadIdx.x & 63, l = t & 7;
     const bool in = s < G.ng;
     bool act = in;
@@ -979,6 +989,12 @@ __global__ void __launch_bounds__(256) k_ghost_relax(GhostRows<T> G, int is_p, c
     }
     x[c] = v;
     next[s] = v;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_ghost_relax(GhostRows<T> G, int is_p, const T *b, T *x, const T *prev,
+                                                     T *next, Dims d, int only) {
+    ghost_relax_rows(G, is_p, b, x, prev, next, d, only);
 }
 
 template <typename T>
@@ -1254,6 +1270,23 @@ __global__ void __launch_bounds__(kFinThreads) k_sum_partials(const double *part
         for (int a = 0; a < nv; a++) out[a] = sh[a][0];
 }
 
+// k_sum_partials into device-mapped host memory, then the epoch (k_publish)
+__global__ void __launch_bounds__(kFinThreads) k_sum_publish(const double *partial, long nblk, int nv, double *out,
+                                                             int reduce_max, unsigned *epoch_out, unsigned epoch) {
+    __shared__ double sh[4][kFinThreads];
+    sum_columns(partial, nblk, nv, reduce_max, sh);
+    if (threadIdx.x != 0) return;
+    for (int a = 0; a < nv; a++) out[a] = sh[a][0];
+    __threadfence_system();
+    *reinterpret_cast<volatile unsigned *>(epoch_out) = epoch;
+}
+
+void launch_sum_publish(hipStream_t st, const double *partial, long nblk, int nv, double *out, int reduce_max,
+                        unsigned *epoch_out, unsigned epoch) {
+    hipLaunchKernelGGL(k_sum_publish, dim3(1), dim3(kFinThreads), 0, st, partial, nblk, nv, out, reduce_max, epoch_out,
+                       epoch);
+}
+
 void launch_sum_partials(hipStream_t st, const double *partial, long nblk, int nv, double *out, int reduce_max) {
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kFinThreads), 0, st, partial, nblk, nv, out, reduce_max);
 }
@@ -1445,9 +1478,8 @@ __global__ void __launch_bounds__(256) k_d2f(Dims d, const double *a, float *b) 
 }
 // b = (float) a, and x = the first smoother colour from a zero start; two
 // cells of a row per lane
-__global__ void __launch_bounds__(256) k_d2f_first(Dims d, SysCoef<float> S, const uint8_t *flag, const double *a,
-                                                   float *b, float *x) {
-    const int i0 = 2 * (blockIdx.x * 64 + threadIdx.x), j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
+__device__ inline void d2f_first(const Dims &d, const SysCoef<float> &S, const uint8_t *flag, const double *a,
+                                 float *b, float *x, int i0, int j, int k) {
     if (i0 >= d.nx || j >= d.ny) return;
     const long q0 = cidx(d, i0, j, k);
     const double2 av = *reinterpret_cast<const double2 *>(a + q0);
@@ -1463,6 +1495,10 @@ __global__ void __launch_bounds__(256) k_d2f_first(Dims d, SysCoef<float> S, con
         b[q0] = b0;
         x[q0] = x0;
     }
+}
+__global__ void __launch_bounds__(256) k_d2f_first(Dims d, SysCoef<float> S, const uint8_t *flag, const double *a,
+                                                   float *b, float *x) {
+    d2f_first(d, S, flag, a, b, x, 2 * (blockIdx.x * 64 + threadIdx.x), blockIdx.y * 4 + threadIdx.y, blockIdx.z);
 }
 __global__ void __launch_bounds__(256) k_add_f2d(Dims d, const float *e, double *x) {
     const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
@@ -1510,6 +1546,162 @@ template <typename T>
 void launch_copy(hipStream_t st, const Dims &d, const T *a, T *b) {
     hipLaunchKernelGGL((k_copy<T>), igrid(d), dim3(64, 4), 0, st, d, a, b);
 }
+
+// ---------------------------------------------------------------------------
+// The three momentum systems in one launch: blockIdx.y is the component, whose
+// operands come from a table in device memory (read as scalars). They share
+// the grid, the flags and the ghost stencils; one launch in place of three
+// saves two launch latencies per stage where the grid is small (a launch of
+// any size up to 64^3 takes 4 to 5 us with its gap) and two kernel tails
+// where it is large. Components outside `mask` return at once.
+// ---------------------------------------------------------------------------
+template <typename T>
+__global__ void __launch_bounds__(256) k_mom_colour(Dims d, const MomTable<T> *M, unsigned mask, const uint8_t *flag,
+                                                    int color, int zero_in, GhostRows<T> G, int prev, unsigned ngb,
+                                                    unsigned gx, unsigned gy) {
+    const unsigned c = blockIdx.y, w = blockIdx.x;
+    if (!((mask >> c) & 1u)) return;
+    const SysCoef<T> S = M->S[c];
+    const T *b = M->b[c];
+    T *x = M->x[c];
+    if (w < ngb) {
+        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const T *)M->gv[c][prev], M->gv[c][prev ^ 1], color,
+                             threadIdx.x, ghost_row_of_lane(w));
+        return;
+    }
+    rbgs_cell(d, S, flag, b, x, color, zero_in, xcd_map(w - ngb, gridDim.x - ngb, gx, gy));
+}
+
+template <int BY>
+__global__ void __launch_bounds__(64 * BY) k_mom_colour_quad(Dims d, const MomTable<float> *M, unsigned mask,
+                                                             const uint8_t *flag, int color, int zero_in,
+                                                             GhostRows<float> G, int prev, unsigned ngb, unsigned gx,
+                                                             unsigned gy) {
+    const unsigned c = blockIdx.y, w = blockIdx.x;
+    if (!((mask >> c) & 1u)) return;
+    const SysCoef<float> S = M->S[c];
+    const float *b = M->b[c];
+    float *x = M->x[c];
+    if (w < ngb) {
+        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const float *)M->gv[c][prev], M->gv[c][prev ^ 1], color,
+                             threadIdx.x, ghost_row_of_lane(w));
+        return;
+    }
+    rbgs_quad<BY>(d, S, flag, b, x, color, zero_in, xcd_map(w - ngb, gridDim.x - ngb, gx, gy));
+}
+
+// relaxation of the first colour's ghost rows after a zero start
+template <typename T>
+__global__ void __launch_bounds__(256) k_mom_ghost(Dims d, const MomTable<T> *M, unsigned mask, GhostRows<T> G,
+                                                   int only) {
+    const unsigned c = blockIdx.y;
+    if (!((mask >> c) & 1u)) return;
+    ghost_relax_rows(G, 0, M->b[c], M->x[c], (const T *)nullptr, M->gv[c][0], d, only);
+}
+
+template <typename T>
+int launch_mom_colour(hipStream_t st, const Dims &d, const MomTable<T> *M, unsigned mask, const uint8_t *flag,
+                      int color, int zero_in, const GhostRows<T> &G, int prev) {
+    // ghost rows ride in the launch once a first relaxation has set their values
+    const bool gh = G.ng > 0 && !zero_in;
+    if (gh && prev < 0) abort();
+    if constexpr (std::is_same<T, float>::value) {
+        if (d.nx >= kQuadMinRow) {
+            const unsigned ngb = gh ? colour_ghost_blocks(G.ng, 64 * 8) : 0u;
+            const unsigned gx = ((d.nx + 3) / 4 + 63) / 64, gy = (d.ny + 7) / 8;
+            hipLaunchKernelGGL((k_mom_colour_quad<8>), dim3(ngb + gx * gy * d.nz, 3), dim3(64, 8), 0, st, d, M, mask,
+                               flag, color, zero_in, G, prev, ngb, gx, gy);
+            return gh ? prev ^ 1 : prev;
+        }
+    }
+    const unsigned ngb = gh ? colour_ghost_blocks(G.ng, 64 * 4) : 0u;
+    const unsigned gx = ((d.nx + 1) / 2 + 63) / 64, gy = (d.ny + 3) / 4;
+    hipLaunchKernelGGL((k_mom_colour<T>), dim3(ngb + gx * gy * d.nz, 3), dim3(64, 4), 0, st, d, M, mask, flag, color,
+                       zero_in, G, prev, ngb, gx, gy);
+    return gh ? prev ^ 1 : prev;
+}
+
+template <typename T>
+void launch_mom_ghost(hipStream_t st, const Dims &d, const MomTable<T> *M, unsigned mask, const GhostRows<T> &G,
+                      int only) {
+    hipLaunchKernelGGL((k_mom_ghost<T>), dim3((G.ng + 31) / 32, 3), dim3(256), 0, st, d, M, mask, G, only);
+}
+
+template <bool STORE>
+__global__ void __launch_bounds__(256) k_mom_residual(Dims d, const MomTable<double> *M, unsigned mask,
+                                                      GhostRows<double> G, const uint8_t *flag, double *partial,
+                                                      unsigned ngb, unsigned gx, unsigned gy) {
+    const unsigned c = blockIdx.y;
+    if (!((mask >> c) & 1u)) return;
+    const SysCoef<double> S = M->S[c];
+    const NormSpec off{0, nullptr, nullptr, nullptr, nullptr, -1};
+    double acc[2] = {0, 0};
+    residual_block<STORE>(d, S, G, flag, M->b[c], (const double *)M->x[c], M->r[c], off, blockIdx.x, gridDim.x, ngb,
+                          gx, gy, acc);
+    const double a1[1] = {acc[0]};
+    bsum<1>(a1, partial, (long)blockIdx.x * 3 + c);
+}
+
+void launch_mom_residual(hipStream_t st, const Dims &d, const MomTable<double> *M, unsigned mask,
+                         const GhostRows<double> &G, const uint8_t *flag, bool store, double *partial) {
+    const dim3 grid(agrid_blocks(d, G.ng), 3);
+    if (store)
+        hipLaunchKernelGGL(k_mom_residual<true>, grid, dim3(64, 4), 0, st, d, M, mask, G, flag, partial,
+                           ghost_blocks(G.ng), pgx(d), pgy(d));
+    else
+        hipLaunchKernelGGL(k_mom_residual<false>, grid, dim3(64, 4), 0, st, d, M, mask, G, flag, partial,
+                           ghost_blocks(G.ng), pgx(d), pgy(d));
+}
+
+// FP32 right-hand sides of a correction, b (from x = 0) or the residual,
+// with the first smoother colour
+__global__ void __launch_bounds__(256) k_mom_d2f_first(Dims d, const MomTable<double> *M, const MomTable<float> *M32,
+                                                       unsigned mask, const uint8_t *flag, int from_b) {
+    const unsigned c = blockIdx.z / d.nz, k = blockIdx.z % d.nz;
+    if (!((mask >> c) & 1u)) return;
+    const SysCoef<float> S = M32->S[c];
+    d2f_first(d, S, flag, from_b ? M->b[c] : M->r[c], M32->brw[c], M32->x[c], 2 * (blockIdx.x * 64 + threadIdx.x),
+              blockIdx.y * 4 + threadIdx.y, k);
+}
+
+// x = e, or x += e
+__global__ void __launch_bounds__(256) k_mom_add(Dims d, const MomTable<double> *M, const MomTable<float> *M32,
+                                                 unsigned mask, int add) {
+    const unsigned c = blockIdx.z / d.nz, k = blockIdx.z % d.nz;
+    const int i0 = 2 * (blockIdx.x * 64 + threadIdx.x), j = blockIdx.y * 4 + threadIdx.y;
+    if (!((mask >> c) & 1u) || i0 >= d.nx || j >= d.ny) return;
+    const long q = cidx(d, i0, j, k);
+    const float2 e = *reinterpret_cast<const float2 *>(M32->x[c] + q);
+    double2 *x = reinterpret_cast<double2 *>(M->x[c] + q);
+    double2 v = make_double2((double)e.x, (double)e.y);
+    if (add) {
+        const double2 o = *x;
+        v.x = o.x + v.x;
+        v.y = o.y + v.y;
+    }
+    if (i0 + 1 < d.nx) *x = v;
+    else M->x[c][q] = v.x;
+}
+
+void launch_mom_d2f_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
+                          unsigned mask, const uint8_t *flag, bool from_b) {
+    dim3 g = jgrid(d);
+    g.z *= 3;
+    hipLaunchKernelGGL(k_mom_d2f_first, g, dim3(64, 4), 0, st, d, M, M32, mask, flag, from_b ? 1 : 0);
+}
+void launch_mom_add(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
+                    unsigned mask, bool add) {
+    dim3 g = jgrid(d);
+    g.z *= 3;
+    hipLaunchKernelGGL(k_mom_add, g, dim3(64, 4), 0, st, d, M, M32, mask, add ? 1 : 0);
+}
+#define INST_MOM(T)                                                                                                 \
+    template int launch_mom_colour<T>(hipStream_t, const Dims &, const MomTable<T> *, unsigned, const uint8_t *, int, \
+                                      int, const GhostRows<T> &, int);                                              \
+    template void launch_mom_ghost<T>(hipStream_t, const Dims &, const MomTable<T> *, unsigned, const GhostRows<T> &, \
+                                      int);
+INST_MOM(double)
+INST_MOM(float)
 
 // ---------------------------------------------------------------------------
 // multigrid transfers

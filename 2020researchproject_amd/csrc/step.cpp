@@ -228,6 +228,14 @@ static void read_sums(IBMSolver *s, int nv) {
     wait_epoch(s->stream, s->sums_h_epoch, e);
 }
 
+// The sums (maxima) of nv columns of block partials, formed straight into
+// sums_h and awaited there
+static void sum_read(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
+    const unsigned e = ++s->sums_epoch;
+    launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d, reduce_max, s->sums_d_epoch, e);
+    wait_epoch(s->stream, s->sums_h_epoch, e);
+}
+
 // Finalize kernel `op` over the block partials, with the resulting scalars
 // published into host memory, then a wait for them there: no copy and no
 // stream synchronisation on the Krylov loop's path (each end of iteration
@@ -597,8 +605,7 @@ static void smooth(IBMSolver *s, const Dims &d, const SysCoef<T> &S, const Ghost
                 // the first colour from a zero start writes every cell;
                 // first_done: the kernel that wrote b already wrote it
                 const bool z = zero_init && sw == 0 && c == 0;
-                if (level >= 0) snprintf(nm, sizeof nm, "rbgs_L%d", level);
-                else snprintf(nm, sizeof nm, "mom_rbgs");
+                snprintf(nm, sizeof nm, "rbgs_L%d", level);
                 // Ghost rows are relaxed after each colour, those of the
                 // colour just updated (the others keep their values); past a
                 // zero start that happens inside the colour launch itself.
@@ -620,8 +627,7 @@ static void smooth(IBMSolver *s, const Dims &d, const SysCoef<T> &S, const Ghost
     T *cur = x, *nxt = xalt;
     for (int sw = 0; sw < sweeps; sw++) {
         const bool z = zero_init && sw == 0;
-        if (level >= 0) snprintf(nm, sizeof nm, "rbgs_fused_L%d", level);
-        else snprintf(nm, sizeof nm, "mom_rbgs_fused");
+        snprintf(nm, sizeof nm, "rbgs_fused_L%d", level);
         TIMED(nm, n * ((z ? 2 : 3) * sizeof(T) + 1),
               launch_rbgs_fused<T>(s->stream, d, S, flag, b, cur, nxt, z ? 1 : 0));
         if (G.ng) {
@@ -1404,22 +1410,31 @@ static void solve_system(IBMSolver *s, int sk, const double *b, double *x, doubl
 }
 
 // ---------------------------------------------------------------------------
-// Momentum solves of the mixed-Krylov mode: FP32 red-black Gauss-Seidel
-// sweeps inside FP64 iterative refinement. The Helmholtz operator
-// (1 + sum K) I - sum K_nb is strongly diagonally dominant wherever
-// dt / (Re h^2) is small: a Jacobi sweep then contracts fluid rows by
-// rho_J = max sum K / (1 + sum K) and a red-black sweep by about rho_J^2, so
-// m sweeps per round reduce the correction's residual by rho_J^(2m) until FP32
-// rounding (~1e-7) limits it. Each round: FP32 right-hand side (the FP64
-// residual; the first colour written in the same launch), m sweeps from zero,
-// x += e in FP64, FP64 residual and its norm. The stopping test is the
-// reference's ||b - A x|| <= tol ||b|| in FP64. Where rho_J^2 > 0.03 (few
-// sweeps would not do) the BiCGSTAB path solves instead, as it does for a
-// component whose residual stops falling by at least 10x per round.
+// Momentum solves by red-black Gauss-Seidel sweeps, the three components in
+// each launch. The Helmholtz operator (1 + sum K) I - sum K_nb is strongly
+// diagonally dominant wherever dt / (Re h^2) is small: a Jacobi sweep then
+// contracts fluid rows by rho_J = max sum K / (1 + sum K) and a red-black
+// sweep by about rho_J^2.
+//   FP64 mode: sweeps on the system itself from x = 0, as many as the
+//     estimated rate asks for, then the FP64 residual norm; further rounds at
+//     the rate the last one showed.
+//   Mixed-Krylov mode: FP32 sweeps inside FP64 refinement. Each round: FP32
+//     right-hand side (the FP64 residual; the first colour written in the same
+//     launch), m sweeps from zero, x += e in FP64, FP64 residual and its norm.
+// The stopping test is the reference's ||b - A x|| <= tol ||b|| in FP64.
+// A component whose residual stops falling by at least 10x per round goes to
+// BiCGSTAB, as do all three where the rate is above kMomMaxRate. FP64, sphere
+// 256 x 128 x 128 at 1e-12: 6 sweeps (12 launches of 70 us) and one residual
+// against 5 BiCGSTAB iterations of 8 kernels per component.
 // ---------------------------------------------------------------------------
-static const double kMomRoundTarget = 1e-6;  // residual reduction aimed at per round
-static const double kMomMaxRate = 0.03;      // largest rho_J^2 for which sweeps are used
-static const int kMomMaxRounds = 8;
+static const double kMomRoundTarget = 1e-6;  // residual reduction aimed at per FP32 round
+// Largest rho_J^2 for which sweeps are used, the largest measured: ms per step
+// at 1e-12, sweeps against BiCGSTAB (its three solves on streams of their
+// own), FP64 / mixed: cavity 64^3 at rate 0.145 2.56 : 3.15 / 2.40 : 3.02,
+// 96^3 at 0.337 4.26 : 5.26 / 3.86 : 5.04, 128^3 at 0.008 5.27 : 6.25 / 5.73 :
+// 6.51, at 0.246 6.18 : 8.27 / 6.29 : 8.34, at 0.505 7.52 : 10.41 / 7.28 : 10.10
+static const double kMomMaxRate = 0.5;
+static const int kMomMaxRounds = 8; 
 
 static int momentum_sweeps(IBMSolver *s) {
     if (s->mom_sweeps >= 0) return s->mom_sweeps;
@@ -1429,82 +1444,132 @@ static int momentum_sweeps(IBMSolver *s) {
     for (int k = 0; k < s->Nz; k++) mx[2] = std::max(mx[2], H1(s->kD, k) + H1(s->kU, k));
     const double sk = mx[0] + mx[1] + mx[2], rj = sk / (1 + sk), rate = rj * rj;
     s->mom_rate = rate;
+    const double target = s->precision == IBM3D_PREC_FP64 ? 0.5 * s->tol : kMomRoundTarget;
     s->mom_sweeps = (rate > 0 && rate <= kMomMaxRate)
-                        ? std::max(2, (int)std::ceil(std::log(kMomRoundTarget) / std::log(rate))) : 0;
+                        ? std::max(2, (int)std::ceil(std::log(target) / std::log(rate))) : 0;
     return s->mom_sweeps;
 }
 
-// Sweeps for a round that must reduce the residual by `need` (< 1): enough
-// at the estimated rate with a factor 2 to spare, at least one, at most the
-// full round's count.
-static int momentum_round_sweeps(const IBMSolver *s, double need) {
-    const double f = std::max(need, kMomRoundTarget) * 0.5;
-    return std::min(s->mom_sweeps, std::max(1, (int)std::ceil(std::log(f) / std::log(s->mom_rate))));
+// Sweeps for a round that must reduce the residual by `need` (< 1) at `rate`
+// per sweep: enough with a factor 2 to spare, at least one, at most `most`.
+static int momentum_round_sweeps(double need, double rate, int most) {
+    return std::min(most, std::max(1, (int)std::ceil(std::log(0.5 * need) / std::log(rate))));
 }
 
-// The three momentum solves by refinement; components that do not converge
-// this way are solved by solve_system. bn: the stopping norms.
-static void momentum_refine(IBMSolver *s, const double bn[3]) {
+void build_momentum_tables(IBMSolver *s) {
+    const size_t ng = std::max(s->ng, 1);
+    s->mgv64.alloc(6 * ng);
+    MomTable<double> t{};
+    for (int c = 0; c < 3; c++) {
+        t.S[c] = s->sys[c].S64;
+        t.b[c] = t.brw[c] = s->b[c].p;
+        t.x[c] = s->us[c].p;
+        t.r[c] = s->precision == IBM3D_PREC_FP64 ? nullptr : c == 0 ? s->ref_r64.p : s->mlane[c - 1].v[0].p;
+        for (int k = 0; k < 2; k++) t.gv[c][k] = s->mgv64.p + (2 * c + k) * ng;
+    }
+    s->mt64.upload(&t, 1);
+    if (s->precision == IBM3D_PREC_FP64) return;
+    s->mgv32.alloc(6 * ng);
+    MomTable<float> f{};
+    for (int c = 0; c < 3; c++) {
+        f.S[c] = s->sys[c].S32;
+        f.b[c] = f.brw[c] = c == 0 ? s->ref_rhs32.p : s->mlane[c - 1].d32[0].p;
+        f.x[c] = c == 0 ? s->ref_e32.p : s->mlane[c - 1].d32[1].p;
+        for (int k = 0; k < 2; k++) f.gv[c][k] = s->mgv32.p + (2 * c + k) * ng;
+    }
+    s->mt32.upload(&f, 1);
+}
+
+// n sweeps of the components in mask (zero: from a zero start, whose first
+// colour is already written when first_done); `prev`: where the ghost values
+// are, in and out.
+template <typename T>
+static void momentum_smooth(IBMSolver *s, const MomTable<T> *M, unsigned mask, int n, bool zero, bool first_done,
+                            int &prev) {
+    const Dims &d = s->d;
+    const GhostRows<T> &G = grows<T>(s->gmom);
+    const double cb = ncells(s) * __builtin_popcount(mask);
+    for (int sw = 0; sw < n; sw++)
+        for (int c = 0; c < 2; c++) {
+            const bool z = zero && sw == 0 && c == 0;
+            if (!(z && first_done))
+                TIMED("mom_rbgs", cb * ((z ? 1.5 : 2) * sizeof(T) + 1),
+                      prev = launch_mom_colour<T>(s->stream, d, M, mask, s->flag.p, c, z ? 1 : 0, G, prev));
+            if (z && G.ng) {
+                TIMED("mom_ghost", 0, launch_mom_ghost<T>(s->stream, d, M, mask, G, c));
+                prev = 0;
+            }
+        }
+}
+
+// The three momentum solves by sweeps; components that do not converge this
+// way are solved by solve_system. bn: the stopping norms.
+static void momentum_sweep_solve(IBMSolver *s, const double bn[3]) {
     const Dims &d = s->d;
     const int m = momentum_sweeps(s);
     const double cb = ncells(s);
     const long na = apply_partials(d, s->gmom.G64.ng);
-    const NormSpec off{0, nullptr, nullptr, nullptr, nullptr, -1};
-    double *r64[3] = {s->ref_r64.p, s->mlane[0].v[0].p, s->mlane[1].v[0].p};
-    float *rhs32[3] = {s->ref_rhs32.p, s->mlane[0].d32[0].p, s->mlane[1].d32[0].p};
-    float *e32[3] = {s->ref_e32.p, s->mlane[0].d32[1].p, s->mlane[1].d32[1].p};
-    double rn[3] = {0, 0, 0};
-    int sweeps[3] = {0, 0, 0};
-    bool active[3], fallback[3] = {false, false, false};
+    const bool f64 = s->precision == IBM3D_PREC_FP64;
+    double rn[3] = {0, 0, 0}, rate[3] = {s->mom_rate, s->mom_rate, s->mom_rate};
+    int sweeps[3] = {0, 0, 0}, prev = -1;
+    bool fallback[3] = {false, false, false};
+    unsigned mask = 0;
     for (int l = 0; l < 3; l++) {
         // a zero right-hand side has the zero solution; a non-finite one
         // stays active, so its residual reports the error
-        active[l] = bn[l] != 0;
-        if (!active[l]) {
-            launch_zero<double>(s->stream, d, s->us[l].p);
-            report_solve(s, l, 0.0, 0);
+        if (bn[l] != 0) {
+            mask |= 1u << l;
+            rn[l] = bn[l];
+            continue;
         }
+        launch_zero<double>(s->stream, d, s->us[l].p);
+        report_solve(s, l, 0.0, 0);
     }
-    for (int round = 0; round < kMomMaxRounds; round++) {
-        bool any = false;
-        for (int l = 0; l < 3; l++) {
-            if (!active[l]) continue;
-            any = true;
-            const SysCoef<double> &S64 = s->sys[l].S64;
-            const SysCoef<float> &S32 = s->sys[l].S32;
-            // right-hand side of the correction (b itself from x = 0) in FP32,
-            // with the first smoother colour from a zero start
-            // the first round aims at the FP32 limit, later ones at what is left
-            const int mr = round ? momentum_round_sweeps(s, s->tol * bn[l] / rn[l]) : m;
-            TIMED("mom_d2f", cb * 17, launch_d2f_first(s->stream, d, S32, s->flag.p, round ? r64[l] : s->b[l].p,
-                                                       rhs32[l], e32[l]));
-            smooth<float>(s, d, S32, s->gmom.G32, s->flag.p, rhs32[l], e32[l], s->ref_e32b.p, mr, true, -1, true);
-            sweeps[l] += mr;
-            if (round) TIMED("mom_add_f2d", cb * 20, launch_add_f2d(s->stream, d, e32[l], s->us[l].p));
-            else TIMED("mom_f2d", cb * 12, launch_f2d(s->stream, d, e32[l], s->us[l].p));
-            TIMED("mom_residual64", 3 * cb * 8,
-                  launch_residual<double>(s->stream, d, S64, s->gmom.G64, s->flag.p, s->b[l].p, s->us[l].p, r64[l],
-                                          off, s->partial.p));
-            launch_sum_partials(s->stream, s->partial.p, na, 2, s->sums.p + 3 + 2 * l, 0);
+    for (int round = 0; mask && round < kMomMaxRounds; round++) {
+        const double act = __builtin_popcount(mask);
+        // the first round aims at the tolerance (FP64) or the FP32 limit,
+        // later ones at what the worst component still lacks
+        int mr = m;
+        if (round) {
+            mr = 1;
+            for (int l = 0; l < 3; l++)
+                if (mask >> l & 1) {
+                    double need = s->tol * bn[l] / rn[l];
+                    if (!f64) need = std::max(need, kMomRoundTarget);
+                    mr = std::max(mr, momentum_round_sweeps(need, rate[l], m));
+                }
         }
-        if (!any) break;
-        read_sums(s, 9);
+        if (f64) {
+            momentum_smooth<double>(s, s->mt64.p, mask, mr, round == 0, false, prev);
+        } else {
+            TIMED("mom_d2f", act * cb * 17, launch_mom_d2f_first(s->stream, d, s->mt64.p, s->mt32.p, mask, s->flag.p,
+                                                                 round == 0));
+            momentum_smooth<float>(s, s->mt32.p, mask, mr, true, true, prev);
+            TIMED("mom_add", act * cb * (round ? 20 : 12),
+                  launch_mom_add(s->stream, d, s->mt64.p, s->mt32.p, mask, round > 0));
+        }
+        TIMED("mom_residual64", act * cb * (f64 ? 2 : 3) * 8,
+              launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p, !f64, s->partial.p));
+        sum_read(s, na, 3);
         for (int l = 0; l < 3; l++) {
-            if (!active[l]) continue;
-            const double r = std::sqrt(s->sums_h[3 + 2 * l]);
+            if (!(mask >> l & 1)) continue;
+            sweeps[l] += mr;
+            const double r = std::sqrt(s->sums_h[l]);
             const bool stalled = round > 0 && !(r <= 0.1 * rn[l]);
+            // rate shown by this round's sweeps (FP64: from ||b||), kept below 1
+            if (f64) rate[l] = std::min(0.5, std::max(1e-6, std::pow(r / rn[l], 1.0 / mr)));
             rn[l] = r;
             if (!std::isfinite(r) || r <= s->tol * bn[l]) {
-                active[l] = false;
+                mask &= ~(1u << l);
                 report_solve(s, l, r / bn[l], sweeps[l]);
             } else if (stalled) {
-                active[l] = false;
+                mask &= ~(1u << l);
                 fallback[l] = true;
             }
         }
     }
     for (int l = 0; l < 3; l++)
-        if (active[l] || fallback[l]) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
+        if ((mask >> l & 1) || fallback[l]) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1600,10 +1665,10 @@ static void do_step(IBMSolver *s) {
     // momentum Helmholtz solves: the three at once on their lanes, or one
     // after the other (mixed defect-correction mode, and under the per-kernel
     // timers, whose events are recorded on the solver's stream)
-    if (s->precision == IBM3D_PREC_MIXED_KRYLOV && s->mom_solver == 0 && momentum_sweeps(s) > 0) {
+    if (s->precision != IBM3D_PREC_MIXED && s->mom_solver == 0 && momentum_sweeps(s) > 0) {
         double bn[3];
         mom_norms(bn);
-        momentum_refine(s, bn);
+        momentum_sweep_solve(s, bn);
     } else if (s->mom_lanes && s->timing == 0 && s->precision != IBM3D_PREC_MIXED) {
         momentum_concurrent(s, mom_norms);
     } else {

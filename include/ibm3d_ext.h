@@ -84,13 +84,14 @@ void IBMSolver_set_mg_relaxation(IBMSolver *, double omega);
    No counterpart in the reference. */
 int IBMSolver_get_pressure_mg_bits(IBMSolver *);
 
-/* Momentum Helmholtz solver of the IBM3D_PREC_MIXED_KRYLOV mode. 0
-   (default): FP32 red-black Gauss-Seidel sweeps inside FP64 iterative
-   refinement where the operator is diagonally dominant enough for a few
-   sweeps per round (max over cells of sum K / (1 + sum K) squared <= 0.03),
-   BiCGSTAB elsewhere and for any component whose residual stops falling;
-   1: always BiCGSTAB (FP64, Jacobi preconditioner, FP32 stored directions).
-   Both stop on the reference's test ||b - A x|| <= tol ||b|| in FP64. */
+/* Momentum Helmholtz solver of the IBM3D_PREC_FP64 and _MIXED_KRYLOV modes.
+   0 (default): red-black Gauss-Seidel sweeps, in FP64 on the system itself or
+   (mixed) in FP32 inside FP64 iterative refinement, where the operator is
+   diagonally dominant enough (max over cells of sum K / (1 + sum K) squared
+   <= 0.5), BiCGSTAB elsewhere and for any component whose residual stops
+   falling; 1: always BiCGSTAB (FP64, Jacobi preconditioner; mixed: FP32 stored
+   directions). All stop on the reference's test ||b - A x|| <= tol ||b|| in
+   FP64; IBMSolver_get_last_iters counts sweeps or iterations. */
 void IBMSolver_set_momentum_solver(IBMSolver *, int mode);
 
 /* Copies a field to host memory in the reference layout (see above). Solid

@@ -50,3 +50,40 @@ def test_fields_cross_the_host_boundary_unchanged(new_gpu, I, cases, shape):
         inner = list(sl)
         inner[ax] = slice(None)
         np.testing.assert_allclose(f[tuple(inner)], 0.5 * (u[tuple(lo)] + u[tuple(hi)]), rtol=1e-13, atol=1e-13)
+
+
+MOMENTUM_CASES = [
+    # (set-up, grid, further arguments): remainders of the launch shapes, with
+    # and without a body, sweep rates from 0.002 to just below the largest one
+    ("cavity", (17, 13, 11), dict(Re=100.0)),
+    ("cavity", (130, 9, 10), dict(Re=100.0, dt=0.001)),
+    ("cavity", (40, 40, 40), dict(Re=20.0, dt=0.008)),
+    ("sphere", (66, 33, 35), dict()),
+    ("sphere", (131, 24, 25), dict()),
+]
+
+
+@pytest.mark.parametrize("precision", [0, 2], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("kind,grid,kw", MOMENTUM_CASES)
+def test_batched_momentum_sweeps_match_bicgstab(new_gpu, cases, kind, grid, kw, precision):
+    """Two steps with the momentum sweeps of the three components in one
+    launch against BiCGSTAB at tol 1e-12: both solve the same systems, so the
+    fields agree to the tolerance times the conditioning of a strongly
+    diagonally dominant system (a few), 1e-10 with room for the projection."""
+    out = []
+    for mode in (0, 1):
+        s = new_gpu()
+        s.set_momentum_solver(mode)
+        if kind == "cavity":
+            cases.setup_cavity(s, shape=grid, tol=1e-12, precision=precision, **kw)
+        else:
+            cases.setup_sphere(s, *grid, tol=1e-12, precision=precision, **kw)
+        s.iterate(2)
+        assert (s.last_norms()[:3] <= 1e-12).all()
+        out.append([s.get(n) for n in ("U1_STAR", "U2_STAR", "U3_STAR", "U1", "U2", "U3")])
+    scale = max(np.nanmax(np.abs(a[2:-2, 2:-2, 2:-2])) for a in out[1])
+    for a, b in zip(*out):
+        a, b = a[2:-2, 2:-2, 2:-2], b[2:-2, 2:-2, 2:-2]
+        m = np.isfinite(b)
+        assert np.array_equal(np.isfinite(a), m)
+        assert np.abs(a[m] - b[m]).max() <= 1e-10 * scale
