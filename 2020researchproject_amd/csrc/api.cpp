@@ -233,6 +233,7 @@ void IBMSolver_set_mg_params(IBMSolver *s, double gamma, int pre, int post, int 
     if (pre < 0 || post < 0 || pre + post == 0 || pre > 16 || post > 16) fatal("invalid multigrid sweep counts");
     if (smoother != 0 && smoother != 1) fatal("multigrid smoother must be 0 or 1");
     if (!std::isfinite(gamma)) fatal("multigrid coarsening threshold gamma must be finite");
+    s->mg_custom = true;
     s->mg_gamma = gamma;
     s->mg_pre = pre;
     s->mg_post = post;
@@ -242,6 +243,7 @@ void IBMSolver_set_mg_params(IBMSolver *s, double gamma, int pre, int post, int 
 void IBMSolver_set_mg_relaxation(IBMSolver *s, double omega) {
     if (s->assembled) fatal("IBMSolver_set_mg_relaxation must precede IBMSolver_assemble");
     if (!(omega > 0 && omega < 2)) fatal("multigrid over-relaxation factor must lie in (0, 2)");
+    s->mg_custom = true;
     s->mg_omega = omega;
 }
 
@@ -253,6 +255,7 @@ int IBMSolver_get_pressure_mg_bits(IBMSolver *s) {
 void IBMSolver_set_mg_light_levels(IBMSolver *s, int from_level) {
     if (s->assembled) fatal("IBMSolver_set_mg_light_levels must precede IBMSolver_assemble");
     if (from_level < 0) fatal("multigrid light levels: from_level must be 0 or positive");
+    s->mg_custom = true;
     s->mg_light_from = from_level;
 }
 
@@ -650,6 +653,7 @@ static void alloc_fields(IBMSolver *s) {
     long nb = conv_rhs_blocks(s->d) + 64;
     nb = std::max(nb, apply_partials(s->d, s->ng) + 64);
     nb = std::max(nb, vec_partials(s->d) + 64);
+    nb = std::max(nb, separable_partials(s->d));
     s->partial.alloc((size_t)nb * 4);
 }
 
@@ -785,7 +789,9 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
         s->conv_ready = false;
     }
     if (s->precision != IBM3D_PREC_MIXED) build_momentum_tables(s);
-    build_mg(s);
+    build_separable(s);
+    s->mg.clear();
+    if (!s->sep_on) ensure_mg(s);
     s->assembled = true;
     HIP_CHECK(hipStreamSynchronize(s->stream));
 }
@@ -924,6 +930,7 @@ extern "C" int IBMSolver_get_ghost_cells(IBMSolver *s, int *out) {
 }
 
 extern "C" int IBMSolver_get_mg_levels(IBMSolver *s, int *out, int max) {
+    if (s->assembled) ensure_mg(s);
     const int n = (int)s->mg.size();
     for (int l = 0; l < n && l < max && out; l++) {
         out[3 * l] = s->mg[l].d.nx;

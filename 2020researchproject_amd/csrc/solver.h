@@ -8,6 +8,7 @@
 
 #include "../../include/ibm3d.h"
 #include "common.h"
+#include "separable.h"
 #include "solver_kernels.h"
 #include "step_kernels.h"
 
@@ -225,6 +226,7 @@ struct _ibm_solver {
     int mg_pre = 2, mg_post = 2; // smoothing sweeps per level
     int mg_smoother = 1;         // 0 fused red-black sweeps, 1 one launch per colour
     int mg_light_from = 1;       // levels >= this (if > 0) smooth with one sweep before and after
+    bool mg_custom = false;      // a multigrid setter was called: the pressure solve is the multigrid one
     double mg_omega = 1.3;       // over-relaxation factor of the pressure multigrid smoother
     int mom_solver = 0;          // IBMSolver_set_momentum_solver: 0 automatic, 1 BiCGSTAB
     int mom_sweeps = -1;         // FP32 sweeps per refinement round of the momentum solves (0: not used; -1: unset)
@@ -289,7 +291,11 @@ struct _ibm_solver {
 
     ibm::SysData sys[4];                  // u1, u2, u3, p
     long pin = -1;
-    std::vector<ibm::MGLevel> mg;         // mg[0] = fine pressure level
+    std::vector<ibm::MGLevel> mg;         // mg[0] = fine pressure level; empty until ensure_mg
+    // direct pressure solve of a box without a body (build_separable)
+    bool sep_on = false;
+    ibm::SeparableSys sep{};
+    ibm::DBuf<double> sep_mat[3][3];      // V, Vi, lam per axis
     std::vector<ibm::VGraph> vgraphs;     // captured V-cycles per (input, output)
     ibm::Krylov kry;
     ibm::GmresData gm;                    // SOLVER_GMRES / SOLVER_PCG / SOLVER_AMG scratch (pressure)
@@ -347,6 +353,8 @@ void build_system(const IBMSolver *s, const std::vector<double> *D[3], const std
 // step.cpp
 void iterate_impl(IBMSolver *s, int steps, bool verbose);
 void build_mg(IBMSolver *s);
+void ensure_mg(IBMSolver *s);
+void build_separable(IBMSolver *s);
 void build_momentum_tables(IBMSolver *s);
 double max_div_impl(IBMSolver *s);
 void body_force_impl(IBMSolver *s, double *dst);

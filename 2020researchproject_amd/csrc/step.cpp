@@ -222,11 +222,13 @@ static void wait_published(hipStream_t st, KPub *pub_h, unsigned e) { wait_epoch
 
 // The first nv sums, copied by a small kernel into device-mapped host memory
 // (sums_h) and awaited there
-static void read_sums(IBMSolver *s, int nv) {
+static unsigned publish_sums(IBMSolver *s, int nv) {
     const unsigned e = ++s->sums_epoch;
     launch_publish(s->stream, s->sums.p, nv, s->sums_d, s->sums_d_epoch, e);
-    wait_epoch(s->stream, s->sums_h_epoch, e);
+    return e;
 }
+
+static void read_sums(IBMSolver *s, int nv) { wait_epoch(s->stream, s->sums_h_epoch, publish_sums(s, nv)); }
 
 // The sums (maxima) of nv columns of block partials, formed straight into
 // sums_h and awaited there
@@ -240,12 +242,18 @@ static void sum_read(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
 // published into host memory, then a wait for them there: no copy and no
 // stream synchronisation on the Krylov loop's path (each end of iteration
 // otherwise costs a copy and a wake-up of the host thread).
-static void finalize_read(IBMSolver *s, int op, long nblk, int nv) {
+static unsigned finalize_publish(IBMSolver *s, int op, long nblk, int nv) {
     const unsigned e = ++s->pub_epoch;
     launch_finalize(s->stream, op, s->partial.p, nblk, nv, s->ks.p, &s->pub_d->ks, &s->pub_d->epoch, e);
+    return e;
+}
+
+static void finalize_wait(IBMSolver *s, unsigned e) {
     wait_published(s->stream, s->pub_h, e);
     memcpy((void *)s->ks_h, (const void *)&s->pub_h->ks, sizeof(KScal));
 }
+
+static void finalize_read(IBMSolver *s, int op, long nblk, int nv) { finalize_wait(s, finalize_publish(s, op, nblk, nv)); }
 
 // ---------------------------------------------------------------------------
 // multigrid hierarchy of the pressure system
@@ -256,6 +264,10 @@ static const long kDenseCells = 3000;
 // levels with at least this many cells restrict their residual with two
 // launches (residual, then restriction), smaller ones with one
 static const long kSplitRestrictCells = 1L << 20;
+
+// ratio of the largest to the smallest nonzero eigenvalue above which FP32
+// cycles are not tried
+static const double kFp32CycleSpan = 1e5;
 
 static void level_geometry(IBMSolver *s, MGLevel &L, const std::vector<double> &xf, const std::vector<double> &yf,
                            const std::vector<double> &zf) {
@@ -548,6 +560,73 @@ void build_mg(IBMSolver *s) {
     if (s->precision != IBM3D_PREC_FP64) {
         s->mg[0].r32.alloc(s->d.ncell);
         s->mg[0].xa32.alloc(s->d.ncell);
+    }
+}
+
+// The hierarchy, where it is not there yet: a solver whose pressure system is
+// solved directly builds it only if a solve falls back.
+void ensure_mg(IBMSolver *s) {
+    if (!s->mg.empty()) return;
+    DevBytesScope account(&s->dev_bytes);
+    build_mg(s);
+    HIP_CHECK(hipStreamSynchronize(s->stream));
+}
+
+// Direct pressure solve (separable.hip) where the system allows it: no solid
+// or ghost cell, every axis symmetric in its cell widths (all but a periodic
+// axis that is not uniform), and the solver asked for is the default one
+// (BiCGSTAB with the multigrid preconditioner, no multigrid setting changed).
+// Time per step at tol 1e-12, multigrid / direct: cavity 32^3 1.43 / 0.31 ms,
+// 64^3 (FP64) 2.34 / 0.40, 128^3 5.62 / 1.13, channel 64 x 48 x 32 4.85 / 0.29.
+// The transforms grow as the axis length per cell: at 128^3 they are 163 us
+// of the step. Axes beyond the LDS tiles (400 cells) take the multigrid path.
+void build_separable(IBMSolver *s) {
+    s->sep_on = false;
+    if (s->solver_type != SOLVER_BiCGSTAB || s->precond_type != PRECOND_AMG || s->precision == IBM3D_PREC_MIXED
+        || s->mg_custom)
+        return;
+    const Dims &d = s->d;
+    for (int k = 0; k < d.nz; k++)
+        for (int j = 0; j < d.ny; j++)
+            for (int i = 0; i < d.nx; i++)
+                if (s->flag_dev_h[cidx(d, i, j, k)] != F_FLUID) return;
+    const int n[3] = {d.nx, d.ny, d.nz};
+    if (!separable_fits(n)) return;
+    const std::vector<double> *w[3] = {&s->dx, &s->dy, &s->dz};
+    std::vector<double> m[3][3];
+    double lo = 0, hi = 0, low[3];
+    for (int a = 0; a < 3; a++) {
+        const auto &h = s->sys[3].h[a];
+        int same = a;  // an earlier axis with the same operator
+        for (int o = a - 1; o >= 0; o--)
+            if (n[o] == n[a] && *w[o] == *w[a] && s->sys[3].S64.ax[o].periodic == s->sys[3].S64.ax[a].periodic
+                && std::equal(h, h + 4, s->sys[3].h[o]))
+                same = o;
+        if (same < a) for (int c = 0; c < 3; c++) m[a][c] = m[same][c];
+        else if (!separable_axis(n[a], s->sys[3].S64.ax[a].periodic, h, w[a]->data() + 2, m[a][0], m[a][1], m[a][2]))
+            return;
+        const std::vector<double> &lam = m[a][2];
+        if (s->p_singular != (lam[0] == 0) && s->p_singular) return;
+        low[a] = n[a] > 1 ? lam[1] : 0;
+        lo += lam[0];
+        hi += lam[n[a] - 1];
+    }
+    if (!s->p_singular && !(lo > 0)) return;
+    for (int a = 0; a < 3; a++) {
+        for (int c = 0; c < 3; c++) s->sep_mat[a][c].upload(m[a][c]);
+        s->sep.ax[a] = {s->sep_mat[a][0].p, s->sep_mat[a][1].p, s->sep_mat[a][2].p, n[a], (n[a] + 15) / 16 * 16};
+    }
+    s->sep.pinned = s->p_singular;
+    s->sep_on = true;
+    // Mixed-Krylov mode: where a solve of a pinned system falls back, its FP32
+    // cycles stall if the eigenvalues span more than FP32 resolves. They
+    // stalled in the first step of the channel 192 x 96 x 128 (span 5e7) and
+    // took 14 to 39 iterations against 10 of the FP64 cycle; on the cavity
+    // 128^3 (2e4) they needed as many as the FP64 cycle.
+    if (s->p_singular) {
+        for (int a = 0; a < 3; a++)
+            if (low[a] > 0 && (lo == 0 || low[a] < lo)) lo = low[a];
+        if (lo > 0 && hi > kFp32CycleSpan * lo) s->p_mg64 = true;
     }
 }
 
@@ -1374,6 +1453,42 @@ static void momentum_concurrent(IBMSolver *s, F &&norms) {
     for (int c = 0; c < 3; c++) report_solve(s, c, rel[c], it[c]);
 }
 
+// Direct pressure solve and refinement: x = A^-1 b, then x += A^-1 (b - A x)
+// until the FP64 residual meets the tolerance. One round reaches the rounding
+// level of the transforms (1e-12 .. 1e-10 of ||b||), a second one that of the
+// residual. norm() gives the stopping norm (a host read), called once the
+// first round is enqueued. A solve whose residual no longer halves is left to
+// the iterative path (false); its reason is the tolerance, not the method.
+template <typename F>
+static bool separable_solve(IBMSolver *s, const double *b, double *x, F &&norm, double *bnorm) {
+    const Dims &d = s->d;
+    const NormSpec ns{1, s->ks1d[0].p, s->ks1d[1].p, s->ks1d[2].p, s->flag.p, s->pin};
+    double *r = s->kry.v64[0].p, *s1 = s->kry.v64[1].p, *s2 = s->kry.v64[2].p;
+    const double cb = ncells(s) * 8;
+    double last = 0;
+    for (int round = 1;; round++) {
+        TIMED("separable", (round > 1 ? 7 : 6) * cb,
+              launch_separable(s->stream, d, s->sep, round > 1 ? r : b, s1, s2, x, round > 1, s->partial.p));
+        TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r,
+                                                          ns, s->partial.p));
+        const unsigned e = finalize_publish(s, 4, apply_partials(d, 0), 2);
+        if (round == 1) *bnorm = norm();
+        finalize_wait(s, e);
+        if (*bnorm == 0) {
+            launch_zero<double>(s->stream, d, x);
+            report_solve(s, 3, 0, 0);
+            return true;
+        }
+        const double rn = std::sqrt(s->ks_h->rrn);
+        if (rn <= s->tol * *bnorm || !std::isfinite(rn)) {
+            report_solve(s, 3, rn / *bnorm, round);
+            return true;
+        }
+        if (round > 1 && rn > 0.5 * last) return false;
+        last = rn;
+    }
+}
+
 static void solve_system(IBMSolver *s, int sk, const double *b, double *x, double bnorm) {
     const int prec = sk == 3 ? (s->precond_type == PRECOND_AMG ? 2 : 1) : 1;
     NormSpec ns{0, nullptr, nullptr, nullptr, nullptr, -1};
@@ -1381,6 +1496,7 @@ static void solve_system(IBMSolver *s, int sk, const double *b, double *x, doubl
     const int maxit = sk == 3 ? 1000 : 200;  // src/ibm3d_setup.c:1413, 1467
     double rel = 0;
     int it;
+    if (sk == 3) ensure_mg(s);
     if (sk == 3 && s->solver_type != SOLVER_BiCGSTAB && s->precision != IBM3D_PREC_MIXED) {
         // multigrid cycles in FP32 in the mixed-Krylov mode; SOLVER_AMG is the
         // cycle itself, with no separate preconditioner
@@ -1699,9 +1815,16 @@ static void do_step(IBMSolver *s) {
                              : ax == 1 ? (hi ? s->g1d[9].p : s->g1d[8].p) : (hi ? s->g1d[11].p : s->g1d[10].p);
             launch_bc_rhs(s->stream, s->geo, opp, ax, hi, 3, Kf, s->sys[3].gamma[ax][hi], s->bp.p);
         }
-    read_sums(s, 1);
-    const double bnp = std::sqrt(s->sums_h[0] + s->sys[3].bc_norm2 + pnorm[3]);
-    solve_system(s, 3, s->bp.p, s->pp.p, bnp);
+    const unsigned pe = publish_sums(s, 1);
+    auto poisson_norm = [&] {
+        wait_epoch(s->stream, s->sums_h_epoch, pe);
+        return std::sqrt(s->sums_h[0] + s->sys[3].bc_norm2 + pnorm[3]);
+    };
+    double bnp = 0;
+    if (!s->sep_on || !separable_solve(s, s->bp.p, s->pp.p, poisson_norm, &bnp)) {
+        if (!s->sep_on) bnp = poisson_norm();
+        solve_system(s, 3, s->bp.p, s->pp.p, bnp);
+    }
     TIMED("outer_sol", 0, launch_outer(s->stream, s->geo, opp, s->pp.p, nullptr, nullptr, 3, 0));
     // K3: projection
     {

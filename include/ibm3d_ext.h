@@ -57,7 +57,11 @@ void IBMSolver_set_precision(IBMSolver *, int mode);
    smoother 0: each sweep is one fused launch (both colours), ghost rows
    relaxed after each sweep; 1: one launch per colour, ghost rows relaxed
    after each colour. Defaults 3.5, 2, 2, 1. gamma must be finite; pre and
-   post 0..16, not both 0. Must be called before IBMSolver_assemble. */
+   post 0..16, not both 0. Must be called before IBMSolver_assemble.
+   A box without a body under SOLVER_BiCGSTAB with PRECOND_AMG solves its
+   pressure directly (eigenvectors of the three axes, refined until the
+   stopping test holds) in the modes FP64 and MIXED_KRYLOV; calling this or
+   one of the next two functions selects BiCGSTAB with these cycles there. */
 void IBMSolver_set_mg_params(IBMSolver *, double gamma, int pre, int post, int smoother);
 /* Levels from `from_level` down (when from_level > 0) smooth with one sweep
    before and one after the coarse correction instead of pre/post; 0 smooths
@@ -76,11 +80,14 @@ void IBMSolver_set_mg_light_levels(IBMSolver *, int from_level);
    preconditioner changes: the stopping test is the same. Before
    IBMSolver_assemble. No counterpart in the reference. */
 void IBMSolver_set_mg_relaxation(IBMSolver *, double omega);
-/* Precision of the pressure multigrid cycle the solver uses now: 32 or 64
-   (0 before IBMSolver_assemble). In IBM3D_PREC_MIXED_KRYLOV it is 32 until a
+/* Precision of the pressure multigrid cycle the solver uses now, or would use
+   where it solves the pressure directly: 32 or 64 (0 before
+   IBMSolver_assemble). In IBM3D_PREC_MIXED_KRYLOV it is 32 until a
    pressure solve stalls twice (a residual falling less than tenfold over
    three BiCGSTAB iterations, each time followed by a restart from the true
    residual); the solver then keeps the FP64 cycle for its remaining steps.
+   A directly solved, pinned system whose eigenvalues span more than 1e5
+   starts at 64.
    No counterpart in the reference. */
 int IBMSolver_get_pressure_mg_bits(IBMSolver *);
 
@@ -114,8 +121,8 @@ void IBMSolver_get_last_iters(IBMSolver *, int out[4]);
    fastest): writes 3*count ints when out != NULL, returns count. */
 int IBMSolver_get_ghost_cells(IBMSolver *, int *out);
 
-/* Shapes of the pressure multigrid levels built by IBMSolver_assemble
-   (level 0 = the fine grid): writes nx, ny, nz of up to max levels into out
+/* Shapes of the pressure multigrid levels built by IBMSolver_assemble, or by
+   this call where the pressure is solved directly (level 0 = the fine grid): writes nx, ny, nz of up to max levels into out
    when out != NULL, returns the number of levels. */
 int IBMSolver_get_mg_levels(IBMSolver *, int *out, int max);
 
