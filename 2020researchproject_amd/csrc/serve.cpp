@@ -297,8 +297,8 @@ double IBMSolver_estimate_device_bytes(int Nx, int Ny, int Nz, int precision, in
     const double coarse = 1.5 * cells;
     const double mg = cells * (8.0 * 2 + (mixed ? 4.0 * 2 : 0))
         + coarse * (8.0 * 4 + 2 + (mixed ? 4.0 * 4 : 0)) + (cells + coarse) * 1;
-    // dense inverse of the coarsest level (at most 3000 rows; FP64, + FP32)
-    // and the pivot scratch of its inversion
+    // dense inverse of the coarsest level (at most 3000 rows; FP64, + FP32);
+    // the pivot scratch of its inversion (0.8 MB) is part of the last term
     const double n = std::min(3000.0, (double)Nx * Ny * Nz);
     const double dense = n * n * (8 + (mixed ? 4 : 0)) + 2 * 8.0 * n;
     // reduction partials, ghost lists, 1-D metrics and folded coefficients

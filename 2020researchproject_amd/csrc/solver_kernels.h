@@ -264,10 +264,11 @@ template <typename T>
 void launch_coarse_solve(hipStream_t st, const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const T *b, T *x,
                          int sweeps, int singular, const double *dxyz);
 
-// In-place Gauss-Jordan inversion without pivoting of the n x n row-major
-// matrix A (diagonally dominant M-matrix rows); rowp, colp: n doubles of
-// scratch.
-void gauss_jordan_invert(hipStream_t st, double *A, int n, double *rowp, double *colp);
+// In-place Gauss-Jordan inversion without pivoting (beyond blocks of 16) of
+// the n x n row-major matrix A of row pitch ld (diagonally dominant M-matrix
+// rows); scratch: gauss_jordan_scratch(n) doubles.
+size_t gauss_jordan_scratch(int n);
+void gauss_jordan_invert(hipStream_t st, double *A, int n, long ld, double *scratch);
 void launch_d2f_flat(hipStream_t st, const double *a, float *b, long n);
 // x[rows[r]] = sum_c Ainv[r][c] rhs[c], rhs[c] = b[rows[c]]; singular: the
 // volume-weighted mean of b over fluid rows is removed first and the pinned

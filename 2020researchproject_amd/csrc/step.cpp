@@ -348,10 +348,9 @@ static void build_dense(IBMSolver *s, MGLevel &L) {
     L.dinv64.upload(A);
     L.drow.upload(rows);
     L.dvol.upload(vol);
-    DBuf<double> rowp, colp;
-    rowp.alloc(n);
-    colp.alloc(n);
-    gauss_jordan_invert(s->stream, L.dinv64.p, n, rowp.p, colp.p);
+    DBuf<double> scratch;
+    scratch.alloc(gauss_jordan_scratch(n));
+    gauss_jordan_invert(s->stream, L.dinv64.p, n, n, scratch.p);
     if (s->precision != IBM3D_PREC_FP64) {
         L.dinv32.alloc((size_t)n * n);
         launch_d2f_flat(s->stream, L.dinv64.p, L.dinv32.p, (long)n * n);
