@@ -610,7 +610,6 @@ static void alloc_fields(IBMSolver *s) {
     s->p.alloc(n); s->pn.alloc(n); s->pp.alloc(n); s->bp.alloc(n);
     if (s->turb_type != TURBMODEL_NONE)
         for (int a = 0; a < 6; a++) s->tau[a].alloc(n);
-    for (int v = 0; v < 8; v++) s->kry.v64[v].alloc(n);
     if (s->precision != IBM3D_PREC_MIXED) {
         // lanes of the concurrent momentum solves (components 1 and 2)
         HipGlobalLock lk(hip_global_mutex());
@@ -780,6 +779,10 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
     s->sys[3].S64.pin = s->sys[3].S32.pin = s->pin;
     bc_rows_norm(s);
 
+    // the Krylov vectors, then the direct pressure solve, whose set-up takes
+    // them (and memory that the other fields will use) as scratch
+    for (auto &v : s->kry.v64) v.alloc(d.ncell);
+    build_separable(s);
     alloc_fields(s);
     {
         const long ext[3] = {(long)s->Ny * s->Nz, (long)(s->Nx + 4) * s->Nz, (long)(s->Nx + 4) * (s->Ny + 4)};
@@ -789,7 +792,6 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
         s->conv_ready = false;
     }
     if (s->precision != IBM3D_PREC_MIXED) build_momentum_tables(s);
-    build_separable(s);
     s->mg.clear();
     if (!s->sep_on) ensure_mg(s);
     s->assembled = true;

@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "common.h"
+#include "solver_kernels.h"
 
 namespace ibm {
 
@@ -20,6 +21,22 @@ struct SeparableSys {
     int pinned;  // the row of cell (0, 0, 0) is x = b; the problem is otherwise singular
 };
 
+// Ghost rows of an immersed body (capacitance matrix method). The box's
+// operator A holds in every fluid row; a right-hand side mu at the ghost cells
+// makes its solution also meet the ghost rows R x = b_g:
+//   (R A^-1 E) mu = b_g - R A^-1 b_fluid,  x = A^-1 (b_fluid + E mu).
+// y0..z1: rows and planes that hold ghost cells or their stencil points (end
+// exclusive), g0..g1: planes with ghost cells.
+struct SeparableBody {
+    const uint8_t *flag;
+    GhostRows<double> G;
+    const double *inv64;  // inverse of R A^-1 E, row pitch ld; one of the two
+    const float *inv32;
+    int ld;
+    double *t;            // ng: right-hand side of the ghost rows
+    int y0, y1, z0, z1, g0, g1;
+};
+
 // Host: eigenvalues (ascending) and matrices of one axis from its folded
 // coefficients cm, cp, dm, dp (n each) and cell widths; false when the axis
 // has no such form (a periodic axis that is not uniform).
@@ -32,5 +49,20 @@ bool separable_fits(const int n[3]);  // the axes fit the kernels' LDS tiles
 long separable_partials(const Dims &d);
 void launch_separable(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, double *s1, double *s2,
                       double *x, bool add, double *partial);
+// the same with a body (not pinned); s3: a third scratch vector. Solid cells
+// get x = b (+= b).
+void launch_separable_body(hipStream_t st, const Dims &d, const SeparableSys &S, const SeparableBody &B,
+                           const double *b, double *s1, double *s2, double *s3, double *x, bool add);
+
+// Columns of R A^-1 E for the nsrc ghost cells src[c] = {i, j, slot} of plane
+// k: out[slot(g) * ld + slot(c)]. loc: 9 per ghost row, the places of its
+// stencil points (8, -1: none) and of its cell in the box [lo, hi); h: a
+// scratch vector; green: kGreenVecs scratch vectors, each for `per` sources
+constexpr int kGreenVecs = 6;
+struct GreenScratch { double *v[kGreenVecs]; int per; };
+struct GreenBox { int lo[3], hi[3]; };
+void launch_green_plane(hipStream_t st, const Dims &d, const SeparableSys &S, int k, const int3 *src, int nsrc,
+                        const GreenBox &box, const GhostRows<double> &G, const int *loc, double *h,
+                        const GreenScratch &green, double *out, long ld);
 
 }  // namespace ibm

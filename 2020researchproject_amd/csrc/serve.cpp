@@ -289,6 +289,19 @@ double IBMSolver_estimate_device_bytes(int Nx, int Ny, int Nz, int precision, in
     // (+ a second FP32 correction in mode 2); mode 1: 8 FP32 Krylov vectors
     if (mixed) per += 8 + 4 + 4 + (precision == IBM3D_PREC_MIXED_KRYLOV ? 4 : 0);
     if (precision == IBM3D_PREC_MIXED) per += 4 * 8;
+    // the multigrid hierarchy, or the ghost rows' capacitance matrix of a
+    // direct pressure solve, which is limited to its size
+    // reduction partials, ghost lists, 1-D metrics and folded coefficients
+    return cells * per + ibm::multigrid_bytes(d, precision) + 16.0 * (1 << 20);
+}
+
+double IBMSolver_get_device_bytes(IBMSolver *s) { return (double)s->dev_bytes; }
+
+}  // extern "C"
+
+double ibm::multigrid_bytes(const ibm::Dims &d, int precision) {
+    const double cells = (double)d.ncell;
+    const bool mixed = precision != IBM3D_PREC_FP64;
     // multigrid (build_mg): fine-level residual and smoother scratch (FP64,
     // + FP32); coarse levels x, b, r, second smoother buffer (FP64, + FP32),
     // flag and face-mask bytes, and one interpolation-mask byte per cell of
@@ -299,12 +312,6 @@ double IBMSolver_estimate_device_bytes(int Nx, int Ny, int Nz, int precision, in
         + coarse * (8.0 * 4 + 2 + (mixed ? 4.0 * 4 : 0)) + (cells + coarse) * 1;
     // dense inverse of the coarsest level (at most 3000 rows; FP64, + FP32);
     // the pivot scratch of its inversion (0.8 MB) is part of the last term
-    const double n = std::min(3000.0, (double)Nx * Ny * Nz);
-    const double dense = n * n * (8 + (mixed ? 4 : 0)) + 2 * 8.0 * n;
-    // reduction partials, ghost lists, 1-D metrics and folded coefficients
-    return cells * per + mg + dense + 16.0 * (1 << 20);
+    const double n = std::min(3000.0, (double)d.nx * d.ny * d.nz);
+    return mg + n * n * (8 + (mixed ? 4 : 0)) + 2 * 8.0 * n;
 }
-
-double IBMSolver_get_device_bytes(IBMSolver *s) { return (double)s->dev_bytes; }
-
-}  // extern "C"

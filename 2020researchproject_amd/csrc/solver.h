@@ -296,6 +296,11 @@ struct _ibm_solver {
     bool sep_on = false;
     ibm::SeparableSys sep{};
     ibm::DBuf<double> sep_mat[3][3];      // V, Vi, lam per axis
+    // with a body: its ghost rows (build_capacitance)
+    bool cap_on = false;
+    ibm::SeparableBody cap{};
+    ibm::DBuf<double> cap_inv64, cap_t;
+    ibm::DBuf<float> cap_inv32;
     std::vector<ibm::VGraph> vgraphs;     // captured V-cycles per (input, output)
     ibm::Krylov kry;
     ibm::GmresData gm;                    // SOLVER_GMRES / SOLVER_PCG / SOLVER_AMG scratch (pressure)
@@ -370,6 +375,10 @@ void polyhedron_cpt_grid(const Polyhedron *poly, int nx, int ny, int nz, const d
                          const double *z, double *f, double maxd);
 int polyhedron_cpt_grid_noalloc(const Polyhedron *poly, int nx, int ny, int nz, const double *x, const double *y,
                                 const double *z, double *f, double maxd);
+
+// serve.cpp: what IBMSolver_estimate_device_bytes counts for the multigrid
+// hierarchy
+double multigrid_bytes(const Dims &d, int precision);
 
 // export.cpp
 void export_result_impl(IBMSolver *s, const char *filename);

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <sched.h>
 
+#include "../../include/ibm3d_serve.h"
 #include "solver.h"
 
 #include <type_traits>
@@ -571,26 +572,145 @@ void ensure_mg(IBMSolver *s) {
     HIP_CHECK(hipStreamSynchronize(s->stream));
 }
 
-// Direct pressure solve (separable.hip) where the system allows it: no solid
-// or ghost cell, every axis symmetric in its cell widths (all but a periodic
-// axis that is not uniform), and the solver asked for is the default one
-// (BiCGSTAB with the multigrid preconditioner, no multigrid setting changed).
-// Time per step at tol 1e-12, multigrid / direct: cavity 32^3 1.43 / 0.31 ms,
-// 64^3 (FP64) 2.34 / 0.40, 128^3 5.62 / 1.13, channel 64 x 48 x 32 4.85 / 0.29.
+// The ghost rows of a body for the direct pressure solve: R A^-1 E column by
+// column (A^-1 of the unit vectors of the ghost cells), and its inverse. False
+// where the method does not apply: the box alone is singular, a fluid cell
+// borders a solid one that is no ghost cell, or there is no room.
+// Room: what the estimate of a solver's memory holds for the multigrid
+// hierarchy, which is then not built (and, for the inversion, for the fields
+// that are not there yet). The inverse is kept in FP64; in mixed-Krylov mode,
+// if only FP32 fits, in FP32 (the correction of a refinement round, as the
+// FP32 cycles are): canopy 160 x 80 x 48, 6579 ghost cells, 346 MB in FP64.
+// Assembly with the hierarchy / with this: sphere 256 x 128 x 128 (3568 ghost
+// cells) 134 / 119 ms, 133 x 67 x 61 37 / 19, the canopy 36 / 121.
+static bool build_capacitance(IBMSolver *s) {
+    const Dims &d = s->d;
+    const int ng = s->ng, n[3] = {d.nx, d.ny, d.nz};
+    if (s->p_singular || ng == 0) return false;
+    long ghosts = 0;
+    for (int k = 0; k < d.nz; k++)
+        for (int j = 0; j < d.ny; j++)
+            for (int i = 0; i < d.nx; i++) {
+                const long q = cidx(d, i, j, k), st[3] = {1, d.sy, d.sz};
+                const int id[3] = {i, j, k};
+                ghosts += s->flag_dev_h[q] == F_GHOST;
+                if (s->flag_dev_h[q] != F_FLUID) continue;
+                for (int a = 0; a < 3; a++)
+                    for (int side = -1; side <= 1; side += 2) {
+                        const int o = id[a] + side;
+                        const bool in = o >= 0 && o < n[a];
+                        if (!in && !s->sys[3].S64.ax[a].periodic) continue;
+                        if (s->flag_dev_h[q + (in ? side : -side * (n[a] - 1)) * st[a]] == F_SOLID) return false;
+                    }
+            }
+    if (ghosts != ng) return false;
+    const int ld = (ng + 15) / 16 * 16;
+    const double full = 8.0 * ld * ld, room = multigrid_bytes(d, s->precision);
+    const double all = IBMSolver_estimate_device_bytes(s->Nx, s->Ny, s->Nz, s->precision, s->turb_type != TURBMODEL_NONE);
+    const bool wide = full <= room;
+    if (!wide && (s->precision == IBM3D_PREC_FP64 || full / 2 > room || s->dev_bytes + 1.5 * full > all)) return false;
+
+    // places of the ghost cells and their stencil points
+    GreenBox box{{d.nx, d.ny, d.nz}, {0, 0, 0}};
+    std::vector<int> at(27 * (size_t)ng, -1);
+    s->cap.g0 = d.nz;
+    s->cap.g1 = 0;
+    for (int g = 0; g < ng; g++)
+        for (int l = 0; l < 9; l++) {
+            const long q = l < 8 ? s->ghosts[g].src[l] : s->ghosts[g].cell;
+            if (q < 0) continue;
+            const int id[3] = {(int)((q - d.off) % d.sz % d.sy), (int)((q - d.off) % d.sz / d.sy),
+                               (int)((q - d.off) / d.sz)};
+            for (int a = 0; a < 3; a++) {
+                if (id[a] < 0 || id[a] >= n[a]) return false;
+                box.lo[a] = std::min(box.lo[a], id[a]);
+                box.hi[a] = std::max(box.hi[a], id[a] + 1);
+                at[27 * (size_t)g + 3 * l + a] = id[a];
+            }
+            if (l == 8) {
+                s->cap.g0 = std::min(s->cap.g0, id[2]);
+                s->cap.g1 = std::max(s->cap.g1, id[2] + 1);
+            }
+        }
+    const long bx = box.hi[0] - box.lo[0], by = box.hi[1] - box.lo[1], bz = box.hi[2] - box.lo[2];
+    std::vector<int> loc(9 * (size_t)ng, -1);
+    for (size_t e = 0; e < loc.size(); e++)
+        if (at[3 * e] >= 0)
+            loc[e] = (int)(((at[3 * e + 2] - box.lo[2]) * by + at[3 * e + 1] - box.lo[1]) * bx + at[3 * e] - box.lo[0]);
+    // sources plane by plane
+    std::vector<std::vector<int3>> plane(d.nz);
+    for (int g = 0; g < ng; g++) {
+        const int *c = &at[27 * (size_t)g + 24];
+        plane[c[2]].push_back({c[0], c[1], g});
+    }
+    std::vector<int3> src;
+    for (const auto &p : plane) src.insert(src.end(), p.begin(), p.end());
+
+    size_t scratch_bytes = 0;
+    DBuf<int> dloc;
+    DBuf<int3> dsrc;
+    DBuf<double> scratch, wide_inv;
+    {
+        DevBytesScope temporary(&scratch_bytes);
+        dloc.upload(loc);
+        dsrc.upload(src);
+        scratch.alloc(gauss_jordan_scratch(ng));
+        if (!wide) wide_inv.alloc((size_t)ld * ld);
+    }
+    if (wide) s->cap_inv64.alloc((size_t)ld * ld);
+    double *inv = wide ? s->cap_inv64.p : wide_inv.p;
+    s->cap_t.alloc(ld);
+    GreenScratch green{};
+    green.per = (int)std::min(1024L, d.ncell / (bx * by * bz));
+    for (int v = 0; v < kGreenVecs; v++) green.v[v] = s->kry.v64[2 + v].p;
+    size_t done = 0;
+    for (int k = 0; k < d.nz; k++) {
+        if (plane[k].empty()) continue;
+        launch_green_plane(s->stream, d, s->sep, k, dsrc.p + done, (int)plane[k].size(), box, s->gp.G64, dloc.p,
+                           s->kry.v64[1].p, green, inv, ld);
+        done += plane[k].size();
+    }
+    gauss_jordan_invert(s->stream, inv, ng, ld, scratch.p);
+    if (!wide) {
+        s->cap_inv32.alloc((size_t)ld * ld);
+        launch_d2f_flat(s->stream, inv, s->cap_inv32.p, (long)ld * ld);
+    }
+    HIP_CHECK(hipStreamSynchronize(s->stream));  // the scratch is freed here
+    s->cap.flag = s->flag.p;
+    s->cap.G = s->gp.G64;
+    s->cap.inv64 = wide ? s->cap_inv64.p : nullptr;
+    s->cap.inv32 = wide ? nullptr : s->cap_inv32.p;
+    s->cap.ld = ld;
+    s->cap.t = s->cap_t.p;
+    s->cap.y0 = box.lo[1]; s->cap.y1 = box.hi[1];
+    s->cap.z0 = box.lo[2]; s->cap.z1 = box.hi[2];
+    return true;
+}
+
+// Direct pressure solve (separable.hip) where the system allows it: every axis
+// symmetric in its cell widths (all but a periodic axis that is not uniform),
+// no body or one that build_capacitance takes, and the solver asked for is the
+// default one (BiCGSTAB with the multigrid preconditioner, no multigrid
+// setting changed). Time per step at tol 1e-12, multigrid / direct: cavity
+// 32^3 1.43 / 0.31 ms, 64^3 (FP64) 2.34 / 0.40, 128^3 5.62 / 1.13, channel
+// 64 x 48 x 32 4.85 / 0.29; with a body: sphere 98 x 47 x 51 (FP64) 2.78 /
+// 0.44, 133 x 67 x 61 3.15 / 0.68, 256 x 128 x 128 8.56 / 2.16, canopy 160 x
+// 80 x 48 5.25 / 0.97.
 // The transforms grow as the axis length per cell: at 128^3 they are 163 us
 // of the step. Axes beyond the LDS tiles (400 cells) take the multigrid path.
 void build_separable(IBMSolver *s) {
-    s->sep_on = false;
+    s->sep_on = s->cap_on = false;
     if (s->solver_type != SOLVER_BiCGSTAB || s->precond_type != PRECOND_AMG || s->precision == IBM3D_PREC_MIXED
         || s->mg_custom)
         return;
     const Dims &d = s->d;
+    bool body = false;
     for (int k = 0; k < d.nz; k++)
         for (int j = 0; j < d.ny; j++)
-            for (int i = 0; i < d.nx; i++)
-                if (s->flag_dev_h[cidx(d, i, j, k)] != F_FLUID) return;
+            for (int i = 0; i < d.nx; i++) body |= s->flag_dev_h[cidx(d, i, j, k)] != F_FLUID;
     const int n[3] = {d.nx, d.ny, d.nz};
     if (!separable_fits(n)) return;
+    if (body && (s->p_singular || s->ng == 0)) return;
     const std::vector<double> *w[3] = {&s->dx, &s->dy, &s->dz};
     std::vector<double> m[3][3];
     double lo = 0, hi = 0, low[3];
@@ -616,6 +736,10 @@ void build_separable(IBMSolver *s) {
         s->sep.ax[a] = {s->sep_mat[a][0].p, s->sep_mat[a][1].p, s->sep_mat[a][2].p, n[a], (n[a] + 15) / 16 * 16};
     }
     s->sep.pinned = s->p_singular;
+    if (body) {
+        s->sep_on = s->cap_on = build_capacitance(s);
+        return;
+    }
     s->sep_on = true;
     // Mixed-Krylov mode: where a solve of a pinned system falls back, its FP32
     // cycles stall if the eigenvalues span more than FP32 resolves. They
@@ -1466,11 +1590,16 @@ static bool separable_solve(IBMSolver *s, const double *b, double *x, F &&norm, 
     const double cb = ncells(s) * 8;
     double last = 0;
     for (int round = 1;; round++) {
-        TIMED("separable", (round > 1 ? 7 : 6) * cb,
-              launch_separable(s->stream, d, s->sep, round > 1 ? r : b, s1, s2, x, round > 1, s->partial.p));
+        const double *rhs = round > 1 ? r : b;
+        if (s->cap_on)
+            TIMED("separable_body", (round > 1 ? 10 : 9) * cb + (double)s->cap.G.ng * s->cap.ld * (s->cap.inv64 ? 8 : 4),
+                  launch_separable_body(s->stream, d, s->sep, s->cap, rhs, s1, s2, s->kry.v64[3].p, x, round > 1));
+        else
+            TIMED("separable", (round > 1 ? 7 : 6) * cb,
+                  launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, round > 1, s->partial.p));
         TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r,
                                                           ns, s->partial.p));
-        const unsigned e = finalize_publish(s, 4, apply_partials(d, 0), 2);
+        const unsigned e = finalize_publish(s, 4, apply_partials(d, s->gp.G64.ng), 2);
         if (round == 1) *bnorm = norm();
         finalize_wait(s, e);
         if (*bnorm == 0) {
@@ -1479,13 +1608,21 @@ static bool separable_solve(IBMSolver *s, const double *b, double *x, F &&norm, 
             return true;
         }
         const double rn = std::sqrt(s->ks_h->rrn);
-        if (rn <= s->tol * *bnorm || !std::isfinite(rn)) {
+        if (rn <= s->tol * *bnorm) {
             report_solve(s, 3, rn / *bnorm, round);
             return true;
         }
-        if (round > 1 && rn > 0.5 * last) return false;
+        if (!(round == 1 || rn <= 0.5 * last) || !std::isfinite(rn)) break;
         last = rn;
     }
+    // with a body the memory of the capacitance matrix is the hierarchy's: the
+    // solver goes over to the iterative path for good
+    if (s->cap_on) {
+        s->sep_on = s->cap_on = false;
+        s->cap_inv64.free();
+        s->cap_inv32.free();
+    }
+    return false;
 }
 
 static void solve_system(IBMSolver *s, int sk, const double *b, double *x, double bnorm) {
@@ -1820,8 +1957,9 @@ static void do_step(IBMSolver *s) {
         return std::sqrt(s->sums_h[0] + s->sys[3].bc_norm2 + pnorm[3]);
     };
     double bnp = 0;
-    if (!s->sep_on || !separable_solve(s, s->bp.p, s->pp.p, poisson_norm, &bnp)) {
-        if (!s->sep_on) bnp = poisson_norm();
+    const bool direct = s->sep_on;
+    if (!direct || !separable_solve(s, s->bp.p, s->pp.p, poisson_norm, &bnp)) {
+        if (!direct) bnp = poisson_norm();
         solve_system(s, 3, s->bp.p, s->pp.p, bnp);
     }
     TIMED("outer_sol", 0, launch_outer(s->stream, s->geo, opp, s->pp.p, nullptr, nullptr, 3, 0));

@@ -58,10 +58,12 @@ void IBMSolver_set_precision(IBMSolver *, int mode);
    relaxed after each sweep; 1: one launch per colour, ghost rows relaxed
    after each colour. Defaults 3.5, 2, 2, 1. gamma must be finite; pre and
    post 0..16, not both 0. Must be called before IBMSolver_assemble.
-   A box without a body under SOLVER_BiCGSTAB with PRECOND_AMG solves its
-   pressure directly (eigenvectors of the three axes, refined until the
-   stopping test holds) in the modes FP64 and MIXED_KRYLOV; calling this or
-   one of the next two functions selects BiCGSTAB with these cycles there. */
+   SOLVER_BiCGSTAB with PRECOND_AMG solves the pressure directly in the modes
+   FP64 and MIXED_KRYLOV (eigenvectors of the three axes, a dense inverse for
+   the ghost rows of a body, refined until the stopping test holds) where the
+   periodic axes are uniform and a body has a pressure-type boundary and not
+   too many ghost cells for the grid; calling this or one of the next two
+   functions selects BiCGSTAB with these cycles there. */
 void IBMSolver_set_mg_params(IBMSolver *, double gamma, int pre, int post, int smoother);
 /* Levels from `from_level` down (when from_level > 0) smooth with one sweep
    before and one after the coarse correction instead of pre/post; 0 smooths
