@@ -752,6 +752,8 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
         s->ks1d[0].upload(kx); s->ks1d[1].upload(ky); s->ks1d[2].upload(kz);
     }
 
+    build_outer_rules(s);
+
     // flags and level set in device layout (all padded cells)
     s->flag_dev_h.assign(d.ncell, F_FLUID);
     std::vector<double> lv(d.ncell, 0.5);

@@ -246,6 +246,7 @@ struct _ibm_solver {
     ibm::Dims d{};
     ibm::Geo geo{};
     ibm::DBuf<double> g1d[12];       // dx dy dz xc yc zc kW kE kS kN kD kU
+    ibm::DBuf<ibm::OuterRule> outer_rules;  // build_outer_rules
     ibm::DBuf<double> ks1d[3];       // kW+kE, kS+kN, kD+kU (interior, unpadded)
     ibm::DBuf<uint8_t> flag;
     ibm::DBuf<double> lvset;
@@ -361,6 +362,7 @@ void build_mg(IBMSolver *s);
 void ensure_mg(IBMSolver *s);
 void build_separable(IBMSolver *s);
 void build_momentum_tables(IBMSolver *s);
+void build_outer_rules(IBMSolver *s);
 double max_div_impl(IBMSolver *s);
 void body_force_impl(IBMSolver *s, double *dst);
 void body_force_read(IBMSolver *s, double out[3]);

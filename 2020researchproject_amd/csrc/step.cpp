@@ -99,10 +99,10 @@ static double ncells(const IBMSolver *s) { return (double)s->Nx * s->Ny * s->Nz;
 // ---------------------------------------------------------------------------
 // boundary data
 // ---------------------------------------------------------------------------
-enum { BCD_U = 0, BCD_P = 1, BCD_USOL = 2, BCD_PSOL = 3 };
+enum { BCD_FIELDS, BCD_PSOL };
 
-// Builds the face data for one use: velocity at time t (BCD_U, BCD_USOL),
-// pressure at t (BCD_P) or the increment p_bc(t + dt) - p_bc(t) (BCD_PSOL).
+// Builds the face data for one use: velocity and pressure at time t
+// (BCD_FIELDS) or the increment p_bc(t + dt) - p_bc(t) (BCD_PSOL).
 // VAL_FUNC faces are evaluated on the host over the reference's tangential
 // ranges and uploaded; norm2[c] returns 2 sum g^2 of their BC rows.
 static OuterParams make_outer(IBMSolver *s, int what, double t, double norm2[4]) {
@@ -178,11 +178,102 @@ static bool conv_outflow(IBMSolver *s, int init) {
     return any;
 }
 
+// Rules of the outer layers (k_outer) for every kind of field, axis, side and
+// layer.  <- src/ibm3d_fracstep.c:855-1906
+static OuterRule outer_rule(const IBMSolver *s, int kind, int ax, int hi, int layer) {
+    const int n[3] = {s->Nx, s->Ny, s->Nz}, N = n[ax];
+    const std::vector<double> *width[3] = {&s->dx, &s->dy, &s->dz}, *centre[3] = {&s->xc, &s->yc, &s->zc};
+    const std::vector<double> &cc = *centre[ax];
+    const int o1 = hi ? N : -1, o2 = hi ? N + 1 : -2, q0 = hi ? N - 1 : 0, q1 = hi ? N - 2 : 1;
+    const bool vel = kind < 3, first = layer == 0;
+    const IBMSolverBCType t = s->bc[face_bc(ax, hi)].type;
+    OuterRule r{0, {0, 0}, {first ? q0 : q1, q0}, 0, 0};
+    switch (t) {
+    case BC_ALL_PERIODIC:
+        r.c[0] = 1;
+        r.n[0] = (first ? o1 : o2) + (hi ? -N : N);
+        return r;
+    case BC_VELOCITY_PERIODIC:
+        if (!vel) break;
+        r.c[0] = 1;
+        r.n[0] = (first ? o1 : o2) + (hi ? -N : N);
+        return r;
+    case BC_VELOCITY_COMPONENT:
+        if (vel) break;
+        r.c[0] = 1;
+        return r;
+    case BC_FREE_SLIP_WALL:
+        if (kind == ax) break;
+        r.c[0] = 1;
+        return r;
+    case BC_PRESSURE:
+        if (vel) {  // linear extrapolation, layer by layer
+            const double s1 = std::fabs(H1(cc, o1) - H1(cc, q0)), s0 = std::fabs(H1(cc, q0) - H1(cc, q1));
+            const double a1 = (s1 + s0) / s0, b1 = -s1 / s0;
+            r.n[0] = q0;
+            r.n[1] = q1;
+            r.c[0] = a1;
+            r.c[1] = b1;
+            if (first) return r;
+            const double s2 = std::fabs(H1(cc, o2) - H1(cc, o1)), a2 = (s2 + s1) / s1, b2 = -s2 / s1;
+            r.c[0] = a2 * a1 + b2;
+            r.c[1] = a2 * b1;
+            return r;
+        }
+        break;
+    case BC_CONVECTIVE_OUTFLOW:
+        break;
+    default:
+        r.keep = 1;
+        return r;
+    }
+    // the boundary value, by linear interpolation (zero on a free-slip wall);
+    // the low z face takes the x widths for the pressure, src/ibm3d_fracstep.c:1792-1800
+    const std::vector<double> &dd =
+        kind == OUT_P && ax == 2 && !hi && t != BC_CONVECTIVE_OUTFLOW ? s->dx : *width[ax];
+    const double ao = first ? H1(dd, o1) / 2 : H1(dd, o2) / 2 + H1(dd, o1);
+    const double bi = first ? H1(dd, q0) / 2 : H1(dd, q0) + H1(dd, q1) / 2;
+    r.g = t == BC_FREE_SLIP_WALL ? 0.0 : (ao + bi) / bi;
+    r.c[0] = -ao / bi;
+    return r;
+}
+
+void build_outer_rules(IBMSolver *s) {
+    std::vector<OuterRule> t;
+    for (int kind = 0; kind < 5; kind++)
+        for (int e = 0; e < 12; e++) t.push_back(outer_rule(s, kind, e / 4, e / 2 % 2, e % 2));
+    s->outer_rules.upload(t);
+}
+
+// Boundary data of the systems comp..comp+n-1 into their right-hand sides;
+// faces whose data are zero for all of them take no part.
+static void bc_rhs(IBMSolver *s, const OuterParams &op, int comp, int n) {
+    BcRhs p{};
+    p.n = n;
+    p.comp = comp;
+    for (int c = 0; c < n; c++) p.b[c] = comp < 3 ? s->b[c].p : s->bp.p;
+    for (int ax = 0; ax < 3; ax++)
+        for (int hi = 0; hi < 2; hi++) {
+            const HostBC &B = s->bc[face_bc(ax, hi)];
+            const bool on = comp < 3 ? B.type == BC_VELOCITY_COMPONENT || B.type == BC_CONVECTIVE_OUTFLOW
+                                     : (B.type == BC_PRESSURE || B.type == BC_VELOCITY_PERIODIC) && B.val_type == VAL_FUNC;
+            bool any = false;
+            for (int c = 0; on && c < n; c++) {
+                const FaceBC &F = op.face[ax][hi];
+                if (F.garr || F.g[comp + c] != 0) p.gamma[c][ax][hi] = s->sys[comp + c].gamma[ax][hi];
+                any |= p.gamma[c][ax][hi] != 0;
+            }
+            if (!any) continue;
+            p.K[ax][hi] = s->g1d[6 + 2 * ax + hi].p;
+            p.face[p.nface++] = 2 * ax + hi;
+        }
+    TIMED("bc_rhs", 0, launch_bc_rhs(s->stream, s->geo, op, p));
+}
+
 static void update_outer(IBMSolver *s) {
-    OuterParams ou = make_outer(s, BCD_U, s->time, nullptr);
-    TIMED("outer_u", 0, launch_outer(s->stream, s->geo, ou, s->u[0].p, s->u[1].p, s->u[2].p, 0, 0));
-    OuterParams opp = make_outer(s, BCD_P, s->time, nullptr);
-    TIMED("outer_p", 0, launch_outer(s->stream, s->geo, opp, s->p.p, nullptr, nullptr, 1, 0));
+    const OuterParams op = make_outer(s, BCD_FIELDS, s->time, nullptr);
+    TIMED("outer", 0, launch_outer(s->stream, s->d, op, s->outer_rules.p, {{s->u[0].p, s->u[1].p, s->u[2].p, s->p.p},
+                                                           {0, 1, 2, OUT_P}, 4}));
 }
 
 static void update_ghost(IBMSolver *s) {
@@ -223,20 +314,22 @@ static void wait_published(hipStream_t st, KPub *pub_h, unsigned e) { wait_epoch
 
 // The first nv sums, copied by a small kernel into device-mapped host memory
 // (sums_h) and awaited there
-static unsigned publish_sums(IBMSolver *s, int nv) {
+static void read_sums(IBMSolver *s, int nv) {
     const unsigned e = ++s->sums_epoch;
     launch_publish(s->stream, s->sums.p, nv, s->sums_d, s->sums_d_epoch, e);
+    wait_epoch(s->stream, s->sums_h_epoch, e);
+}
+
+// The sums (maxima) of nv columns of block partials, formed straight into
+// sums_h (sum_publish: the epoch to wait for) and awaited there
+static unsigned sum_publish(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
+    const unsigned e = ++s->sums_epoch;
+    launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d, reduce_max, s->sums_d_epoch, e);
     return e;
 }
 
-static void read_sums(IBMSolver *s, int nv) { wait_epoch(s->stream, s->sums_h_epoch, publish_sums(s, nv)); }
-
-// The sums (maxima) of nv columns of block partials, formed straight into
-// sums_h and awaited there
 static void sum_read(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
-    const unsigned e = ++s->sums_epoch;
-    launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d, reduce_max, s->sums_d_epoch, e);
-    wait_epoch(s->stream, s->sums_h_epoch, e);
+    wait_epoch(s->stream, s->sums_h_epoch, sum_publish(s, nblk, nv, reduce_max));
 }
 
 // Finalize kernel `op` over the block partials, with the resulting scalars
@@ -1888,25 +1981,23 @@ static void do_step(IBMSolver *s) {
         TIMED("k1_conv_rhs", cn * (16 * 8 + 1),
               launch_conv_rhs(s->stream, s->geo, sp, s->flag.p, u3, U3, s->p.p, Np, N, b, tau_ptrs(s),
                               s->partial.p));
-        launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
     }
-    const bool conv = conv_outflow(s, 0);
+    // squared norms of the right-hand sides: straight to the host, or to where
+    // the outflow faces' norms join them
+    bool conv = false;
+    for (const HostBC &B : s->bc) conv |= B.type == BC_CONVECTIVE_OUTFLOW;
+    unsigned me = 0;
+    if (conv) launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
+    else me = sum_publish(s, conv_rhs_blocks(s->d), 3);
+    conv_outflow(s, 0);
     double fnorm[4];
-    const OuterParams ob = make_outer(s, BCD_USOL, s->time, fnorm);
-    for (int l = 0; l < 3; l++)
-        for (int ax = 0; ax < 3; ax++)
-            for (int hi = 0; hi < 2; hi++) {
-                const double gm = s->sys[l].gamma[ax][hi];
-                const IBMSolverBCType t = s->bc[face_bc(ax, hi)].type;
-                if (gm == 0 || (t != BC_VELOCITY_COMPONENT && t != BC_CONVECTIVE_OUTFLOW)) continue;
-                const double *Kf = ax == 0 ? (hi ? s->g1d[7].p : s->g1d[6].p)
-                                 : ax == 1 ? (hi ? s->g1d[9].p : s->g1d[8].p) : (hi ? s->g1d[11].p : s->g1d[10].p);
-                launch_bc_rhs(s->stream, s->geo, ob, ax, hi, l, Kf, gm, s->b[l].p);
-            }
+    const OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm);
+    bc_rhs(s, ob, 0, 3);
     // stopping norms of the momentum solves: the right-hand sides' sums
     // (host read) plus the BC rows' and forcing parts
     auto mom_norms = [&](double bn[3]) {
-        read_sums(s, conv ? kConvNormSlot + 18 : 3);
+        if (conv) read_sums(s, kConvNormSlot + 18);
+        else wait_epoch(s->stream, s->sums_h_epoch, me);
         for (int l = 0; l < 3; l++) {
             double bn2 = s->sums_h[l] + s->sys[l].bc_norm2 + fnorm[l];
             for (int f = 0; conv && f < 6; f++)
@@ -1930,7 +2021,7 @@ static void do_step(IBMSolver *s) {
     }
     // outer layers of the three solutions from their BC rows (the per-component
     // fill of each u* with the solve's boundary data, all three in one pass)
-    TIMED("outer_sol", 0, launch_outer(s->stream, s->geo, ob, s->us[0].p, s->us[1].p, s->us[2].p, 0, 0));
+    TIMED("outer_sol", 0, launch_outer(s->stream, s->d, ob, s->outer_rules.p, {{s->us[0].p, s->us[1].p, s->us[2].p}, {0, 1, 2}, 3}));
     // K2: U*, Poisson RHS
     {
         const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};
@@ -1939,19 +2030,11 @@ static void do_step(IBMSolver *s) {
         const double *Fc[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
         TIMED("k2_poisson_rhs", cn * (4 * 8 + 1),
               launch_poisson_rhs(s->stream, s->geo, sp, s->flag.p, s->pin, Fc, s->bp.p, s->partial.p));
-        launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 1, s->sums.p, 0);
     }
+    const unsigned pe = sum_publish(s, conv_rhs_blocks(s->d), 1);
     double pnorm[4];
     const OuterParams opp = make_outer(s, BCD_PSOL, s->time, pnorm);
-    for (int ax = 0; ax < 3; ax++)
-        for (int hi = 0; hi < 2; hi++) {
-            const IBMSolverBCType t = s->bc[face_bc(ax, hi)].type;
-            if ((t != BC_PRESSURE && t != BC_VELOCITY_PERIODIC) || s->bc[face_bc(ax, hi)].val_type != VAL_FUNC) continue;
-            const double *Kf = ax == 0 ? (hi ? s->g1d[7].p : s->g1d[6].p)
-                             : ax == 1 ? (hi ? s->g1d[9].p : s->g1d[8].p) : (hi ? s->g1d[11].p : s->g1d[10].p);
-            launch_bc_rhs(s->stream, s->geo, opp, ax, hi, 3, Kf, s->sys[3].gamma[ax][hi], s->bp.p);
-        }
-    const unsigned pe = publish_sums(s, 1);
+    bc_rhs(s, opp, 3, 1);
     auto poisson_norm = [&] {
         wait_epoch(s->stream, s->sums_h_epoch, pe);
         return std::sqrt(s->sums_h[0] + s->sys[3].bc_norm2 + pnorm[3]);
@@ -1962,7 +2045,7 @@ static void do_step(IBMSolver *s) {
         if (!direct) bnp = poisson_norm();
         solve_system(s, 3, s->bp.p, s->pp.p, bnp);
     }
-    TIMED("outer_sol", 0, launch_outer(s->stream, s->geo, opp, s->pp.p, nullptr, nullptr, 3, 0));
+    TIMED("outer_sol", 0, launch_outer(s->stream, s->d, opp, s->outer_rules.p, {{s->pp.p}, {OUT_DP}, 1}));
     // K3: projection
     {
         const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};

@@ -78,10 +78,33 @@ void launch_poisson_rhs(hipStream_t st, const Geo &g, const StepParams &sp, cons
 void launch_update(hipStream_t st, const Geo &g, const StepParams &sp, const uint8_t *flag, const double *p,
                    const double *pp, const double *const us[3], const double *const F[3], double *pn,
                    double *const un[3], double *const G[3]);
-void launch_outer(hipStream_t st, const Geo &g, const OuterParams &op, double *f1, double *f2, double *f3,
-                  int mode, int comp);
-void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, int ax, int hi, int comp,
-                   const double *Kf, double gamma, double *b);
+// Fields whose outer layers are filled. kind: 0..2 velocity component, OUT_P
+// pressure, OUT_DP solution of the pressure-correction system.
+enum { OUT_P = 3, OUT_DP = 4 };
+struct OuterFields {
+    double *f[4];
+    int kind[4];
+    int n;
+};
+// Rule of an outer position: value = g * (boundary value) + sum_t c[t] (value
+// at position n[t] of the axis); keep: not written. Table [kind][axis][hi][layer].
+struct OuterRule {
+    double g, c[2];
+    int n[2], keep, pad;
+};
+constexpr int kOuterRules = 5 * 12;
+void launch_outer(hipStream_t st, const Dims &d, const OuterParams &op, const OuterRule *rules,
+                  const OuterFields &fs);
+// Boundary data of the right-hand sides b[0..n) of components comp..comp+n-1:
+// faces 2 axis + hi; gamma[c][axis][hi] 0: no share; K: face coefficients
+struct BcRhs {
+    double *b[3];
+    int n, comp;
+    int face[6], nface;
+    double gamma[3][3][2];
+    const double *K[3][2];
+};
+void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p);
 void launch_ghost_update(hipStream_t st, const GhostCell *gc, int ng, const int *level_start, int nlevels,
                          double *old, double *u1, double *u2, double *u3, double *p);
 void launch_solid_nan(hipStream_t st, const Dims &d, const uint8_t *flag, double *u1, double *u2, double *u3,

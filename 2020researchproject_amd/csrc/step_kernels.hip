@@ -14,6 +14,8 @@
 // one 512-byte x-row segment per array.
 #include "step_kernels.h"
 
+#include <algorithm>
+
 namespace ibm {
 
 #define C1(a, i) ((a)[(i) + 2])
@@ -273,115 +275,66 @@ __global__ void __launch_bounds__(256) k_update(Geo g, StepParams sp, const uint
 
 // ---------------------------------------------------------------------------
 // Outer boundary layers.  <- src/ibm3d_fracstep.c:855-1906
-// One launch per axis (x, then y, then z: the y and z passes read corner
-// values the previous passes wrote). Tangential ranges as in the reference:
-// x faces (j,k) interior; y faces i padded, k interior; z faces i, j padded.
-// mode: 0 = velocity fields (3), 1 = pressure, 2 = solution fill of the
-// momentum system (BC rows, component `comp`), 3 = solution fill of the
-// pressure-correction system.
+// One launch for the six faces and all fields. The reference fills x, then y,
+// then z faces, each reading the corner values that the previous ones wrote;
+// here a thread evaluates those itself: an outer value is a constant plus at
+// most two values further in on its axis, which may in turn be outer on an
+// earlier axis. Tangential ranges as in the reference: x faces (j, k)
+// interior; y faces i padded, k interior; z faces i, j padded. One value per
+// thread, its rule read from a table made at assembly: bound by the launch and
+// a chain of dependent loads. 32^3: 5.8 us for the four fields, 3 launches per
+// step (a launch per axis was 12 of 5.6 us); rules evaluated in the kernel, all
+// layers and fields in one thread, took 33 us.
 // ---------------------------------------------------------------------------
-__device__ inline void face_pos(int n, int hi, int &o1, int &o2, int &q0, int &q1) {
-    if (hi) { o1 = n; o2 = n + 1; q0 = n - 1; q1 = n - 2; }
-    else { o1 = -1; o2 = -2; q0 = 0; q1 = 1; }
-}
-
 __device__ inline double bcval(const FaceBC &f, int comp, int t1, int t2, int n2) {
     if (f.garr) return f.garr[((long)comp * f.n1 + (t1 + f.t1off)) * n2 + (t2 + f.t2off)];
     return f.g[comp];
 }
 
-__global__ void k_outer(Geo g, OuterParams op, int ax, double *f1, double *f2, double *f3, int mode, int comp) {
-    const Dims &d = g.d;
-    const int hi = blockIdx.z;
-    int a0, a1, b0, b1;
-    if (ax == 0) { a0 = 0; a1 = d.ny; b0 = 0; b1 = d.nz; }
-    else if (ax == 1) { a0 = -2; a1 = d.nx + 2; b0 = 0; b1 = d.nz; }
-    else { a0 = -2; a1 = d.nx + 2; b0 = -2; b1 = d.ny + 2; }
+// value of f at (i, j, k), outer positions on the axes up to AX evaluated;
+// rules: of f's kind
+template <int AX>
+__device__ inline double outer_value(const Dims &d, const OuterParams &op, const OuterRule *rules, const double *f,
+                                     int comp, int i, int j, int k) {
+    const int n = AX == 0 ? i : AX == 1 ? j : k, N = AX == 0 ? d.nx : AX == 1 ? d.ny : d.nz;
+    if (n >= 0 && n < N) {
+        if constexpr (AX == 0) return f[cidx(d, i, j, k)];
+        else return outer_value<AX - 1>(d, op, rules, f, comp, i, j, k);
+    }
+    const int hi = n >= N, layer = hi ? n - N : -1 - n;
+    const OuterRule &r = rules[(2 * AX + hi) * 2 + layer];
+    if (r.keep) return f[cidx(d, i, j, k)];
+    double v = 0;
+    if (r.g != 0)
+        v = r.g * bcval(op.face[AX][hi], comp, AX == 0 ? j : i, AX == 2 ? j : k, AX == 2 ? d.ny + 4 : d.nz);
+#pragma unroll 1
+    for (int t = 0; t < 2; t++) {
+        const double c = r.c[t];
+        if (c == 0) continue;
+        const int m = r.n[t], x = AX == 0 ? m : i, y = AX == 1 ? m : j, z = AX == 2 ? m : k;
+        // a position that is not interior on this axis (a single cell wide) is taken as it is
+        double w;
+        if (AX == 0 || m < 0 || m >= N) w = f[cidx(d, x, y, z)];
+        else w = outer_value<AX == 0 ? 0 : AX - 1>(d, op, rules, f, comp, x, y, z);
+        v += c * w;
+    }
+    return v;
+}
+
+__global__ void k_outer(Dims d, OuterParams op, const OuterRule *rules, OuterFields fs) {
+    // one value per thread: face, layer and field
+    const int ax = blockIdx.z % 6 / 2, hi = blockIdx.z % 2, layer = blockIdx.z / 6 % 2, e = blockIdx.z / 12;
+    const int a0 = ax == 0 ? 0 : -2, a1 = ax == 0 ? d.ny : d.nx + 2;
+    const int b0 = ax == 2 ? -2 : 0, b1 = ax == 2 ? d.ny + 2 : d.nz;
     const int t1 = a0 + blockIdx.x * blockDim.x + threadIdx.x;
     const int t2 = b0 + blockIdx.y * blockDim.y + threadIdx.y;
     if (t1 >= a1 || t2 >= b1) return;
-    const FaceBC &F = op.face[ax][hi];
     const int N = ax == 0 ? d.nx : ax == 1 ? d.ny : d.nz;
-    const long st = ax == 0 ? 1 : ax == 1 ? d.sy : d.sz;
-    // linear index of position n along the normal
-    long base;
-    if (ax == 0) base = cidx(d, 0, t1, t2);
-    else if (ax == 1) base = cidx(d, t1, 0, t2);
-    else base = cidx(d, t1, t2, 0);
-    int o1, o2, q0, q1;
-    face_pos(N, hi, o1, o2, q0, q1);
-    const double *dd = ax == 0 ? g.dx : ax == 1 ? g.dy : g.dz;
-    const double *cc = ax == 0 ? g.xc : ax == 1 ? g.yc : g.zc;
-    const int n2 = ax == 0 ? d.nz : ax == 1 ? d.nz : d.ny + 4;
-
-    for (int layer = 1; layer <= 2; layer++) {
-        const int o = layer == 1 ? o1 : o2, qq = layer == 1 ? q0 : q1;
-        const long co = base + o * st, cq = base + qq * st;
-        // Dirichlet interpolation distances (ao outer, bi inner)
-        const double *dl = (mode == 1 && ax == 2 && !hi && F.type != BCT_CONVECTIVE) ? g.dx : dd;  // :1792-1800 spacing quirk
-        double ao, bi;
-        if (layer == 1) { ao = C1(dl, o1) / 2; bi = C1(dl, q0) / 2; }
-        else { ao = C1(dl, o2) / 2 + C1(dl, o1); bi = C1(dl, q0) + C1(dl, q1) / 2; }
-        // extrapolation spacings of the pressure outlet for velocity
-        int n1, nn2;
-        double so, si;
-        if (layer == 1) {
-            n1 = q0; nn2 = q1;
-            so = hi ? C1(cc, o1) - C1(cc, q0) : C1(cc, q0) - C1(cc, o1);
-            si = hi ? C1(cc, q0) - C1(cc, q1) : C1(cc, q1) - C1(cc, q0);
-        } else {
-            n1 = o1; nn2 = q0;
-            so = hi ? C1(cc, o2) - C1(cc, o1) : C1(cc, o1) - C1(cc, o2);
-            si = hi ? C1(cc, o1) - C1(cc, q0) : C1(cc, q0) - C1(cc, o1);
-        }
-        const long cn1 = base + n1 * st, cn2 = base + nn2 * st;
-        const long cw = base + (hi ? o - N : o + N) * st;  // periodic image
-        if (mode == 0 || mode == 2) {
-            double *ff[3] = {f1, f2, f3};
-            const int l0 = mode == 0 ? 0 : comp, l1 = mode == 0 ? 3 : comp + 1;
-            for (int l = l0; l < l1; l++) {
-                double *a = ff[mode == 0 ? l : 0];
-                switch (F.type) {
-                case BCT_VELOCITY:
-                case BCT_CONVECTIVE: {
-                    const double gv = bcval(F, l, t1, t2, n2);
-                    a[co] = (ao + bi) / bi * gv - ao / bi * a[cq];
-                    break;
-                }
-                case BCT_PRESSURE:
-                    a[co] = (so + si) / si * a[cn1] - so / si * a[cn2];
-                    break;
-                case BCT_FREE_SLIP:
-                    a[co] = (l == ax) ? -ao / bi * a[cq] : a[cq];
-                    break;
-                case BCT_ALL_PERIODIC:
-                case BCT_VELOCITY_PERIODIC:
-                    a[co] = a[cw];
-                    break;
-                default:;
-                }
-            }
-        } else {
-            double *a = f1;
-            switch (F.type) {
-            case BCT_VELOCITY:
-            case BCT_FREE_SLIP:
-                a[co] = a[cq];
-                break;
-            case BCT_PRESSURE:
-            case BCT_VELOCITY_PERIODIC:
-            case BCT_CONVECTIVE: {
-                const double gv = bcval(F, 3, t1, t2, n2);
-                a[co] = (ao + bi) / bi * gv - ao / bi * a[cq];
-                break;
-            }
-            case BCT_ALL_PERIODIC:
-                a[co] = a[cw];
-                break;
-            default:;
-            }
-        }
-    }
+    const int kind = fs.kind[e], n = hi ? N + layer : -1 - layer;
+    double *f = fs.f[e];
+    const int i = ax == 0 ? n : t1, j = ax == 0 ? t1 : ax == 1 ? n : t2, k = ax == 2 ? n : t2;
+    // (itself where the rule keeps it)
+    f[cidx(d, i, j, k)] = outer_value<2>(d, op, rules + 12 * kind, f, min(kind, 3), i, j, k);
 }
 
 // ---------------------------------------------------------------------------
@@ -501,27 +454,34 @@ long launch_conv_outflow(hipStream_t st, const Geo &g, int ax, int hi, double uc
 // Inhomogeneous boundary data folded into the right-hand side of the first
 // interior cell: b += K_face * gamma * g (the outer row x_o = alpha x_q +
 // gamma g eliminated from the fluid row). The BC rows' own right-hand side
-// enters the stopping norm on the host.
+// enters the stopping norm on the host. One launch for all faces and fields: a
+// cell on several faces belongs to the first of them, whose thread adds the
+// others' shares too (a launch per face and field was 18 launches per cavity
+// step, 2.7 us each at 32^3).
 // ---------------------------------------------------------------------------
-__global__ void k_bc_rhs(Geo g, OuterParams op, int ax, int hi, int comp, const double *Kf, double gamma,
-                         double *b) {
+__global__ void k_bc_rhs(Geo g, OuterParams op, BcRhs p) {
     const Dims &d = g.d;
-    int a1, b1;
-    if (ax == 0) { a1 = d.ny; b1 = d.nz; }
-    else if (ax == 1) { a1 = d.nx; b1 = d.nz; }
-    else { a1 = d.nx; b1 = d.ny; }
+    const int fc = p.face[blockIdx.z], ax = fc / 2, hi = fc % 2;
+    const int n[3] = {d.nx, d.ny, d.nz};
     const int t1 = blockIdx.x * blockDim.x + threadIdx.x;
     const int t2 = blockIdx.y * blockDim.y + threadIdx.y;
-    if (t1 >= a1 || t2 >= b1) return;
-    const FaceBC &F = op.face[ax][hi];
-    const int N = ax == 0 ? d.nx : ax == 1 ? d.ny : d.nz;
-    const int n = hi ? N - 1 : 0;
-    long q;
-    if (ax == 0) q = cidx(d, n, t1, t2);
-    else if (ax == 1) q = cidx(d, t1, n, t2);
-    else q = cidx(d, t1, t2, n);
-    const int n2 = ax == 0 ? d.nz : ax == 1 ? d.nz : d.ny + 4;
-    b[q] += C1(Kf, n) * gamma * bcval(F, comp, t1, t2, n2);
+    if (t1 >= (ax == 0 ? d.ny : d.nx) || t2 >= (ax == 2 ? d.ny : d.nz)) return;
+    const int at = hi ? n[ax] - 1 : 0;
+    const int i = ax == 0 ? at : t1, j = ax == 0 ? t1 : ax == 1 ? at : t2, k = ax == 2 ? at : t2;
+    double v[3] = {0, 0, 0};
+    for (int e = 0; e < p.nface; e++) {
+        const int a = p.face[e] / 2, h = p.face[e] % 2;
+        const int m = a == 0 ? i : a == 1 ? j : k;
+        if (m != (h ? n[a] - 1 : 0)) continue;
+        if (e < (int)blockIdx.z) return;  // an earlier face's cell
+        const double kf = C1(p.K[a][h], m);
+        for (int c = 0; c < p.n; c++)
+            if (p.gamma[c][a][h] != 0)
+                v[c] += kf * p.gamma[c][a][h]
+                    * bcval(op.face[a][h], p.comp + c, a == 0 ? j : i, a == 2 ? j : k, a == 2 ? d.ny + 4 : d.nz);
+    }
+    const long q = cidx(d, i, j, k);
+    for (int c = 0; c < p.n; c++) p.b[c][q] += v[c];
 }
 
 // ---------------------------------------------------------------------------
@@ -827,28 +787,17 @@ void launch_update(hipStream_t st, const Geo &g, const StepParams &sp, const uin
                        F[0], F[1], F[2], pn, un[0], un[1], un[2], G[0], G[1], G[2]);
 }
 
-void launch_outer(hipStream_t st, const Geo &g, const OuterParams &op, double *f1, double *f2, double *f3,
-                  int mode, int comp) {
-    const Dims &d = g.d;
-    for (int ax = 0; ax < 3; ax++) {
-        int n1, n2;
-        if (ax == 0) { n1 = d.ny; n2 = d.nz; }
-        else if (ax == 1) { n1 = d.nx + 4; n2 = d.nz; }
-        else { n1 = d.nx + 4; n2 = d.ny + 4; }
-        dim3 grid((n1 + 15) / 16, (n2 + 15) / 16, 2);
-        hipLaunchKernelGGL(k_outer, grid, dim3(16, 16), 0, st, g, op, ax, f1, f2, f3, mode, comp);
-    }
+void launch_outer(hipStream_t st, const Dims &d, const OuterParams &op, const OuterRule *rules,
+                  const OuterFields &fs) {
+    const int m1 = std::max(d.ny, d.nx + 4), m2 = std::max(d.nz, d.ny + 4);
+    hipLaunchKernelGGL(k_outer, dim3((m1 + 15) / 16, (m2 + 15) / 16, 12 * fs.n), dim3(16, 16), 0, st, d, op, rules, fs);
 }
 
-void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, int ax, int hi, int comp,
-                   const double *Kf, double gamma, double *b) {
+void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p) {
     const Dims &d = g.d;
-    int a1, b1;
-    if (ax == 0) { a1 = d.ny; b1 = d.nz; }
-    else if (ax == 1) { a1 = d.nx; b1 = d.nz; }
-    else { a1 = d.nx; b1 = d.ny; }
-    hipLaunchKernelGGL(k_bc_rhs, dim3((a1 + 15) / 16, (b1 + 15) / 16), dim3(16, 16), 0, st, g, op, ax, hi, comp,
-                       Kf, gamma, b);
+    if (p.nface == 0) return;
+    const int m1 = std::max(d.nx, d.ny), m2 = std::max(d.ny, d.nz);
+    hipLaunchKernelGGL(k_bc_rhs, dim3((m1 + 15) / 16, (m2 + 15) / 16, p.nface), dim3(16, 16), 0, st, g, op, p);
 }
 
 void launch_ghost_update(hipStream_t st, const GhostCell *gc, int ng, const int *level_start, int nlevels,

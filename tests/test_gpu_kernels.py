@@ -238,3 +238,55 @@ def test_direct_pressure_solve_with_a_body_matches_multigrid(new_gpu, I, cases, 
         assert np.array_equal(np.isfinite(a), m[n])
         ref = out[1][n][m[n]]
         assert np.linalg.norm(a[m[n]] - ref) <= 2 * tol * span * (speed if n != "P" else np.linalg.norm(ref)), n
+
+
+OUTER_CASES = [
+    # boundary types per face (west, east, south, north, down, up)
+    ("velocity", "pressure", "slip", "slip", "wall", "wall"),
+    ("func", "pressure", "pressure", "func", "pressure", "slip"),
+    ("periodic", "periodic", "wall", "pressure", "pressure", "pressure"),
+    ("slip", "velocity", "uperiodic", "uperiodic", "periodic", "periodic"),
+]
+
+
+@pytest.mark.parametrize("shape", [(6, 4, 8), (34, 18, 20)])
+@pytest.mark.parametrize("faces", OUTER_CASES)
+def test_outer_layers_match_the_oracle(new_gpu, new_oracle, I, faces, shape):
+    """Both outer layers, edges and corners of the four fields from random
+    interior ones, on stretched axes where they may be: an outer value is a
+    short sum of products, so the two agree to a few roundings (1e-12 of the
+    largest value, which extrapolation at edges and corners can raise)."""
+    periodic = [faces[2 * a] == "periodic" or faces[2 * a] == "uperiodic" for a in range(3)]
+    out = []
+    for new in (new_gpu, new_oracle):
+        s = new()
+        f = [np.linspace(0.0, 1.0, n + 1) if p else tanh_faces(n, 0.0, 1.0 + a, 1.2)
+             for a, (n, p) in enumerate(zip(shape, periodic))]
+        s.set_grid(*f)
+        s.set_params(100.0, 0.002)
+        for d, t in zip((I.DIR_WEST, I.DIR_EAST, I.DIR_SOUTH, I.DIR_NORTH, I.DIR_DOWN, I.DIR_UP), faces):
+            if t == "velocity":
+                s.set_bc(d, I.BC_VELOCITY_COMPONENT, I.VAL_CONST, 1.0, 0.25, -0.5)
+            elif t == "func":
+                s.set_bc(d, I.BC_VELOCITY_COMPONENT, I.VAL_FUNC, *[
+                    (lambda c: lambda t, x, y, z: c + x + 2 * y * z)(c) for c in (1.0, 2.0, 3.0)])
+            elif t == "pressure":
+                s.set_bc(d, I.BC_PRESSURE, I.VAL_CONST, 0.75)
+            elif t == "uperiodic":
+                s.set_bc(d, I.BC_VELOCITY_PERIODIC, I.VAL_CONST, 0.5)
+            else:
+                s.set_bc(d, {"slip": I.BC_FREE_SLIP_WALL, "wall": I.BC_STATIONARY_WALL,
+                             "periodic": I.BC_ALL_PERIODIC}[t])
+        s.set_obstacle(None)
+        s.set_linear_solver(I.SOLVER_BiCGSTAB, I.PRECOND_AMG, 1e-10)
+        s.assemble()
+        s.init_flow_const(0, 0, 0, 0)
+        rng = np.random.default_rng(5)
+        for n in ("U1", "U2", "U3", "P"):
+            s.set(n, rng.standard_normal(s.shape))
+        s.iterate(0)
+        out.append({n: s.get(n) for n in ("U1", "U2", "U3", "P")})
+    for n, a in out[0].items():
+        b = out[1][n]
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), n
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), n
