@@ -21,12 +21,15 @@ struct SeparableSys {
     int pinned;  // the row of cell (0, 0, 0) is x = b; the problem is otherwise singular
 };
 
+struct GreenBox { int lo[3], hi[3]; };  // end exclusive
+
 // Ghost rows of an immersed body (capacitance matrix method). The box's
 // operator A holds in every fluid row; a right-hand side mu at the ghost cells
 // makes its solution also meet the ghost rows R x = b_g:
 //   (R A^-1 E) mu = b_g - R A^-1 b_fluid,  x = A^-1 (b_fluid + E mu).
-// y0..z1: rows and planes that hold ghost cells or their stencil points (end
-// exclusive), g0..g1: planes with ghost cells.
+// look: the box of the ghost cells and their stencil points, cells: that of the
+// ghost cells; fluid, ghost: masks of the interior cells, one word per 16 cells
+// of a row.
 struct SeparableBody {
     const uint8_t *flag;
     GhostRows<double> G;
@@ -34,7 +37,8 @@ struct SeparableBody {
     const float *inv32;
     int ld;
     double *t;            // ng: right-hand side of the ghost rows
-    int y0, y1, z0, z1, g0, g1;
+    const uint16_t *fluid, *ghost;
+    GreenBox look, cells;
 };
 
 // Host: eigenvalues (ascending) and matrices of one axis from its folded
@@ -60,7 +64,6 @@ void launch_separable_body(hipStream_t st, const Dims &d, const SeparableSys &S,
 // scratch vector; green: kGreenVecs scratch vectors, each for `per` sources
 constexpr int kGreenVecs = 6;
 struct GreenScratch { double *v[kGreenVecs]; int per; };
-struct GreenBox { int lo[3], hi[3]; };
 void launch_green_plane(hipStream_t st, const Dims &d, const SeparableSys &S, int k, const int3 *src, int nsrc,
                         const GreenBox &box, const GhostRows<double> &G, const int *loc, double *h,
                         const GreenScratch &green, double *out, long ld);

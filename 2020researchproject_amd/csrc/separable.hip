@@ -10,114 +10,161 @@
 // division and its inverse, the y and x transforms back. Each launch reads and
 // writes the field once and keeps the intermediate of its two products in LDS.
 // Work: 12 n flops per cell (n: mean axis length), at 128^3 3.2 GFLOP, 41 us at
-// the chip's FP64 matrix rate. Measured at 128^3: 55, 60 and 47 us (20 TFLOP/s,
-// bound by the operand loads of one 16 x 16 tile per wave); at 32^3 4.6, 6.8
-// and 4.7 us, the length of a small launch. A BiCGSTAB iteration with two
-// multigrid cycles took 420 us at 128^3 and 190 us at 32^3, and there were 10
-// and 6 of them per step.
+// the chip's FP64 matrix rate. Measured at 128^3: 32, 34 and 33 us (32 TFLOP/s;
+// 55, 60 and 47 us with one tile per wave at a time: bound by the operands'
+// way through the L2); at 32^3 4.6, 7.0 and 5.7 us, the length of a small
+// launch. A BiCGSTAB iteration with two multigrid cycles took 420 us at 128^3
+// and 190 us at 32^3, and there were 10 and 6 of them per step.
 #include "separable.h"
 
 #include <algorithm>
 #include <cmath>
 #include <numeric>
+#include <type_traits>
 
 namespace ibm {
 
 typedef double mfma_acc __attribute__((ext_vector_type(4)));
 
-constexpr int kSepThreads = 256;
+constexpr int kSepThreads = 512;  // at most; 256 where the tiles feed no more waves
 constexpr int kSepWaves = kSepThreads / 64;
-// LDS row padding: the four lane groups of an operand read, four rows apart,
-// then use different banks
-constexpr int kSepPad = 4;
+__device__ inline int sep_waves() { return blockDim.x >> 6; }
+// LDS row padding (doubles) of a tile read by columns and by rows: the lane
+// groups of an operand read then use different banks
+constexpr int kSepPadCol = 8, kSepPadRow = 2;
 
-// 16 x 16 tile of a product with K = 16 chunks: lane l holds row (of A) or
-// column (of B) l % 16, and the elements 16 c + 4 (l / 16) + 0 .. 3 of the
-// summed index in chunk c (any order serves as long as A and B agree). Result
-// element r of a lane: row 4 r + l / 16, column l % 16.
-template <typename FA, typename FB>
-__device__ inline mfma_acc sep_tile(int chunks, FA a, FB b) {
-    mfma_acc acc = {0, 0, 0, 0};
-    const int k0 = 4 * ((threadIdx.x & 63) >> 4);
-    double av[4], bv[4], an[4], bn[4];
-    a(k0, av);
-    b(k0, bv);
+// MR x NR tiles of 16 x 16 of a product with 16 `chunks` summed elements: lane l
+// holds row (of A) or column (of B) l % 16, and of chunk c the elements 16 c +
+// sep_k(l, 0 .. 3) (any order serves as long as A and B agree; this one loads
+// 64 contiguous bytes of 16 rows at once). a(r, k0, v) and b(s, k0, v) load
+// those of row tile r and column tile s. Result element e of a lane: row 4 e +
+// l / 16, column l % 16. The operands come through the L2 of the XCD, whose
+// rate bounds the large grids: a tile product reads MR + NR operands for MR NR
+// products.
+__device__ inline int sep_k(int g, int t) { return 2 * g + (t & 1) + 8 * (t >> 1); }
+
+template <int MR, int NR, typename FA, typename FB>
+__device__ inline void sep_tiles(int chunks, FA a, FB b, mfma_acc (&acc)[MR][NR]) {
+    double av[MR][4], bv[NR][4], an[MR][4], bn[NR][4];
+#pragma unroll
+    for (int r = 0; r < MR; r++) {
+        a(r, 0, av[r]);
+#pragma unroll
+        for (int s = 0; s < NR; s++) acc[r][s] = {0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int s = 0; s < NR; s++) b(s, 0, bv[s]);
     for (int c = 1; c <= chunks; c++) {
-        const int kn = 16 * min(c, chunks - 1) + k0;  // the next chunk's operands, in flight during the products
-        a(kn, an);
-        b(kn, bn);
+        const int kn = 16 * min(c, chunks - 1);  // the next chunk's operands, in flight during the products
+#pragma unroll
+        for (int r = 0; r < MR; r++) a(r, kn, an[r]);
+#pragma unroll
+        for (int s = 0; s < NR; s++) b(s, kn, bn[s]);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < MR; r++)
+#pragma unroll
+                for (int s = 0; s < NR; s++)
+                    acc[r][s] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r][t], bv[s][t], acc[r][s], 0, 0, 0);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t], bv[t], acc, 0, 0, 0);
-            av[t] = an[t];
-            bv[t] = bn[t];
+#pragma unroll
+            for (int r = 0; r < MR; r++) av[r][t] = an[r][t];
+#pragma unroll
+            for (int s = 0; s < NR; s++) bv[s][t] = bn[s][t];
         }
     }
-    return acc;
 }
 
-__device__ inline void sep_load4(const double *p, double (&v)[4]) {
-    const double2 a = *reinterpret_cast<const double2 *>(p), b = *reinterpret_cast<const double2 *>(p + 2);
+// four consecutive-in-pairs elements of a row (p: row start + chunk + 2 g)
+__device__ inline void sep_row(const double *p, double (&v)[4]) {
+    const double2 a = *reinterpret_cast<const double2 *>(p), b = *reinterpret_cast<const double2 *>(p + 8);
     v[0] = a.x;
     v[1] = a.y;
     v[2] = b.x;
     v[3] = b.y;
 }
 
-// What the first transform reads of b at a cell: everything, only fluid cells,
-// or only ghost cells (the result is then added to y)
-enum { SEP_ALL, SEP_FLUID, SEP_GHOST };
+// Macro tiles of MR x NR over mt x nt tiles, one per wave at a time: f(m, n)
+// with m, n the first tile of each; tiles past the end are clamped by the
+// operand loads and skipped by the stores
+template <int MR, int NR, typename F>
+__device__ inline void sep_macro(int mt, int nt, F f) {
+    const int gn = (nt + NR - 1) / NR, total = (mt + MR - 1) / MR * gn;
+    for (int w = threadIdx.x >> 6; w < total; w += sep_waves()) f(w / gn * MR, w % gn * NR);
+}
+
+// Cells that the first transform reads: all, or those of a bit mask (16 cells
+// of a row per word); with SEP_ADD the result is added to y
+enum { SEP_ALL, SEP_MASK, SEP_ADD };
 
 // y(l, m, k) = sum_ij Vi_x[l][i] Vi_y[m][j] b(i, j, k) for the l of one block
-// of 16 nb and all m: plane k = k0 + blockIdx.y
-template <int WHAT>
+// of 16 nb and all m: plane k = k0 + blockIdx.y; i and j over the tiles
+// [i0, i1) and [j0, j1) (b is 0 elsewhere)
+template <int WHAT, int MR, int NR>
 __global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableAxis X, SeparableAxis Y, const double *b,
-                                                        const uint8_t *flag, double *y, int nb, int k0) {
+                                                        const uint16_t *mask, double *y, int nb, int pitch, int k0,
+                                                        int i0, int i1, int j0, int j1) {
     extern __shared__ double sep_lds[];
-    const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-    const int k = k0 + blockIdx.y, l0 = blockIdx.x * 16 * nb, pitch = 16 * nb + kSepPad;
-    const int mt = Y.np / 16, nt = min(nb, (X.np - l0) / 16);
-    for (int w = wave; w < mt * nt; w += kSepWaves) {
-        const int j0 = 16 * (w / nt), c0 = 16 * (w % nt);
-        const long q0 = cidx(d, 0, min(j0 + ln, d.ny - 1), k);
-        const double *vx = X.Vi + (long)(l0 + c0 + ln) * X.np;
-        const mfma_acc t = sep_tile(
-            X.np / 16,
-            [&](int i, double (&v)[4]) {
-                sep_load4(b + q0 + i, v);
-                unsigned f = 0;
-                if (WHAT != SEP_ALL) f = *reinterpret_cast<const unsigned *>(flag + q0 + i);
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const unsigned fq = f >> 8 * q & 0xFF;
-                    const bool in = WHAT == SEP_ALL || fq == (WHAT == SEP_FLUID ? F_FLUID : F_GHOST);
-                    v[q] = in && i + q < d.nx ? v[q] : 0.0;  // not what lies past the row
-                }
-            },
-            [&](int i, double (&v)[4]) { sep_load4(vx + i, v); });
-#pragma unroll
-        for (int r = 0; r < 4; r++) sep_lds[(j0 + 4 * r + g) * pitch + c0 + ln] = t[r];
-    }
-    __syncthreads();
-    for (int w = wave; w < mt * nt; w += kSepWaves) {
-        const int m0 = 16 * (w / nt), c0 = 16 * (w % nt);
-        const double *vy = Y.Vi + (long)(m0 + ln) * Y.np;
-        const double *col = sep_lds + c0 + ln;
-        const mfma_acc t = sep_tile(
-            Y.np / 16, [&](int j, double (&v)[4]) { sep_load4(vy + j, v); },
-            [&](int j, double (&v)[4]) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = col[(j + q) * pitch];
-            });
-        const int l = l0 + c0 + ln;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int m = m0 + 4 * r + g;
-            if (l >= d.nx || m >= d.ny) continue;
-            const long q = cidx(d, l, m, k);
-            y[q] = WHAT == SEP_GHOST ? y[q] + t[r] : t[r];
+    const int ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const int k = k0 + blockIdx.y, l0 = blockIdx.x * 16 * nb;
+    const int jt = j1 - j0, mt = Y.np / 16, nt = min(nb, (X.np - l0) / 16);
+    sep_macro<MR, NR>(jt, nt, [&](int m, int n) {
+        long q0[MR];
+        const double *vx[NR];
+        const uint16_t *in[MR];
+        for (int r = 0; r < MR; r++) {
+            const int j = min(16 * (j0 + m + r) + ln, d.ny - 1);
+            q0[r] = cidx(d, 16 * i0 + 2 * g, j, k);
+            in[r] = mask + ((long)k * d.ny + j) * (X.np / 16) + i0;
         }
-    }
+        for (int s = 0; s < NR; s++) vx[s] = X.Vi + (long)(l0 + 16 * min(n + s, nt - 1) + ln) * X.np + 16 * i0 + 2 * g;
+        mfma_acc t[MR][NR];
+        sep_tiles<MR, NR>(
+            i1 - i0,
+            [&](int r, int i, double (&v)[4]) {
+                sep_row(b + q0[r] + i, v);
+                const unsigned f = WHAT != SEP_ALL ? (unsigned)in[r][i >> 4] >> 2 * g : 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++)  // not what lies past the row, or outside the mask
+                    if (WHAT == SEP_ALL ? 16 * i0 + i + sep_k(g, e) >= d.nx : !(f >> sep_k(0, e) & 1)) v[e] = 0.0;
+            },
+            [&](int s, int i, double (&v)[4]) { sep_row(vx[s] + i, v); }, t);
+#pragma unroll
+        for (int r = 0; r < MR; r++)
+#pragma unroll
+            for (int s = 0; s < NR; s++)
+                if (m + r < jt && n + s < nt)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        sep_lds[(16 * (m + r) + 4 * e + g) * pitch + 16 * (n + s) + ln] = t[r][s][e];
+    });
+    __syncthreads();
+    sep_macro<MR, NR>(mt, nt, [&](int m, int n) {
+        const double *vy[MR], *col[NR];
+        for (int r = 0; r < MR; r++) vy[r] = Y.Vi + (long)(16 * min(m + r, mt - 1) + ln) * Y.np + 16 * j0 + 2 * g;
+        for (int s = 0; s < NR; s++) col[s] = sep_lds + 16 * min(n + s, nt - 1) + ln;
+        mfma_acc t[MR][NR];
+        sep_tiles<MR, NR>(
+            jt, [&](int r, int j, double (&v)[4]) { sep_row(vy[r] + j, v); },
+            [&](int s, int j, double (&v)[4]) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = col[s][(j + sep_k(g, e)) * pitch];
+            },
+            t);
+#pragma unroll
+        for (int r = 0; r < MR; r++)
+#pragma unroll
+            for (int s = 0; s < NR; s++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int row = 16 * (m + r) + 4 * e + g, l = l0 + 16 * (n + s) + ln;
+                    if (n + s >= nt || l >= d.nx || row >= d.ny) continue;
+                    const long q = cidx(d, l, row, k);
+                    y[q] = WHAT == SEP_ADD ? y[q] + t[r][s][e] : t[r][s][e];
+                }
+    });
 }
 
 // w(l, m, k) = sum_n V_z[k][n] u(l, m, n), u = (sum_k Vi_z[n][k] y(l, m, k)) /
@@ -128,73 +175,97 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableAxis X,
 // partial gets the block's share of the solution at that cell.
 // Planes k of the tiles [t0, t1) are written. UNIT: y is a unit vector in z, 1
 // in plane ku for every l and m.
-template <bool UNIT>
-__global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, const double *y, double *w_out, int nb,
+template <bool UNIT, int MR, int NR>
+__global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, const double *y, double *w_out, int nb, int pitch,
                                                        int t0, int t1, int ku, double *partial) {
     extern __shared__ double sep_lds[];
-    __shared__ double first[kSepThreads / 64 + 1];
+    __shared__ double first[kSepWaves];
     const SeparableAxis &Z = S.ax[2];
     const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-    const int m = blockIdx.y, l0 = blockIdx.x * 16 * nb, pitch = 16 * nb + kSepPad;
+    const int m = blockIdx.y, l0 = blockIdx.x * 16 * nb;
     const int zt = Z.np / 16, nt = min(nb, (S.ax[0].np - l0) / 16);
     double shift = 0;  // the added multiple of the unit vector
     if (S.pinned) {
         double z = 0;
-        for (int k = threadIdx.x; k < d.nz; k += kSepThreads) z += Z.Vi[k] * y[cidx(d, 0, 0, k)];
+        for (int k = threadIdx.x; k < d.nz; k += blockDim.x) z += Z.Vi[k] * y[cidx(d, 0, 0, k)];
         for (int o = 32; o > 0; o >>= 1) z += __shfl_down(z, o, 64);
         if ((threadIdx.x & 63) == 0) first[wave] = z;
         __syncthreads();
         z = 0;
-        for (int q = 0; q < kSepWaves; q++) z += first[q];
+        for (int q = 0; q < sep_waves(); q++) z += first[q];
         shift = -z / (S.ax[0].Vi[0] * S.ax[1].Vi[0] * Z.Vi[0]);
     }
     const double lm = S.ax[1].lam[m];
     const double um = S.pinned ? S.ax[1].Vi[(long)m * S.ax[1].np] * shift : 0.0;
-    for (int w = wave; w < zt * nt; w += kSepWaves) {
-        const int n0 = 16 * (w / nt), c0 = 16 * (w % nt);
-        const int l = min(l0 + c0 + ln, d.nx - 1);
-        const double *vz = Z.Vi + (long)(n0 + ln) * Z.np, *col = y + cidx(d, l, m, 0);
-        mfma_acc t;
-        if (UNIT)
-            for (int r = 0; r < 4; r++) t[r] = Z.Vi[(long)(n0 + 4 * r + g) * Z.np + ku];
-        else t = sep_tile(
-            zt, [&](int k, double (&v)[4]) { sep_load4(vz + k, v); },
-            [&](int k, double (&v)[4]) {
+    sep_macro<MR, NR>(zt, nt, [&](int zr, int n) {
+        const double *vz[MR], *col[NR];
+        for (int r = 0; r < MR; r++) vz[r] = Z.Vi + (long)(16 * min(zr + r, zt - 1) + ln) * Z.np + 2 * g;
+        for (int s = 0; s < NR; s++) col[s] = y + cidx(d, min(l0 + 16 * (n + s) + ln, d.nx - 1), m, 0);
+        mfma_acc t[MR][NR];
+        if constexpr (UNIT) {
+            for (int r = 0; r < MR; r++)
+                for (int s = 0; s < NR; s++)
+                    for (int e = 0; e < 4; e++)
+                        t[r][s][e] = Z.Vi[(long)(16 * min(zr + r, zt - 1) + 4 * e + g) * Z.np + ku];
+        } else {
+            sep_tiles<MR, NR>(
+                zt, [&](int r, int k, double (&v)[4]) { sep_row(vz[r] + k, v); },
+                [&](int s, int k, double (&v)[4]) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = col[min(k + q, d.nz - 1) * d.sz];
-            });
-        const double ll = S.ax[0].lam[l] + lm;
-        const double ul = S.pinned ? S.ax[0].Vi[(long)l * S.ax[0].np] * um : 0.0;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int n = n0 + 4 * r + g;
-            double v = 0;
-            if (n < d.nz) {
-                const double den = ll + Z.lam[n];
-                v = den != 0 ? (t[r] + (S.pinned ? ul * Z.Vi[(long)n * Z.np] : 0.0)) / den : 0.0;
-            }
-            sep_lds[n * pitch + c0 + ln] = v;
+                    for (int e = 0; e < 4; e++) v[e] = col[s][min(k + sep_k(g, e), d.nz - 1) * d.sz];
+                },
+                t);
         }
-    }
+#pragma unroll
+        for (int s = 0; s < NR; s++) {
+            const int l = min(l0 + 16 * (n + s) + ln, d.nx - 1);
+            const double ll = S.ax[0].lam[l] + lm;
+            const double ul = S.pinned ? S.ax[0].Vi[(long)l * S.ax[0].np] * um : 0.0;
+#pragma unroll
+            for (int r = 0; r < MR; r++)
+                if (zr + r < zt && n + s < nt)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int row = 16 * (zr + r) + 4 * e + g;
+                        double v = 0;
+                        if (row < d.nz) {
+                            const double den = ll + Z.lam[row];
+                            v = t[r][s][e];
+                            if (S.pinned) v += ul * Z.Vi[(long)row * Z.np];
+                            v = den != 0 ? v / den : 0.0;
+                        }
+                        sep_lds[row * pitch + 16 * (n + s) + ln] = v;
+                    }
+        }
+    });
     __syncthreads();
     double mine = 0;
-    for (int w = wave; w < (t1 - t0) * nt; w += kSepWaves) {
-        const int k0 = 16 * (t0 + w / nt), c0 = 16 * (w % nt);
-        const double *vz = Z.V + (long)(k0 + ln) * Z.np, *col = sep_lds + c0 + ln;
-        const mfma_acc t = sep_tile(
-            zt, [&](int n, double (&v)[4]) { sep_load4(vz + n, v); },
-            [&](int n, double (&v)[4]) {
+    sep_macro<MR, NR>(t1 - t0, nt, [&](int zr, int n) {
+        const double *vz[MR], *col[NR];
+        for (int r = 0; r < MR; r++) vz[r] = Z.V + (long)(16 * min(t0 + zr + r, t1 - 1) + ln) * Z.np + 2 * g;
+        for (int s = 0; s < NR; s++) col[s] = sep_lds + 16 * min(n + s, nt - 1) + ln;
+        mfma_acc t[MR][NR];
+        sep_tiles<MR, NR>(
+            zt, [&](int r, int k, double (&v)[4]) { sep_row(vz[r] + k, v); },
+            [&](int s, int k, double (&v)[4]) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = col[(n + q) * pitch];
-            });
-        const int l = l0 + c0 + ln;
+                for (int e = 0; e < 4; e++) v[e] = col[s][(k + sep_k(g, e)) * pitch];
+            },
+            t);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int k = k0 + 4 * r + g;
-            if (l < d.nx && k < d.nz) w_out[cidx(d, l, m, k)] = t[r];
+        for (int s = 0; s < NR; s++) {
+            const int l = l0 + 16 * (n + s) + ln;
+            if (n + s >= nt || l >= d.nx) continue;
+#pragma unroll
+            for (int r = 0; r < MR; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int k = 16 * (t0 + zr + r) + 4 * e + g;
+                    if (t0 + zr + r < t1 && k < d.nz) w_out[cidx(d, l, m, k)] = t[r][s][e];
+                }
+            if (S.pinned && t0 + zr == 0 && g == 0) mine += S.ax[0].V[l] * t[0][s][0];
         }
-        if (S.pinned && k0 == 0 && g == 0 && l < d.nx) mine += S.ax[0].V[l] * t[0];
-    }
+    });
     if (!S.pinned) return;
     mine *= S.ax[1].V[m];
     for (int o = 32; o > 0; o >>= 1) mine += __shfl_down(mine, o, 64);
@@ -203,80 +274,102 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, c
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0;
-        for (int q = 0; q < kSepWaves; q++) s += first[q];
+        for (int q = 0; q < sep_waves(); q++) s += first[q];
         partial[blockIdx.x + (long)gridDim.x * m] = s;
     }
 }
 
-// x(i, j, k) = or += sum_lm V_x[i][l] V_y[j][m] w(l, m, k) for all i, the rows j
-// of a block of 16 nb from tile t0 (of the tiles below t1) and plane k = k0 +
-// blockIdx.y. pinned: plus the constant that gives cell (0, 0, 0) its
-// right-hand side (np partial sums of its value). flag: solid cells take b.
+// x(i, j, k) = or += sum_lm V_x[i][l] V_y[j][m] w(l, m, k) for the rows j of a
+// block of 16 nb from tile t0 (of the tiles below t1) and plane k = k0 +
+// blockIdx.y; columns of the tiles [i0, i1). pinned: plus the constant that
+// gives cell (0, 0, 0) its right-hand side (np partial sums of its value).
+// flag: solid cells take b.
+template <int MR, int NR>
 __global__ void __launch_bounds__(kSepThreads) k_sep_back(Dims d, SeparableAxis X, SeparableAxis Y, const double *w_in,
-                                                          double *x, int nb, int t0, int t1, int k0, int add,
+                                                          double *x, int nb, int t0, int t1, int i0, int i1, int k0, int add,
                                                           int pinned, const double *b, const uint8_t *flag,
                                                           const double *partial, int np) {
     extern __shared__ double sep_lds[];
-    __shared__ double first[kSepThreads / 64];
+    __shared__ double first[kSepWaves];
     const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-    const int k = k0 + blockIdx.y, j0 = 16 * (t0 + blockIdx.x * nb), pitch = X.np + kSepPad;
+    const int k = k0 + blockIdx.y, j0 = 16 * (t0 + blockIdx.x * nb), pitch = X.np + kSepPadRow;
     const int xt = X.np / 16, jt = min(nb, t1 - j0 / 16);
     double base = 0;
     if (pinned) {
         double s = 0;
-        for (int q = threadIdx.x; q < np; q += kSepThreads) s += partial[q];
+        for (int q = threadIdx.x; q < np; q += blockDim.x) s += partial[q];
         for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
         if ((threadIdx.x & 63) == 0) first[wave] = s;
     }
-    for (int w = wave; w < jt * xt; w += kSepWaves) {
-        const int r0 = 16 * (w / xt), c0 = 16 * (w % xt);
-        const int l = min(c0 + ln, d.nx - 1);
-        const double *vy = Y.V + (long)(j0 + r0 + ln) * Y.np, *col = w_in + cidx(d, l, 0, k);
-        const mfma_acc t = sep_tile(
-            Y.np / 16, [&](int m, double (&v)[4]) { sep_load4(vy + m, v); },
-            [&](int m, double (&v)[4]) {
+    sep_macro<MR, NR>(jt, xt, [&](int jr, int n) {
+        const double *vy[MR], *col[NR];
+        for (int r = 0; r < MR; r++) vy[r] = Y.V + (long)(j0 + 16 * min(jr + r, jt - 1) + ln) * Y.np + 2 * g;
+        for (int s = 0; s < NR; s++) col[s] = w_in + cidx(d, min(16 * (n + s) + ln, d.nx - 1), 0, k);
+        mfma_acc t[MR][NR];
+        sep_tiles<MR, NR>(
+            Y.np / 16, [&](int r, int m, double (&v)[4]) { sep_row(vy[r] + m, v); },
+            [&](int s, int m, double (&v)[4]) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = col[(long)min(m + q, d.ny - 1) * d.sy];
-            });
+                for (int e = 0; e < 4; e++) v[e] = col[s][(long)min(m + sep_k(g, e), d.ny - 1) * d.sy];
+            },
+            t);
 #pragma unroll
-        for (int r = 0; r < 4; r++) sep_lds[(r0 + 4 * r + g) * pitch + c0 + ln] = t[r];
-    }
+        for (int r = 0; r < MR; r++)
+#pragma unroll
+            for (int s = 0; s < NR; s++)
+                if (jr + r < jt && n + s < xt)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        sep_lds[(16 * (jr + r) + 4 * e + g) * pitch + 16 * (n + s) + ln] = t[r][s][e];
+    });
     __syncthreads();
     if (pinned) {
         double s = 0;
-        for (int q = 0; q < kSepWaves; q++) s += first[q];
+        for (int q = 0; q < sep_waves(); q++) s += first[q];
         base = b[cidx(d, 0, 0, 0)] - s;
     }
-    for (int w = wave; w < jt * xt; w += kSepWaves) {
-        const int r0 = 16 * (w / xt), i0 = 16 * (w % xt);
-        const double *vx = X.V + (long)(i0 + ln) * X.np, *row = sep_lds + (r0 + ln) * pitch;
-        const mfma_acc t = sep_tile(
-            xt, [&](int l, double (&v)[4]) { sep_load4(row + l, v); },
-            [&](int l, double (&v)[4]) { sep_load4(vx + l, v); });
-        const int i = i0 + ln;
+    sep_macro<MR, NR>(jt, i1 - i0, [&](int jr, int n) {
+        const double *vx[NR], *row[MR];
+        for (int r = 0; r < MR; r++) row[r] = sep_lds + (16 * min(jr + r, jt - 1) + ln) * pitch + 2 * g;
+        for (int s = 0; s < NR; s++) vx[s] = X.V + (long)(16 * min(i0 + n + s, i1 - 1) + ln) * X.np + 2 * g;
+        mfma_acc t[MR][NR];
+        sep_tiles<MR, NR>(
+            xt, [&](int r, int l, double (&v)[4]) { sep_row(row[r] + l, v); },
+            [&](int s, int l, double (&v)[4]) { sep_row(vx[s] + l, v); }, t);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j = j0 + r0 + 4 * r + g;
-            if (i >= d.nx || j >= d.ny) continue;
-            const long q = cidx(d, i, j, k);
-            const double v = flag && flag[q] == F_SOLID ? b[q] : t[r] + base;
-            x[q] = add ? x[q] + v : v;
-        }
-    }
+        for (int r = 0; r < MR; r++)
+#pragma unroll
+            for (int s = 0; s < NR; s++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int i = 16 * (i0 + n + s) + ln, j = j0 + 16 * (jr + r) + 4 * e + g;
+                    if (jr + r >= jt || i0 + n + s >= i1 || i >= d.nx || j >= d.ny) continue;
+                    const long q = cidx(d, i, j, k);
+                    const double v = flag && flag[q] == F_SOLID ? b[q] : t[r][s][e] + base;
+                    x[q] = add ? x[q] + v : v;
+                }
+    });
 }
 
 static int sep_pad16(int n) { return (n + 15) / 16 * 16; }
 
-// LDS of a block of nb tiles of 16 beside a padded axis of np (its larger
-// layout: np rows of 16 nb, or 16 nb rows of np)
-static size_t sep_lds_bytes(int nb, int np) {
-    return std::max((size_t)np * (16 * nb + kSepPad), (size_t)16 * nb * (np + kSepPad)) * sizeof(double);
+// LDS of a workgroup: two fit a compute unit (with 64 KB the last kernel takes
+// 103 us at 256 x 128 x 128 instead of 71: two row tiles need 66 KB)
+constexpr size_t kSepLds = 80 * 1024;
+
+// Row pitch of a column-read tile of nb tiles of 16 beside a padded axis of np
+// (less padding on the longest axes), and the LDS of a block in its larger
+// layout: np rows of 16 nb, or 16 nb rows of np
+static int sep_pitch(int nb, int np) {
+    return 16 * nb + (np * (16 * nb + kSepPadCol) * sizeof(double) <= kSepLds ? kSepPadCol : kSepPadCol / 2);
 }
-constexpr size_t kSepLds = 64 * 1024;
+static size_t sep_lds_bytes(int nb, int np) {
+    return std::max((size_t)np * sep_pitch(nb, np), (size_t)16 * nb * (np + kSepPadRow)) * sizeof(double);
+}
 
 // Tiles of 16 per block along an axis of `tiles` tiles beside `other` blocks
 // of the grid: as many as leave a workgroup for every compute unit and fit
-// the LDS, up to four (the matrices are then read by fewer workgroups).
+// the LDS, up to four (the operands are then read by fewer workgroups).
 static int sep_block(int tiles, int other, int np) {
     for (int nb = 4; nb > 1; nb /= 2)
         if (tiles >= nb && (long)((tiles + nb - 1) / nb) * other >= 256 && sep_lds_bytes(nb, np) <= kSepLds) return nb;
@@ -289,13 +382,35 @@ bool separable_fits(const int n[3]) {
 
 long separable_partials(const Dims &d) { return (long)(sep_pad16(d.nx) / 16) * d.ny; }
 
+// Calls f with the macro tile for mt x nt tiles per workgroup and the threads:
+// 2 x 2 where that leaves one for each of four waves, else 2 tiles along the
+// longer side (rows: the first two kernels, columns: the last), else 1 x 1;
+// eight waves where there are macro tiles for them and the grid alone does not
+// fill the chip. Last kernel, canopy 160 x 80 x 48: 28 us with 1 x 1 and four
+// waves, 19 with 1 x 2 and eight.
+template <int N> using SepInt = std::integral_constant<int, N>;
+template <typename F>
+static void sep_shape(int mt, int nt, bool rows, long groups, F f) {
+    const int m2 = (mt + 1) / 2, n2 = (nt + 1) / 2;
+    const auto threads = [&](int tiles) { return groups < 1024 && tiles > 4 ? 512 : 256; };
+    if (mt > 1 && nt > 1 && m2 * n2 >= 4) f(SepInt<2>(), SepInt<2>(), threads(m2 * n2));
+    else if (rows && m2 * nt >= 3) f(SepInt<2>(), SepInt<1>(), threads(m2 * nt));
+    else if (!rows && mt * n2 >= 3) f(SepInt<1>(), SepInt<2>(), threads(mt * n2));
+    else f(SepInt<1>(), SepInt<1>(), threads(mt * nt));
+}
+
+struct SepRange { int i0, i1, j0, j1, k0, k1; };  // cells; i and j in whole tiles of 16
+
 template <int WHAT>
-static void sep_xy(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, const uint8_t *flag,
-                   double *y, int k0, int k1) {
-    const int xt = S.ax[0].np / 16, nb = sep_block(xt, k1 - k0, S.ax[1].np);
-    hipLaunchKernelGGL((k_sep_xy<WHAT>), dim3((xt + nb - 1) / nb, k1 - k0), dim3(kSepThreads),
-                       (size_t)S.ax[1].np * (16 * nb + kSepPad) * sizeof(double), st, d, S.ax[0], S.ax[1], b, flag, y,
-                       nb, k0);
+static void sep_xy(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, const uint16_t *mask,
+                   double *y, const SepRange &in) {
+    const int xt = S.ax[0].np / 16, nk = in.k1 - in.k0, nb = sep_block(xt, nk, S.ax[1].np), gx = (xt + nb - 1) / nb;
+    const int pitch = sep_pitch(nb, S.ax[1].np);
+    sep_shape(S.ax[1].np / 16, nb, true, (long)gx * nk, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_xy<WHAT, mr(), nr()>), dim3(gx, nk), dim3(threads),
+                           (size_t)S.ax[1].np * pitch * sizeof(double), st, d, S.ax[0], S.ax[1], b, mask, y, nb, pitch,
+                           in.k0, in.i0 / 16, (in.i1 + 15) / 16, in.j0 / 16, (in.j1 + 15) / 16);
+    });
 }
 
 // planes [k0, k1) (whole tiles of 16); returns the number of partial sums
@@ -303,26 +418,34 @@ template <bool UNIT>
 static int sep_z(hipStream_t st, const Dims &d, const SeparableSys &S, const double *y, double *w, int k0, int k1,
                  int ku, double *partial) {
     const int xt = S.ax[0].np / 16, nb = sep_block(xt, d.ny, S.ax[2].np), g = (xt + nb - 1) / nb;
-    hipLaunchKernelGGL((k_sep_z<UNIT>), dim3(g, d.ny), dim3(kSepThreads),
-                       (size_t)S.ax[2].np * (16 * nb + kSepPad) * sizeof(double), st, d, S, y, w, nb, k0 / 16,
-                       (k1 + 15) / 16, ku, partial);
+    const int pitch = sep_pitch(nb, S.ax[2].np);
+    sep_shape(S.ax[2].np / 16, nb, true, (long)g * d.ny, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_z<UNIT, mr(), nr()>), dim3(g, d.ny), dim3(threads),
+                           (size_t)S.ax[2].np * pitch * sizeof(double), st, d, S, y, w, nb, pitch, k0 / 16,
+                           (k1 + 15) / 16, ku, partial);
+    });
     return g * d.ny;
 }
 
-// rows [j0, j1) (whole tiles of 16) of the planes [k0, k1)
-static void sep_back(hipStream_t st, const Dims &d, const SeparableSys &S, const double *w, double *x, int j0, int j1,
-                     int k0, int k1, bool add, const double *b, const uint8_t *flag, const double *partial, int np) {
-    const int t0 = j0 / 16, t1 = (j1 + 15) / 16, nb = sep_block(t1 - t0, k1 - k0, S.ax[0].np);
-    hipLaunchKernelGGL(k_sep_back, dim3((t1 - t0 + nb - 1) / nb, k1 - k0), dim3(kSepThreads),
-                       (size_t)16 * nb * (S.ax[0].np + kSepPad) * sizeof(double), st, d, S.ax[0], S.ax[1], w, x, nb,
-                       t0, t1, k0, add ? 1 : 0, partial ? S.pinned : 0, b, flag, partial, np);
+static void sep_back(hipStream_t st, const Dims &d, const SeparableSys &S, const double *w, double *x,
+                     const SepRange &o, bool add, const double *b, const uint8_t *flag, const double *partial,
+                     int np) {
+    const int t0 = o.j0 / 16, t1 = (o.j1 + 15) / 16, nk = o.k1 - o.k0, nb = sep_block(t1 - t0, nk, S.ax[0].np);
+    const int gy = (t1 - t0 + nb - 1) / nb;
+    sep_shape(nb, S.ax[0].np / 16, false, (long)gy * nk, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_back<mr(), nr()>), dim3(gy, nk), dim3(threads),
+                           (size_t)16 * nb * (S.ax[0].np + kSepPadRow) * sizeof(double), st, d, S.ax[0], S.ax[1], w,
+                           x, nb, t0, t1, o.i0 / 16, (o.i1 + 15) / 16, o.k0, add ? 1 : 0, partial ? S.pinned : 0, b,
+                           flag, partial, np);
+    });
 }
 
 void launch_separable(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, double *s1, double *s2,
                       double *x, bool add, double *partial) {
-    sep_xy<SEP_ALL>(st, d, S, b, nullptr, s1, 0, d.nz);
+    const SepRange all{0, d.nx, 0, d.ny, 0, d.nz};
+    sep_xy<SEP_ALL>(st, d, S, b, nullptr, s1, all);
     const int np = sep_z<false>(st, d, S, s1, s2, 0, d.nz, 0, partial);
-    sep_back(st, d, S, s2, x, 0, d.ny, 0, d.nz, add, b, nullptr, partial, np);
+    sep_back(st, d, S, s2, x, all, add, b, nullptr, partial, np);
 }
 
 // ---------------------------------------------------------------------------
@@ -331,7 +454,7 @@ void launch_separable(hipStream_t st, const Dims &d, const SeparableSys &S, cons
 // One solve is two passes of the transforms, the first one's last two limited
 // to the planes and rows the ghost rows look at, and one product with the
 // inverse of the ghost rows' matrix: 256 x 128 x 128 with 3568 ghost cells
-// 0.63 ms, of it 32 us for the product (102 MB); BiCGSTAB with multigrid
+// 0.34 ms, of it 32 us for the product (102 MB); BiCGSTAB with multigrid
 // cycles took 7 iterations of 0.95 ms.
 // t_g = b_g - (R y)_g
 __global__ void k_cap_rhs(GhostRows<double> G, const double *b, const double *y, double *t) {
@@ -369,18 +492,21 @@ void launch_separable_body(hipStream_t st, const Dims &d, const SeparableSys &S,
                            const double *b, double *s1, double *s2, double *s3, double *x, bool add) {
     // A^-1 b_fluid where the ghost rows look; then the ghost cells' part is
     // added to its transform
-    sep_xy<SEP_FLUID>(st, d, S, b, B.flag, s1, 0, d.nz);
-    sep_z<false>(st, d, S, s1, s2, B.z0, B.z1, 0, nullptr);
-    sep_back(st, d, S, s2, s3, B.y0, B.y1, B.z0, B.z1, false, b, nullptr, nullptr, 0);
+    const SepRange all{0, d.nx, 0, d.ny, 0, d.nz};
+    const SepRange look{B.look.lo[0], B.look.hi[0], B.look.lo[1], B.look.hi[1], B.look.lo[2], B.look.hi[2]};
+    const SepRange cells{B.cells.lo[0], B.cells.hi[0], B.cells.lo[1], B.cells.hi[1], B.cells.lo[2], B.cells.hi[2]};
+    sep_xy<SEP_MASK>(st, d, S, b, B.fluid, s1, all);
+    sep_z<false>(st, d, S, s1, s2, look.k0, look.k1, 0, nullptr);
+    sep_back(st, d, S, s2, s3, look, false, b, nullptr, nullptr, 0);
     const int ng = B.G.ng;
     hipLaunchKernelGGL(k_cap_rhs, dim3((ng + 63) / 64), dim3(64), 0, st, B.G, b, s3, B.t);
     if (B.inv64)
         hipLaunchKernelGGL((k_cap_apply<double>), dim3((ng + 3) / 4), dim3(256), 0, st, B.G, B.inv64, B.ld, B.t, s3);
     else
         hipLaunchKernelGGL((k_cap_apply<float>), dim3((ng + 3) / 4), dim3(256), 0, st, B.G, B.inv32, B.ld, B.t, s3);
-    sep_xy<SEP_GHOST>(st, d, S, s3, B.flag, s1, B.g0, B.g1);
+    sep_xy<SEP_ADD>(st, d, S, s3, B.ghost, s1, cells);
     sep_z<false>(st, d, S, s1, s2, 0, d.nz, 0, nullptr);
-    sep_back(st, d, S, s2, x, 0, d.ny, 0, d.nz, add, b, B.flag, nullptr, 0);
+    sep_back(st, d, S, s2, x, all, add, b, B.flag, nullptr, 0);
 }
 
 // A^-1 e_c in the box, for the unit vectors of the ghost cells c = src0 +
@@ -391,43 +517,52 @@ __global__ void __launch_bounds__(kSepThreads) k_cap_green(Dims d, SeparableAxis
                                                            const int3 *src, int src0, GreenBox box,
                                                            GreenScratch out) {
     extern __shared__ double sep_lds[];
-    const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-    const int k = box.lo[2] + blockIdx.y, j0 = 16 * (box.lo[1] / 16 + blockIdx.x), pitch = X.np + kSepPad;
+    const int ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const int k = box.lo[2] + blockIdx.y, j0 = 16 * (box.lo[1] / 16 + blockIdx.x), pitch = X.np + kSepPadRow;
     const int xt = X.np / 16, x0 = box.lo[0] / 16, x1 = (box.hi[0] + 15) / 16;
     const int3 c = src[src0 + blockIdx.z];
     double *fy = sep_lds + 16 * pitch;  // Vi_y[m][j of the source]
-    for (int m = threadIdx.x; m < Y.np; m += kSepThreads) fy[m] = Y.Vi[(long)m * Y.np + c.y];
+    for (int m = threadIdx.x; m < Y.np; m += blockDim.x) fy[m] = Y.Vi[(long)m * Y.np + c.y];
     __syncthreads();
-    for (int w = wave; w < xt; w += kSepWaves) {
-        const int l = min(16 * w + ln, d.nx - 1);
-        const double *vy = Y.V + (long)(j0 + ln) * Y.np, *col = h + cidx(d, l, 0, k);
-        const double fx = X.Vi[(long)l * X.np + c.x];
-        const mfma_acc t = sep_tile(
-            Y.np / 16, [&](int m, double (&v)[4]) { sep_load4(vy + m, v); },
-            [&](int m, double (&v)[4]) {
+    sep_macro<1, 2>(1, xt, [&](int, int n) {
+        const double *vy = Y.V + (long)(j0 + ln) * Y.np + 2 * g, *col[2];
+        for (int s = 0; s < 2; s++) col[s] = h + cidx(d, min(16 * (n + s) + ln, d.nx - 1), 0, k);
+        mfma_acc t[1][2];
+        sep_tiles<1, 2>(
+            Y.np / 16, [&](int, int m, double (&v)[4]) { sep_row(vy + m, v); },
+            [&](int s, int m, double (&v)[4]) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) v[q] = col[(long)min(m + q, d.ny - 1) * d.sy] * fy[m + q];
-            });
+                for (int e = 0; e < 4; e++) {
+                    const int q = m + sep_k(g, e);
+                    v[e] = col[s][(long)min(q, d.ny - 1) * d.sy] * fy[q];
+                }
+            },
+            t);
+        for (int s = 0; s < 2 && n + s < xt; s++) {
+            const int l = 16 * (n + s) + ln;
+            const double fx = X.Vi[(long)l * X.np + c.x];
 #pragma unroll
-        for (int r = 0; r < 4; r++) sep_lds[(4 * r + g) * pitch + 16 * w + ln] = t[r] * fx;
-    }
+            for (int e = 0; e < 4; e++) sep_lds[(4 * e + g) * pitch + l] = t[0][s][e] * fx;
+        }
+    });
     __syncthreads();
     const int bx = box.hi[0] - box.lo[0], by = box.hi[1] - box.lo[1], bz = box.hi[2] - box.lo[2];
     double *o = out.v[blockIdx.z / out.per] + (long)(blockIdx.z % out.per) * bx * by * bz
         + (long)(k - box.lo[2]) * bx * by;
-    for (int w = x0 + wave; w < x1; w += kSepWaves) {
-        const int i = 16 * w + ln;
-        const double *vx = X.V + (long)i * X.np, *row = sep_lds + ln * pitch;
-        const mfma_acc t = sep_tile(
-            xt, [&](int l, double (&v)[4]) { sep_load4(row + l, v); },
-            [&](int l, double (&v)[4]) { sep_load4(vx + l, v); });
+    sep_macro<1, 1>(1, x1 - x0, [&](int, int n) {
+        const int i = 16 * (x0 + n) + ln;
+        const double *vx = X.V + (long)i * X.np + 2 * g, *row = sep_lds + ln * pitch + 2 * g;
+        mfma_acc t[1][1];
+        sep_tiles<1, 1>(
+            xt, [&](int, int l, double (&v)[4]) { sep_row(row + l, v); },
+            [&](int, int l, double (&v)[4]) { sep_row(vx + l, v); }, t);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j = j0 + 4 * r + g;
+        for (int e = 0; e < 4; e++) {
+            const int j = j0 + 4 * e + g;
             if (i >= box.lo[0] && i < box.hi[0] && j >= box.lo[1] && j < box.hi[1])
-                o[(long)(j - box.lo[1]) * bx + i - box.lo[0]] = t[r];
+                o[(long)(j - box.lo[1]) * bx + i - box.lo[0]] = t[0][0][e];
         }
-    }
+    });
 }
 
 // the ghost rows of those columns
@@ -452,8 +587,8 @@ void launch_green_plane(hipStream_t st, const Dims &d, const SeparableSys &S, in
     const int jt = (box.hi[1] + 15) / 16 - box.lo[1] / 16, batch = kGreenVecs * green.per;
     for (int c = 0; c < nsrc; c += batch) {
         const int n = std::min(batch, nsrc - c);
-        hipLaunchKernelGGL(k_cap_green, dim3(jt, box.hi[2] - box.lo[2], n), dim3(kSepThreads),
-                           (16 * (size_t)(S.ax[0].np + kSepPad) + S.ax[1].np) * sizeof(double), st, d, S.ax[0],
+        hipLaunchKernelGGL(k_cap_green, dim3(jt, box.hi[2] - box.lo[2], n), dim3(256),
+                           (16 * (size_t)(S.ax[0].np + kSepPadRow) + S.ax[1].np) * sizeof(double), st, d, S.ax[0],
                            S.ax[1], h, src, c, box, green);
         hipLaunchKernelGGL(k_cap_rows, dim3((G.ng + 255) / 256, n), dim3(256), 0, st, G, loc, src, c, vol, green, out,
                            ld);

@@ -704,10 +704,8 @@ static bool build_capacitance(IBMSolver *s) {
     if (!wide && (s->precision == IBM3D_PREC_FP64 || full / 2 > room || s->dev_bytes + 1.5 * full > all)) return false;
 
     // places of the ghost cells and their stencil points
-    GreenBox box{{d.nx, d.ny, d.nz}, {0, 0, 0}};
+    GreenBox box{{d.nx, d.ny, d.nz}, {0, 0, 0}}, cells = box;
     std::vector<int> at(27 * (size_t)ng, -1);
-    s->cap.g0 = d.nz;
-    s->cap.g1 = 0;
     for (int g = 0; g < ng; g++)
         for (int l = 0; l < 9; l++) {
             const long q = l < 8 ? s->ghosts[g].src[l] : s->ghosts[g].cell;
@@ -719,10 +717,9 @@ static bool build_capacitance(IBMSolver *s) {
                 box.lo[a] = std::min(box.lo[a], id[a]);
                 box.hi[a] = std::max(box.hi[a], id[a] + 1);
                 at[27 * (size_t)g + 3 * l + a] = id[a];
-            }
-            if (l == 8) {
-                s->cap.g0 = std::min(s->cap.g0, id[2]);
-                s->cap.g1 = std::max(s->cap.g1, id[2] + 1);
+                if (l < 8) continue;
+                cells.lo[a] = std::min(cells.lo[a], id[a]);
+                cells.hi[a] = std::max(cells.hi[a], id[a] + 1);
             }
         }
     const long bx = box.hi[0] - box.lo[0], by = box.hi[1] - box.lo[1], bz = box.hi[2] - box.lo[2];
@@ -775,8 +772,20 @@ static bool build_capacitance(IBMSolver *s) {
     s->cap.inv32 = wide ? nullptr : s->cap_inv32.p;
     s->cap.ld = ld;
     s->cap.t = s->cap_t.p;
-    s->cap.y0 = box.lo[1]; s->cap.y1 = box.hi[1];
-    s->cap.z0 = box.lo[2]; s->cap.z1 = box.hi[2];
+    s->cap.look = box;
+    s->cap.cells = cells;
+    const int words = s->sep.ax[0].np / 16;
+    for (int m = 0; m < 2; m++) {
+        std::vector<uint16_t> bits((size_t)words * d.ny * d.nz, 0);
+        for (int k = 0; k < d.nz; k++)
+            for (int j = 0; j < d.ny; j++)
+                for (int i = 0; i < d.nx; i++)
+                    if (s->flag_dev_h[cidx(d, i, j, k)] == (m ? F_GHOST : F_FLUID))
+                        bits[((size_t)k * d.ny + j) * words + i / 16] |= 1 << i % 16;
+        s->cap_mask[m].upload(bits);
+    }
+    s->cap.fluid = s->cap_mask[0].p;
+    s->cap.ghost = s->cap_mask[1].p;
     return true;
 }
 
@@ -785,12 +794,12 @@ static bool build_capacitance(IBMSolver *s) {
 // no body or one that build_capacitance takes, and the solver asked for is the
 // default one (BiCGSTAB with the multigrid preconditioner, no multigrid
 // setting changed). Time per step at tol 1e-12, multigrid / direct: cavity
-// 32^3 1.43 / 0.31 ms, 64^3 (FP64) 2.34 / 0.40, 128^3 5.62 / 1.13, channel
+// 32^3 1.43 / 0.31 ms, 64^3 (FP64) 2.34 / 0.40, 128^3 5.62 / 1.07, channel
 // 64 x 48 x 32 4.85 / 0.29; with a body: sphere 98 x 47 x 51 (FP64) 2.78 /
-// 0.44, 133 x 67 x 61 3.15 / 0.68, 256 x 128 x 128 8.56 / 2.16, canopy 160 x
-// 80 x 48 5.25 / 0.97.
-// The transforms grow as the axis length per cell: at 128^3 they are 163 us
-// of the step. Axes beyond the LDS tiles (400 cells) take the multigrid path.
+// 0.44, 133 x 67 x 61 3.15 / 0.61, 256 x 128 x 128 8.56 / 1.9, canopy 160 x
+// 80 x 48 5.25 / 0.86 (the rest of the step as it was then).
+// The transforms grow as the axis length per cell: at 128^3 they are 100 us
+// of the step. Axes beyond the LDS tiles (512 cells) take the multigrid path.
 void build_separable(IBMSolver *s) {
     s->sep_on = s->cap_on = false;
     if (s->solver_type != SOLVER_BiCGSTAB || s->precond_type != PRECOND_AMG || s->precision == IBM3D_PREC_MIXED

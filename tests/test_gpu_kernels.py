@@ -119,7 +119,7 @@ SEPARABLE_CASES = [
     # remainders of the 16-wide tiles, one to several tiles per workgroup, the
     # smallest boxes, the longest axis whose tile fits the LDS and the next
     ("cavity", (4, 3, 2)), ("cavity", (8, 8, 8)), ("cavity", (17, 16, 15)), ("cavity", (33, 47, 20)),
-    ("cavity", (64, 48, 33)), ("cavity", (130, 36, 65)), ("cavity", (20, 272, 18)), ("cavity", (10, 9, 400)),
+    ("cavity", (9, 10, 512)), ("cavity", (528, 8, 8)), ("cavity", (64, 48, 33)), ("cavity", (130, 36, 65)), ("cavity", (20, 272, 18)), ("cavity", (10, 9, 400)),
     ("cavity", (416, 10, 9)), ("channel", (16, 12, 8)), ("channel", (34, 18, 22)), ("channel", (64, 70, 80)),
     ("pressure", (32, 20, 12)), ("pressure", (49, 33, 18)), ("outflow", (49, 33, 18)),
 ]
