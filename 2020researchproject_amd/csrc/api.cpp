@@ -785,6 +785,7 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
     // them (and memory that the other fields will use) as scratch
     for (auto &v : s->kry.v64) v.alloc(d.ncell);
     build_separable(s);
+    build_separable_momentum(s);
     alloc_fields(s);
     {
         const long ext[3] = {(long)s->Ny * s->Nz, (long)(s->Nx + 4) * s->Nz, (long)(s->Nx + 4) * (s->Ny + 4)};

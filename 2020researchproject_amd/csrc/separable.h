@@ -8,16 +8,17 @@
 
 namespace ibm {
 
-// Spectral form of the system sum_a T_a x = b whose 1-D operators T_a (after
-// the boundary folds) are symmetric in the scalar product of the cell widths:
-// T_a = V diag(lam) Vi, Vi V = I. Matrices are row-major, padded with zeros to
-// a multiple of 16 on both sides; lam is ascending.
+// Spectral form of the system (c0 + sum_a T_a) x = b whose 1-D operators T_a
+// (after the boundary folds) are symmetric in a scalar product with positive
+// weights: T_a = V diag(lam) Vi, Vi V = I. Matrices are row-major, padded with
+// zeros to a multiple of 16 on both sides; lam is ascending.
 struct SeparableAxis {
     const double *V, *Vi, *lam;
     int n, np;
 };
 struct SeparableSys {
     SeparableAxis ax[3];
+    double c0;   // the operator is c0 + the sum of the three
     int pinned;  // the row of cell (0, 0, 0) is x = b; the problem is otherwise singular
 };
 
@@ -42,10 +43,11 @@ struct SeparableBody {
 };
 
 // Host: eigenvalues (ascending) and matrices of one axis from its folded
-// coefficients cm, cp, dm, dp (n each) and cell widths; false when the axis
-// has no such form (a periodic axis that is not uniform).
-bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], const double *width,
-                    std::vector<double> &V, std::vector<double> &Vi, std::vector<double> &lam);
+// coefficients cm, cp, dm, dp (n each); false when the axis has no such form (a
+// periodic axis that is not uniform, an extrapolated outlet that couples the
+// wrong way).
+bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], std::vector<double> &V,
+                    std::vector<double> &Vi, std::vector<double> &lam);
 
 // x = A^-1 b (add: x += A^-1 b) up to rounding, all in the padded layout d;
 // s1, s2: scratch vectors of that layout, partial: separable_partials doubles
@@ -53,7 +55,17 @@ bool separable_fits(const int n[3]);  // the axes fit the kernels' LDS tiles
 long separable_partials(const Dims &d);
 void launch_separable(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, double *s1, double *s2,
                       double *x, bool add, double *partial);
-// the same with a body (not pinned); s3: a third scratch vector. Solid cells
+// n systems of one shape at once (not pinned): x[c] = A_c^-1 b[c]; s1, s2: n
+// scratch vectors each
+constexpr int kSepBatch = 3;
+struct SeparableBatch {
+    SeparableSys S[kSepBatch];
+    const double *in[kSepBatch];
+    double *out[kSepBatch];
+};
+void launch_separable_batch(hipStream_t st, const Dims &d, int n, const SeparableSys *S, const double *const *b,
+                            double *const *s1, double *const *s2, double *const *x);
+// launch_separable with a body (not pinned); s3: a third scratch vector. Solid cells
 // get x = b (+= b).
 void launch_separable_body(hipStream_t st, const Dims &d, const SeparableSys &S, const SeparableBody &B,
                            const double *b, double *s1, double *s2, double *s3, double *x, bool add);

@@ -103,10 +103,12 @@ enum { SEP_ALL, SEP_MASK, SEP_ADD };
 // of 16 nb and all m: plane k = k0 + blockIdx.y; i and j over the tiles
 // [i0, i1) and [j0, j1) (b is 0 elsewhere)
 template <int WHAT, int MR, int NR>
-__global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableAxis X, SeparableAxis Y, const double *b,
-                                                        const uint16_t *mask, double *y, int nb, int pitch, int k0,
-                                                        int i0, int i1, int j0, int j1) {
+__global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableBatch B, const uint16_t *mask, int nb,
+                                                        int pitch, int k0, int i0, int i1, int j0, int j1) {
     extern __shared__ double sep_lds[];
+    const SeparableAxis &X = B.S[blockIdx.z].ax[0], &Y = B.S[blockIdx.z].ax[1];
+    const double *b = B.in[blockIdx.z];
+    double *y = B.out[blockIdx.z];
     const int ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
     const int k = k0 + blockIdx.y, l0 = blockIdx.x * 16 * nb;
     const int jt = j1 - j0, mt = Y.np / 16, nt = min(nb, (X.np - l0) / 16);
@@ -168,7 +170,7 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableAxis X,
 }
 
 // w(l, m, k) = sum_n V_z[k][n] u(l, m, n), u = (sum_k Vi_z[n][k] y(l, m, k)) /
-// (lam_l + lam_m + lam_n), for one row m = blockIdx.y and a block of 16 nb l.
+// (c0 + lam_l + lam_m + lam_n), for one row m = blockIdx.y and a block of 16 nb l.
 // pinned: b is changed at cell (0, 0, 0) so that the singular problem has a
 // solution (the other rows do not see that row), by the multiple of its unit
 // vector that takes out the zero mode, and the zero mode of the solution is 0;
@@ -176,10 +178,13 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_xy(Dims d, SeparableAxis X,
 // Planes k of the tiles [t0, t1) are written. UNIT: y is a unit vector in z, 1
 // in plane ku for every l and m.
 template <bool UNIT, int MR, int NR>
-__global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, const double *y, double *w_out, int nb, int pitch,
-                                                       int t0, int t1, int ku, double *partial) {
+__global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableBatch B, int nb, int pitch, int t0, int t1,
+                                                       int ku, double *partial) {
     extern __shared__ double sep_lds[];
     __shared__ double first[kSepWaves];
+    const SeparableSys &S = B.S[blockIdx.z];
+    const double *y = B.in[blockIdx.z];
+    double *w_out = B.out[blockIdx.z];
     const SeparableAxis &Z = S.ax[2];
     const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
     const int m = blockIdx.y, l0 = blockIdx.x * 16 * nb;
@@ -195,7 +200,7 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, c
         for (int q = 0; q < sep_waves(); q++) z += first[q];
         shift = -z / (S.ax[0].Vi[0] * S.ax[1].Vi[0] * Z.Vi[0]);
     }
-    const double lm = S.ax[1].lam[m];
+    const double lm = S.c0 + S.ax[1].lam[m];
     const double um = S.pinned ? S.ax[1].Vi[(long)m * S.ax[1].np] * shift : 0.0;
     sep_macro<MR, NR>(zt, nt, [&](int zr, int n) {
         const double *vz[MR], *col[NR];
@@ -285,12 +290,14 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_z(Dims d, SeparableSys S, c
 // gives cell (0, 0, 0) its right-hand side (np partial sums of its value).
 // flag: solid cells take b.
 template <int MR, int NR>
-__global__ void __launch_bounds__(kSepThreads) k_sep_back(Dims d, SeparableAxis X, SeparableAxis Y, const double *w_in,
-                                                          double *x, int nb, int t0, int t1, int i0, int i1, int k0, int add,
-                                                          int pinned, const double *b, const uint8_t *flag,
-                                                          const double *partial, int np) {
+__global__ void __launch_bounds__(kSepThreads) k_sep_back(Dims d, SeparableBatch B, int nb, int t0, int t1, int i0, int i1,
+                                                          int k0, int add, int pinned, const double *b,
+                                                          const uint8_t *flag, const double *partial, int np) {
     extern __shared__ double sep_lds[];
     __shared__ double first[kSepWaves];
+    const SeparableAxis &X = B.S[blockIdx.z].ax[0], &Y = B.S[blockIdx.z].ax[1];
+    const double *w_in = B.in[blockIdx.z];
+    double *x = B.out[blockIdx.z];
     const int wave = threadIdx.x >> 6, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
     const int k = k0 + blockIdx.y, j0 = 16 * (t0 + blockIdx.x * nb), pitch = X.np + kSepPadRow;
     const int xt = X.np / 16, jt = min(nb, t1 - j0 / 16);
@@ -402,50 +409,64 @@ static void sep_shape(int mt, int nt, bool rows, long groups, F f) {
 struct SepRange { int i0, i1, j0, j1, k0, k1; };  // cells; i and j in whole tiles of 16
 
 template <int WHAT>
-static void sep_xy(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, const uint16_t *mask,
-                   double *y, const SepRange &in) {
-    const int xt = S.ax[0].np / 16, nk = in.k1 - in.k0, nb = sep_block(xt, nk, S.ax[1].np), gx = (xt + nb - 1) / nb;
-    const int pitch = sep_pitch(nb, S.ax[1].np);
-    sep_shape(S.ax[1].np / 16, nb, true, (long)gx * nk, [&](auto mr, auto nr, int threads) {
-        hipLaunchKernelGGL((k_sep_xy<WHAT, mr(), nr()>), dim3(gx, nk), dim3(threads),
-                           (size_t)S.ax[1].np * pitch * sizeof(double), st, d, S.ax[0], S.ax[1], b, mask, y, nb, pitch,
-                           in.k0, in.i0 / 16, (in.i1 + 15) / 16, in.j0 / 16, (in.j1 + 15) / 16);
+static void sep_xy(hipStream_t st, const Dims &d, int n, const SeparableBatch &B, const uint16_t *mask,
+                   const SepRange &in) {
+    const int xt = B.S[0].ax[0].np / 16, np = B.S[0].ax[1].np, nk = in.k1 - in.k0;
+    const int nb = sep_block(xt, nk * n, np), gx = (xt + nb - 1) / nb, pitch = sep_pitch(nb, np);
+    sep_shape(np / 16, nb, true, (long)gx * nk * n, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_xy<WHAT, mr(), nr()>), dim3(gx, nk, n), dim3(threads),
+                           (size_t)np * pitch * sizeof(double), st, d, B, mask, nb, pitch, in.k0, in.i0 / 16,
+                           (in.i1 + 15) / 16, in.j0 / 16, (in.j1 + 15) / 16);
     });
 }
 
 // planes [k0, k1) (whole tiles of 16); returns the number of partial sums
 template <bool UNIT>
-static int sep_z(hipStream_t st, const Dims &d, const SeparableSys &S, const double *y, double *w, int k0, int k1,
-                 int ku, double *partial) {
-    const int xt = S.ax[0].np / 16, nb = sep_block(xt, d.ny, S.ax[2].np), g = (xt + nb - 1) / nb;
-    const int pitch = sep_pitch(nb, S.ax[2].np);
-    sep_shape(S.ax[2].np / 16, nb, true, (long)g * d.ny, [&](auto mr, auto nr, int threads) {
-        hipLaunchKernelGGL((k_sep_z<UNIT, mr(), nr()>), dim3(g, d.ny), dim3(threads),
-                           (size_t)S.ax[2].np * pitch * sizeof(double), st, d, S, y, w, nb, pitch, k0 / 16,
-                           (k1 + 15) / 16, ku, partial);
+static int sep_z(hipStream_t st, const Dims &d, int n, const SeparableBatch &B, int k0, int k1, int ku,
+                 double *partial) {
+    const int xt = B.S[0].ax[0].np / 16, np = B.S[0].ax[2].np;
+    const int nb = sep_block(xt, d.ny * n, np), g = (xt + nb - 1) / nb, pitch = sep_pitch(nb, np);
+    sep_shape(np / 16, nb, true, (long)g * d.ny * n, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_z<UNIT, mr(), nr()>), dim3(g, d.ny, n), dim3(threads),
+                           (size_t)np * pitch * sizeof(double), st, d, B, nb, pitch, k0 / 16, (k1 + 15) / 16, ku,
+                           partial);
     });
     return g * d.ny;
 }
 
-static void sep_back(hipStream_t st, const Dims &d, const SeparableSys &S, const double *w, double *x,
-                     const SepRange &o, bool add, const double *b, const uint8_t *flag, const double *partial,
-                     int np) {
-    const int t0 = o.j0 / 16, t1 = (o.j1 + 15) / 16, nk = o.k1 - o.k0, nb = sep_block(t1 - t0, nk, S.ax[0].np);
-    const int gy = (t1 - t0 + nb - 1) / nb;
-    sep_shape(nb, S.ax[0].np / 16, false, (long)gy * nk, [&](auto mr, auto nr, int threads) {
-        hipLaunchKernelGGL((k_sep_back<mr(), nr()>), dim3(gy, nk), dim3(threads),
-                           (size_t)16 * nb * (S.ax[0].np + kSepPadRow) * sizeof(double), st, d, S.ax[0], S.ax[1], w,
-                           x, nb, t0, t1, o.i0 / 16, (o.i1 + 15) / 16, o.k0, add ? 1 : 0, partial ? S.pinned : 0, b,
-                           flag, partial, np);
+static void sep_back(hipStream_t st, const Dims &d, int n, const SeparableBatch &B, const SepRange &o, bool add,
+                     const double *b, const uint8_t *flag, const double *partial, int partials) {
+    const int t0 = o.j0 / 16, t1 = (o.j1 + 15) / 16, nk = o.k1 - o.k0, np = B.S[0].ax[0].np;
+    const int nb = sep_block(t1 - t0, nk * n, np), gy = (t1 - t0 + nb - 1) / nb;
+    sep_shape(nb, np / 16, false, (long)gy * nk * n, [&](auto mr, auto nr, int threads) {
+        hipLaunchKernelGGL((k_sep_back<mr(), nr()>), dim3(gy, nk, n), dim3(threads),
+                           (size_t)16 * nb * (np + kSepPadRow) * sizeof(double), st, d, B, nb, t0, t1, o.i0 / 16,
+                           (o.i1 + 15) / 16, o.k0, add ? 1 : 0, partial ? B.S[0].pinned : 0, b, flag, partial,
+                           partials);
     });
+}
+
+void launch_separable_batch(hipStream_t st, const Dims &d, int n, const SeparableSys *S, const double *const *b,
+                            double *const *s1, double *const *s2, double *const *x) {
+    SeparableBatch B[3]{};
+    for (int c = 0; c < n; c++)
+        for (int p = 0; p < 3; p++) {
+            B[p].S[c] = S[c];
+            B[p].in[c] = p == 0 ? b[c] : p == 1 ? s1[c] : s2[c];
+            B[p].out[c] = p == 0 ? s1[c] : p == 1 ? s2[c] : x[c];
+        }
+    const SepRange all{0, d.nx, 0, d.ny, 0, d.nz};
+    sep_xy<SEP_ALL>(st, d, n, B[0], nullptr, all);
+    sep_z<false>(st, d, n, B[1], 0, d.nz, 0, nullptr);
+    sep_back(st, d, n, B[2], all, false, nullptr, nullptr, nullptr, 0);
 }
 
 void launch_separable(hipStream_t st, const Dims &d, const SeparableSys &S, const double *b, double *s1, double *s2,
                       double *x, bool add, double *partial) {
     const SepRange all{0, d.nx, 0, d.ny, 0, d.nz};
-    sep_xy<SEP_ALL>(st, d, S, b, nullptr, s1, all);
-    const int np = sep_z<false>(st, d, S, s1, s2, 0, d.nz, 0, partial);
-    sep_back(st, d, S, s2, x, all, add, b, nullptr, partial, np);
+    sep_xy<SEP_ALL>(st, d, 1, {{S}, {b}, {s1}}, nullptr, all);
+    const int np = sep_z<false>(st, d, 1, {{S}, {s1}, {s2}}, 0, d.nz, 0, partial);
+    sep_back(st, d, 1, {{S}, {s2}, {x}}, all, add, b, nullptr, partial, np);
 }
 
 // ---------------------------------------------------------------------------
@@ -495,18 +516,18 @@ void launch_separable_body(hipStream_t st, const Dims &d, const SeparableSys &S,
     const SepRange all{0, d.nx, 0, d.ny, 0, d.nz};
     const SepRange look{B.look.lo[0], B.look.hi[0], B.look.lo[1], B.look.hi[1], B.look.lo[2], B.look.hi[2]};
     const SepRange cells{B.cells.lo[0], B.cells.hi[0], B.cells.lo[1], B.cells.hi[1], B.cells.lo[2], B.cells.hi[2]};
-    sep_xy<SEP_MASK>(st, d, S, b, B.fluid, s1, all);
-    sep_z<false>(st, d, S, s1, s2, look.k0, look.k1, 0, nullptr);
-    sep_back(st, d, S, s2, s3, look, false, b, nullptr, nullptr, 0);
+    sep_xy<SEP_MASK>(st, d, 1, {{S}, {b}, {s1}}, B.fluid, all);
+    sep_z<false>(st, d, 1, {{S}, {s1}, {s2}}, look.k0, look.k1, 0, nullptr);
+    sep_back(st, d, 1, {{S}, {s2}, {s3}}, look, false, b, nullptr, nullptr, 0);
     const int ng = B.G.ng;
     hipLaunchKernelGGL(k_cap_rhs, dim3((ng + 63) / 64), dim3(64), 0, st, B.G, b, s3, B.t);
     if (B.inv64)
         hipLaunchKernelGGL((k_cap_apply<double>), dim3((ng + 3) / 4), dim3(256), 0, st, B.G, B.inv64, B.ld, B.t, s3);
     else
         hipLaunchKernelGGL((k_cap_apply<float>), dim3((ng + 3) / 4), dim3(256), 0, st, B.G, B.inv32, B.ld, B.t, s3);
-    sep_xy<SEP_ADD>(st, d, S, s3, B.ghost, s1, cells);
-    sep_z<false>(st, d, S, s1, s2, 0, d.nz, 0, nullptr);
-    sep_back(st, d, S, s2, x, all, add, b, B.flag, nullptr, 0);
+    sep_xy<SEP_ADD>(st, d, 1, {{S}, {s3}, {s1}}, B.ghost, cells);
+    sep_z<false>(st, d, 1, {{S}, {s1}, {s2}}, 0, d.nz, 0, nullptr);
+    sep_back(st, d, 1, {{S}, {s2}, {x}}, all, add, b, B.flag, nullptr, 0);
 }
 
 // A^-1 e_c in the box, for the unit vectors of the ghost cells c = src0 +
@@ -583,7 +604,7 @@ void launch_green_plane(hipStream_t st, const Dims &d, const SeparableSys &S, in
                         const GreenBox &box, const GhostRows<double> &G, const int *loc, double *h,
                         const GreenScratch &green, double *out, long ld) {
     const long vol = (long)(box.hi[0] - box.lo[0]) * (box.hi[1] - box.lo[1]) * (box.hi[2] - box.lo[2]);
-    sep_z<true>(st, d, S, h, h, box.lo[2], box.hi[2], k, nullptr);
+    sep_z<true>(st, d, 1, {{S}, {h}, {h}}, box.lo[2], box.hi[2], k, nullptr);
     const int jt = (box.hi[1] + 15) / 16 - box.lo[1] / 16, batch = kGreenVecs * green.per;
     for (int c = 0; c < nsrc; c += batch) {
         const int n = std::min(batch, nsrc - c);
@@ -644,16 +665,14 @@ static bool tridiagonal_eigen(std::vector<double> &d, std::vector<double> &e, st
     return true;
 }
 
-bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], const double *width,
-                    std::vector<double> &V, std::vector<double> &Vi, std::vector<double> &lam) {
+bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], std::vector<double> &V,
+                    std::vector<double> &Vi, std::vector<double> &lam) {
     const std::vector<double> &cm = coef[0], &cp = coef[1], &dm = coef[2], &dp = coef[3];
-    std::vector<double> q, ev;
+    std::vector<double> q, ev, w(n, 1.0);  // w: square roots of the weights
     if (periodic) {
         // uniform spacing: Fourier modes
         for (int i = 0; i < n; i++)
-            if (std::fabs(cm[i] - cm[0]) > 1e-10 * cm[0] || std::fabs(cp[i] - cm[0]) > 1e-10 * cm[0] ||
-                std::fabs(width[i] - width[0]) > 1e-10 * width[0])
-                return false;
+            if (std::fabs(cm[i] - cm[0]) > 1e-10 * cm[0] || std::fabs(cp[i] - cm[0]) > 1e-10 * cm[0]) return false;
         for (int m = 0; m < n; m++) {
             const int f = (m + 1) / 2;  // 0, 1, 1, 2, 2, ...
             ev.push_back(2 * cm[0] * (1 - std::cos(2 * M_PI * f / n)));
@@ -668,10 +687,10 @@ bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], con
         ev.resize(n);
         for (int i = 0; i < n; i++) ev[i] = dm[i] + dp[i];
         for (int i = 0; i + 1 < n; i++) {
-            // width_i cp_i = width_(i+1) cm_(i+1): the operator is symmetric
-            const double a = cp[i] * width[i], b = cm[i + 1] * width[i + 1];
-            if (std::fabs(a - b) > 1e-9 * std::fabs(a) || !(a > 0)) return false;
-            e[i] = -0.5 * (a + b) / std::sqrt(width[i] * width[i + 1]);
+            // weight_i cp_i = weight_(i+1) cm_(i+1): the operator is symmetric
+            if (!(cp[i] > 0) || !(cm[i + 1] > 0)) return false;
+            w[i + 1] = w[i] * std::sqrt(cp[i] / cm[i + 1]);
+            e[i] = -std::sqrt(cp[i] * cm[i + 1]);
         }
         if (!tridiagonal_eigen(ev, e, q)) return false;
     }
@@ -690,8 +709,8 @@ bool separable_axis(int n, bool periodic, const std::vector<double> coef[4], con
         lam[m] = zero && m == 0 ? 0.0 : v;
         for (int i = 0; i < n; i++) {
             const double z = q[(size_t)order[m] * n + i];
-            V[(size_t)i * np + m] = z / std::sqrt(width[i]);
-            Vi[(size_t)m * np + i] = z * std::sqrt(width[i]);
+            V[(size_t)i * np + m] = z / w[i];
+            Vi[(size_t)m * np + i] = z * w[i];
         }
     }
     return true;

@@ -297,6 +297,10 @@ struct _ibm_solver {
     bool sep_on = false;
     ibm::SeparableSys sep{};
     ibm::DBuf<double> sep_mat[3][3];      // V, Vi, lam per axis
+    // momentum systems of a box without a body (build_separable_momentum)
+    bool sep_mom_on = false;
+    ibm::SeparableSys sep_mom[3]{};
+    ibm::DBuf<double> sep_mom_mat[9][3];
     // with a body: its ghost rows (build_capacitance)
     bool cap_on = false;
     ibm::SeparableBody cap{};
@@ -323,8 +327,10 @@ struct _ibm_solver {
 
 namespace ibm {
 
-// slots of IBMSolver::sums: 0..11 reductions of the step kernels, 12..29 the
-// convective outflow faces' BC-row norms (3 per face, bc[] order)
+// slots of IBMSolver::sums: 0..11 reductions of the step kernels (0..2 the
+// momentum right-hand sides), 12..29 the convective outflow faces' BC-row norms
+// (3 per face, bc[] order)
+constexpr int kPoissonSlot = 4, kMomResidualSlot = 8;
 constexpr int kSumSlots = 32;
 constexpr int kConvNormSlot = 12;
 // fields of up to this many values (1 MiB) cross between host and device
@@ -362,6 +368,7 @@ void iterate_impl(IBMSolver *s, int steps, bool verbose);
 void build_mg(IBMSolver *s);
 void ensure_mg(IBMSolver *s);
 void build_separable(IBMSolver *s);
+void build_separable_momentum(IBMSolver *s);
 void build_momentum_tables(IBMSolver *s);
 void build_outer_rules(IBMSolver *s);
 double max_div_impl(IBMSolver *s);

@@ -321,13 +321,15 @@ static void read_sums(IBMSolver *s, int nv) {
 }
 
 // The sums (maxima) of nv columns of block partials, formed straight into
-// sums_h (sum_publish: the epoch to wait for) and awaited there
-static unsigned sum_publish(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
+// sums_h[slot..] (sum_publish: the epoch to wait for; an earlier one's sums are
+// then there too)
+static unsigned sum_publish(IBMSolver *s, long nblk, int nv, int reduce_max = 0, int slot = 0) {
     const unsigned e = ++s->sums_epoch;
-    launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d, reduce_max, s->sums_d_epoch, e);
+    launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d + slot, reduce_max, s->sums_d_epoch, e);
     return e;
 }
 
+// and awaited there
 static void sum_read(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
     wait_epoch(s->stream, s->sums_h_epoch, sum_publish(s, nblk, nv, reduce_max));
 }
@@ -813,18 +815,16 @@ void build_separable(IBMSolver *s) {
     const int n[3] = {d.nx, d.ny, d.nz};
     if (!separable_fits(n)) return;
     if (body && (s->p_singular || s->ng == 0)) return;
-    const std::vector<double> *w[3] = {&s->dx, &s->dy, &s->dz};
     std::vector<double> m[3][3];
     double lo = 0, hi = 0, low[3];
     for (int a = 0; a < 3; a++) {
         const auto &h = s->sys[3].h[a];
         int same = a;  // an earlier axis with the same operator
         for (int o = a - 1; o >= 0; o--)
-            if (n[o] == n[a] && *w[o] == *w[a] && s->sys[3].S64.ax[o].periodic == s->sys[3].S64.ax[a].periodic
-                && std::equal(h, h + 4, s->sys[3].h[o]))
+            if (s->sys[3].S64.ax[o].periodic == s->sys[3].S64.ax[a].periodic && std::equal(h, h + 4, s->sys[3].h[o]))
                 same = o;
         if (same < a) for (int c = 0; c < 3; c++) m[a][c] = m[same][c];
-        else if (!separable_axis(n[a], s->sys[3].S64.ax[a].periodic, h, w[a]->data() + 2, m[a][0], m[a][1], m[a][2]))
+        else if (!separable_axis(n[a], s->sys[3].S64.ax[a].periodic, h, m[a][0], m[a][1], m[a][2]))
             return;
         const std::vector<double> &lam = m[a][2];
         if (s->p_singular != (lam[0] == 0) && s->p_singular) return;
@@ -837,6 +837,7 @@ void build_separable(IBMSolver *s) {
         for (int c = 0; c < 3; c++) s->sep_mat[a][c].upload(m[a][c]);
         s->sep.ax[a] = {s->sep_mat[a][0].p, s->sep_mat[a][1].p, s->sep_mat[a][2].p, n[a], (n[a] + 15) / 16 * 16};
     }
+    s->sep.c0 = 0;
     s->sep.pinned = s->p_singular;
     if (body) {
         s->sep_on = s->cap_on = build_capacitance(s);
@@ -853,6 +854,49 @@ void build_separable(IBMSolver *s) {
             if (low[a] > 0 && (lo == 0 || low[a] < lo)) lo = low[a];
         if (lo > 0 && hi > kFp32CycleSpan * lo) s->p_mg64 = true;
     }
+}
+
+// Direct solve of the three momentum systems of a box without a body, batched in
+// three launches. Time per step at tol 1e-12, sweeps / direct (mixed-Krylov, in
+// brackets FP64 where it differs): cavity 32^3 0.20 / 0.12 ms, 64^3 0.28 / 0.19,
+// 128^3 1.00 / 0.73, 192^3 3.1 (4.7) / 3.07, 256^3 7.95 (9.8) / 7.7, 320 x 96 x
+// 96 1.43 / 1.34, 480 x 64 x 64 0.91 (1.05) / 0.94: taken on every grid that the
+// transforms take. With a body the sweeps stay: the ghost rows of three systems
+// would need three more dense inverses.
+void build_separable_momentum(IBMSolver *s) {
+    s->sep_mom_on = false;
+    const Dims &d = s->d;
+    const int n[3] = {d.nx, d.ny, d.nz};
+    if (s->precision == IBM3D_PREC_MIXED || s->ng > 0 || !separable_fits(n)) return;
+    for (int k = 0; k < d.nz; k++)
+        for (int j = 0; j < d.ny; j++)
+            for (int i = 0; i < d.nx; i++)
+                if (s->flag_dev_h[cidx(d, i, j, k)] != F_FLUID) return;
+    int used = 0;
+    struct Axis { int c, a, slot; };
+    std::vector<Axis> known;
+    for (int c = 0; c < 3; c++) {
+        for (int a = 0; a < 3; a++) {
+            const auto &h = s->sys[c].h[a];
+            int slot = -1;  // an earlier axis with the same operator
+            for (const Axis &o : known)
+                if (s->sys[o.c].S64.ax[o.a].periodic == s->sys[c].S64.ax[a].periodic
+                    && std::equal(h, h + 4, s->sys[o.c].h[o.a]))
+                    slot = o.slot;
+            if (slot < 0) {
+                std::vector<double> m[3];
+                if (!separable_axis(n[a], s->sys[c].S64.ax[a].periodic, h, m[0], m[1], m[2])) return;
+                slot = used++;
+                for (int e = 0; e < 3; e++) s->sep_mom_mat[slot][e].upload(m[e]);
+                known.push_back({c, a, slot});
+            }
+            DBuf<double> *m = s->sep_mom_mat[slot];
+            s->sep_mom[c].ax[a] = {m[0].p, m[1].p, m[2].p, n[a], (n[a] + 15) / 16 * 16};
+        }
+        s->sep_mom[c].c0 = s->sys[c].S64.c0;
+        s->sep_mom[c].pinned = 0;
+    }
+    s->sep_mom_on = true;
 }
 
 template <typename T> static const T *dinv(const MGLevel &L);
@@ -1681,41 +1725,44 @@ static void momentum_concurrent(IBMSolver *s, F &&norms) {
 // Direct pressure solve and refinement: x = A^-1 b, then x += A^-1 (b - A x)
 // until the FP64 residual meets the tolerance. One round reaches the rounding
 // level of the transforms (1e-12 .. 1e-10 of ||b||), a second one that of the
-// residual. norm() gives the stopping norm (a host read), called once the
-// first round is enqueued. A solve whose residual no longer halves is left to
-// the iterative path (false); its reason is the tolerance, not the method.
-template <typename F>
-static bool separable_solve(IBMSolver *s, const double *b, double *x, F &&norm, double *bnorm) {
+// residual. A solve whose residual no longer halves is left to the iterative
+// path (false); its reason is the tolerance, not the method. separable_round
+// enqueues a round and returns the epoch of its residual's norms.
+static unsigned separable_round(IBMSolver *s, const double *b, double *x, bool first) {
     const Dims &d = s->d;
     const NormSpec ns{1, s->ks1d[0].p, s->ks1d[1].p, s->ks1d[2].p, s->flag.p, s->pin};
     double *r = s->kry.v64[0].p, *s1 = s->kry.v64[1].p, *s2 = s->kry.v64[2].p;
     const double cb = ncells(s) * 8;
+    const double *rhs = first ? b : r;
+    if (s->cap_on)
+        TIMED("separable_body", (first ? 9 : 10) * cb + (double)s->cap.G.ng * s->cap.ld * (s->cap.inv64 ? 8 : 4),
+              launch_separable_body(s->stream, d, s->sep, s->cap, rhs, s1, s2, s->kry.v64[3].p, x, !first));
+    else
+        TIMED("separable", (first ? 6 : 7) * cb,
+              launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, !first, s->partial.p));
+    TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r, ns,
+                                                      s->partial.p));
+    return finalize_publish(s, 4, apply_partials(d, s->gp.G64.ng), 2);
+}
+
+// The rounds after the first, whose norms come with epoch e; bn: stopping norm
+static bool separable_finish(IBMSolver *s, const double *b, double *x, unsigned e, double bn) {
     double last = 0;
     for (int round = 1;; round++) {
-        const double *rhs = round > 1 ? r : b;
-        if (s->cap_on)
-            TIMED("separable_body", (round > 1 ? 10 : 9) * cb + (double)s->cap.G.ng * s->cap.ld * (s->cap.inv64 ? 8 : 4),
-                  launch_separable_body(s->stream, d, s->sep, s->cap, rhs, s1, s2, s->kry.v64[3].p, x, round > 1));
-        else
-            TIMED("separable", (round > 1 ? 7 : 6) * cb,
-                  launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, round > 1, s->partial.p));
-        TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r,
-                                                          ns, s->partial.p));
-        const unsigned e = finalize_publish(s, 4, apply_partials(d, s->gp.G64.ng), 2);
-        if (round == 1) *bnorm = norm();
         finalize_wait(s, e);
-        if (*bnorm == 0) {
-            launch_zero<double>(s->stream, d, x);
+        if (bn == 0) {
+            launch_zero<double>(s->stream, s->d, x);
             report_solve(s, 3, 0, 0);
             return true;
         }
         const double rn = std::sqrt(s->ks_h->rrn);
-        if (rn <= s->tol * *bnorm) {
-            report_solve(s, 3, rn / *bnorm, round);
+        if (rn <= s->tol * bn) {
+            report_solve(s, 3, rn / bn, round);
             return true;
         }
         if (!(round == 1 || rn <= 0.5 * last) || !std::isfinite(rn)) break;
         last = rn;
+        e = separable_round(s, b, x, false);
     }
     // with a body the memory of the capacitance matrix is the hierarchy's: the
     // solver goes over to the iterative path for good
@@ -1857,8 +1904,10 @@ static void momentum_smooth(IBMSolver *s, const MomTable<T> *M, unsigned mask, i
 }
 
 // The three momentum solves by sweeps; components that do not converge this
-// way are solved by solve_system. bn: the stopping norms.
-static void momentum_sweep_solve(IBMSolver *s, const double bn[3]) {
+// way are solved by solve_system. norms(bn, e): the stopping norms, once epoch e
+// of the sums is there.
+template <typename F>
+static void momentum_sweep_solve(IBMSolver *s, F &&norms) {
     const Dims &d = s->d;
     const int m = momentum_sweeps(s);
     const double cb = ncells(s);
@@ -1867,18 +1916,8 @@ static void momentum_sweep_solve(IBMSolver *s, const double bn[3]) {
     double rn[3] = {0, 0, 0}, rate[3] = {s->mom_rate, s->mom_rate, s->mom_rate};
     int sweeps[3] = {0, 0, 0}, prev = -1;
     bool fallback[3] = {false, false, false};
-    unsigned mask = 0;
-    for (int l = 0; l < 3; l++) {
-        // a zero right-hand side has the zero solution; a non-finite one
-        // stays active, so its residual reports the error
-        if (bn[l] != 0) {
-            mask |= 1u << l;
-            rn[l] = bn[l];
-            continue;
-        }
-        launch_zero<double>(s->stream, d, s->us[l].p);
-        report_solve(s, l, 0.0, 0);
-    }
+    unsigned mask = 7;
+    double bn[3];
     for (int round = 0; mask && round < kMomMaxRounds; round++) {
         const double act = __builtin_popcount(mask);
         // the first round aims at the tolerance (FP64) or the FP32 limit,
@@ -1904,11 +1943,26 @@ static void momentum_sweep_solve(IBMSolver *s, const double bn[3]) {
         }
         TIMED("mom_residual64", act * cb * (f64 ? 2 : 3) * 8,
               launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p, !f64, s->partial.p));
-        sum_read(s, na, 3);
+        const unsigned e = sum_publish(s, na, 3, 0, kMomResidualSlot);
+        if (round == 0) {
+            // the norms are read behind the first round's launches
+            norms(bn, e);
+            for (int l = 0; l < 3; l++) {
+                // a zero right-hand side has the zero solution; a non-finite
+                // one stays active, so its residual reports the error
+                rn[l] = bn[l];
+                if (bn[l] != 0) continue;
+                mask &= ~(1u << l);
+                launch_zero<double>(s->stream, d, s->us[l].p);
+                report_solve(s, l, 0.0, 0);
+            }
+        } else {
+            wait_epoch(s->stream, s->sums_h_epoch, e);
+        }
         for (int l = 0; l < 3; l++) {
             if (!(mask >> l & 1)) continue;
             sweeps[l] += mr;
-            const double r = std::sqrt(s->sums_h[l]);
+            const double r = std::sqrt(s->sums_h[kMomResidualSlot + l]);
             const bool stalled = round > 0 && !(r <= 0.1 * rn[l]);
             // rate shown by this round's sweeps (FP64: from ||b||), kept below 1
             if (f64) rate[l] = std::min(0.5, std::max(1e-6, std::pow(r / rn[l], 1.0 / mr)));
@@ -1924,6 +1978,35 @@ static void momentum_sweep_solve(IBMSolver *s, const double bn[3]) {
     }
     for (int l = 0; l < 3; l++)
         if ((mask >> l & 1) || fallback[l]) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
+}
+
+// The three momentum solves by the transforms, and their residuals' norms to
+// sums_h
+static void momentum_direct(IBMSolver *s) {
+    const double cb = ncells(s) * 8 * 3;
+    const double *b[3];
+    double *s1[3], *s2[3], *x[3];
+    for (int l = 0; l < 3; l++) {
+        b[l] = s->b[l].p;
+        s1[l] = s->kry.v64[1 + l].p;
+        s2[l] = s->kry.v64[4 + l].p;
+        x[l] = s->us[l].p;
+    }
+    TIMED("mom_separable", 6 * cb, launch_separable_batch(s->stream, s->d, 3, s->sep_mom, b, s1, s2, x));
+    TIMED("mom_residual64", 2 * cb,
+          launch_mom_residual(s->stream, s->d, s->mt64.p, 7, s->gmom.G64, s->flag.p, false, s->partial.p));
+    sum_publish(s, apply_partials(s->d, 0), 3, 0, kMomResidualSlot);
+}
+
+// whether all of them meet the tolerance (bn: stopping norms)
+static bool momentum_direct_met(IBMSolver *s, const double bn[3]) {
+    double r[3];
+    for (int l = 0; l < 3; l++) {
+        r[l] = std::sqrt(s->sums_h[kMomResidualSlot + l]);
+        if (!(r[l] <= s->tol * bn[l])) return false;
+    }
+    for (int l = 0; l < 3; l++) report_solve(s, l, bn[l] != 0 ? r[l] / bn[l] : 0.0, bn[l] != 0);
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -2000,13 +2083,14 @@ static void do_step(IBMSolver *s) {
     else me = sum_publish(s, conv_rhs_blocks(s->d), 3);
     conv_outflow(s, 0);
     double fnorm[4];
-    const OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm);
+    OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm), opp{};
     bc_rhs(s, ob, 0, 3);
-    // stopping norms of the momentum solves: the right-hand sides' sums
-    // (host read) plus the BC rows' and forcing parts
-    auto mom_norms = [&](double bn[3]) {
-        if (conv) read_sums(s, kConvNormSlot + 18);
-        else wait_epoch(s->stream, s->sums_h_epoch, me);
+    // stopping norms of the momentum solves: the right-hand sides' sums, plus
+    // the BC rows' and forcing parts; read once epoch e of the sums is there
+    // (before the solves where outflow faces have their share: the whole table
+    // of sums is read then)
+    double bn[3];
+    auto form_norms = [&] {
         for (int l = 0; l < 3; l++) {
             double bn2 = s->sums_h[l] + s->sys[l].bc_norm2 + fnorm[l];
             for (int f = 0; conv && f < 6; f++)
@@ -2014,46 +2098,65 @@ static void do_step(IBMSolver *s) {
             bn[l] = std::sqrt(bn2);
         }
     };
-    // momentum Helmholtz solves: the three at once on their lanes, or one
-    // after the other (mixed defect-correction mode, and under the per-kernel
-    // timers, whose events are recorded on the solver's stream)
-    if (s->precision != IBM3D_PREC_MIXED && s->mom_solver == 0 && momentum_sweeps(s) > 0) {
-        double bn[3];
-        mom_norms(bn);
-        momentum_sweep_solve(s, bn);
-    } else if (s->mom_lanes && s->timing == 0 && s->precision != IBM3D_PREC_MIXED) {
-        momentum_concurrent(s, mom_norms);
-    } else {
-        double bn[3];
-        mom_norms(bn);
-        for (int l = 0; l < 3; l++) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
+    if (conv) {
+        read_sums(s, kConvNormSlot + 18);
+        form_norms();
     }
-    // outer layers of the three solutions from their BC rows (the per-component
-    // fill of each u* with the solve's boundary data, all three in one pass)
-    TIMED("outer_sol", 0, launch_outer(s->stream, s->d, ob, s->outer_rules.p, {{s->us[0].p, s->us[1].p, s->us[2].p}, {0, 1, 2}, 3}));
-    // K2: U*, Poisson RHS
-    {
+    auto mom_norms = [&](double out[3], unsigned e) {
+        wait_epoch(s->stream, s->sums_h_epoch, e);
+        if (!conv) form_norms();
+        std::copy(bn, bn + 3, out);
+    };
+    // momentum Helmholtz solves: by sweeps; else the three at once on their
+    // lanes, or one after the other (mixed defect-correction mode, and under
+    // the per-kernel timers, whose events are recorded on the solver's stream)
+    auto mom_iterate = [&](unsigned e) {
+        if (s->precision != IBM3D_PREC_MIXED && s->mom_solver == 0 && momentum_sweeps(s) > 0) {
+            momentum_sweep_solve(s, mom_norms);
+        } else if (s->mom_lanes && s->timing == 0 && s->precision != IBM3D_PREC_MIXED) {
+            momentum_concurrent(s, [&](double out[3]) { mom_norms(out, e); });
+        } else {
+            double n3[3];
+            mom_norms(n3, e);
+            for (int l = 0; l < 3; l++) solve_system(s, l, s->b[l].p, s->us[l].p, n3[l]);
+        }
+    };
+    // or directly: the residuals are then looked at together with the
+    // pressure's, and the step goes on from the iterative solves if one of them
+    // is not below the tolerance
+    bool mom_open = s->sep_mom_on && s->mom_solver == 0;
+    if (mom_open) momentum_direct(s);
+    else mom_iterate(conv ? s->sums_epoch : me);
+    const bool direct = s->sep_on;
+    double bnp = 0;
+    unsigned fe = 0;
+    for (;;) {
+        // outer layers of the three solutions from their BC rows (the per-component
+        // fill of each u* with the solve's boundary data, all three in one pass)
+        TIMED("outer_sol", 0, launch_outer(s->stream, s->d, ob, s->outer_rules.p,
+                                           {{s->us[0].p, s->us[1].p, s->us[2].p}, {0, 1, 2}, 3}));
+        // K2: U*, Poisson RHS
         const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};
         double *Fs[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
         TIMED("k2_face_star", cn * (4 * 8 + 3 * 8 + 1), launch_face_star(s->stream, s->geo, sp, s->flag.p, us3, s->p.p, Fs));
         const double *Fc[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
         TIMED("k2_poisson_rhs", cn * (4 * 8 + 1),
               launch_poisson_rhs(s->stream, s->geo, sp, s->flag.p, s->pin, Fc, s->bp.p, s->partial.p));
-    }
-    const unsigned pe = sum_publish(s, conv_rhs_blocks(s->d), 1);
-    double pnorm[4];
-    const OuterParams opp = make_outer(s, BCD_PSOL, s->time, pnorm);
-    bc_rhs(s, opp, 3, 1);
-    auto poisson_norm = [&] {
+        const unsigned pe = sum_publish(s, conv_rhs_blocks(s->d), 1, 0, kPoissonSlot);
+        double pnorm[4];
+        opp = make_outer(s, BCD_PSOL, s->time, pnorm);
+        bc_rhs(s, opp, 3, 1);
+        if (direct) fe = separable_round(s, s->bp.p, s->pp.p, true);
         wait_epoch(s->stream, s->sums_h_epoch, pe);
-        return std::sqrt(s->sums_h[0] + s->sys[3].bc_norm2 + pnorm[3]);
-    };
-    double bnp = 0;
-    const bool direct = s->sep_on;
-    if (!direct || !separable_solve(s, s->bp.p, s->pp.p, poisson_norm, &bnp)) {
-        if (!direct) bnp = poisson_norm();
-        solve_system(s, 3, s->bp.p, s->pp.p, bnp);
+        bnp = std::sqrt(s->sums_h[kPoissonSlot] + s->sys[3].bc_norm2 + pnorm[3]);
+        if (!mom_open) break;
+        if (!conv) form_norms();
+        mom_open = false;
+        if (momentum_direct_met(s, bn)) break;
+        mom_iterate(pe);
+        ob = make_outer(s, BCD_FIELDS, s->time, fnorm);  // its buffers hold the pressure's data now
     }
+    if (!direct || !separable_finish(s, s->bp.p, s->pp.p, fe, bnp)) solve_system(s, 3, s->bp.p, s->pp.p, bnp);
     TIMED("outer_sol", 0, launch_outer(s->stream, s->d, opp, s->outer_rules.p, {{s->pp.p}, {OUT_DP}, 1}));
     // K3: projection
     {

@@ -94,13 +94,15 @@ void IBMSolver_set_mg_relaxation(IBMSolver *, double omega);
 int IBMSolver_get_pressure_mg_bits(IBMSolver *);
 
 /* Momentum Helmholtz solver of the IBM3D_PREC_FP64 and _MIXED_KRYLOV modes.
-   0 (default): red-black Gauss-Seidel sweeps, in FP64 on the system itself or
-   (mixed) in FP32 inside FP64 iterative refinement, where the operator is
+   0 (default): in a box without a body directly, in FP64 (eigenvectors of the
+   three axes, where the periodic ones are uniform); else, or if that misses
+   the tolerance, red-black Gauss-Seidel sweeps, in FP64 on the system itself
+   or (mixed) in FP32 inside FP64 iterative refinement, where the operator is
    diagonally dominant enough (max over cells of sum K / (1 + sum K) squared
    <= 0.5), BiCGSTAB elsewhere and for any component whose residual stops
    falling; 1: always BiCGSTAB (FP64, Jacobi preconditioner; mixed: FP32 stored
    directions). All stop on the reference's test ||b - A x|| <= tol ||b|| in
-   FP64; IBMSolver_get_last_iters counts sweeps or iterations. */
+   FP64; IBMSolver_get_last_iters counts sweeps or iterations (1: direct). */
 void IBMSolver_set_momentum_solver(IBMSolver *, int mode);
 
 /* Copies a field to host memory in the reference layout (see above). Solid

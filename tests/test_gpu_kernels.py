@@ -290,3 +290,30 @@ def test_outer_layers_match_the_oracle(new_gpu, new_oracle, I, faces, shape):
         b = out[1][n]
         assert np.array_equal(np.isfinite(a), np.isfinite(b)), n
         assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), n
+
+
+@pytest.mark.parametrize("precision", [0, 2], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("kind,shape", [("channel", (34, 18, 22)), ("channel", (64, 48, 32)),
+                                        ("pressure", (49, 33, 18)), ("outflow", (49, 33, 18))])
+def test_momentum_of_boxes_matches_bicgstab(new_gpu, I, cases, kind, shape, precision):
+    """Periodic axes, walls, free slip and outlets (the axis of a pressure
+    outlet extrapolates the velocity and may leave the direct solve to the
+    sweeps) against BiCGSTAB at tol 1e-12, as for the sweeps: 1e-10 with room
+    for the projection."""
+    out = []
+    for mode in (0, 1):
+        s = new_gpu()
+        s.set_momentum_solver(mode)
+        s.set_precision(precision)
+        if kind == "channel":
+            cases.setup_channel(s, *shape, tol=1e-12, precision=precision)
+        else:
+            setup_duct(s, I, shape, kind, 1e-12)
+        s.iterate(2)
+        assert (s.last_norms()[:3] <= 1e-12).all()
+        if mode == 0 and kind == "channel":
+            assert list(s.last_iters()[:3]) == [1, 1, 1]
+        out.append([s.get(n)[2:-2, 2:-2, 2:-2] for n in ("U1_STAR", "U2_STAR", "U3_STAR", "U1", "U2", "U3")])
+    scale = max(np.abs(a).max() for a in out[1])
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() <= 1e-10 * scale
