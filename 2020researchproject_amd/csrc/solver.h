@@ -274,6 +274,7 @@ struct _ibm_solver {
     bool mom_lanes = false;
     double *sums_h = nullptr;        // pinned
     double *gm_h = nullptr;          // pinned, 64 scalars of the GMRES / PCG solvers
+    char *stage_h = nullptr;         // pinned, kStageSlots chunks of kStageChunk: large fields on their way to the host
     double *io_h = nullptr, *io_d = nullptr;  // device-mapped host memory, kIoDoubles: small fields in the host layout
 
     // ghost cells
@@ -336,6 +337,11 @@ constexpr int kConvNormSlot = 12;
 // fields of up to this many values (1 MiB) cross between host and device
 // through mapped memory that the layout kernel itself reads or writes
 constexpr size_t kIoDoubles = 1u << 17;
+// those of at least kStageMin bytes go to the host through a ring of pinned
+// chunks (8 MiB per solver, from its first read of such a field on: 1 ms once,
+// which smaller fields do not earn back: 2.5 MB 0.15 against 0.17 ms)
+constexpr size_t kStageMin = 8u << 20, kStageChunk = 1u << 20;
+constexpr int kStageSlots = 8, kStageThreads = 4;
 constexpr int kConvSpeedSlot = 31;  // convection speed of the face being advanced
 
 // Errors of one case (rejected input, a non-finite residual, a lost Krylov

@@ -317,3 +317,23 @@ def test_momentum_of_boxes_matches_bicgstab(new_gpu, I, cases, kind, shape, prec
     scale = max(np.abs(a).max() for a in out[1])
     for a, b in zip(*out):
         assert np.abs(a - b).max() <= 1e-10 * scale
+
+
+@pytest.mark.parametrize("shape", [(124, 92, 86), (128, 92, 92), (150, 110, 97)])
+def test_large_fields_reach_the_host_unchanged(new_gpu, cases, shape):
+    """Cell and face fields of just below, at and above the size that crosses
+    through the ring of pinned chunks (8 MiB; the ring's 8 chunks of 1 MiB used
+    once, and again with a part of a chunk left): as set, bit for bit, twice."""
+    s = new_gpu()
+    cases.setup_cavity(s, shape=shape, tol=1e-8)
+    rng = np.random.default_rng(11)
+    a = {n: rng.standard_normal(s.shape) for n in ("U1", "P")}
+    for n, v in a.items():
+        s.set(n, v)
+    for _ in range(2):
+        for n, v in a.items():
+            np.testing.assert_array_equal(s.get(n), v)
+    s.iterate(0)
+    u, f = s.get("U1"), s.get("FACE_U1")
+    np.testing.assert_allclose(f[:, 2:-2, 2:-2], 0.5 * (u[1:-2, 2:-2, 2:-2] + u[2:-1, 2:-2, 2:-2]),
+                               rtol=1e-13, atol=1e-13)
