@@ -231,7 +231,7 @@ struct _ibm_solver {
     int mom_solver = 0;          // IBMSolver_set_momentum_solver: 0 automatic, 1 BiCGSTAB
     int mom_sweeps = -1;         // FP32 sweeps per refinement round of the momentum solves (0: not used; -1: unset)
     ibm::DBuf<ibm::MomTable<double>> mt64;  // operands of the batched momentum launches
-    ibm::DBuf<ibm::MomTable<float>> mt32;   // mixed-Krylov mode: the FP32 corrections
+    ibm::DBuf<ibm::MomTable<float>> mt32, mt32b;  // mixed-Krylov mode: the FP32 corrections of the first and second round
     ibm::DBuf<double> mgv64;     // ghost values of the three components (two buffers each)
     ibm::DBuf<float> mgv32;
     double mom_rate = 0;         // estimated red-black sweep contraction of the momentum operators
@@ -272,6 +272,7 @@ struct _ibm_solver {
     ibm::MomLane mlane[2];
     hipEvent_t ev_rhs = nullptr;     // momentum right-hand sides formed (solver's stream)
     bool mom_lanes = false;
+    bool lanes_used = false;         // the lanes' vectors hold values of a BiCGSTAB solve
     double *sums_h = nullptr;        // pinned
     double *gm_h = nullptr;          // pinned, 64 scalars of the GMRES / PCG solvers
     char *stage_h = nullptr;         // pinned, kStageSlots chunks of kStageChunk: large fields on their way to the host

@@ -130,16 +130,23 @@ int launch_mom_colour(hipStream_t st, const Dims &d, const MomTable<T> *M, unsig
 template <typename T>
 void launch_mom_ghost(hipStream_t st, const Dims &d, const MomTable<T> *M, unsigned mask, const GhostRows<T> &G,
                       int only);
-// residuals (written to M->r when store) with partial[3 blk + c] = the block's
-// share of ||b_c - A_c x_c||^2, apply_partials blocks
+// residuals with partial[3 blk + c] = the block's share of ||b_c - A_c x_c||^2,
+// apply_partials blocks; MOM_STORE: written to M->r; MOM_JACOBI: the solution is
+// in M->r, and with a Jacobi step goes to M->x
+enum MomResidual { MOM_NORMS, MOM_STORE, MOM_JACOBI };
 void launch_mom_residual(hipStream_t st, const Dims &d, const MomTable<double> *M, unsigned mask,
-                         const GhostRows<double> &G, const uint8_t *flag, bool store, double *partial);
+                         const GhostRows<double> &G, const uint8_t *flag, MomResidual what, double *partial);
 // FP32 right-hand sides M32->b from M->b or M->r, and the first colour in M32->x
 void launch_mom_d2f_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
                           unsigned mask, const uint8_t *flag, bool from_b);
-// M->x = M32->x, or (add) M->x += M32->x
+// x = e (M32), x or (to_r) r = e0 + e (M0 given) or, with add, x += e
 void launch_mom_add(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
-                    unsigned mask, bool add);
+                    const MomTable<float> *M0, unsigned mask, bool add, bool to_r);
+// residual of x = e (Ma), in FP32 as the right-hand side of Mb with its first
+// colour; block partials of the squared norms
+void launch_mom_residual_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *Ma,
+                               const MomTable<float> *Mb, unsigned mask, const GhostRows<double> &G,
+                               const uint8_t *flag, double *partial);
 
 // BiCGSTAB pieces
 template <typename T>

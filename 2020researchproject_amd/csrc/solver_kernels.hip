@@ -355,11 +355,62 @@ __device__ inline double nscale(const NormSpec &ns, const Dims &d, int i, int j,
 
 // One block of the residual r = b - A x (blocks below ngb: ghost rows, the
 // others cell pairs, XCD-contiguous of `nb` blocks in all): acc gets the
-// block's lanes' shares of ||r||^2 and ||D^-1 r||^2. STORE: r is written.
-template <bool STORE, typename T>
+// block's lanes' shares of ||r||^2 and ||D^-1 r||^2. The sink takes r: two
+// cells of a row with their flags (skipping ghost cells), and ghost rows.
+template <typename T>
+struct ResidualStore {
+    T *r;
+    __device__ void pair(const Dims &d, int i0, int, int, long q0, unsigned, T v0, T v1, bool g0, bool g1) const {
+        store_pair_skip(d, i0, q0, r, v0, v1, g0, g1);
+    }
+    __device__ void ghost(int, long c, T v) const { r[c] = v; }
+};
+struct ResidualDrop {
+    template <typename T>
+    __device__ void pair(const Dims &, int, int, int, long, unsigned, T, T, bool, bool) const {}
+    template <typename T>
+    __device__ void ghost(int, long, T) const {}
+};
+// FP32 right-hand side of a correction and the first smoother colour on it
+struct ResidualCorrection {
+    const SysCoef<float> &S;
+    float *b, *x;
+    __device__ void pair(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1, bool g0,
+                         bool g1) const {
+        const float b0 = (float)v0, b1 = (float)v1;
+        const float d0 = stencil_diag(S, i0, j, k, q0), d1 = stencil_diag(S, min(i0 + 1, d.nx - 1), j, k, q0 + 1);
+        store_pair_skip(d, i0, q0, b, b0, b1, g0, g1);
+        store_pair_skip(d, i0, q0, x, first_colour_of(S, fv & 0xFFu, i0, j, k, q0, b0, d0),
+                        first_colour_of(S, fv >> 8, i0 + 1, j, k, q0 + 1, b1, d1), g0, g1);
+    }
+    __device__ void ghost(int, long c, double v) const {
+        b[c] = (float)v;
+        x[c] = 0;
+    }
+};
+// out = x + r / diagonal
+struct ResidualJacobi {
+    const SysCoef<double> &S;
+    const GhostRows<double> &G;
+    const double *x;
+    double *out;
+    __device__ void pair(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1, bool g0,
+                         bool g1) const {
+        const double2 o = *reinterpret_cast<const double2 *>(x + q0);
+        const double d0 = stencil_diag(S, i0, j, k, q0), d1 = stencil_diag(S, min(i0 + 1, d.nx - 1), j, k, q0 + 1);
+        store_pair_skip(d, i0, q0, out, o.x + ((fv & 0xFFu) == F_FLUID ? v0 / d0 : 0.0),
+                        o.y + (fv >> 8 == F_FLUID ? v1 / d1 : 0.0), g0, g1);
+    }
+    __device__ void ghost(int s, long c, double v) const {
+        const double dg = S.is_p ? 1 - G.wself[s] : 1 + G.wself[s];
+        out[c] = x[c] + (dg != 0 ? v / dg : 0.0);
+    }
+};
+
+template <typename SINK, typename T, typename TX>
 __device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const GhostRows<T> &G,
                                       const uint8_t *__restrict__ flag, const T *__restrict__ b,
-                                      const T *__restrict__ x, T *__restrict__ r, const NormSpec &ns, unsigned wb,
+                                      const TX *__restrict__ x, const SINK &sink, const NormSpec &ns, unsigned wb,
                                       unsigned nb, unsigned ngb, unsigned gx, unsigned gy, double (&acc)[2]) {
     using T2 = typename Vec2<T>::type;
     if (wb < ngb) {
@@ -368,7 +419,7 @@ __device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const 
             long c;
             const T yv = ghost_row_apply<T>(G, S.is_p, x, s, c);
             const T rv = b[c] - yv;
-            if (STORE) r[c] = rv;
+            sink.ghost(s, c, rv);
             acc[0] = acc[1] = (double)rv * (double)rv;
         }
     } else {
@@ -403,7 +454,7 @@ __device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const 
                     gh[o] = !ident && f == F_GHOST;  // written by the ghost blocks
                     on[o] = i0 + o < d.nx && (ident || f == F_FLUID);
                 }
-                if (STORE) store_pair_skip(d, i0, q0, r, v[0], v[1], gh[0], gh[1]);
+                sink.pair(d, i0, j, k, q0, fv[kk], v[0], v[1], gh[0], gh[1]);
 #pragma unroll
                 for (int o = 0; o < 2; o++) {
                     if (!on[o]) continue;
@@ -423,7 +474,7 @@ __global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRow
                                                   const T *__restrict__ x, T *__restrict__ r, NormSpec ns,
                                                   double *partial, unsigned ngb, unsigned gx, unsigned gy) {
     double acc[2] = {0, 0};
-    residual_block<true>(d, S, G, flag, b, x, r, ns, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    residual_block(d, S, G, flag, b, x, ResidualStore<T>{r}, ns, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
     bsum<2>(acc, partial, blockIdx.x);
 }
 
@@ -1627,30 +1678,62 @@ void launch_mom_ghost(hipStream_t st, const Dims &d, const MomTable<T> *M, unsig
     hipLaunchKernelGGL((k_mom_ghost<T>), dim3((G.ng + 31) / 32, 3), dim3(256), 0, st, d, M, mask, G, only);
 }
 
-template <bool STORE>
-__global__ void __launch_bounds__(256) k_mom_residual(Dims d, const MomTable<double> *M, unsigned mask,
-                                                      GhostRows<double> G, const uint8_t *flag, double *partial,
-                                                      unsigned ngb, unsigned gx, unsigned gy) {
+// Residuals of the three systems: WHAT 0 their norms only, 1 also r, 2 of the
+// FP32 solution of the first round (x there), r as the FP32 right-hand side of
+// the next one with its first colour. The last saves the pass that forms x in
+// FP64 and the one that rounds r: 256 x 128 x 128, 31 and 40 us of the 170 that
+// a round's end took. 3: of the sum of the two rounds' corrections (kept in r),
+// with a Jacobi step on it into x: two FP32 corrections leave about 4e-15 of the
+// solution, of one sign where the flow is uniform, and through the mass flux of a
+// convective outlet that shifted the pressure of the sphere 133 x 67 x 61 by
+// 6e-10 of its norm (now 2e-12); a third round in its place costs 60 us.
+template <int WHAT>
+__global__ void __launch_bounds__(256) k_mom_residual(Dims d, const MomTable<double> *M, const MomTable<float> *Ma,
+                                                      const MomTable<float> *Mb, unsigned mask, GhostRows<double> G,
+                                                      const uint8_t *flag, double *partial, unsigned ngb, unsigned gx,
+                                                      unsigned gy) {
     const unsigned c = blockIdx.y;
     if (!((mask >> c) & 1u)) return;
     const SysCoef<double> S = M->S[c];
     const NormSpec off{0, nullptr, nullptr, nullptr, nullptr, -1};
     double acc[2] = {0, 0};
-    residual_block<STORE>(d, S, G, flag, M->b[c], (const double *)M->x[c], M->r[c], off, blockIdx.x, gridDim.x, ngb,
-                          gx, gy, acc);
+    const double *b = M->b[c], *x = M->x[c];
+    if constexpr (WHAT == 2) {
+        const SysCoef<float> S32 = Mb->S[c];
+        residual_block(d, S, G, flag, b, (const float *)Ma->x[c], ResidualCorrection{S32, Mb->brw[c], Mb->x[c]}, off,
+                       blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    } else if constexpr (WHAT == 3) {
+        residual_block(d, S, G, flag, b, (const double *)M->r[c], ResidualJacobi{S, G, M->r[c], M->x[c]}, off,
+                       blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    } else if constexpr (WHAT == 1) {
+        residual_block(d, S, G, flag, b, x, ResidualStore<double>{M->r[c]}, off, blockIdx.x, gridDim.x, ngb, gx, gy,
+                       acc);
+    } else {
+        residual_block(d, S, G, flag, b, x, ResidualDrop{}, off, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    }
     const double a1[1] = {acc[0]};
     bsum<1>(a1, partial, (long)blockIdx.x * 3 + c);
 }
 
 void launch_mom_residual(hipStream_t st, const Dims &d, const MomTable<double> *M, unsigned mask,
-                         const GhostRows<double> &G, const uint8_t *flag, bool store, double *partial) {
+                         const GhostRows<double> &G, const uint8_t *flag, MomResidual what, double *partial) {
     const dim3 grid(agrid_blocks(d, G.ng), 3);
-    if (store)
-        hipLaunchKernelGGL(k_mom_residual<true>, grid, dim3(64, 4), 0, st, d, M, mask, G, flag, partial,
+    if (what == MOM_JACOBI)
+        hipLaunchKernelGGL(k_mom_residual<3>, grid, dim3(64, 4), 0, st, d, M, nullptr, nullptr, mask, G, flag, partial,
+                           ghost_blocks(G.ng), pgx(d), pgy(d));
+    else if (what == MOM_STORE)
+        hipLaunchKernelGGL(k_mom_residual<1>, grid, dim3(64, 4), 0, st, d, M, nullptr, nullptr, mask, G, flag, partial,
                            ghost_blocks(G.ng), pgx(d), pgy(d));
     else
-        hipLaunchKernelGGL(k_mom_residual<false>, grid, dim3(64, 4), 0, st, d, M, mask, G, flag, partial,
+        hipLaunchKernelGGL(k_mom_residual<0>, grid, dim3(64, 4), 0, st, d, M, nullptr, nullptr, mask, G, flag, partial,
                            ghost_blocks(G.ng), pgx(d), pgy(d));
+}
+
+void launch_mom_residual_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *Ma,
+                               const MomTable<float> *Mb, unsigned mask, const GhostRows<double> &G,
+                               const uint8_t *flag, double *partial) {
+    hipLaunchKernelGGL(k_mom_residual<2>, dim3(agrid_blocks(d, G.ng), 3), dim3(64, 4), 0, st, d, M, Ma, Mb, mask, G,
+                       flag, partial, ghost_blocks(G.ng), pgx(d), pgy(d));
 }
 
 // FP32 right-hand sides of a correction, b (from x = 0) or the residual,
@@ -1664,23 +1747,28 @@ __global__ void __launch_bounds__(256) k_mom_d2f_first(Dims d, const MomTable<do
               blockIdx.y * 4 + threadIdx.y, k);
 }
 
-// x = e, or x += e
+// x = e, x += e, or x or r = e0 + e
 __global__ void __launch_bounds__(256) k_mom_add(Dims d, const MomTable<double> *M, const MomTable<float> *M32,
-                                                 unsigned mask, int add) {
+                                                 const MomTable<float> *M0, unsigned mask, int add, int to_r) {
     const unsigned c = blockIdx.z / d.nz, k = blockIdx.z % d.nz;
     const int i0 = 2 * (blockIdx.x * 64 + threadIdx.x), j = blockIdx.y * 4 + threadIdx.y;
     if (!((mask >> c) & 1u) || i0 >= d.nx || j >= d.ny) return;
     const long q = cidx(d, i0, j, k);
     const float2 e = *reinterpret_cast<const float2 *>(M32->x[c] + q);
-    double2 *x = reinterpret_cast<double2 *>(M->x[c] + q);
+    double *out = (to_r ? M->r[c] : M->x[c]) + q;
+    double2 *x = reinterpret_cast<double2 *>(out);
     double2 v = make_double2((double)e.x, (double)e.y);
-    if (add) {
+    if (M0) {
+        const float2 o = *reinterpret_cast<const float2 *>(M0->x[c] + q);
+        v.x = (double)o.x + v.x;
+        v.y = (double)o.y + v.y;
+    } else if (add) {
         const double2 o = *x;
         v.x = o.x + v.x;
         v.y = o.y + v.y;
     }
     if (i0 + 1 < d.nx) *x = v;
-    else M->x[c][q] = v.x;
+    else *out = v.x;
 }
 
 void launch_mom_d2f_first(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
@@ -1690,10 +1778,10 @@ void launch_mom_d2f_first(hipStream_t st, const Dims &d, const MomTable<double> 
     hipLaunchKernelGGL(k_mom_d2f_first, g, dim3(64, 4), 0, st, d, M, M32, mask, flag, from_b ? 1 : 0);
 }
 void launch_mom_add(hipStream_t st, const Dims &d, const MomTable<double> *M, const MomTable<float> *M32,
-                    unsigned mask, bool add) {
+                    const MomTable<float> *M0, unsigned mask, bool add, bool to_r) {
     dim3 g = jgrid(d);
     g.z *= 3;
-    hipLaunchKernelGGL(k_mom_add, g, dim3(64, 4), 0, st, d, M, M32, mask, add ? 1 : 0);
+    hipLaunchKernelGGL(k_mom_add, g, dim3(64, 4), 0, st, d, M, M32, M0, mask, add ? 1 : 0, to_r ? 1 : 0);
 }
 #define INST_MOM(T)                                                                                                 \
     template int launch_mom_colour<T>(hipStream_t, const Dims &, const MomTable<T> *, unsigned, const uint8_t *, int, \

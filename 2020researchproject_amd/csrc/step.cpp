@@ -313,25 +313,20 @@ static void wait_epoch(hipStream_t st, unsigned *ep, unsigned e) {
 static void wait_published(hipStream_t st, KPub *pub_h, unsigned e) { wait_epoch(st, &pub_h->epoch, e); }
 
 // The first nv sums, copied by a small kernel into device-mapped host memory
-// (sums_h) and awaited there
-static void read_sums(IBMSolver *s, int nv) {
+// (sums_h); returns the epoch to wait for
+static unsigned publish_sums(IBMSolver *s, int nv) {
     const unsigned e = ++s->sums_epoch;
     launch_publish(s->stream, s->sums.p, nv, s->sums_d, s->sums_d_epoch, e);
-    wait_epoch(s->stream, s->sums_h_epoch, e);
+    return e;
 }
 
 // The sums (maxima) of nv columns of block partials, formed straight into
-// sums_h[slot..] (sum_publish: the epoch to wait for; an earlier one's sums are
-// then there too)
+// sums_h[slot..]; returns the epoch to wait for (an earlier one's sums are then
+// there too)
 static unsigned sum_publish(IBMSolver *s, long nblk, int nv, int reduce_max = 0, int slot = 0) {
     const unsigned e = ++s->sums_epoch;
     launch_sum_publish(s->stream, s->partial.p, nblk, nv, s->sums_d + slot, reduce_max, s->sums_d_epoch, e);
     return e;
-}
-
-// and awaited there
-static void sum_read(IBMSolver *s, long nblk, int nv, int reduce_max = 0) {
-    wait_epoch(s->stream, s->sums_h_epoch, sum_publish(s, nblk, nv, reduce_max));
 }
 
 // Finalize kernel `op` over the block partials, with the resulting scalars
@@ -1572,6 +1567,7 @@ static void report_solve(IBMSolver *s, int sk, double rel, int it) {
 // overlaps them.
 template <typename F>
 static void momentum_concurrent(IBMSolver *s, F &&norms) {
+    s->lanes_used = true;
     const Dims &d = s->d;
     const GhostRows<double> &G = s->gmom.G64;
     const uint8_t *flag = s->flag.p;
@@ -1820,14 +1816,24 @@ static void solve_system(IBMSolver *s, int sk, const double *b, double *x, doubl
 //     estimated rate asks for, then the FP64 residual norm; further rounds at
 //     the rate the last one showed.
 //   Mixed-Krylov mode: FP32 sweeps inside FP64 refinement. Each round: FP32
-//     right-hand side (the FP64 residual; the first colour written in the same
-//     launch), m sweeps from zero, x += e in FP64, FP64 residual and its norm.
+//     right-hand side (b, then the FP64 residual; the first colour written in
+//     the same launch), m sweeps from zero, FP64 residual and its norm of the
+//     sum of the corrections.
 // The stopping test is the reference's ||b - A x|| <= tol ||b|| in FP64.
 // A component whose residual stops falling by at least 10x per round goes to
 // BiCGSTAB, as do all three where the rate is above kMomMaxRate. FP64, sphere
 // 256 x 128 x 128 at 1e-12: 6 sweeps (12 launches of 70 us) and one residual
 // against 5 BiCGSTAB iterations of 8 kernels per component.
 // ---------------------------------------------------------------------------
+// Contraction of a sweep at ghost rows, which lag the fluid rows they
+// interpolate, whatever the fluid rows' rate: 1.6e-3 to 2.9e-3 measured on the
+// spheres 98 x 47 x 51 and 133 x 67 x 61 and the canopy 160 x 80 x 48. With the
+// fluid rows' rate alone (1e-4, 5e-4, 2e-8) the first round had a sweep or two
+// too few and a round more followed (sphere 133 x 67 x 61: 70 us against 22 for
+// a sweep more). What that third round gave beyond the tolerance a Jacobi step
+// gives as well (k_mom_residual<3>, 8 us); at larger rates there were two
+// rounds, and the step would gain less (256 x 128 x 128: 70 us).
+static const double kMomGhostRate = 3e-3;
 static const double kMomRoundTarget = 1e-6;  // residual reduction aimed at per FP32 round
 // Largest rho_J^2 for which sweeps are used, the largest measured: ms per step
 // at 1e-12, sweeps against BiCGSTAB (its three solves on streams of their
@@ -1843,7 +1849,8 @@ static int momentum_sweeps(IBMSolver *s) {
     for (int i = 0; i < s->Nx; i++) mx[0] = std::max(mx[0], H1(s->kW, i) + H1(s->kE, i));
     for (int j = 0; j < s->Ny; j++) mx[1] = std::max(mx[1], H1(s->kS, j) + H1(s->kN, j));
     for (int k = 0; k < s->Nz; k++) mx[2] = std::max(mx[2], H1(s->kD, k) + H1(s->kU, k));
-    const double sk = mx[0] + mx[1] + mx[2], rj = sk / (1 + sk), rate = rj * rj;
+    const double sk = mx[0] + mx[1] + mx[2], rj = sk / (1 + sk);
+    const double rate = s->ng > 0 ? std::max(rj * rj, kMomGhostRate) : rj * rj;
     s->mom_rate = rate;
     const double target = s->precision == IBM3D_PREC_FP64 ? 0.5 * s->tol : kMomRoundTarget;
     s->mom_sweeps = (rate > 0 && rate <= kMomMaxRate)
@@ -1879,6 +1886,8 @@ void build_momentum_tables(IBMSolver *s) {
         for (int k = 0; k < 2; k++) f.gv[c][k] = s->mgv32.p + (2 * c + k) * ng;
     }
     s->mt32.upload(&f, 1);
+    for (int c = 0; c < 3; c++) f.x[c] = c == 0 ? s->ref_e32b.p : reinterpret_cast<float *>(s->mlane[c - 1].v[1].p);
+    s->mt32b.upload(&f, 1);
 }
 
 // n sweeps of the components in mask (zero: from a zero start, whose first
@@ -1903,81 +1912,115 @@ static void momentum_smooth(IBMSolver *s, const MomTable<T> *M, unsigned mask, i
         }
 }
 
-// The three momentum solves by sweeps; components that do not converge this
-// way are solved by solve_system. norms(bn, e): the stopping norms, once epoch e
-// of the sums is there.
-template <typename F>
-static void momentum_sweep_solve(IBMSolver *s, F &&norms) {
+// One round of sweeps of the components in mask, ending with the residuals'
+// norms on their way to sums_h. FP32: rounds 0 and 1 keep their corrections e0
+// and e1 apart; x = e0 + e1 is formed when both are there (x = e0 if round 0 is
+// to be the only one; with a Jacobi step where the ghost rows bound the rate),
+// and r only where a third round follows.
+struct MomSweeps {
+    int round = 0, prev = -1, sweeps[3] = {0, 0, 0};
+};
+static unsigned momentum_sweep_round(IBMSolver *s, MomSweeps &st, unsigned mask, int n, bool only) {
     const Dims &d = s->d;
-    const int m = momentum_sweeps(s);
-    const double cb = ncells(s);
-    const long na = apply_partials(d, s->gmom.G64.ng);
+    const int round = st.round++;
+    const double act = __builtin_popcount(mask), cb = ncells(s);
     const bool f64 = s->precision == IBM3D_PREC_FP64;
-    double rn[3] = {0, 0, 0}, rate[3] = {s->mom_rate, s->mom_rate, s->mom_rate};
-    int sweeps[3] = {0, 0, 0}, prev = -1;
-    bool fallback[3] = {false, false, false};
+    const bool jacobi = !f64 && round == 1 && s->ng > 0 && s->mom_rate <= kMomGhostRate;
+    if (f64) {
+        momentum_smooth<double>(s, s->mt64.p, mask, n, round == 0, false, st.prev);
+    } else {
+        const MomTable<float> *m32 = round == 1 ? s->mt32b.p : s->mt32.p;
+        if (round > 1)
+            TIMED("mom_residual64", act * cb * 3 * 8,
+                  launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p, MOM_STORE, s->partial.p));
+        if (round != 1)
+            TIMED("mom_d2f", act * cb * 17,
+                  launch_mom_d2f_first(s->stream, d, s->mt64.p, m32, mask, s->flag.p, round == 0));
+        momentum_smooth<float>(s, m32, mask, n, true, true, st.prev);
+        if (round || only)
+            TIMED("mom_add", act * cb * (round > 1 ? 20 : round ? 16 : 12),
+                  launch_mom_add(s->stream, d, s->mt64.p, m32, round == 1 ? s->mt32.p : nullptr, mask, round > 1,
+                                 jacobi));
+    }
+    if (!f64 && round == 0)
+        TIMED("mom_residual64", act * cb * 20,
+              launch_mom_residual_first(s->stream, d, s->mt64.p, s->mt32.p, s->mt32b.p, mask, s->gmom.G64, s->flag.p,
+                                        s->partial.p));
+    else
+        TIMED("mom_residual64", act * cb * (jacobi ? 3 : 2) * 8,
+              launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p,
+                                  jacobi ? MOM_JACOBI : MOM_NORMS, s->partial.p));
+    for (int l = 0; l < 3; l++) st.sweeps[l] += mask >> l & 1 ? n : 0;
+    return sum_publish(s, apply_partials(d, s->gmom.G64.ng), 3, 0, kMomResidualSlot);
+}
+
+// The rounds that the estimated rate asks for (FP64: one; FP32: a second one
+// where the tolerance is below what one reaches), without a look at the norms:
+// they are read together with the pressure's.
+static unsigned momentum_sweeps_start(IBMSolver *s, MomSweeps &st) {
+    if (s->lanes_used && s->precision != IBM3D_PREC_FP64) {
+        // the second round's corrections share these vectors with the lanes'
+        // BiCGSTAB; the smoother reads (times zero) the padding beside the rows
+        for (auto &L : s->mlane) launch_fill(s->stream, L.v[1].p, s->d.ncell, 0.0);
+        s->lanes_used = false;
+    }
+    const bool two = s->precision != IBM3D_PREC_FP64 && s->tol < kMomRoundTarget;
+    const int m = momentum_sweeps(s);
+    const unsigned e = momentum_sweep_round(s, st, 7, m, !two);
+    if (!two) return e;
+    const double need = std::max(s->tol / kMomRoundTarget, kMomRoundTarget);
+    return momentum_sweep_round(s, st, 7, momentum_round_sweeps(need, s->mom_rate, m), false);
+}
+
+// Whether the three solves meet the tolerance (bn: stopping norms) after the
+// rounds begun; false when more was done: further rounds at what the worst
+// component still lacks and, for a component that does not converge this way,
+// solve_system.
+static bool momentum_sweeps_finish(IBMSolver *s, MomSweeps &st, const double bn[3]) {
+    const int m = momentum_sweeps(s);
+    const bool f64 = s->precision == IBM3D_PREC_FP64;
+    double rn[3] = {bn[0], bn[1], bn[2]}, rate[3] = {s->mom_rate, s->mom_rate, s->mom_rate};
     unsigned mask = 7;
-    double bn[3];
-    for (int round = 0; mask && round < kMomMaxRounds; round++) {
-        const double act = __builtin_popcount(mask);
-        // the first round aims at the tolerance (FP64) or the FP32 limit,
-        // later ones at what the worst component still lacks
-        int mr = m;
-        if (round) {
-            mr = 1;
-            for (int l = 0; l < 3; l++)
-                if (mask >> l & 1) {
-                    double need = s->tol * bn[l] / rn[l];
-                    if (!f64) need = std::max(need, kMomRoundTarget);
-                    mr = std::max(mr, momentum_round_sweeps(need, rate[l], m));
-                }
-        }
-        if (f64) {
-            momentum_smooth<double>(s, s->mt64.p, mask, mr, round == 0, false, prev);
-        } else {
-            TIMED("mom_d2f", act * cb * 17, launch_mom_d2f_first(s->stream, d, s->mt64.p, s->mt32.p, mask, s->flag.p,
-                                                                 round == 0));
-            momentum_smooth<float>(s, s->mt32.p, mask, mr, true, true, prev);
-            TIMED("mom_add", act * cb * (round ? 20 : 12),
-                  launch_mom_add(s->stream, d, s->mt64.p, s->mt32.p, mask, round > 0));
-        }
-        TIMED("mom_residual64", act * cb * (f64 ? 2 : 3) * 8,
-              launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p, !f64, s->partial.p));
-        const unsigned e = sum_publish(s, na, 3, 0, kMomResidualSlot);
-        if (round == 0) {
-            // the norms are read behind the first round's launches
-            norms(bn, e);
-            for (int l = 0; l < 3; l++) {
-                // a zero right-hand side has the zero solution; a non-finite
-                // one stays active, so its residual reports the error
-                rn[l] = bn[l];
-                if (bn[l] != 0) continue;
-                mask &= ~(1u << l);
-                launch_zero<double>(s->stream, d, s->us[l].p);
-                report_solve(s, l, 0.0, 0);
-            }
-        } else {
-            wait_epoch(s->stream, s->sums_h_epoch, e);
-        }
+    bool fallback[3] = {false, false, false};
+    for (int l = 0; l < 3; l++) {
+        // a zero right-hand side has the zero solution; a non-finite one stays
+        // active, so its residual reports the error
+        if (bn[l] != 0) continue;
+        mask &= ~(1u << l);
+        launch_zero<double>(s->stream, s->d, s->us[l].p);
+        report_solve(s, l, 0.0, 0);
+    }
+    for (int mr = 0, looked = 0;; looked++) {
         for (int l = 0; l < 3; l++) {
             if (!(mask >> l & 1)) continue;
-            sweeps[l] += mr;
             const double r = std::sqrt(s->sums_h[kMomResidualSlot + l]);
-            const bool stalled = round > 0 && !(r <= 0.1 * rn[l]);
-            // rate shown by this round's sweeps (FP64: from ||b||), kept below 1
-            if (f64) rate[l] = std::min(0.5, std::max(1e-6, std::pow(r / rn[l], 1.0 / mr)));
+            const bool stalled = looked > 0 && !(r <= 0.1 * rn[l]);
+            // rate shown by the sweeps looked at (FP64: from ||b||), kept below 1
+            if (f64)
+                rate[l] = std::min(0.5, std::max(1e-6, std::pow(r / rn[l], 1.0 / (looked ? mr : st.sweeps[l]))));
             rn[l] = r;
             if (!std::isfinite(r) || r <= s->tol * bn[l]) {
                 mask &= ~(1u << l);
-                report_solve(s, l, r / bn[l], sweeps[l]);
+                report_solve(s, l, r / bn[l], st.sweeps[l]);
             } else if (stalled) {
                 mask &= ~(1u << l);
                 fallback[l] = true;
             }
         }
+        if (looked == 0 && mask == 0) return true;
+        if (mask == 0 || st.round >= kMomMaxRounds) break;
+        mr = 1;
+        for (int l = 0; l < 3; l++)
+            if (mask >> l & 1) {
+                double need = s->tol * bn[l] / rn[l];
+                if (!f64) need = std::max(need, kMomRoundTarget);
+                mr = std::max(mr, momentum_round_sweeps(need, rate[l], m));
+            }
+        wait_epoch(s->stream, s->sums_h_epoch, momentum_sweep_round(s, st, mask, mr, false));
     }
     for (int l = 0; l < 3; l++)
         if ((mask >> l & 1) || fallback[l]) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
+    return false;
 }
 
 // The three momentum solves by the transforms, and their residuals' norms to
@@ -1994,7 +2037,7 @@ static void momentum_direct(IBMSolver *s) {
     }
     TIMED("mom_separable", 6 * cb, launch_separable_batch(s->stream, s->d, 3, s->sep_mom, b, s1, s2, x));
     TIMED("mom_residual64", 2 * cb,
-          launch_mom_residual(s->stream, s->d, s->mt64.p, 7, s->gmom.G64, s->flag.p, false, s->partial.p));
+          launch_mom_residual(s->stream, s->d, s->mt64.p, 7, s->gmom.G64, s->flag.p, MOM_NORMS, s->partial.p));
     sum_publish(s, apply_partials(s->d, 0), 3, 0, kMomResidualSlot);
 }
 
@@ -2078,17 +2121,18 @@ static void do_step(IBMSolver *s) {
     // the outflow faces' norms join them
     bool conv = false;
     for (const HostBC &B : s->bc) conv |= B.type == BC_CONVECTIVE_OUTFLOW;
-    unsigned me = 0;
-    if (conv) launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
-    else me = sum_publish(s, conv_rhs_blocks(s->d), 3);
-    conv_outflow(s, 0);
+    if (conv) {
+        launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
+        conv_outflow(s, 0);
+        publish_sums(s, kConvNormSlot + 18);
+    } else {
+        sum_publish(s, conv_rhs_blocks(s->d), 3);
+    }
     double fnorm[4];
     OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm), opp{};
     bc_rhs(s, ob, 0, 3);
     // stopping norms of the momentum solves: the right-hand sides' sums, plus
-    // the BC rows' and forcing parts; read once epoch e of the sums is there
-    // (before the solves where outflow faces have their share: the whole table
-    // of sums is read then)
+    // the BC rows' and forcing parts
     double bn[3];
     auto form_norms = [&] {
         for (int l = 0; l < 3; l++) {
@@ -2098,35 +2142,37 @@ static void do_step(IBMSolver *s) {
             bn[l] = std::sqrt(bn2);
         }
     };
-    if (conv) {
-        read_sums(s, kConvNormSlot + 18);
+    auto read_norms = [&](double out[3]) {
+        wait_epoch(s->stream, s->sums_h_epoch, s->sums_epoch);
         form_norms();
-    }
-    auto mom_norms = [&](double out[3], unsigned e) {
-        wait_epoch(s->stream, s->sums_h_epoch, e);
-        if (!conv) form_norms();
         std::copy(bn, bn + 3, out);
     };
-    // momentum Helmholtz solves: by sweeps; else the three at once on their
-    // lanes, or one after the other (mixed defect-correction mode, and under
-    // the per-kernel timers, whose events are recorded on the solver's stream)
-    auto mom_iterate = [&](unsigned e) {
-        if (s->precision != IBM3D_PREC_MIXED && s->mom_solver == 0 && momentum_sweeps(s) > 0) {
-            momentum_sweep_solve(s, mom_norms);
+    // momentum Helmholtz solves: directly, or by sweeps, with a look at the
+    // residuals together with the pressure's (the step goes on from further
+    // solves if one of them is not below the tolerance); else the three at once
+    // on their lanes, or one after the other (mixed defect-correction mode, and
+    // under the per-kernel timers, whose events are recorded on the solver's
+    // stream)
+    const bool sweep = s->precision != IBM3D_PREC_MIXED && s->mom_solver == 0 && momentum_sweeps(s) > 0;
+    MomSweeps sweeps;
+    auto mom_iterate = [&] {
+        if (sweep) {
+            wait_epoch(s->stream, s->sums_h_epoch, momentum_sweeps_start(s, sweeps));
+            form_norms();
+            momentum_sweeps_finish(s, sweeps, bn);
         } else if (s->mom_lanes && s->timing == 0 && s->precision != IBM3D_PREC_MIXED) {
-            momentum_concurrent(s, [&](double out[3]) { mom_norms(out, e); });
+            momentum_concurrent(s, read_norms);
         } else {
             double n3[3];
-            mom_norms(n3, e);
+            read_norms(n3);
             for (int l = 0; l < 3; l++) solve_system(s, l, s->b[l].p, s->us[l].p, n3[l]);
         }
     };
-    // or directly: the residuals are then looked at together with the
-    // pressure's, and the step goes on from the iterative solves if one of them
-    // is not below the tolerance
-    bool mom_open = s->sep_mom_on && s->mom_solver == 0;
-    if (mom_open) momentum_direct(s);
-    else mom_iterate(conv ? s->sums_epoch : me);
+    const bool mom_direct = s->sep_mom_on && s->mom_solver == 0;
+    bool mom_open = mom_direct || sweep;
+    if (mom_direct) momentum_direct(s);
+    else if (sweep) momentum_sweeps_start(s, sweeps);
+    else mom_iterate();
     const bool direct = s->sep_on;
     double bnp = 0;
     unsigned fe = 0;
@@ -2150,10 +2196,14 @@ static void do_step(IBMSolver *s) {
         wait_epoch(s->stream, s->sums_h_epoch, pe);
         bnp = std::sqrt(s->sums_h[kPoissonSlot] + s->sys[3].bc_norm2 + pnorm[3]);
         if (!mom_open) break;
-        if (!conv) form_norms();
+        form_norms();
         mom_open = false;
-        if (momentum_direct_met(s, bn)) break;
-        mom_iterate(pe);
+        if (mom_direct) {
+            if (momentum_direct_met(s, bn)) break;
+            mom_iterate();
+        } else if (momentum_sweeps_finish(s, sweeps, bn)) {
+            break;
+        }
         ob = make_outer(s, BCD_FIELDS, s->time, fnorm);  // its buffers hold the pressure's data now
     }
     if (!direct || !separable_finish(s, s->bp.p, s->pp.p, fe, bnp)) solve_system(s, 3, s->bp.p, s->pp.p, bnp);
@@ -2255,7 +2305,7 @@ void body_force_impl(IBMSolver *s, double *dst) {
 
 void body_force_read(IBMSolver *s, double out[3]) {
     body_force_impl(s, s->sums.p);
-    read_sums(s, 3);
+    wait_epoch(s->stream, s->sums_h_epoch, publish_sums(s, 3));
     for (int a = 0; a < 3; a++) out[a] = s->sums_h[a];
 }
 
@@ -2263,7 +2313,7 @@ double max_div_impl(IBMSolver *s) {
     const double *U3[3] = {s->F[0].p, s->F[1].p, s->F[2].p};
     launch_maxdiv(s->stream, s->geo, s->flag.p, s->pin, U3, s->partial.p);
     launch_sum_partials(s->stream, s->partial.p, maxdiv_blocks(s->d), 1, s->sums.p, 1);
-    read_sums(s, 1);
+    wait_epoch(s->stream, s->sums_h_epoch, publish_sums(s, 1));
     return s->sums_h[0];
 }
 
