@@ -658,6 +658,7 @@ static void alloc_fields(IBMSolver *s) {
     nb = std::max(nb, apply_partials(s->d, s->ng) + 64);
     nb = std::max(nb, vec_partials(s->d) + 64);
     nb = std::max(nb, separable_partials(s->d));
+    // (a pressure solve's own sums follow those of its right-hand side)
     s->partial.alloc((size_t)nb * 4);
 }
 

@@ -332,7 +332,7 @@ namespace ibm {
 // slots of IBMSolver::sums: 0..11 reductions of the step kernels (0..2 the
 // momentum right-hand sides), 12..29 the convective outflow faces' BC-row norms
 // (3 per face, bc[] order)
-constexpr int kPoissonSlot = 4, kMomResidualSlot = 8;
+constexpr int kPoissonSlot = 4, kPressureSlot = 5, kMomResidualSlot = 8;
 constexpr int kSumSlots = 32;
 constexpr int kConvNormSlot = 12;
 // fields of up to this many values (1 MiB) cross between host and device

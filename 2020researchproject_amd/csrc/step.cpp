@@ -247,7 +247,7 @@ void build_outer_rules(IBMSolver *s) {
 
 // Boundary data of the systems comp..comp+n-1 into their right-hand sides;
 // faces whose data are zero for all of them take no part.
-static void bc_rhs(IBMSolver *s, const OuterParams &op, int comp, int n) {
+static void bc_rhs(IBMSolver *s, const OuterParams &op, int comp, int n, const SumRiders &sums = {}) {
     BcRhs p{};
     p.n = n;
     p.comp = comp;
@@ -267,7 +267,7 @@ static void bc_rhs(IBMSolver *s, const OuterParams &op, int comp, int n) {
             p.K[ax][hi] = s->g1d[6 + 2 * ax + hi].p;
             p.face[p.nface++] = 2 * ax + hi;
         }
-    TIMED("bc_rhs", 0, launch_bc_rhs(s->stream, s->geo, op, p));
+    TIMED("bc_rhs", 0, launch_bc_rhs(s->stream, s->geo, op, p, sums));
 }
 
 static void update_outer(IBMSolver *s) {
@@ -329,22 +329,29 @@ static unsigned sum_publish(IBMSolver *s, long nblk, int nv, int reduce_max = 0,
     return e;
 }
 
+// The same sums as a rider of a boundary launch: nblk x nv partials to
+// sums_h[slot..]; the last rider's epoch is s->sums_epoch
+static void add_rider(IBMSolver *s, SumRiders &sums, const double *partial, long nblk, int nv, int slot) {
+    sums.r[sums.n].partial = partial;
+    sums.r[sums.n].nblk = nblk;
+    sums.r[sums.n].nv = nv;
+    sums.r[sums.n].out = s->sums_d + slot;
+    if (sums.n++ == 0) {
+        sums.epoch_out = s->sums_d_epoch;
+        sums.epoch = ++s->sums_epoch;
+    }
+}
+
 // Finalize kernel `op` over the block partials, with the resulting scalars
 // published into host memory, then a wait for them there: no copy and no
 // stream synchronisation on the Krylov loop's path (each end of iteration
 // otherwise costs a copy and a wake-up of the host thread).
-static unsigned finalize_publish(IBMSolver *s, int op, long nblk, int nv) {
+static void finalize_read(IBMSolver *s, int op, long nblk, int nv) {
     const unsigned e = ++s->pub_epoch;
     launch_finalize(s->stream, op, s->partial.p, nblk, nv, s->ks.p, &s->pub_d->ks, &s->pub_d->epoch, e);
-    return e;
-}
-
-static void finalize_wait(IBMSolver *s, unsigned e) {
     wait_published(s->stream, s->pub_h, e);
     memcpy((void *)s->ks_h, (const void *)&s->pub_h->ks, sizeof(KScal));
 }
-
-static void finalize_read(IBMSolver *s, int op, long nblk, int nv) { finalize_wait(s, finalize_publish(s, op, nblk, nv)); }
 
 // ---------------------------------------------------------------------------
 // multigrid hierarchy of the pressure system
@@ -1723,9 +1730,10 @@ static void momentum_concurrent(IBMSolver *s, F &&norms) {
 // level of the transforms (1e-12 .. 1e-10 of ||b||), a second one that of the
 // residual. A solve whose residual no longer halves is left to the iterative
 // path (false); its reason is the tolerance, not the method. separable_round
-// enqueues a round and returns the epoch of its residual's norms.
-static unsigned separable_round(IBMSolver *s, const double *b, double *x, bool first) {
+// enqueues a round, up to the partial sums of its residual's norms.
+static void separable_round(IBMSolver *s, const double *b, double *x, bool first) {
     const Dims &d = s->d;
+    double *partial = s->partial.p + conv_rhs_blocks(d);  // behind the right-hand side's
     const NormSpec ns{1, s->ks1d[0].p, s->ks1d[1].p, s->ks1d[2].p, s->flag.p, s->pin};
     double *r = s->kry.v64[0].p, *s1 = s->kry.v64[1].p, *s2 = s->kry.v64[2].p;
     const double cb = ncells(s) * 8;
@@ -1735,30 +1743,35 @@ static unsigned separable_round(IBMSolver *s, const double *b, double *x, bool f
               launch_separable_body(s->stream, d, s->sep, s->cap, rhs, s1, s2, s->kry.v64[3].p, x, !first));
     else
         TIMED("separable", (first ? 6 : 7) * cb,
-              launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, !first, s->partial.p));
+              launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, !first, partial));
     TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r, ns,
-                                                      s->partial.p));
-    return finalize_publish(s, 4, apply_partials(d, s->gp.G64.ng), 2);
+                                                      partial));
 }
 
-// The rounds after the first, whose norms come with epoch e; bn: stopping norm
-static bool separable_finish(IBMSolver *s, const double *b, double *x, unsigned e, double bn) {
+// Whether the first round, whose norms are in sums_h, met the tolerance (bn:
+// stopping norm), and the rounds after it; `more`: whether there were any
+static bool separable_finish(IBMSolver *s, const double *b, double *x, double bn, bool &more) {
     double last = 0;
     for (int round = 1;; round++) {
-        finalize_wait(s, e);
         if (bn == 0) {
             launch_zero<double>(s->stream, s->d, x);
+            more = true;
             report_solve(s, 3, 0, 0);
             return true;
         }
-        const double rn = std::sqrt(s->ks_h->rrn);
+        const double rn = std::sqrt(s->sums_h[kPressureSlot + 1]);
         if (rn <= s->tol * bn) {
             report_solve(s, 3, rn / bn, round);
             return true;
         }
         if (!(round == 1 || rn <= 0.5 * last) || !std::isfinite(rn)) break;
         last = rn;
-        e = separable_round(s, b, x, false);
+        more = true;
+        separable_round(s, b, x, false);
+        const unsigned e = ++s->sums_epoch;
+        launch_sum_publish(s->stream, s->partial.p + conv_rhs_blocks(s->d), apply_partials(s->d, s->gp.G64.ng), 2,
+                           s->sums_d + kPressureSlot, 0, s->sums_d_epoch, e);
+        wait_epoch(s->stream, s->sums_h_epoch, e);
     }
     // with a body the memory of the capacitance matrix is the hierarchy's: the
     // solver goes over to the iterative path for good
@@ -1912,15 +1925,15 @@ static void momentum_smooth(IBMSolver *s, const MomTable<T> *M, unsigned mask, i
         }
 }
 
-// One round of sweeps of the components in mask, ending with the residuals'
-// norms on their way to sums_h. FP32: rounds 0 and 1 keep their corrections e0
+// One round of sweeps of the components in mask, ending with the partial sums
+// of the residuals' norms. FP32: rounds 0 and 1 keep their corrections e0
 // and e1 apart; x = e0 + e1 is formed when both are there (x = e0 if round 0 is
 // to be the only one; with a Jacobi step where the ghost rows bound the rate),
 // and r only where a third round follows.
 struct MomSweeps {
     int round = 0, prev = -1, sweeps[3] = {0, 0, 0};
 };
-static unsigned momentum_sweep_round(IBMSolver *s, MomSweeps &st, unsigned mask, int n, bool only) {
+static void momentum_sweep_round(IBMSolver *s, MomSweeps &st, unsigned mask, int n, bool only) {
     const Dims &d = s->d;
     const int round = st.round++;
     const double act = __builtin_popcount(mask), cb = ncells(s);
@@ -1951,13 +1964,17 @@ static unsigned momentum_sweep_round(IBMSolver *s, MomSweeps &st, unsigned mask,
               launch_mom_residual(s->stream, d, s->mt64.p, mask, s->gmom.G64, s->flag.p,
                                   jacobi ? MOM_JACOBI : MOM_NORMS, s->partial.p));
     for (int l = 0; l < 3; l++) st.sweeps[l] += mask >> l & 1 ? n : 0;
-    return sum_publish(s, apply_partials(d, s->gmom.G64.ng), 3, 0, kMomResidualSlot);
+}
+
+// the norms of the last momentum residual, in a launch of their own or riding
+static unsigned momentum_publish(IBMSolver *s) {
+    return sum_publish(s, apply_partials(s->d, s->gmom.G64.ng), 3, 0, kMomResidualSlot);
 }
 
 // The rounds that the estimated rate asks for (FP64: one; FP32: a second one
 // where the tolerance is below what one reaches), without a look at the norms:
 // they are read together with the pressure's.
-static unsigned momentum_sweeps_start(IBMSolver *s, MomSweeps &st) {
+static void momentum_sweeps_start(IBMSolver *s, MomSweeps &st) {
     if (s->lanes_used && s->precision != IBM3D_PREC_FP64) {
         // the second round's corrections share these vectors with the lanes'
         // BiCGSTAB; the smoother reads (times zero) the padding beside the rows
@@ -1966,10 +1983,10 @@ static unsigned momentum_sweeps_start(IBMSolver *s, MomSweeps &st) {
     }
     const bool two = s->precision != IBM3D_PREC_FP64 && s->tol < kMomRoundTarget;
     const int m = momentum_sweeps(s);
-    const unsigned e = momentum_sweep_round(s, st, 7, m, !two);
-    if (!two) return e;
+    momentum_sweep_round(s, st, 7, m, !two);
+    if (!two) return;
     const double need = std::max(s->tol / kMomRoundTarget, kMomRoundTarget);
-    return momentum_sweep_round(s, st, 7, momentum_round_sweeps(need, s->mom_rate, m), false);
+    momentum_sweep_round(s, st, 7, momentum_round_sweeps(need, s->mom_rate, m), false);
 }
 
 // Whether the three solves meet the tolerance (bn: stopping norms) after the
@@ -2016,15 +2033,16 @@ static bool momentum_sweeps_finish(IBMSolver *s, MomSweeps &st, const double bn[
                 if (!f64) need = std::max(need, kMomRoundTarget);
                 mr = std::max(mr, momentum_round_sweeps(need, rate[l], m));
             }
-        wait_epoch(s->stream, s->sums_h_epoch, momentum_sweep_round(s, st, mask, mr, false));
+        momentum_sweep_round(s, st, mask, mr, false);
+        wait_epoch(s->stream, s->sums_h_epoch, momentum_publish(s));
     }
     for (int l = 0; l < 3; l++)
         if ((mask >> l & 1) || fallback[l]) solve_system(s, l, s->b[l].p, s->us[l].p, bn[l]);
     return false;
 }
 
-// The three momentum solves by the transforms, and their residuals' norms to
-// sums_h
+// The three momentum solves by the transforms, and the partial sums of their
+// residuals' norms
 static void momentum_direct(IBMSolver *s) {
     const double cb = ncells(s) * 8 * 3;
     const double *b[3];
@@ -2038,7 +2056,6 @@ static void momentum_direct(IBMSolver *s) {
     TIMED("mom_separable", 6 * cb, launch_separable_batch(s->stream, s->d, 3, s->sep_mom, b, s1, s2, x));
     TIMED("mom_residual64", 2 * cb,
           launch_mom_residual(s->stream, s->d, s->mt64.p, 7, s->gmom.G64, s->flag.p, MOM_NORMS, s->partial.p));
-    sum_publish(s, apply_partials(s->d, 0), 3, 0, kMomResidualSlot);
 }
 
 // whether all of them meet the tolerance (bn: stopping norms)
@@ -2125,12 +2142,14 @@ static void do_step(IBMSolver *s) {
         launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
         conv_outflow(s, 0);
         publish_sums(s, kConvNormSlot + 18);
-    } else {
-        sum_publish(s, conv_rhs_blocks(s->d), 3);
     }
     double fnorm[4];
     OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm), opp{};
-    bc_rhs(s, ob, 0, 3);
+    {
+        SumRiders norms{};
+        if (!conv) add_rider(s, norms, s->partial.p, conv_rhs_blocks(s->d), 3, 0);
+        bc_rhs(s, ob, 0, 3, norms);
+    }
     // stopping norms of the momentum solves: the right-hand sides' sums, plus
     // the BC rows' and forcing parts
     double bn[3];
@@ -2157,7 +2176,8 @@ static void do_step(IBMSolver *s) {
     MomSweeps sweeps;
     auto mom_iterate = [&] {
         if (sweep) {
-            wait_epoch(s->stream, s->sums_h_epoch, momentum_sweeps_start(s, sweeps));
+            momentum_sweeps_start(s, sweeps);
+            wait_epoch(s->stream, s->sums_h_epoch, momentum_publish(s));
             form_norms();
             momentum_sweeps_finish(s, sweeps, bn);
         } else if (s->mom_lanes && s->timing == 0 && s->precision != IBM3D_PREC_MIXED) {
@@ -2173,14 +2193,26 @@ static void do_step(IBMSolver *s) {
     if (mom_direct) momentum_direct(s);
     else if (sweep) momentum_sweeps_start(s, sweeps);
     else mom_iterate();
+    // outer layers of p' and K3, the projection (its results are not the
+    // fields yet, so it may run before the solves have been looked at)
+    auto project = [&](const SumRiders &sums) {
+        TIMED("outer_sol", 0, launch_outer(s->stream, s->d, opp, s->outer_rules.p, {{s->pp.p}, {OUT_DP}, 1}, sums));
+        const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};
+        const double *Fs[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
+        double *un[3] = {s->un[0].p, s->un[1].p, s->un[2].p};
+        double *Fn[3] = {s->Fn[0].p, s->Fn[1].p, s->Fn[2].p};
+        TIMED("k3_update", cn * (15 * 8 + 1),
+              launch_update(s->stream, s->geo, sp, s->flag.p, s->p.p, s->pp.p, us3, Fs, s->pn.p, un, Fn));
+    };
     const bool direct = s->sep_on;
     double bnp = 0;
-    unsigned fe = 0;
     for (;;) {
         // outer layers of the three solutions from their BC rows (the per-component
         // fill of each u* with the solve's boundary data, all three in one pass)
+        SumRiders mom{}, pres{};
+        if (mom_open) add_rider(s, mom, s->partial.p, apply_partials(s->d, s->gmom.G64.ng), 3, kMomResidualSlot);
         TIMED("outer_sol", 0, launch_outer(s->stream, s->d, ob, s->outer_rules.p,
-                                           {{s->us[0].p, s->us[1].p, s->us[2].p}, {0, 1, 2}, 3}));
+                                           {{s->us[0].p, s->us[1].p, s->us[2].p}, {0, 1, 2}, 3}, mom));
         // K2: U*, Poisson RHS
         const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};
         double *Fs[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
@@ -2188,12 +2220,18 @@ static void do_step(IBMSolver *s) {
         const double *Fc[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
         TIMED("k2_poisson_rhs", cn * (4 * 8 + 1),
               launch_poisson_rhs(s->stream, s->geo, sp, s->flag.p, s->pin, Fc, s->bp.p, s->partial.p));
-        const unsigned pe = sum_publish(s, conv_rhs_blocks(s->d), 1, 0, kPoissonSlot);
         double pnorm[4];
         opp = make_outer(s, BCD_PSOL, s->time, pnorm);
-        bc_rhs(s, opp, 3, 1);
-        if (direct) fe = separable_round(s, s->bp.p, s->pp.p, true);
-        wait_epoch(s->stream, s->sums_h_epoch, pe);
+        if (!direct) add_rider(s, pres, s->partial.p, conv_rhs_blocks(s->d), 1, kPoissonSlot);
+        bc_rhs(s, opp, 3, 1, pres);
+        if (direct) {
+            separable_round(s, s->bp.p, s->pp.p, true);
+            add_rider(s, pres, s->partial.p, conv_rhs_blocks(s->d), 1, kPoissonSlot);
+            add_rider(s, pres, s->partial.p + conv_rhs_blocks(s->d), apply_partials(s->d, s->gp.G64.ng), 2,
+                      kPressureSlot);
+            project(pres);
+        }
+        wait_epoch(s->stream, s->sums_h_epoch, s->sums_epoch);
         bnp = std::sqrt(s->sums_h[kPoissonSlot] + s->sys[3].bc_norm2 + pnorm[3]);
         if (!mom_open) break;
         form_norms();
@@ -2206,17 +2244,12 @@ static void do_step(IBMSolver *s) {
         }
         ob = make_outer(s, BCD_FIELDS, s->time, fnorm);  // its buffers hold the pressure's data now
     }
-    if (!direct || !separable_finish(s, s->bp.p, s->pp.p, fe, bnp)) solve_system(s, 3, s->bp.p, s->pp.p, bnp);
-    TIMED("outer_sol", 0, launch_outer(s->stream, s->d, opp, s->outer_rules.p, {{s->pp.p}, {OUT_DP}, 1}));
-    // K3: projection
-    {
-        const double *us3[3] = {s->us[0].p, s->us[1].p, s->us[2].p};
-        const double *Fs[3] = {s->Fs[0].p, s->Fs[1].p, s->Fs[2].p};
-        double *un[3] = {s->un[0].p, s->un[1].p, s->un[2].p};
-        double *Fn[3] = {s->Fn[0].p, s->Fn[1].p, s->Fn[2].p};
-        TIMED("k3_update", cn * (15 * 8 + 1),
-              launch_update(s->stream, s->geo, sp, s->flag.p, s->p.p, s->pp.p, us3, Fs, s->pn.p, un, Fn));
+    bool more = !direct;
+    if (!direct || !separable_finish(s, s->bp.p, s->pp.p, bnp, more)) {
+        more = true;
+        solve_system(s, 3, s->bp.p, s->pp.p, bnp);
     }
+    if (more) project({});
     // pointer swaps  <- src/ibm3d_fracstep.c:795-804
     for (int l = 0; l < 3; l++) {
         std::swap(s->u[l], s->un[l]);

@@ -86,6 +86,20 @@ struct OuterFields {
     int kind[4];
     int n;
 };
+// Sums of columns of block partials that ride in a boundary launch as one more
+// workgroup and go to device-mapped host memory, with the epoch after the last.
+struct SumRiders {
+    struct {
+        const double *partial;
+        long nblk;
+        int nv;
+        double *out;
+    } r[2];
+    int n;
+    unsigned *epoch_out;
+    unsigned epoch;
+};
+
 // Rule of an outer position: value = g * (boundary value) + sum_t c[t] (value
 // at position n[t] of the axis); keep: not written. Table [kind][axis][hi][layer].
 struct OuterRule {
@@ -94,7 +108,7 @@ struct OuterRule {
 };
 constexpr int kOuterRules = 5 * 12;
 void launch_outer(hipStream_t st, const Dims &d, const OuterParams &op, const OuterRule *rules,
-                  const OuterFields &fs);
+                  const OuterFields &fs, const SumRiders &sums = {});
 // Boundary data of the right-hand sides b[0..n) of components comp..comp+n-1:
 // faces 2 axis + hi; gamma[c][axis][hi] 0: no share; K: face coefficients
 struct BcRhs {
@@ -104,7 +118,7 @@ struct BcRhs {
     double gamma[3][3][2];
     const double *K[3][2];
 };
-void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p);
+void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p, const SumRiders &sums = {});
 void launch_ghost_update(hipStream_t st, const GhostCell *gc, int ng, const int *level_start, int nlevels,
                          double *old, double *u1, double *u2, double *u3, double *p);
 void launch_solid_nan(hipStream_t st, const Dims &d, const uint8_t *flag, double *u1, double *u2, double *u3,

@@ -321,7 +321,41 @@ __device__ inline double outer_value(const Dims &d, const OuterParams &op, const
     return v;
 }
 
-__global__ void k_outer(Dims d, OuterParams op, const OuterRule *rules, OuterFields fs) {
+// One workgroup of 256 threads: fixed-order sums. Riding beside a boundary
+// launch it costs no launch of its own (5 us on small grids, four per step), and
+// there is no chain between the two.
+constexpr int kRiderThreads = 256;
+__device__ inline void run_riders(const SumRiders &sums) {
+    __shared__ double sh[kRiderThreads / 64];
+    const int t = threadIdx.x + blockDim.x * threadIdx.y;
+    for (int e = 0; e < sums.n; e++) {
+        const auto &R = sums.r[e];
+        for (int a = 0; a < R.nv; a++) {
+            double acc[4] = {0, 0, 0, 0};
+            long b = t;
+            for (; b + 3 * kRiderThreads < R.nblk; b += 4 * kRiderThreads)
+#pragma unroll
+                for (int u = 0; u < 4; u++) acc[u] += R.partial[(b + u * kRiderThreads) * R.nv + a];
+            for (; b < R.nblk; b += kRiderThreads) acc[0] += R.partial[b * R.nv + a];
+            double v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+            if ((t & 63) == 0) sh[t >> 6] = v;
+            __syncthreads();
+            if (t == 0) R.out[a] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+            __syncthreads();
+        }
+    }
+    if (t != 0) return;
+    __threadfence_system();
+    *reinterpret_cast<volatile unsigned *>(sums.epoch_out) = sums.epoch;
+}
+
+__global__ void __launch_bounds__(kRiderThreads) k_outer(Dims d, OuterParams op, const OuterRule *rules,
+                                                         OuterFields fs, SumRiders sums) {
+    if ((int)blockIdx.z == 12 * fs.n) {
+        if (blockIdx.x == 0 && blockIdx.y == 0) run_riders(sums);
+        return;
+    }
     // one value per thread: face, layer and field
     const int ax = blockIdx.z % 6 / 2, hi = blockIdx.z % 2, layer = blockIdx.z / 6 % 2, e = blockIdx.z / 12;
     const int a0 = ax == 0 ? 0 : -2, a1 = ax == 0 ? d.ny : d.nx + 2;
@@ -459,7 +493,11 @@ long launch_conv_outflow(hipStream_t st, const Geo &g, int ax, int hi, double uc
 // others' shares too (a launch per face and field was 18 launches per cavity
 // step, 2.7 us each at 32^3).
 // ---------------------------------------------------------------------------
-__global__ void k_bc_rhs(Geo g, OuterParams op, BcRhs p) {
+__global__ void __launch_bounds__(kRiderThreads) k_bc_rhs(Geo g, OuterParams op, BcRhs p, SumRiders sums) {
+    if ((int)blockIdx.z == p.nface) {
+        if (blockIdx.x == 0 && blockIdx.y == 0) run_riders(sums);
+        return;
+    }
     const Dims &d = g.d;
     const int fc = p.face[blockIdx.z], ax = fc / 2, hi = fc % 2;
     const int n[3] = {d.nx, d.ny, d.nz};
@@ -788,16 +826,18 @@ void launch_update(hipStream_t st, const Geo &g, const StepParams &sp, const uin
 }
 
 void launch_outer(hipStream_t st, const Dims &d, const OuterParams &op, const OuterRule *rules,
-                  const OuterFields &fs) {
+                  const OuterFields &fs, const SumRiders &sums) {
     const int m1 = std::max(d.ny, d.nx + 4), m2 = std::max(d.nz, d.ny + 4);
-    hipLaunchKernelGGL(k_outer, dim3((m1 + 15) / 16, (m2 + 15) / 16, 12 * fs.n), dim3(16, 16), 0, st, d, op, rules, fs);
+    hipLaunchKernelGGL(k_outer, dim3((m1 + 15) / 16, (m2 + 15) / 16, 12 * fs.n + (sums.n > 0)), dim3(16, 16), 0, st, d, op,
+                       rules, fs, sums);
 }
 
-void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p) {
+void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p, const SumRiders &sums) {
     const Dims &d = g.d;
-    if (p.nface == 0) return;
-    const int m1 = std::max(d.nx, d.ny), m2 = std::max(d.ny, d.nz);
-    hipLaunchKernelGGL(k_bc_rhs, dim3((m1 + 15) / 16, (m2 + 15) / 16, p.nface), dim3(16, 16), 0, st, g, op, p);
+    const int nz = p.nface + (sums.n > 0);
+    if (nz == 0) return;
+    const int m1 = p.nface ? std::max(d.nx, d.ny) : 1, m2 = p.nface ? std::max(d.ny, d.nz) : 1;
+    hipLaunchKernelGGL(k_bc_rhs, dim3((m1 + 15) / 16, (m2 + 15) / 16, nz), dim3(16, 16), 0, st, g, op, p, sums);
 }
 
 void launch_ghost_update(hipStream_t st, const GhostCell *gc, int ng, const int *level_start, int nlevels,
