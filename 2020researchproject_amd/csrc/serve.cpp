@@ -311,7 +311,7 @@ double ibm::multigrid_bytes(const ibm::Dims &d, int precision) {
     const double mg = cells * (8.0 * 2 + (mixed ? 4.0 * 2 : 0))
         + coarse * (8.0 * 4 + 2 + (mixed ? 4.0 * 4 : 0)) + (cells + coarse) * 1;
     // dense inverse of the coarsest level (at most 3000 rows; FP64, + FP32);
-    // the pivot scratch of its inversion (0.8 MB) is part of the last term
+    // the pivot scratch of its inversion (3 MB) is part of the last term
     const double n = std::min(3000.0, (double)d.nx * d.ny * d.nz);
     return mg + n * n * (8 + (mixed ? 4 : 0)) + 2 * 8.0 * n;
 }

@@ -271,7 +271,7 @@ template <typename T>
 void launch_coarse_solve(hipStream_t st, const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const T *b, T *x,
                          int sweeps, int singular, const double *dxyz);
 
-// In-place Gauss-Jordan inversion without pivoting (beyond blocks of 16) of
+// In-place Gauss-Jordan inversion without pivoting of
 // the n x n row-major matrix A of row pitch ld (diagonally dominant M-matrix
 // rows); scratch: gauss_jordan_scratch(n) doubles.
 size_t gauss_jordan_scratch(int n);

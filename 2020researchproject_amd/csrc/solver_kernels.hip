@@ -2020,47 +2020,83 @@ void launch_coarse_solve(hipStream_t st, const Dims &d, const SysCoef<T> &S, con
 // ---------------------------------------------------------------------------
 // exact coarsest-level solve through a precomputed dense inverse
 // ---------------------------------------------------------------------------
-// Gauss-Jordan inversion by blocks of 16 pivots: a panel launch inverts the
-// 16 x 16 pivot block and forms the pivot rows times that inverse, an update
-// launch subtracts (pivot columns) x (those rows) from the whole matrix on the
-// FP64 matrix cores. Bound by reading and writing the matrix once per block,
-// n / 16 times in all (one pivot at a time it was n times). With it, assembly
-// of the sphere 133 x 67 x 61 took 37 ms instead of 64, and the serving mix of
-// six jobs 276 ms instead of 392.
-constexpr int kGjBlock = 16, kGjTile = 64;
+// Gauss-Jordan inversion by blocks of 64 pivots: a panel launch inverts the
+// pivot block and forms the pivot rows times that inverse, an update launch
+// subtracts (pivot columns) x (those rows) from the whole matrix, both on the
+// FP64 matrix cores. Bound by reading and writing the matrix once per block, n /
+// 64 times in all, and by the chain of the pivot block: n = 6579 (346 MB) 103
+// blocks of 240 + 86 us, with blocks of 16 412 of 140 + 12; n = 512 0.73 against
+// 0.53 ms. Assembly of the sphere 133 x 67 x 61 (n = 1900 then) took 64 ms with
+// one pivot at a time and 37 with blocks of 16.
+constexpr int kGjBlock = 64;
 
 __device__ inline double gj_read(const double *A, int n, long ld, int r, int c) {
     return r < n && c < n ? A[r * ld + c] : (r == c ? 1.0 : 0.0);  // past the edge: the identity
 }
 
-// rowp [16][ldp]: pivot rows times the block's inverse (the inverse itself in
-// the block's own columns); colp [n][16]: pivot columns
+// rowp [64][ldp]: pivot rows times the block's inverse (the inverse itself in
+// the block's own columns); colp [ldp][64]: pivot columns
 __global__ void __launch_bounds__(256) k_gj_panel(const double *A, int n, long ld, int p, double *rowp, long ldp,
                                                   double *colp) {
-    __shared__ double M[kGjBlock][kGjBlock + 1];
-    const int r = threadIdx.x / kGjBlock, c = threadIdx.x % kGjBlock;
-    M[r][c] = gj_read(A, n, ld, p + r, p + c);
-    __syncthreads();
+    typedef double acc4 __attribute__((ext_vector_type(4)));
+    __shared__ double M[kGjBlock][kGjBlock + 2];
+    __shared__ double buf[2][2][kGjBlock];  // of two pivots in turn: row, column
+    // a thread holds 4 x 4 of the pivot block
+    const int r0 = threadIdx.x / 16 * 4, c0 = threadIdx.x % 16 * 4;
+    double v[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) v[a][b] = gj_read(A, n, ld, p + r0 + a, p + c0 + b);
     for (int k = 0; k < kGjBlock; k++) {
-        const double piv = 1 / M[k][k], row = c == k ? piv : M[k][c] * piv;
-        const double v = r == k ? row : (c == k ? 0.0 : M[r][c]) - M[r][k] * row;
+        double *row = buf[k & 1][0], *col = buf[k & 1][1];
+        const int kr = k - r0, kc = k - c0;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            if (a == kr)
+#pragma unroll
+                for (int b = 0; b < 4; b++) row[c0 + b] = v[a][b];
+            if (a == kc)
+#pragma unroll
+                for (int b = 0; b < 4; b++) col[r0 + b] = v[b][a];
+        }
         __syncthreads();
-        M[r][c] = v;
-        __syncthreads();
+        const double piv = 1 / row[k];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const double x = b == kc ? piv : row[c0 + b] * piv;
+#pragma unroll
+            for (int a = 0; a < 4; a++) v[a][b] = a == kr ? x : (b == kc ? 0.0 : v[a][b]) - col[r0 + a] * x;
+        }
     }
-    const int i0 = blockIdx.x * kGjTile;
-    for (int e = threadIdx.x; e < kGjTile * kGjBlock; e += 256) {
-        const int j = i0 + e % kGjTile, q = e / kGjTile;
-        if (j >= ldp) continue;
-        double v = 0;
-        if (j >= p && j < p + kGjBlock) v = M[q][j - p];
-        else
-            for (int k = 0; k < kGjBlock; k++) v += M[q][k] * gj_read(A, n, ld, p + k, j);
-        rowp[q * ldp + j] = v;
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) M[r0 + a][c0 + b] = v[a][b];
+    __syncthreads();
+    const int j0 = blockIdx.x * kGjBlock, ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const int j = j0 + 16 * (threadIdx.x >> 6) + ln;
+    if (j0 == p) {
+        for (int e = threadIdx.x; e < kGjBlock * kGjBlock; e += 256)
+            rowp[e / kGjBlock * ldp + j0 + e % kGjBlock] = M[e / kGjBlock][e % kGjBlock];
+    } else {
+        acc4 acc[4] = {};
+        for (int k0 = 4 * g; k0 < kGjBlock; k0 += 16) {
+            double bv[4];
+            for (int t = 0; t < 4; t++) bv[t] = gj_read(A, n, ld, p + k0 + t, j);
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int m = 0; m < 4; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(M[16 * m + ln][k0 + t], bv[t], acc[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) rowp[(16 * m + 4 * r + g) * ldp + j] = acc[m][r];
     }
-    for (int e = threadIdx.x; e < kGjTile * kGjBlock; e += 256) {
-        const int i = i0 + e / kGjBlock, q = e % kGjBlock;
-        if (i < ldp) colp[(long)i * kGjBlock + q] = gj_read(A, n, ld, i, p + q);
+    for (int e = threadIdx.x; e < kGjBlock * kGjBlock; e += 256) {
+        const int i = j0 + e / kGjBlock, q = e % kGjBlock;
+        colp[(long)i * kGjBlock + q] = gj_read(A, n, ld, i, p + q);
     }
 }
 
@@ -2069,23 +2105,28 @@ __global__ void __launch_bounds__(256) k_gj_update(double *A, int n, long ld, in
                                                    const double *colp) {
     typedef double acc4 __attribute__((ext_vector_type(4)));
     const int ln = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-    const int i0 = blockIdx.y * kGjTile + 16 * (threadIdx.x >> 6);
-    if (i0 >= ldp) return;
-    double cv[4];
-    for (int t = 0; t < 4; t++) cv[t] = -colp[(long)(i0 + ln) * kGjBlock + 4 * g + t];
-    for (int jt = 0; jt < 4; jt++) {
-        const int j0 = blockIdx.x * kGjTile + 16 * jt, j = j0 + ln;
-        if (j0 >= ldp) return;
+    const int i0 = blockIdx.y * kGjBlock + 16 * (threadIdx.x >> 6), j0 = blockIdx.x * kGjBlock;
+    const bool own = blockIdx.y * kGjBlock == p;
+    double cv[kGjBlock / 4];
+#pragma unroll
+    for (int c = 0; c < kGjBlock / 16; c++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) cv[4 * c + t] = -colp[(long)(i0 + ln) * kGjBlock + 16 * c + 4 * g + t];
+    for (int j = j0 + ln; j < j0 + kGjBlock; j += 16) {
         acc4 acc;
         for (int r = 0; r < 4; r++) {
             const int i = i0 + 4 * r + g;
             acc[r] = j0 != p && i < n && j < n ? A[i * ld + j] : 0.0;
         }
-        for (int t = 0; t < 4; t++)
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[t], rowp[(4 * g + t) * ldp + j], acc, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < kGjBlock / 16; c++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[4 * c + t], rowp[(16 * c + 4 * g + t) * ldp + j], acc, 0,
+                                                           0, 0);
         for (int r = 0; r < 4; r++) {
             const int i = i0 + 4 * r + g;
-            if (i < n && j < n) A[i * ld + j] = i0 == p ? rowp[(4 * r + g) * ldp + j] : acc[r];
+            if (i < n && j < n) A[i * ld + j] = own ? rowp[(i - p) * ldp + j] : acc[r];
         }
     }
 }
@@ -2095,7 +2136,7 @@ static int gj_pad(int n) { return (n + kGjBlock - 1) / kGjBlock * kGjBlock; }
 size_t gauss_jordan_scratch(int n) { return 2 * (size_t)kGjBlock * gj_pad(n); }
 
 void gauss_jordan_invert(hipStream_t st, double *A, int n, long ld, double *scratch) {
-    const int ldp = gj_pad(n), tiles = (n + kGjTile - 1) / kGjTile;
+    const int ldp = gj_pad(n), tiles = ldp / kGjBlock;
     double *rowp = scratch, *colp = scratch + (size_t)kGjBlock * ldp;
     for (int p = 0; p < n; p += kGjBlock) {
         hipLaunchKernelGGL(k_gj_panel, dim3(tiles), dim3(256), 0, st, A, n, ld, p, rowp, (long)ldp, colp);

@@ -679,7 +679,7 @@ void ensure_mg(IBMSolver *s) {
 // if only FP32 fits, in FP32 (the correction of a refinement round, as the
 // FP32 cycles are): canopy 160 x 80 x 48, 6579 ghost cells, 346 MB in FP64.
 // Assembly with the hierarchy / with this: sphere 256 x 128 x 128 (3568 ghost
-// cells) 134 / 119 ms, 133 x 67 x 61 37 / 19, the canopy 36 / 121.
+// cells) 134 / 119 ms, 133 x 67 x 61 37 / 20, the canopy 36 / 91.
 static bool build_capacitance(IBMSolver *s) {
     const Dims &d = s->d;
     const int ng = s->ng, n[3] = {d.nx, d.ny, d.nz};

@@ -163,8 +163,7 @@ def test_direct_pressure_solve_matches_multigrid(new_gpu, I, cases, kind, shape)
 @pytest.mark.parametrize("shape", [(18, 18, 18), (26, 22, 18), (30, 30, 26)])
 def test_coarsest_level_inverse_at_block_remainders(new_gpu, cases, shape):
     """Two levels, the coarser one solved through its dense inverse, whose size
-    (729, 1287, 2925 rows) leaves a remainder of the inversion's blocks of 16
-    and tiles of 64: the iteration counts of an exact coarse solve, at most 10
+    (729, 1287, 2925 rows) leaves a remainder of the inversion's blocks of 64: the iteration counts of an exact coarse solve, at most 10
     (6 or 7 on the cavities of even sizes; with an inexact one the cycle
     contracts like its smoother alone and takes several times as many)."""
     s = new_gpu()
