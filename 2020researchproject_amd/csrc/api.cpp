@@ -748,8 +748,21 @@ extern "C" void IBMSolver_assemble(IBMSolver *s) {
     std::vector<double> *g[12] = {&s->dx, &s->dy, &s->dz, &s->xc, &s->yc, &s->zc,
                                   &s->kW, &s->kE, &s->kS, &s->kN, &s->kD, &s->kU};
     for (int a = 0; a < 12; a++) s->g1d[a].upload(*g[a]);
+    {
+        const std::vector<double> *w[3] = {&s->dx, &s->dy, &s->dz}, *c[3] = {&s->xc, &s->yc, &s->zc};
+        const int n[3] = {s->Nx, s->Ny, s->Nz};
+        for (int a = 0; a < 3; a++) {
+            std::vector<AxisMetric> m(n[a] + 4, AxisMetric{});
+            for (int i = -1; i <= n[a]; i++)
+                H1(m, i) = {H1((*w[a]), i) / (H1((*w[a]), i - 1) + H1((*w[a]), i)),
+                            1 / (H1((*c[a]), i) - H1((*c[a]), i - 1)), 1 / H1((*w[a]), i),
+                            1 / (H1((*c[a]), i + 1) - H1((*c[a]), i - 1))};
+            s->metric[a].upload(m);
+        }
+    }
     s->geo = {d, s->g1d[0].p, s->g1d[1].p, s->g1d[2].p, s->g1d[3].p, s->g1d[4].p, s->g1d[5].p,
-              s->g1d[6].p, s->g1d[7].p, s->g1d[8].p, s->g1d[9].p, s->g1d[10].p, s->g1d[11].p};
+              s->g1d[6].p, s->g1d[7].p, s->g1d[8].p, s->g1d[9].p, s->g1d[10].p, s->g1d[11].p,
+              s->metric[0].p, s->metric[1].p, s->metric[2].p};
     {
         std::vector<double> kx(s->Nx), ky(s->Ny), kz(s->Nz);
         for (int i = 0; i < s->Nx; i++) kx[i] = H1(s->kW, i) + H1(s->kE, i);

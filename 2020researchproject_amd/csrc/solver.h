@@ -246,6 +246,7 @@ struct _ibm_solver {
     ibm::Dims d{};
     ibm::Geo geo{};
     ibm::DBuf<double> g1d[12];       // dx dy dz xc yc zc kW kE kS kN kD kU
+    ibm::DBuf<ibm::AxisMetric> metric[3];
     ibm::DBuf<ibm::OuterRule> outer_rules;  // build_outer_rules
     ibm::DBuf<double> ks1d[3];       // kW+kE, kS+kN, kD+kU (interior, unpadded)
     ibm::DBuf<uint8_t> flag;

@@ -6,10 +6,20 @@
 namespace ibm {
 
 // Geometry of one grid: padded 1-D arrays indexed [i + 2] (i = -2 .. n+1).
+// Metrics of one position of an axis, so that the step's kernels need no
+// division: w, the weight of the lower cell in a value at the position's low
+// face (the lower cell's is the width of the upper one over the sum of both),
+// and the reciprocals of the distance of the two cells' centres, of the cell's
+// width and of the distance of its neighbours' centres. Positions -1 .. n.
+struct alignas(32) AxisMetric {
+    double w, rc, rd, r2;
+};
+
 struct Geo {
     Dims d;
     const double *dx, *dy, *dz, *xc, *yc, *zc;
     const double *kW, *kE, *kS, *kN, *kD, *kU;  // dt / (2 Re h dx), interior only
+    const AxisMetric *mx, *my, *mz;
 };
 
 struct StepParams {

@@ -77,7 +77,10 @@ __global__ void k_interp_stag(Geo g, const double *u1, const double *u2, const d
 // K1: convection N (AB2 history) and the Crank-Nicolson momentum RHS of the
 // three components, fused.  <- src/ibm3d_fracstep.c:117-170 and :237-269
 // Writes N (non-fluid: NaN) and b_l (non-fluid rows: 0); accumulates the
-// squared norms of b_l over the interior rows for the stopping test.
+// squared norms of b_l over the interior rows for the stopping test. Bound by
+// its 16 fields: 256 x 128 x 128 176 us, 3.3 TB/s (187 with the 30 divisions per
+// cell that the axis metrics replace; the blocks in contiguous ranges per XCD:
+// 183).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_conv_rhs(Geo g, StepParams sp, const uint8_t *flag,
                                                   const double *u1, const double *u2, const double *u3,
@@ -98,39 +101,33 @@ __global__ void __launch_bounds__(256) k_conv_rhs(Geo g, StepParams sp, const ui
         const long q = cidx(d, i, j, k);
         const long sy = d.sy, sz = d.sz;
         const bool fl = flag[q] == F_FLUID;
-        const double dxm = C1(g.dx, i - 1), dx0 = C1(g.dx, i), dxp = C1(g.dx, i + 1);
-        const double dym = C1(g.dy, j - 1), dy0 = C1(g.dy, j), dyp = C1(g.dy, j + 1);
-        const double dzm = C1(g.dz, k - 1), dz0 = C1(g.dz, k), dzp = C1(g.dz, k + 1);
+        const AxisMetric X0 = C1(g.mx, i), Y0 = C1(g.my, j), Z0 = C1(g.mz, k);
+        const double wxp = C1(g.mx, i + 1).w, wyp = C1(g.my, j + 1).w, wzp = C1(g.mz, k + 1).w;
         const double Uw = U1[q], Ue = U1[q + 1], Vs = U2[q], Vn = U2[q + sy], Wd = U3[q], Wu = U3[q + sz];
         const double kW = C1(g.kW, i), kE = C1(g.kE, i), kS = C1(g.kS, j), kN = C1(g.kN, j);
         const double kD = C1(g.kD, k), kU = C1(g.kU, k);
         const double kc = 1 - kW - kE - kS - kN - kD - kU;
-        const double ddx = C1(g.xc, i + 1) - C1(g.xc, i - 1);
-        const double ddy = C1(g.yc, j + 1) - C1(g.yc, j - 1);
-        const double ddz = C1(g.zc, k + 1) - C1(g.zc, k - 1);
         const double *uu[3] = {u1, u2, u3};
         const double *Np[3] = {Np1, Np2, Np3};
         double *NN[3] = {N1, N2, N3};
         double *bb[3] = {b1, b2, b3};
-        const double dp[3] = {(p[q + 1] - p[q - 1]) / ddx, (p[q + sy] - p[q - sy]) / ddy,
-                              (p[q + sz] - p[q - sz]) / ddz};
+        const double dp[3] = {(p[q + 1] - p[q - 1]) * X0.r2, (p[q + sy] - p[q - sy]) * Y0.r2,
+                              (p[q + sz] - p[q - sz]) * Z0.r2};
 #pragma unroll
         for (int l = 0; l < 3; l++) {
             const double *a = uu[l];
             const double c = a[q], xm = a[q - 1], xp = a[q + 1], ym = a[q - sy], yp = a[q + sy];
             const double zm = a[q - sz], zp = a[q + sz];
             const double npl = Np[l][q];
-            const double uw = (xm * dx0 + c * dxm) / (dxm + dx0);
-            const double ue = (c * dxp + xp * dx0) / (dx0 + dxp);
-            const double us = (ym * dy0 + c * dym) / (dym + dy0);
-            const double un = (c * dyp + yp * dy0) / (dy0 + dyp);
-            const double ud = (zm * dz0 + c * dzm) / (dzm + dz0);
-            const double uu_ = (c * dzp + zp * dz0) / (dz0 + dzp);
-            const double n = (Ue * ue - Uw * uw) / dx0 + (Vn * un - Vs * us) / dy0 + (Wu * uu_ - Wd * ud) / dz0;
+            const double uw = c + X0.w * (xm - c), ue = xp + wxp * (c - xp);
+            const double us = c + Y0.w * (ym - c), un = yp + wyp * (c - yp);
+            const double ud = c + Z0.w * (zm - c), uu_ = zp + wzp * (c - zp);
+            const double n = (Ue * ue - Uw * uw) * X0.rd + (Vn * un - Vs * us) * Y0.rd + (Wu * uu_ - Wd * ud) * Z0.rd;
             double divt = 0;
             if (tau.on) {
                 const double *t1 = tau.t[tau.slot[l][0]], *t2 = tau.t[tau.slot[l][1]], *t3 = tau.t[tau.slot[l][2]];
-                divt = (t1[q + 1] - t1[q - 1]) / ddx + (t2[q + sy] - t2[q - sy]) / ddy + (t3[q + sz] - t3[q - sz]) / ddz;
+                divt = (t1[q + 1] - t1[q - 1]) * X0.r2 + (t2[q + sy] - t2[q - sy]) * Y0.r2
+                    + (t3[q + sz] - t3[q - sz]) * Z0.r2;
             }
             const double b = -sp.dt / 2 * (3 * n - npl) - sp.dt * dp[l] + kc * c
                 + kW * xm + kE * xp + kS * ym + kN * yp + kD * zm + kU * zp
@@ -163,41 +160,29 @@ __global__ void __launch_bounds__(256) k_face_star(Geo g, StepParams sp, const u
     const uint8_t f0 = flag[q];
     if (j < d.ny && k < d.nz) {  // x face i-1/2
         const uint8_t fm = flag[q - 1];
-        const double dm = C1(g.dx, i - 1), d0 = C1(g.dx, i);
-        double v;
-        if ((fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID)) {
-            v = (us1[q - 1] * d0 + us1[q] * dm) / (dm + d0);
-        } else {
-            const double tm = us1[q - 1] + dt * (p[q] - p[q - 2]) / (C1(g.xc, i) - C1(g.xc, i - 2));
-            const double t0 = us1[q] + dt * (p[q + 1] - p[q - 1]) / (C1(g.xc, i + 1) - C1(g.xc, i - 1));
-            v = (tm * d0 + t0 * dm) / (dm + d0) - dt * (p[q] - p[q - 1]) / (C1(g.xc, i) - C1(g.xc, i - 1));
-        }
+        const AxisMetric M = C1(g.mx, i);
+        const double um = us1[q - 1], u0 = us1[q], pm = p[q - 1], p0 = p[q];
+        const double tm = um + dt * (p0 - p[q - 2]) * C1(g.mx, i - 1).r2, t0 = u0 + dt * (p[q + 1] - pm) * M.r2;
+        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
+        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
         F1[q] = v;
     }
     if (i < d.nx && k < d.nz) {  // y face j-1/2
         const uint8_t fm = flag[q - sy];
-        const double dm = C1(g.dy, j - 1), d0 = C1(g.dy, j);
-        double v;
-        if ((fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID)) {
-            v = (us2[q - sy] * d0 + us2[q] * dm) / (dm + d0);
-        } else {
-            const double tm = us2[q - sy] + dt * (p[q] - p[q - 2 * sy]) / (C1(g.yc, j) - C1(g.yc, j - 2));
-            const double t0 = us2[q] + dt * (p[q + sy] - p[q - sy]) / (C1(g.yc, j + 1) - C1(g.yc, j - 1));
-            v = (tm * d0 + t0 * dm) / (dm + d0) - dt * (p[q] - p[q - sy]) / (C1(g.yc, j) - C1(g.yc, j - 1));
-        }
+        const AxisMetric M = C1(g.my, j);
+        const double um = us2[q - sy], u0 = us2[q], pm = p[q - sy], p0 = p[q];
+        const double tm = um + dt * (p0 - p[q - 2 * sy]) * C1(g.my, j - 1).r2, t0 = u0 + dt * (p[q + sy] - pm) * M.r2;
+        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
+        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
         F2[q] = v;
     }
     if (i < d.nx && j < d.ny) {  // z face k-1/2
         const uint8_t fm = flag[q - sz];
-        const double dm = C1(g.dz, k - 1), d0 = C1(g.dz, k);
-        double v;
-        if ((fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID)) {
-            v = (us3[q - sz] * d0 + us3[q] * dm) / (dm + d0);
-        } else {
-            const double tm = us3[q - sz] + dt * (p[q] - p[q - 2 * sz]) / (C1(g.zc, k) - C1(g.zc, k - 2));
-            const double t0 = us3[q] + dt * (p[q + sz] - p[q - sz]) / (C1(g.zc, k + 1) - C1(g.zc, k - 1));
-            v = (tm * d0 + t0 * dm) / (dm + d0) - dt * (p[q] - p[q - sz]) / (C1(g.zc, k) - C1(g.zc, k - 1));
-        }
+        const AxisMetric M = C1(g.mz, k);
+        const double um = us3[q - sz], u0 = us3[q], pm = p[q - sz], p0 = p[q];
+        const double tm = um + dt * (p0 - p[q - 2 * sz]) * C1(g.mz, k - 1).r2, t0 = u0 + dt * (p[q + sz] - pm) * M.r2;
+        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
+        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
         F3[q] = v;
     }
 }
@@ -220,8 +205,8 @@ __global__ void __launch_bounds__(256) k_poisson_rhs(Geo g, StepParams sp, const
         const long q = cidx(d, i, j, k);
         double v = 0;
         if (q != pin && flag[q] == F_FLUID) {
-            v = -1 / (2 * sp.Re) * ((F1[q + 1] - F1[q]) / C1(g.dx, i) + (F2[q + d.sy] - F2[q]) / C1(g.dy, j)
-                                    + (F3[q + d.sz] - F3[q]) / C1(g.dz, k));
+            v = -1 / (2 * sp.Re) * ((F1[q + 1] - F1[q]) * C1(g.mx, i).rd + (F2[q + d.sy] - F2[q]) * C1(g.my, j).rd
+                                    + (F3[q + d.sz] - F3[q]) * C1(g.mz, k).rd);
             const double ks = C1(g.kN, j) + C1(g.kE, i) + C1(g.kS, j) + C1(g.kW, i) + C1(g.kD, k) + C1(g.kU, k);
             const double vn = v / ks;
             nrm[0] = vn * vn;
@@ -255,22 +240,22 @@ __global__ void __launch_bounds__(256) k_update(Geo g, StepParams sp, const uint
     if (i < d.nx && j < d.ny && k < d.nz) {
         pn[q] = (f0 == F_FLUID || f0 == F_GHOST) ? p[q] + pp[q] : nan_d();
         if (f0 == F_FLUID) {
-            un1[q] = us1[q] - dt * (pp[q + 1] - pp[q - 1]) / (C1(g.xc, i + 1) - C1(g.xc, i - 1));
-            un2[q] = us2[q] - dt * (pp[q + sy] - pp[q - sy]) / (C1(g.yc, j + 1) - C1(g.yc, j - 1));
-            un3[q] = us3[q] - dt * (pp[q + sz] - pp[q - sz]) / (C1(g.zc, k + 1) - C1(g.zc, k - 1));
+            un1[q] = us1[q] - dt * (pp[q + 1] - pp[q - 1]) * C1(g.mx, i).r2;
+            un2[q] = us2[q] - dt * (pp[q + sy] - pp[q - sy]) * C1(g.my, j).r2;
+            un3[q] = us3[q] - dt * (pp[q + sz] - pp[q - sz]) * C1(g.mz, k).r2;
         } else if (f0 == F_SOLID) {
             un1[q] = un2[q] = un3[q] = nan_d();
         }
     }
     if (j < d.ny && k < d.nz)
         G1[q] = (flag[q - 1] != F_SOLID && f0 != F_SOLID)
-            ? F1[q] - dt * (pp[q] - pp[q - 1]) / (C1(g.xc, i) - C1(g.xc, i - 1)) : nan_d();
+            ? F1[q] - dt * (pp[q] - pp[q - 1]) * C1(g.mx, i).rc : nan_d();
     if (i < d.nx && k < d.nz)
         G2[q] = (flag[q - sy] != F_SOLID && f0 != F_SOLID)
-            ? F2[q] - dt * (pp[q] - pp[q - sy]) / (C1(g.yc, j) - C1(g.yc, j - 1)) : nan_d();
+            ? F2[q] - dt * (pp[q] - pp[q - sy]) * C1(g.my, j).rc : nan_d();
     if (i < d.nx && j < d.ny)
         G3[q] = (flag[q - sz] != F_SOLID && f0 != F_SOLID)
-            ? F3[q] - dt * (pp[q] - pp[q - sz]) / (C1(g.zc, k) - C1(g.zc, k - 1)) : nan_d();
+            ? F3[q] - dt * (pp[q] - pp[q - sz]) * C1(g.mz, k).rc : nan_d();
 }
 
 // ---------------------------------------------------------------------------
