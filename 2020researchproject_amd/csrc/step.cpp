@@ -272,8 +272,10 @@ static void bc_rhs(IBMSolver *s, const OuterParams &op, int comp, int n, const S
 
 static void update_outer(IBMSolver *s) {
     const OuterParams op = make_outer(s, BCD_FIELDS, s->time, nullptr);
-    TIMED("outer", 0, launch_outer(s->stream, s->d, op, s->outer_rules.p, {{s->u[0].p, s->u[1].p, s->u[2].p, s->p.p},
-                                                           {0, 1, 2, OUT_P}, 4}));
+    // (the ghost cells' values, which update_ghost needs, are saved by the way)
+    TIMED("outer", 0, launch_outer(s->stream, s->d, op, s->outer_rules.p,
+                                   {{s->u[0].p, s->u[1].p, s->u[2].p, s->p.p}, {0, 1, 2, OUT_P}, 4}, {},
+                                   {s->gc.p, s->ng, s->ghost_old.p}));
 }
 
 static void update_ghost(IBMSolver *s) {

@@ -110,6 +110,13 @@ struct SumRiders {
     unsigned epoch;
 };
 
+// Saves the four fields of an outer-layer launch at the ghost cells
+struct GhostSave {
+    const GhostCell *gc;
+    int ng;
+    double *old;
+};
+
 // Rule of an outer position: value = g * (boundary value) + sum_t c[t] (value
 // at position n[t] of the axis); keep: not written. Table [kind][axis][hi][layer].
 struct OuterRule {
@@ -118,7 +125,7 @@ struct OuterRule {
 };
 constexpr int kOuterRules = 5 * 12;
 void launch_outer(hipStream_t st, const Dims &d, const OuterParams &op, const OuterRule *rules,
-                  const OuterFields &fs, const SumRiders &sums = {});
+                  const OuterFields &fs, const SumRiders &sums = {}, const GhostSave &save = {});
 // Boundary data of the right-hand sides b[0..n) of components comp..comp+n-1:
 // faces 2 axis + hi; gamma[c][axis][hi] 0: no share; K: face coefficients
 struct BcRhs {
@@ -129,8 +136,11 @@ struct BcRhs {
     const double *K[3][2];
 };
 void launch_bc_rhs(hipStream_t st, const Geo &g, const OuterParams &op, const BcRhs &p, const SumRiders &sums = {});
+// ordered update of the ghost cells; old: their values before it (GhostSave)
+constexpr int kGhostLevels = 30;
+struct GhostLevels { int start[kGhostLevels + 1], n; };
 void launch_ghost_update(hipStream_t st, const GhostCell *gc, int ng, const int *level_start, int nlevels,
-                         double *old, double *u1, double *u2, double *u3, double *p);
+                         const double *old, double *u1, double *u2, double *u3, double *p);
 void launch_solid_nan(hipStream_t st, const Dims &d, const uint8_t *flag, double *u1, double *u2, double *u3,
                       double *p);
 void launch_sgs(hipStream_t st, const Geo &g, int model, double coef, const VanDriest &vd, const uint8_t *flag,
