@@ -1741,10 +1741,10 @@ static void separable_round(IBMSolver *s, const double *b, double *x, bool first
     const double cb = ncells(s) * 8;
     const double *rhs = first ? b : r;
     if (s->cap_on)
-        TIMED("separable_body", (first ? 9 : 10) * cb + (double)s->cap.G.ng * s->cap.ld * (s->cap.inv64 ? 8 : 4),
+        TIMED("separable_body", 0,  // matrix products: no byte count, they are not bound by it
               launch_separable_body(s->stream, d, s->sep, s->cap, rhs, s1, s2, s->kry.v64[3].p, x, !first));
     else
-        TIMED("separable", (first ? 6 : 7) * cb,
+        TIMED("separable", 0,
               launch_separable(s->stream, d, s->sep, rhs, s1, s2, x, !first, partial));
     TIMED("residual", 3 * cb, launch_residual<double>(s->stream, d, s->sys[3].S64, s->gp.G64, s->flag.p, b, x, r, ns,
                                                       partial));
@@ -2046,7 +2046,6 @@ static bool momentum_sweeps_finish(IBMSolver *s, MomSweeps &st, const double bn[
 // The three momentum solves by the transforms, and the partial sums of their
 // residuals' norms
 static void momentum_direct(IBMSolver *s) {
-    const double cb = ncells(s) * 8 * 3;
     const double *b[3];
     double *s1[3], *s2[3], *x[3];
     for (int l = 0; l < 3; l++) {
@@ -2055,8 +2054,8 @@ static void momentum_direct(IBMSolver *s) {
         s2[l] = s->kry.v64[4 + l].p;
         x[l] = s->us[l].p;
     }
-    TIMED("mom_separable", 6 * cb, launch_separable_batch(s->stream, s->d, 3, s->sep_mom, b, s1, s2, x));
-    TIMED("mom_residual64", 2 * cb,
+    TIMED("mom_separable", 0, launch_separable_batch(s->stream, s->d, 3, s->sep_mom, b, s1, s2, x));
+    TIMED("mom_residual64", ncells(s) * 3 * 16,
           launch_mom_residual(s->stream, s->d, s->mt64.p, 7, s->gmom.G64, s->flag.p, MOM_NORMS, s->partial.p));
 }
 

@@ -11,10 +11,11 @@ boundary and immersed-boundary ghost updates, and the drag/lift reduction
 of the step's fields). Inputs are resident in HBM when the timed region
 starts.
 
-The headline value is the mixed path in Mcell-steps/s: FP64 BiCGSTAB whose
-multigrid preconditioner runs in FP32 (IBM3D_PREC_MIXED_KRYLOV). The plain
-FP64 path runs the same steps for the speed-up. After the timed regions both
-GPU paths and the FP64 CPU oracle run the first steps of the same case from
+The headline value is the mixed path in Mcell-steps/s
+(IBM3D_PREC_MIXED_KRYLOV): FP32 momentum sweeps in FP64 refinement; the
+pressure is solved directly in FP64 where the case allows it, else by FP64
+BiCGSTAB whose multigrid preconditioner runs in FP32. The plain FP64 path
+runs the same steps for the speed-up. After the timed regions both GPU paths and the FP64 CPU oracle run the first steps of the same case from
 the same initial field; their differences (rel-L2 and Linf of u and p,
 max|div U|, drag and lift) are the line's error statement. Prints one JSON
 line.
@@ -317,7 +318,7 @@ def serving_stream(args) -> dict:
     return {
         "value": round(res["mcell_steps_per_s"], 2), "unit": "Mcell-steps/s",
         "workload": f"{len(specs)} cases, Poisson arrivals (mean 50 ms), cavity/sphere, "
-                    "grids 32^3..128x64x64, Re 100-1000, 100-400 steps, tol 1e-10, FP64 BiCGSTAB + FP32 multigrid",
+                    "grids 32^3..128x64x64, Re 100-1000, 100-400 steps, tol 1e-10, mixed precision, direct FP64 pressure where eligible",
         "slots": args.serving_slots, "budget_gib": args.serving_budget_gib,
         "cases": len(specs), "failed": sum(r.state != 2 for r in res["results"]),
         "p50_s": round(res["p50_s"], 3), "p99_s": round(res["p99_s"], 3),
@@ -361,7 +362,7 @@ def main() -> int:
     ap.add_argument("--grid", type=str, default="256x128x128")
     ap.add_argument("--tol", type=float, default=1e-9)
     ap.add_argument("--mixed-mode", type=int, default=2, choices=(1, 2),
-                    help="1: FP64 defect correction around FP32 BiCGSTAB; 2: FP64 BiCGSTAB, FP32 multigrid")
+                    help="1: FP64 defect correction around FP32 BiCGSTAB; 2: FP64 pressure (direct, or BiCGSTAB with FP32 multigrid)")
     ap.add_argument("--copy-calib-mb", type=float, default=0.0,
                     help="also run one plain device copy of this many MiB (calibrates rocprofv3 byte counters)")
     ap.add_argument("--no-fp64", action="store_true")
@@ -404,8 +405,8 @@ def main() -> int:
         "config": {"workload": f"sphere {nx}x{ny}x{nz} cosine-stretched, Re 300, dt 0.002, uniform inflow, "
                                f"{args.outflow} outflow, slip lateral walls, tol {args.tol:g}",
                    "cells": int(cells),
-                   "precision": ("momentum: FP32 red-black sweeps in FP64 refinement; pressure: FP64 BiCGSTAB, "
-                                 "FP32 multigrid preconditioner" if args.mixed_mode == 2 else
+                   "precision": ("momentum: FP32 red-black sweeps in FP64 refinement; pressure: direct FP64 solve, "
+                                 "where ineligible FP64 BiCGSTAB with FP32 multigrid preconditioner" if args.mixed_mode == 2 else
                                  "FP64 defect correction around FP32 multigrid-BiCGSTAB"),
                    "mg_levels": mixed["mg_levels"]},
         "p50_ms": round(float(np.percentile(mixed["step_ms"], 50)), 3),
