@@ -110,7 +110,7 @@ __device__ inline typename Vec2<T>::type load_pair(const TX *p) {
 }
 
 template <typename T, typename TX = T>
-__device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const TX *x, int i0, int j, int k, long q0,
+__device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const TX *x, int i0, int j, int k, long q0,
                                   T yv[2], T xq[2]) {
     using T2 = typename Vec2<T>::type;
     const AxisCoef<T> &AX = S.ax[0], &AY = S.ax[1], &AZ = S.ax[2];
@@ -121,12 +121,12 @@ __device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const TX *
     const T2 yp = load_pair<T>(x + q0 + (long)(jp - j) * d.sy);
     const T2 zm = load_pair<T>(x + q0 + (long)(km - k) * d.sz);
     const T2 zp = load_pair<T>(x + q0 + (long)(kp - k) * d.sz);
-    T xl = (T)x[q0 - 1], xr = (T)x[q0 + 2];
-    if (AX.periodic) {
-        if (i0 == 0) xl = (T)x[q0 + AX.n - 1];
-        if (i0 + 1 == AX.n - 1) xr = (T)x[q0 - i0];
-    }
-    const unsigned mm = S.skip ? *reinterpret_cast<const unsigned short *>(S.fmask + q0) : 0u;
+    // no branch between the loads: the row's ends choose the address, and systems
+    // without a face mask read the flags (in cache) and drop them
+    const T xl = (T)x[AX.periodic && i0 == 0 ? q0 + AX.n - 1 : q0 - 1];
+    const T xr = (T)x[AX.periodic && i0 + 2 >= AX.n ? q0 - i0 : q0 + 2];
+    const unsigned fm = *reinterpret_cast<const unsigned short *>((S.skip ? S.fmask : flag) + q0);
+    const unsigned mm = S.skip ? fm : 0u;
     using P4 = typename Packed4<T>::type;
     const P4 cx0 = reinterpret_cast<const P4 *>(AX.c4)[i0];
     const P4 cx1 = reinterpret_cast<const P4 *>(AX.c4)[i0 + 1 < d.nx ? i0 + 1 : i0];
@@ -135,9 +135,8 @@ __device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const TX *
 #pragma unroll
     for (int o = 0; o < 2; o++) {
         const unsigned m = (mm >> (8 * o)) & 0xFFu;
-        // periodic x, cell i0 + 1 the last of its row: the wrap neighbour
-        T xp = o ? xr : xc.y;
-        if (o == 0 && AX.periodic && i0 == AX.n - 1) xp = (T)x[q0 - i0];
+        // periodic x, the pair at the end of its row: xr is the wrap neighbour
+        const T xp = o || (AX.periodic && i0 == AX.n - 1) ? xr : xc.y;
         const T xm = o ? xc.x : xl;
         const P4 cx = o ? cx1 : cx0;
         T diag = S.c0, off = 0;
@@ -236,14 +235,17 @@ __device__ inline void store_pair_skip(const Dims &d, int i0, long q0, T *a, T v
 // y at ghost row s: is_p ? (1 - ws) x - sum w x : (1 + ws) x + sum w x
 template <typename T, typename TX>
 __device__ inline T ghost_row_apply(const GhostRows<T> &G, int is_p, const TX *x, int s, long &c) {
-    T a = 0;
-#pragma unroll
-    for (int l = 0; l < 8; l++) {
-        const long q = G.src[8 * (long)s + l];
-        if (q >= 0) a += G.w[8 * (long)s + l] * (T)x[q];
-    }
     c = G.cell[s];
     const T ws = G.wself[s], xc = (T)x[c];
+    long q[8];
+    T w[8], v[8];
+#pragma unroll
+    for (int l = 0; l < 8; l++) q[l] = G.src[8 * (long)s + l], w[l] = G.w[8 * (long)s + l];
+#pragma unroll
+    for (int l = 0; l < 8; l++) v[l] = (T)x[q[l] >= 0 ? q[l] : c];
+    T a = 0;
+#pragma unroll
+    for (int l = 0; l < 8; l++) a = q[l] >= 0 ? a + w[l] * v[l] : a;
     return is_p ? (T(1) - ws) * xc - a : (T(1) + ws) * xc + a;
 }
 
@@ -280,7 +282,7 @@ __global__ void __launch_bounds__(256) k_apply(Dims d, SysCoef<T> S, GhostRows<T
                 const long q0 = cidx(d, i0, j, k);
                 fv[kk] = *reinterpret_cast<const unsigned short *>(flag + q0);
                 if (MODE > 0) wv[kk] = *reinterpret_cast<const T2 *>(w + q0);
-                pair_apply(d, S, x, i0, j, k, q0, yv[kk], xq[kk]);
+                pair_apply(d, S, flag, x, i0, j, k, q0, yv[kk], xq[kk]);
             }
 #pragma unroll
             for (int kk = 0; kk < kRedZP; kk++) {
@@ -356,18 +358,24 @@ __device__ inline double nscale(const NormSpec &ns, const Dims &d, int i, int j,
 // One block of the residual r = b - A x (blocks below ngb: ghost rows, the
 // others cell pairs, XCD-contiguous of `nb` blocks in all): acc gets the
 // block's lanes' shares of ||r||^2 and ||D^-1 r||^2. The sink takes r: two
-// cells of a row with their flags (skipping ghost cells), and ghost rows.
+// cells of a row with their flags (skipping ghost cells), and ghost rows. Its
+// form() makes what is stored, with the loads that takes, for all planes
+// before the first put(): a load behind a store waits for the store as well.
 template <typename T>
 struct ResidualStore {
     T *r;
-    __device__ void pair(const Dims &d, int i0, int, int, long q0, unsigned, T v0, T v1, bool g0, bool g1) const {
-        store_pair_skip(d, i0, q0, r, v0, v1, g0, g1);
+    struct Out { T v0, v1; };
+    __device__ Out form(const Dims &, int, int, int, long, unsigned, T v0, T v1) const { return {v0, v1}; }
+    __device__ void put(const Dims &d, int i0, long q0, const Out &o, bool g0, bool g1) const {
+        store_pair_skip(d, i0, q0, r, o.v0, o.v1, g0, g1);
     }
     __device__ void ghost(int, long c, T v) const { r[c] = v; }
 };
 struct ResidualDrop {
+    struct Out {};
     template <typename T>
-    __device__ void pair(const Dims &, int, int, int, long, unsigned, T, T, bool, bool) const {}
+    __device__ Out form(const Dims &, int, int, int, long, unsigned, T, T) const { return {}; }
+    __device__ void put(const Dims &, int, long, const Out &, bool, bool) const {}
     template <typename T>
     __device__ void ghost(int, long, T) const {}
 };
@@ -375,13 +383,16 @@ struct ResidualDrop {
 struct ResidualCorrection {
     const SysCoef<float> &S;
     float *b, *x;
-    __device__ void pair(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1, bool g0,
-                         bool g1) const {
+    struct Out { float b0, b1, x0, x1; };
+    __device__ Out form(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1) const {
         const float b0 = (float)v0, b1 = (float)v1;
         const float d0 = stencil_diag(S, i0, j, k, q0), d1 = stencil_diag(S, min(i0 + 1, d.nx - 1), j, k, q0 + 1);
-        store_pair_skip(d, i0, q0, b, b0, b1, g0, g1);
-        store_pair_skip(d, i0, q0, x, first_colour_of(S, fv & 0xFFu, i0, j, k, q0, b0, d0),
-                        first_colour_of(S, fv >> 8, i0 + 1, j, k, q0 + 1, b1, d1), g0, g1);
+        return {b0, b1, first_colour_of(S, fv & 0xFFu, i0, j, k, q0, b0, d0),
+                first_colour_of(S, fv >> 8, i0 + 1, j, k, q0 + 1, b1, d1)};
+    }
+    __device__ void put(const Dims &d, int i0, long q0, const Out &o, bool g0, bool g1) const {
+        store_pair_skip(d, i0, q0, b, o.b0, o.b1, g0, g1);
+        store_pair_skip(d, i0, q0, x, o.x0, o.x1, g0, g1);
     }
     __device__ void ghost(int, long c, double v) const {
         b[c] = (float)v;
@@ -394,12 +405,14 @@ struct ResidualJacobi {
     const GhostRows<double> &G;
     const double *x;
     double *out;
-    __device__ void pair(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1, bool g0,
-                         bool g1) const {
+    struct Out { double v0, v1; };
+    __device__ Out form(const Dims &d, int i0, int j, int k, long q0, unsigned fv, double v0, double v1) const {
         const double2 o = *reinterpret_cast<const double2 *>(x + q0);
         const double d0 = stencil_diag(S, i0, j, k, q0), d1 = stencil_diag(S, min(i0 + 1, d.nx - 1), j, k, q0 + 1);
-        store_pair_skip(d, i0, q0, out, o.x + ((fv & 0xFFu) == F_FLUID ? v0 / d0 : 0.0),
-                        o.y + (fv >> 8 == F_FLUID ? v1 / d1 : 0.0), g0, g1);
+        return {o.x + ((fv & 0xFFu) == F_FLUID ? v0 / d0 : 0.0), o.y + (fv >> 8 == F_FLUID ? v1 / d1 : 0.0)};
+    }
+    __device__ void put(const Dims &d, int i0, long q0, const Out &o, bool g0, bool g1) const {
+        store_pair_skip(d, i0, q0, out, o.v0, o.v1, g0, g1);
     }
     __device__ void ghost(int s, long c, double v) const {
         const double dg = S.is_p ? 1 - G.wself[s] : 1 + G.wself[s];
@@ -407,7 +420,7 @@ struct ResidualJacobi {
     }
 };
 
-template <typename SINK, typename T, typename TX>
+template <bool NS, typename SINK, typename T, typename TX>
 __device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const GhostRows<T> &G,
                                       const uint8_t *__restrict__ flag, const T *__restrict__ b,
                                       const TX *__restrict__ x, const SINK &sink, const NormSpec &ns, unsigned wb,
@@ -429,60 +442,76 @@ __device__ inline void residual_block(const Dims &d, const SysCoef<T> &S, const 
         if (i0 < d.nx && j < d.ny) {
             T yv[kRedZP][2], xq[kRedZP][2];
             T2 bv[kRedZP];
-            unsigned fv[kRedZP];
+            unsigned fv[kRedZP], nfv[kRedZP];
+            double kx[2], ky, kz[kRedZP];
+            if constexpr (NS) {
+                kx[0] = ns.ksx[i0];
+                kx[1] = ns.ksx[min(i0 + 1, d.nx - 1)];
+                ky = ns.ksy[j];
+            }
 #pragma unroll
             for (int kk = 0; kk < kRedZP; kk++) {
                 const int k = min(k0 + kk, k1 - 1);  // past the last plane: a repeat, discarded
                 const long q0 = cidx(d, i0, j, k);
                 fv[kk] = *reinterpret_cast<const unsigned short *>(flag + q0);
                 bv[kk] = *reinterpret_cast<const T2 *>(b + q0);
-                pair_apply(d, S, x, i0, j, k, q0, yv[kk], xq[kk]);
+                if constexpr (NS) {
+                    nfv[kk] = *reinterpret_cast<const unsigned short *>(ns.flag + q0);
+                    kz[kk] = ns.ksz[k];
+                }
+                pair_apply(d, S, flag, x, i0, j, k, q0, yv[kk], xq[kk]);
             }
+            typename SINK::Out out[kRedZP];
+            bool gh[kRedZP][2];
 #pragma unroll
             for (int kk = 0; kk < kRedZP; kk++) {
-                const int k = k0 + kk;
-                if (k >= k1) break;
+                const int k = min(k0 + kk, k1 - 1);
                 const long q0 = cidx(d, i0, j, k);
                 T v[2];
-                bool on[2], gh[2];
 #pragma unroll
                 for (int o = 0; o < 2; o++) {
                     const unsigned f = (fv[kk] >> (8 * o)) & 0xFFu;
                     const bool ident = q0 + o == S.pin || f == F_SOLID;
                     const T bo = o ? bv[kk].y : bv[kk].x;
                     v[o] = ident ? bo - xq[kk][o] : bo - yv[kk][o];
-                    gh[o] = !ident && f == F_GHOST;  // written by the ghost blocks
-                    on[o] = i0 + o < d.nx && (ident || f == F_FLUID);
-                }
-                sink.pair(d, i0, j, k, q0, fv[kk], v[0], v[1], gh[0], gh[1]);
-#pragma unroll
-                for (int o = 0; o < 2; o++) {
-                    if (!on[o]) continue;
+                    gh[kk][o] = !ident && f == F_GHOST;  // written by the ghost blocks
+                    if (k0 + kk >= k1 || i0 + o >= d.nx || !(ident || f == F_FLUID)) continue;
                     const double rd = (double)v[o];
                     acc[0] += rd * rd;
-                    const double rsc = rd * nscale(ns, d, i0 + o, j, k, q0 + o);
+                    double rsc = rd;
+                    if constexpr (NS) {
+                        const bool fluid = ((nfv[kk] >> (8 * o)) & 0xFFu) == F_FLUID;
+                        rsc *= q0 + o == ns.pin || !fluid ? 1.0 : 1.0 / (kx[o] + ky + kz[kk]);
+                    }
                     acc[1] += rsc * rsc;
                 }
+                out[kk] = sink.form(d, i0, j, k, q0, fv[kk], v[0], v[1]);
             }
+#pragma unroll
+            for (int kk = 0; kk < kRedZP; kk++)
+                if (k0 + kk < k1) sink.put(d, i0, cidx(d, i0, j, k0 + kk), out[kk], gh[kk][0], gh[kk][1]);
         }
     }
 }
 
-template <typename T>
+template <bool NS, typename T>
 __global__ void __launch_bounds__(256) k_residual(Dims d, SysCoef<T> S, GhostRows<T> G,
                                                   const uint8_t *__restrict__ flag, const T *__restrict__ b,
                                                   const T *__restrict__ x, T *__restrict__ r, NormSpec ns,
                                                   double *partial, unsigned ngb, unsigned gx, unsigned gy) {
     double acc[2] = {0, 0};
-    residual_block(d, S, G, flag, b, x, ResidualStore<T>{r}, ns, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+    residual_block<NS>(d, S, G, flag, b, x, ResidualStore<T>{r}, ns, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
     bsum<2>(acc, partial, blockIdx.x);
 }
 
 template <typename T>
 void launch_residual(hipStream_t st, const Dims &d, const SysCoef<T> &S, const GhostRows<T> &G,
                      const uint8_t *flag, const T *b, const T *x, T *r, const NormSpec &ns, double *partial) {
-    hipLaunchKernelGGL((k_residual<T>), dim3(agrid_blocks(d, G.ng)), dim3(64, 4), 0, st, d, S, G, flag, b, x, r, ns,
-                       partial, ghost_blocks(G.ng), pgx(d), pgy(d));
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(agrid_blocks(d, G.ng)), dim3(64, 4), 0, st, d, S, G, flag, b, x, r, ns, partial,
+                           ghost_blocks(G.ng), pgx(d), pgy(d));
+    };
+    ns.on ? launch(k_residual<true, T>) : launch(k_residual<false, T>);
 }
 
 // ---------------------------------------------------------------------------
@@ -1606,18 +1635,44 @@ void launch_copy(hipStream_t st, const Dims &d, const T *a, T *b) {
 // any size up to 64^3 takes 4 to 5 us with its gap) and two kernel tails
 // where it is large. Components outside `mask` return at once.
 // ---------------------------------------------------------------------------
+// A pointer read from memory has no known address space, and what goes through
+// it becomes a flat access, which is waited for with every other one in flight;
+// the tables' pointers are all to device memory and are read as such. With the
+// branches between the loads gone (pair_apply) and the stores last, the two
+// residuals of a mixed round at 256 x 128 x 128 take 72 us in place of 85 on
+// average, the FP64 one 55 in place of 62, the pressure's 35 in place of 44.
+template <typename T>
+__device__ inline T *global_ptr(T *const &p) {
+    using G = __attribute__((address_space(1))) T *;
+    return (T *)*static_cast<const G *>(static_cast<const void *>(&p));
+}
+template <typename T>
+__device__ inline SysCoef<T> global_ptr(const SysCoef<T> &from) {
+    SysCoef<T> S = from;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        S.ax[a].cm = global_ptr(from.ax[a].cm);
+        S.ax[a].cp = global_ptr(from.ax[a].cp);
+        S.ax[a].dm = global_ptr(from.ax[a].dm);
+        S.ax[a].dp = global_ptr(from.ax[a].dp);
+        S.ax[a].c4 = global_ptr(from.ax[a].c4);
+    }
+    S.fmask = global_ptr(from.fmask);
+    return S;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_mom_colour(Dims d, const MomTable<T> *M, unsigned mask, const uint8_t *flag,
                                                     int color, int zero_in, GhostRows<T> G, int prev, unsigned ngb,
                                                     unsigned gx, unsigned gy) {
     const unsigned c = blockIdx.y, w = blockIdx.x;
     if (!((mask >> c) & 1u)) return;
-    const SysCoef<T> S = M->S[c];
-    const T *b = M->b[c];
-    T *x = M->x[c];
+    const SysCoef<T> S = global_ptr(M->S[c]);
+    const T *b = global_ptr(M->b[c]);
+    T *x = global_ptr(M->x[c]);
     if (w < ngb) {
-        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const T *)M->gv[c][prev], M->gv[c][prev ^ 1], color,
-                             threadIdx.x, ghost_row_of_lane(w));
+        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const T *)global_ptr(M->gv[c][prev]),
+                             global_ptr(M->gv[c][prev ^ 1]), color, threadIdx.x, ghost_row_of_lane(w));
         return;
     }
     rbgs_cell(d, S, flag, b, x, color, zero_in, xcd_map(w - ngb, gridDim.x - ngb, gx, gy));
@@ -1630,12 +1685,12 @@ __global__ void __launch_bounds__(64 * BY) k_mom_colour_quad(Dims d, const MomTa
                                                              unsigned gy) {
     const unsigned c = blockIdx.y, w = blockIdx.x;
     if (!((mask >> c) & 1u)) return;
-    const SysCoef<float> S = M->S[c];
-    const float *b = M->b[c];
-    float *x = M->x[c];
+    const SysCoef<float> S = global_ptr(M->S[c]);
+    const float *b = global_ptr(M->b[c]);
+    float *x = global_ptr(M->x[c]);
     if (w < ngb) {
-        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const float *)M->gv[c][prev], M->gv[c][prev ^ 1], color,
-                             threadIdx.x, ghost_row_of_lane(w));
+        ghost_rows_in_colour(d, S, flag, b, x, G, S.is_p, (const float *)global_ptr(M->gv[c][prev]),
+                             global_ptr(M->gv[c][prev ^ 1]), color, threadIdx.x, ghost_row_of_lane(w));
         return;
     }
     rbgs_quad<BY>(d, S, flag, b, x, color, zero_in, xcd_map(w - ngb, gridDim.x - ngb, gx, gy));
@@ -1647,7 +1702,8 @@ __global__ void __launch_bounds__(256) k_mom_ghost(Dims d, const MomTable<T> *M,
                                                    int only) {
     const unsigned c = blockIdx.y;
     if (!((mask >> c) & 1u)) return;
-    ghost_relax_rows(G, 0, M->b[c], M->x[c], (const T *)nullptr, M->gv[c][0], d, only);
+    ghost_relax_rows(G, 0, global_ptr(M->b[c]), global_ptr(M->x[c]), (const T *)nullptr, global_ptr(M->gv[c][0]), d,
+                     only);
 }
 
 template <typename T>
@@ -1694,22 +1750,24 @@ __global__ void __launch_bounds__(256) k_mom_residual(Dims d, const MomTable<dou
                                                       unsigned gy) {
     const unsigned c = blockIdx.y;
     if (!((mask >> c) & 1u)) return;
-    const SysCoef<double> S = M->S[c];
+    const SysCoef<double> S = global_ptr(M->S[c]);
     const NormSpec off{0, nullptr, nullptr, nullptr, nullptr, -1};
     double acc[2] = {0, 0};
-    const double *b = M->b[c], *x = M->x[c];
+    const double *b = global_ptr(M->b[c]), *x = global_ptr(M->x[c]);
     if constexpr (WHAT == 2) {
-        const SysCoef<float> S32 = Mb->S[c];
-        residual_block(d, S, G, flag, b, (const float *)Ma->x[c], ResidualCorrection{S32, Mb->brw[c], Mb->x[c]}, off,
-                       blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+        const SysCoef<float> S32 = global_ptr(Mb->S[c]);
+        residual_block<false>(d, S, G, flag, b, (const float *)global_ptr(Ma->x[c]),
+                              ResidualCorrection{S32, global_ptr(Mb->brw[c]), global_ptr(Mb->x[c])}, off, blockIdx.x,
+                              gridDim.x, ngb, gx, gy, acc);
     } else if constexpr (WHAT == 3) {
-        residual_block(d, S, G, flag, b, (const double *)M->r[c], ResidualJacobi{S, G, M->r[c], M->x[c]}, off,
-                       blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+        double *r = global_ptr(M->r[c]);
+        residual_block<false>(d, S, G, flag, b, (const double *)r, ResidualJacobi{S, G, r, global_ptr(M->x[c])}, off,
+                              blockIdx.x, gridDim.x, ngb, gx, gy, acc);
     } else if constexpr (WHAT == 1) {
-        residual_block(d, S, G, flag, b, x, ResidualStore<double>{M->r[c]}, off, blockIdx.x, gridDim.x, ngb, gx, gy,
-                       acc);
+        residual_block<false>(d, S, G, flag, b, x, ResidualStore<double>{global_ptr(M->r[c])}, off, blockIdx.x,
+                              gridDim.x, ngb, gx, gy, acc);
     } else {
-        residual_block(d, S, G, flag, b, x, ResidualDrop{}, off, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
+        residual_block<false>(d, S, G, flag, b, x, ResidualDrop{}, off, blockIdx.x, gridDim.x, ngb, gx, gy, acc);
     }
     const double a1[1] = {acc[0]};
     bsum<1>(a1, partial, (long)blockIdx.x * 3 + c);
@@ -1742,9 +1800,9 @@ __global__ void __launch_bounds__(256) k_mom_d2f_first(Dims d, const MomTable<do
                                                        unsigned mask, const uint8_t *flag, int from_b) {
     const unsigned c = blockIdx.z / d.nz, k = blockIdx.z % d.nz;
     if (!((mask >> c) & 1u)) return;
-    const SysCoef<float> S = M32->S[c];
-    d2f_first(d, S, flag, from_b ? M->b[c] : M->r[c], M32->brw[c], M32->x[c], 2 * (blockIdx.x * 64 + threadIdx.x),
-              blockIdx.y * 4 + threadIdx.y, k);
+    const SysCoef<float> S = global_ptr(M32->S[c]);
+    d2f_first(d, S, flag, from_b ? global_ptr(M->b[c]) : global_ptr(M->r[c]), global_ptr(M32->brw[c]),
+              global_ptr(M32->x[c]), 2 * (blockIdx.x * 64 + threadIdx.x), blockIdx.y * 4 + threadIdx.y, k);
 }
 
 // x = e, x += e, or x or r = e0 + e
@@ -1754,12 +1812,12 @@ __global__ void __launch_bounds__(256) k_mom_add(Dims d, const MomTable<double> 
     const int i0 = 2 * (blockIdx.x * 64 + threadIdx.x), j = blockIdx.y * 4 + threadIdx.y;
     if (!((mask >> c) & 1u) || i0 >= d.nx || j >= d.ny) return;
     const long q = cidx(d, i0, j, k);
-    const float2 e = *reinterpret_cast<const float2 *>(M32->x[c] + q);
-    double *out = (to_r ? M->r[c] : M->x[c]) + q;
+    const float2 e = *reinterpret_cast<const float2 *>(global_ptr(M32->x[c]) + q);
+    double *out = (to_r ? global_ptr(M->r[c]) : global_ptr(M->x[c])) + q;
     double2 *x = reinterpret_cast<double2 *>(out);
     double2 v = make_double2((double)e.x, (double)e.y);
     if (M0) {
-        const float2 o = *reinterpret_cast<const float2 *>(M0->x[c] + q);
+        const float2 o = *reinterpret_cast<const float2 *>(global_ptr(M0->x[c]) + q);
         v.x = (double)o.x + v.x;
         v.y = (double)o.y + v.y;
     } else if (add) {

@@ -20,6 +20,10 @@ namespace ibm {
 
 #define C1(a, i) ((a)[(i) + 2])
 
+// v is formed here, by every lane: else the compiler turns a select of it into a
+// branch, its loads behind that, one round trip to memory after another
+__device__ inline void form_now(double &v) { asm volatile("" : "+v"(v)); }
+
 __device__ inline double nan_d() { return __builtin_nan(""); }
 
 // ---------------------------------------------------------------------------
@@ -78,10 +82,14 @@ __global__ void k_interp_stag(Geo g, const double *u1, const double *u2, const d
 // three components, fused.  <- src/ibm3d_fracstep.c:117-170 and :237-269
 // Writes N (non-fluid: NaN) and b_l (non-fluid rows: 0); accumulates the
 // squared norms of b_l over the interior rows for the stopping test. Bound by
-// its 16 fields: 256 x 128 x 128 176 us, 3.3 TB/s (187 with the 30 divisions per
-// cell that the axis metrics replace; the blocks in contiguous ranges per XCD:
-// 183).
+// its 16 fields: 256 x 128 x 128 166 us, 3.3 TB/s of those, 4.2 with the halos
+// (175 with the components one after the other: a store between them, or a
+// branch on the turbulence stress or the forcing, holds the next one's loads
+// back, hence the two switches at compile time and the stores at the end; 187
+// with the 30 divisions per cell that the axis metrics replace; the blocks in
+// contiguous ranges per XCD: 8 us more; several planes per thread, 212 registers).
 // ---------------------------------------------------------------------------
+template <bool TAU, bool FA>
 __global__ void __launch_bounds__(256) k_conv_rhs(Geo g, StepParams sp, const uint8_t *flag,
                                                   const double *u1, const double *u2, const double *u3,
                                                   const double *U1, const double *U2, const double *U3,
@@ -113,6 +121,7 @@ __global__ void __launch_bounds__(256) k_conv_rhs(Geo g, StepParams sp, const ui
         double *bb[3] = {b1, b2, b3};
         const double dp[3] = {(p[q + 1] - p[q - 1]) * X0.r2, (p[q + sy] - p[q - sy]) * Y0.r2,
                               (p[q + sz] - p[q - sz]) * Z0.r2};
+        double nv[3], bv[3];
 #pragma unroll
         for (int l = 0; l < 3; l++) {
             const double *a = uu[l];
@@ -122,19 +131,26 @@ __global__ void __launch_bounds__(256) k_conv_rhs(Geo g, StepParams sp, const ui
             const double uw = c + X0.w * (xm - c), ue = xp + wxp * (c - xp);
             const double us = c + Y0.w * (ym - c), un = yp + wyp * (c - yp);
             const double ud = c + Z0.w * (zm - c), uu_ = zp + wzp * (c - zp);
-            const double n = (Ue * ue - Uw * uw) * X0.rd + (Vn * un - Vs * us) * Y0.rd + (Wu * uu_ - Wd * ud) * Z0.rd;
+            double n = (Ue * ue - Uw * uw) * X0.rd + (Vn * un - Vs * us) * Y0.rd + (Wu * uu_ - Wd * ud) * Z0.rd;
             double divt = 0;
-            if (tau.on) {
+            if (TAU) {
                 const double *t1 = tau.t[tau.slot[l][0]], *t2 = tau.t[tau.slot[l][1]], *t3 = tau.t[tau.slot[l][2]];
                 divt = (t1[q + 1] - t1[q - 1]) * X0.r2 + (t2[q + sy] - t2[q - sy]) * Y0.r2
                     + (t3[q + sz] - t3[q - sz]) * Z0.r2;
             }
-            const double b = -sp.dt / 2 * (3 * n - npl) - sp.dt * dp[l] + kc * c
+            double b = -sp.dt / 2 * (3 * n - npl) - sp.dt * dp[l] + kc * c
                 + kW * xm + kE * xp + kS * ym + kN * yp + kD * zm + kU * zp
-                + sp.dt * (sp.fa[l] ? sp.fa[l][q] : sp.force[l]) - sp.dt * divt;
-            NN[l][q] = fl ? n : nan_d();
-            bb[l][q] = fl ? b : 0.0;
-            nrm[l] = fl ? b * b : 0.0;
+                + sp.dt * (FA && sp.fa[l] ? sp.fa[l][q] : sp.force[l]) - sp.dt * divt;
+            form_now(n);
+            form_now(b);
+            nv[l] = fl ? n : nan_d();
+            bv[l] = fl ? b : 0.0;
+        }
+#pragma unroll
+        for (int l = 0; l < 3; l++) {
+            NN[l][q] = nv[l];
+            bb[l][q] = bv[l];
+            nrm[l] = bv[l] * bv[l];
         }
     }
     block_sum_store<3>(nrm, partial, block_linear());
@@ -157,34 +173,27 @@ __global__ void __launch_bounds__(256) k_face_star(Geo g, StepParams sp, const u
     const long q = cidx(d, i, j, k);
     const long sy = d.sy, sz = d.sz;
     const double dt = sp.dt;
-    const uint8_t f0 = flag[q];
-    if (j < d.ny && k < d.nz) {  // x face i-1/2
-        const uint8_t fm = flag[q - 1];
-        const AxisMetric M = C1(g.mx, i);
-        const double um = us1[q - 1], u0 = us1[q], pm = p[q - 1], p0 = p[q];
-        const double tm = um + dt * (p0 - p[q - 2]) * C1(g.mx, i - 1).r2, t0 = u0 + dt * (p[q + 1] - pm) * M.r2;
-        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
-        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
-        F1[q] = v;
-    }
-    if (i < d.nx && k < d.nz) {  // y face j-1/2
-        const uint8_t fm = flag[q - sy];
-        const AxisMetric M = C1(g.my, j);
-        const double um = us2[q - sy], u0 = us2[q], pm = p[q - sy], p0 = p[q];
-        const double tm = um + dt * (p0 - p[q - 2 * sy]) * C1(g.my, j - 1).r2, t0 = u0 + dt * (p[q + sy] - pm) * M.r2;
-        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
-        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
-        F2[q] = v;
-    }
-    if (i < d.nx && j < d.ny) {  // z face k-1/2
-        const uint8_t fm = flag[q - sz];
-        const AxisMetric M = C1(g.mz, k);
-        const double um = us3[q - sz], u0 = us3[q], pm = p[q - sz], p0 = p[q];
-        const double tm = um + dt * (p0 - p[q - 2 * sz]) * C1(g.mz, k - 1).r2, t0 = u0 + dt * (p[q + sz] - pm) * M.r2;
-        const bool body = (fm == F_FLUID && f0 == F_GHOST) || (fm == F_GHOST && f0 == F_FLUID);
-        const double v = body ? u0 + M.w * (um - u0) : t0 + M.w * (tm - t0) - dt * (p0 - pm) * M.rc;
-        F3[q] = v;
-    }
+    // every load is in the padded range: all issue before the first wait, and
+    // the faces past the last cell's are dropped at the stores
+    const uint8_t f0 = flag[q], fx = flag[q - 1], fy = flag[q - sy], fz = flag[q - sz];
+    const double p0 = p[q];
+    const double px[3] = {p[q - 2], p[q - 1], p[q + 1]}, py[3] = {p[q - 2 * sy], p[q - sy], p[q + sy]};
+    const double pz[3] = {p[q - 2 * sz], p[q - sz], p[q + sz]};
+    const double ux = us1[q - 1], vx = us1[q], uy = us2[q - sy], vy = us2[q], uz = us3[q - sz], vz = us3[q];
+    const AxisMetric X = C1(g.mx, i), Y = C1(g.my, j), Z = C1(g.mz, k);
+    const double xr = C1(g.mx, i - 1).r2, yr = C1(g.my, j - 1).r2, zr = C1(g.mz, k - 1).r2;
+    const auto face = [&](uint8_t fm, const AxisMetric &M, double rm, double um, double u0, const double (&pn)[3]) {
+        const double tm = um + dt * (p0 - pn[0]) * rm, t0 = u0 + dt * (pn[2] - pn[1]) * M.r2;
+        const bool body = fm + f0 == F_FLUID + F_GHOST && fm != f0;
+        double vb = u0 + M.w * (um - u0), v = t0 + M.w * (tm - t0) - dt * (p0 - pn[1]) * M.rc;
+        form_now(vb);
+        form_now(v);
+        return body ? vb : v;
+    };
+    const double v1 = face(fx, X, xr, ux, vx, px), v2 = face(fy, Y, yr, uy, vy, py), v3 = face(fz, Z, zr, uz, vz, pz);
+    if (j < d.ny && k < d.nz) F1[q] = v1;
+    if (i < d.nx && k < d.nz) F2[q] = v2;
+    if (i < d.nx && j < d.ny) F3[q] = v3;
 }
 
 // ---------------------------------------------------------------------------
@@ -221,6 +230,8 @@ __global__ void __launch_bounds__(256) k_poisson_rhs(Geo g, StepParams sp, const
 // p_next = p + p' (fluid, ghost) / NaN (solid); u_next = u* - dt grad p'
 // (fluid) / NaN (solid); ghost entries of u_next are left untouched, as in
 // the reference. U_next = U* - dt dp'/dn on faces with no solid side, else NaN.
+// 256 x 128 x 128: 106 us, 6.2 TB/s (121 with the flags looked at before each
+// load).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_update(Geo g, StepParams sp, const uint8_t *flag,
                                                 const double *p, const double *pp,
@@ -236,26 +247,36 @@ __global__ void __launch_bounds__(256) k_update(Geo g, StepParams sp, const uint
     const long q = cidx(d, i, j, k);
     const long sy = d.sy, sz = d.sz;
     const double dt = sp.dt;
-    const uint8_t f0 = flag[q];
+    // every load is in the padded range: all issue before the first wait
+    const uint8_t f0 = flag[q], fx = flag[q - 1], fy = flag[q - sy], fz = flag[q - sz];
+    const double pc = p[q], c = pp[q], xm = pp[q - 1], xp = pp[q + 1], ym = pp[q - sy], yp = pp[q + sy];
+    const double zm = pp[q - sz], zp = pp[q + sz];
+    const double u1 = us1[q], u2 = us2[q], u3 = us3[q], s1 = F1[q], s2 = F2[q], s3 = F3[q];
+    const AxisMetric X = C1(g.mx, i), Y = C1(g.my, j), Z = C1(g.mz, k);
+    const bool in0 = f0 != F_SOLID;
+    double pv = pc + c, n1 = u1 - dt * (xp - xm) * X.r2, n2 = u2 - dt * (yp - ym) * Y.r2;
+    double n3 = u3 - dt * (zp - zm) * Z.r2;
+    double g1 = s1 - dt * (c - xm) * X.rc, g2 = s2 - dt * (c - ym) * Y.rc, g3 = s3 - dt * (c - zm) * Z.rc;
+    for (double *v : {&pv, &n1, &n2, &n3, &g1, &g2, &g3}) form_now(*v);
+    const bool fluid = f0 == F_FLUID;
+    pv = fluid || f0 == F_GHOST ? pv : nan_d();
+    n1 = fluid ? n1 : nan_d();
+    n2 = fluid ? n2 : nan_d();
+    n3 = fluid ? n3 : nan_d();
+    g1 = in0 && fx != F_SOLID ? g1 : nan_d();
+    g2 = in0 && fy != F_SOLID ? g2 : nan_d();
+    g3 = in0 && fz != F_SOLID ? g3 : nan_d();
     if (i < d.nx && j < d.ny && k < d.nz) {
-        pn[q] = (f0 == F_FLUID || f0 == F_GHOST) ? p[q] + pp[q] : nan_d();
-        if (f0 == F_FLUID) {
-            un1[q] = us1[q] - dt * (pp[q + 1] - pp[q - 1]) * C1(g.mx, i).r2;
-            un2[q] = us2[q] - dt * (pp[q + sy] - pp[q - sy]) * C1(g.my, j).r2;
-            un3[q] = us3[q] - dt * (pp[q + sz] - pp[q - sz]) * C1(g.mz, k).r2;
-        } else if (f0 == F_SOLID) {
-            un1[q] = un2[q] = un3[q] = nan_d();
+        pn[q] = pv;
+        if (fluid || f0 == F_SOLID) {
+            un1[q] = n1;
+            un2[q] = n2;
+            un3[q] = n3;
         }
     }
-    if (j < d.ny && k < d.nz)
-        G1[q] = (flag[q - 1] != F_SOLID && f0 != F_SOLID)
-            ? F1[q] - dt * (pp[q] - pp[q - 1]) * C1(g.mx, i).rc : nan_d();
-    if (i < d.nx && k < d.nz)
-        G2[q] = (flag[q - sy] != F_SOLID && f0 != F_SOLID)
-            ? F2[q] - dt * (pp[q] - pp[q - sy]) * C1(g.my, j).rc : nan_d();
-    if (i < d.nx && j < d.ny)
-        G3[q] = (flag[q - sz] != F_SOLID && f0 != F_SOLID)
-            ? F3[q] - dt * (pp[q] - pp[q - sz]) * C1(g.mz, k).rc : nan_d();
+    if (j < d.ny && k < d.nz) G1[q] = g1;
+    if (i < d.nx && k < d.nz) G2[q] = g2;
+    if (i < d.nx && j < d.ny) G3[q] = g3;
 }
 
 // ---------------------------------------------------------------------------
@@ -804,9 +825,14 @@ void launch_conv_rhs(hipStream_t st, const Geo &g, const StepParams &sp, const u
                      const double *const u[3], const double *const U[3], const double *p,
                      const double *const Np[3], double *const N[3], double *const b[3], const TauPtrs &tau,
                      double *partial) {
-    hipLaunchKernelGGL(k_conv_rhs, cell_grid(g.d, 0), dim3(64, 4), 0, st, g, sp, flag, u[0], u[1], u[2],
-                       U[0], U[1], U[2], p, Np[0], Np[1], Np[2], N[0], N[1], N[2], b[0], b[1], b[2], tau,
-                       partial);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, cell_grid(g.d, 0), dim3(64, 4), 0, st, g, sp, flag, u[0], u[1], u[2], U[0], U[1],
+                           U[2], p, Np[0], Np[1], Np[2], N[0], N[1], N[2], b[0], b[1], b[2], tau, partial);
+    };
+    if (sp.fa[0] || sp.fa[1] || sp.fa[2])
+        tau.on ? launch(k_conv_rhs<true, true>) : launch(k_conv_rhs<false, true>);
+    else
+        tau.on ? launch(k_conv_rhs<true, false>) : launch(k_conv_rhs<false, false>);
 }
 
 void launch_face_star(hipStream_t st, const Geo &g, const StepParams &sp, const uint8_t *flag,

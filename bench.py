@@ -15,10 +15,10 @@ The headline value is the mixed path in Mcell-steps/s
 (IBM3D_PREC_MIXED_KRYLOV): FP32 momentum sweeps in FP64 refinement; the
 pressure is solved directly in FP64 where the case allows it, else by FP64
 BiCGSTAB whose multigrid preconditioner runs in FP32. The plain FP64 path
-runs the same steps for the speed-up. After the timed regions both GPU paths and the FP64 CPU oracle run the first steps of the same case from
-the same initial field; their differences (rel-L2 and Linf of u and p,
-max|div U|, drag and lift) are the line's error statement. Prints one JSON
-line.
+runs the same steps for the speed-up. After the timed regions both GPU paths
+and the FP64 CPU oracle run the first steps of the same case from the same
+initial field; their differences (rel-L2 and Linf of u and p, max|div U|, drag
+and lift) are the line's error statement. Prints one JSON line.
 """
 from __future__ import annotations
 
