@@ -658,7 +658,13 @@ static void alloc_fields(IBMSolver *s) {
     nb = std::max(nb, apply_partials(s->d, s->ng) + 64);
     nb = std::max(nb, vec_partials(s->d) + 64);
     nb = std::max(nb, separable_partials(s->d));
-    // (a pressure solve's own sums follow those of its right-hand side)
+    // (a pressure solve's own sums follow those of its right-hand side, the outflow
+    // faces' those of the momentum right-hand sides)
+    long faces = 0;
+    for (int ax = 0; ax < 3; ax++)
+        for (int hi = 0; hi < 2; hi++)
+            if (s->bc[face_bc(ax, hi)].type == BC_CONVECTIVE_OUTFLOW) faces += conv_outflow_blocks(s->d, ax);
+    nb = std::max(nb, conv_rhs_blocks(s->d) + faces);
     s->partial.alloc((size_t)nb * 4);
 }
 

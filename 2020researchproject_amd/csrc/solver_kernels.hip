@@ -110,8 +110,8 @@ __device__ inline typename Vec2<T>::type load_pair(const TX *p) {
 }
 
 template <typename T, typename TX = T>
-__device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const TX *x, int i0, int j, int k, long q0,
-                                  T yv[2], T xq[2]) {
+__device__ inline void pair_apply(const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const TX *x, int i0, int j,
+                                  int k, long q0, T yv[2], T xq[2]) {
     using T2 = typename Vec2<T>::type;
     const AxisCoef<T> &AX = S.ax[0], &AY = S.ax[1], &AZ = S.ax[2];
     const int jm = (j == 0 && AY.periodic) ? AY.n - 1 : j - 1, jp = (j == AY.n - 1 && AY.periodic) ? 0 : j + 1;

@@ -155,29 +155,6 @@ static OuterParams make_outer(IBMSolver *s, int what, double t, double norm2[4])
     return op;
 }
 
-// Convective outflow faces: init copies the first interior cell's velocity,
-// otherwise one upwind step of the face values from the current u; each face
-// leaves its BC-row norms in sums[kConvNormSlot + 3 bc + c]. Returns whether
-// any face has this condition.
-static bool conv_outflow(IBMSolver *s, int init) {
-    bool any = false;
-    for (int ax = 0; ax < 3; ax++)
-        for (int hi = 0; hi < 2; hi++) {
-            const int bci = face_bc(ax, hi);
-            if (s->bc[bci].type != BC_CONVECTIVE_OUTFLOW) continue;
-            any = true;
-            if ((size_t)conv_outflow_blocks(s->d, ax) * 3 > s->partial.n)
-                fatal("convective outflow: partial-sum buffer too small");
-            TIMED("conv_outflow", 0, {
-                const long nb = launch_conv_outflow(s->stream, s->geo, ax, hi, s->bc[bci].uc, s->dt, init, s->u[0].p,
-                                                    s->u[1].p, s->u[2].p, s->conv_g[bci].p, s->sums.p + kConvSpeedSlot,
-                                                    s->partial.p);
-                launch_sum_partials(s->stream, s->partial.p, nb, 3, s->sums.p + kConvNormSlot + 3 * bci, 0);
-            });
-        }
-    return any;
-}
-
 // Rules of the outer layers (k_outer) for every kind of field, axis, side and
 // layer.  <- src/ibm3d_fracstep.c:855-1906
 static OuterRule outer_rule(const IBMSolver *s, int kind, int ax, int hi, int layer) {
@@ -342,6 +319,27 @@ static void add_rider(IBMSolver *s, SumRiders &sums, const double *partial, long
         sums.epoch_out = s->sums_d_epoch;
         sums.epoch = ++s->sums_epoch;
     }
+}
+
+// Convective outflow faces: init copies the first interior cell's velocity,
+// otherwise one upwind step of the face values from the current u; each face
+// leaves its BC-row norms behind the right-hand sides' partials, to be summed into
+// sums_h[kConvNormSlot + 3 bc + c].
+static void conv_outflow(IBMSolver *s, int init, SumRiders *sums) {
+    double *partial = s->partial.p + 3 * conv_rhs_blocks(s->d);
+    for (int ax = 0; ax < 3; ax++)
+        for (int hi = 0; hi < 2; hi++) {
+            const int bci = face_bc(ax, hi);
+            if (s->bc[bci].type != BC_CONVECTIVE_OUTFLOW) continue;
+            if (partial + 3 * conv_outflow_blocks(s->d, ax) > s->partial.p + s->partial.n)
+                fatal("convective outflow: partial-sum buffer too small");
+            long nb = 0;
+            TIMED("conv_outflow", 0,
+                  nb = launch_conv_outflow(s->stream, s->geo, ax, hi, s->bc[bci].uc, s->dt, init, s->u[0].p, s->u[1].p,
+                                           s->u[2].p, s->conv_g[bci].p, s->sums.p + kConvSpeedSlot, partial));
+            if (sums) add_rider(s, *sums, partial, nb, 3, kConvNormSlot + 3 * bci);
+            partial += 3 * nb;
+        }
 }
 
 // Finalize kernel `op` over the block partials, with the resulting scalars
@@ -2135,29 +2133,20 @@ static void do_step(IBMSolver *s) {
               launch_conv_rhs(s->stream, s->geo, sp, s->flag.p, u3, U3, s->p.p, Np, N, b, tau_ptrs(s),
                               s->partial.p));
     }
-    // squared norms of the right-hand sides: straight to the host, or to where
-    // the outflow faces' norms join them
-    bool conv = false;
-    for (const HostBC &B : s->bc) conv |= B.type == BC_CONVECTIVE_OUTFLOW;
-    if (conv) {
-        launch_sum_partials(s->stream, s->partial.p, conv_rhs_blocks(s->d), 3, s->sums.p, 0);
-        conv_outflow(s, 0);
-        publish_sums(s, kConvNormSlot + 18);
-    }
+    // squared norms of the right-hand sides and of the outflow faces' rows
+    SumRiders norms{};
+    add_rider(s, norms, s->partial.p, conv_rhs_blocks(s->d), 3, 0);
+    conv_outflow(s, 0, &norms);
     double fnorm[4];
     OuterParams ob = make_outer(s, BCD_FIELDS, s->time, fnorm), opp{};
-    {
-        SumRiders norms{};
-        if (!conv) add_rider(s, norms, s->partial.p, conv_rhs_blocks(s->d), 3, 0);
-        bc_rhs(s, ob, 0, 3, norms);
-    }
+    bc_rhs(s, ob, 0, 3, norms);
     // stopping norms of the momentum solves: the right-hand sides' sums, plus
     // the BC rows' and forcing parts
     double bn[3];
     auto form_norms = [&] {
         for (int l = 0; l < 3; l++) {
             double bn2 = s->sums_h[l] + s->sys[l].bc_norm2 + fnorm[l];
-            for (int f = 0; conv && f < 6; f++)
+            for (int f = 0; f < 6; f++)
                 if (s->bc[f].type == BC_CONVECTIVE_OUTFLOW) bn2 += s->sums_h[kConvNormSlot + 3 * f + l];
             bn[l] = std::sqrt(bn2);
         }
@@ -2262,7 +2251,7 @@ static void do_step(IBMSolver *s) {
 
 void iterate_impl(IBMSolver *s, int steps, bool verbose) {
     const double t0 = s->time;
-    if (!s->conv_ready) conv_outflow(s, 1);
+    if (!s->conv_ready) conv_outflow(s, 1, nullptr);
     s->conv_ready = true;
     // prologue  <- src/ibm3d_fracstep.c:46-54
     update_outer(s);

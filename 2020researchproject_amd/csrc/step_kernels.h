@@ -98,13 +98,14 @@ struct OuterFields {
 };
 // Sums of columns of block partials that ride in a boundary launch as one more
 // workgroup and go to device-mapped host memory, with the epoch after the last.
+constexpr int kMaxRiders = 7;  // a right-hand side's norms and those of six outflow faces
 struct SumRiders {
     struct {
         const double *partial;
         long nblk;
         int nv;
         double *out;
-    } r[2];
+    } r[kMaxRiders];
     int n;
     unsigned *epoch_out;
     unsigned epoch;

@@ -194,3 +194,34 @@ def test_gpu_convective_sphere_mixed(I, new_oracle, new_gpu, cases):
             rel = np.linalg.norm((a - b)[fl]) / np.linalg.norm(a[fl])
             assert rel < 1e-7, (prec, name, rel)
         assert g.max_div() < 1e-8
+
+
+def three_outlets(I, s, n):
+    """A skew stream in through the low faces, out through convective high ones."""
+    nx, ny, nz = n
+    s.set_grid(stretched(nx, 0.0, 2.0), stretched(ny, 0.0, 1.0, 0.2), np.linspace(0.0, 0.8, nz + 1))
+    s.set_params(50.0, 0.005)
+    s.set_bc(I.DIR_WEST | I.DIR_SOUTH | I.DIR_DOWN, I.BC_VELOCITY_COMPONENT, I.VAL_CONST, 1.0, 0.5, 0.3)
+    s.set_bc(I.DIR_EAST | I.DIR_NORTH | I.DIR_UP, I.BC_CONVECTIVE_OUTFLOW, 0.0)
+    s.set_obstacle(None)
+    s.set_linear_solver(I.SOLVER_BiCGSTAB, I.PRECOND_AMG, 1e-12)
+    s.assemble()
+    s.init_flow_func(lambda x, y, z: 1.0 + 0.1 * math.sin(2.1 * y + 0.5) * math.cos(1.3 * x),
+                     lambda x, y, z: 0.5 + 0.1 * math.sin(1.7 * z) * math.cos(0.9 * x),
+                     lambda x, y, z: 0.3 + 0.1 * math.cos(2.3 * x + y), lambda x, y, z: 0.0)
+    return s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(24, 16, 12), (6, 34, 70)])
+def test_gpu_three_convective_outlets_match_oracle(I, new_oracle, new_gpu, n):
+    """Several faces' norms behind one another in the partial sums; in the second
+    grid the faces leave more of them than the cells do."""
+    o = three_outlets(I, new_oracle(), n)
+    g = three_outlets(I, new_gpu(), n)
+    o.iterate(4)
+    g.iterate(4)
+    for name in ("U1", "U2", "U3", "P"):
+        a, b = o.get(name), g.get(name)
+        scale = max(np.max(np.abs(a)), 1e-30)
+        assert np.max(np.abs(a - b)) / scale < 1e-8, name
