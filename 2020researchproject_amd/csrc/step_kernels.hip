@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(256) k_poisson_rhs(Geo g, StepParams sp, const
 // p_next = p + p' (fluid, ghost) / NaN (solid); u_next = u* - dt grad p'
 // (fluid) / NaN (solid); ghost entries of u_next are left untouched, as in
 // the reference. U_next = U* - dt dp'/dn on faces with no solid side, else NaN.
-// 256 x 128 x 128: 106 us, 6.2 TB/s (121 with the flags looked at before each
+// 256 x 128 x 128: 106 us, 6.1 TB/s (121 with the flags looked at before each
 // load).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_update(Geo g, StepParams sp, const uint8_t *flag,
