@@ -1773,6 +1773,10 @@ static bool separable_finish(IBMSolver *s, const double *b, double *x, double bn
                            s->sums_d + kPressureSlot, 0, s->sums_d_epoch, e);
         wait_epoch(s->stream, s->sums_h_epoch, e);
     }
+    // The iterative solve starts from x = 0 with zero outer layers: its operator
+    // forms 0 * (outer value) at folded faces, and the projection has filled
+    // the outer layers of p' from a solution that may not be finite.
+    launch_fill(s->stream, x, s->d.ncell, 0.0);
     // with a body the memory of the capacitance matrix is the hierarchy's: the
     // solver goes over to the iterative path for good
     if (s->cap_on) {
@@ -2228,6 +2232,7 @@ static void do_step(IBMSolver *s) {
         mom_open = false;
         if (mom_direct) {
             if (momentum_direct_met(s, bn)) break;
+            for (auto &u : s->us) launch_fill(s->stream, u.p, s->d.ncell, 0.0);  // as in separable_finish
             mom_iterate();
         } else if (momentum_sweeps_finish(s, sweeps, bn)) {
             break;

@@ -1,0 +1,77 @@
+"""Calls that leave the direct solves, or that the direct solves must not take
+from the iterative ones: systems they cannot hold, tolerances they cannot
+reach, settings made after assembly."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+H = 0.125  # cell width of the uniform grids below: every face and centre is a binary fraction
+
+
+def setup_surface_body(s, I, cases, kind, shape=(32, 16, 16), tol=1e-12, precision=0):
+    """Inlet, pressure outlet, free slip; a body whose surface runs through
+    cell centres: a sphere of radius 3 h about a cell centre (30 of its 90 ghost
+    cells have phi = 0), or a box with its faces in planes of cell centres."""
+    f = [H * np.arange(n + 1) for n in shape]
+    s.set_grid(*f)
+    s.set_params(100.0, 0.01)
+    s.set_bc(I.DIR_WEST, I.BC_VELOCITY_COMPONENT, I.VAL_CONST, 1.0, 0.0, 0.0)
+    s.set_bc(I.DIR_EAST, I.BC_PRESSURE, I.VAL_CONST, 0.0)
+    s.set_bc(I.DIR_SOUTH | I.DIR_NORTH | I.DIR_DOWN | I.DIR_UP, I.BC_FREE_SLIP_WALL)
+    if kind == "sphere":
+        s.set_obstacle_sphere(*[H * (n // 2 + 0.5) for n in shape], 3 * H)
+    else:
+        lo, hi = [H * (n // 2 - 2.5) for n in shape], [H * (n // 2 + 1.5) for n in shape]
+        s.set_obstacle_stl_bytes(cases.blocks_stl([(lo[0], hi[0], lo[1], hi[1], hi[2])], base=lo[2]))
+    s.set_linear_solver(I.SOLVER_BiCGSTAB, I.PRECOND_AMG, tol)
+    s.set_precision(precision)
+    s.assemble()
+    s.init_flow_const(1.0, 0.0, 0.0, 0.0)
+    return f
+
+
+def span_of(f):
+    """Largest over lowest eigenvalue of the pressure operator, bounded by
+    sum_a 4 / h_a^2 over min_a (pi / (2 L_a))^2."""
+    return sum(4 / np.diff(x).min() ** 2 for x in f) / min((np.pi / (2 * (x[-1] - x[0]))) ** 2 for x in f)
+
+
+def fields(s):
+    return {n: s.get(n)[2:-2, 2:-2, 2:-2] for n in ("U1", "U2", "U3", "P")}
+
+
+def assert_close(out, ref, bound):
+    """Same finite cells, and differences of at most `bound` of the velocity's
+    and the pressure's norm."""
+    m = {n: np.isfinite(a) for n, a in ref.items()}
+    speed = np.sqrt(sum(np.linalg.norm(ref[n][m[n]]) ** 2 for n in ("U1", "U2", "U3")))
+    for n, a in out.items():
+        assert np.array_equal(np.isfinite(a), m[n]), n
+        scale = np.linalg.norm(ref[n][m[n]]) if n == "P" else speed
+        assert np.linalg.norm(a[m[n]] - ref[n][m[n]]) <= bound * scale, n
+
+
+@pytest.mark.parametrize("precision", [0, 2], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["sphere", "box"])
+def test_body_surface_through_cell_centres(new_gpu, new_oracle, I, cases, kind, precision):
+    """Where phi = 0 at a ghost cell its mirror point is the cell itself: the
+    pressure row of that cell is zero and p' stays zero there, in the oracle and
+    in either solve. Both residuals are below tol, so the fields differ by at
+    most 2 tol times the span of the operator's eigenvalues."""
+    tol = 1e-12
+    o = new_oracle()
+    f = setup_surface_body(o, I, cases, kind, tol=tol)
+    o.iterate(3)
+    ref = fields(o)
+    for multigrid in (False, True):
+        s = new_gpu()
+        if multigrid:
+            s.set_mg_relaxation(1.3)
+        setup_surface_body(s, I, cases, kind, tol=tol, precision=precision)
+        assert np.array_equal(s.flags(), o.flags())
+        s.iterate(3)
+        assert (s.last_norms() <= tol).all()
+        assert_close(fields(s), ref, 2 * tol * span_of(f))
