@@ -28,11 +28,12 @@ struct GreenBox { int lo[3], hi[3]; };  // end exclusive
 // operator A holds in every fluid row; a right-hand side mu at the ghost cells
 // makes its solution also meet the ghost rows R x = b_g:
 //   (R A^-1 E) mu = b_g - R A^-1 b_fluid,  x = A^-1 (b_fluid + E mu).
+// A zero row of R (a cell centre on the surface) is x = b.
 // look: the box of the ghost cells and their stencil points, cells: that of the
 // ghost cells; fluid, ghost: masks of the interior cells, one word per 16 cells
 // of a row.
 struct SeparableBody {
-    const uint8_t *flag;
+    const uint8_t *flag;  // F_SOLID: rows x = b, zero ghost rows among them
     GhostRows<double> G;
     const double *inv64;  // inverse of R A^-1 E, row pitch ld; one of the two
     const float *inv32;
@@ -79,5 +80,8 @@ struct GreenScratch { double *v[kGreenVecs]; int per; };
 void launch_green_plane(hipStream_t st, const Dims &d, const SeparableSys &S, int k, const int3 *src, int nsrc,
                         const GreenBox &box, const GhostRows<double> &G, const int *loc, double *h,
                         const GreenScratch &green, double *out, long ld);
+// *bad = 1 if one of a[0 .. n) is not finite (left alone else)
+template <typename T>
+void launch_not_finite(hipStream_t st, const T *a, long n, int *bad);
 
 }  // namespace ibm

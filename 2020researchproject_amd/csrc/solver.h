@@ -310,6 +310,7 @@ struct _ibm_solver {
     ibm::DBuf<double> cap_inv64, cap_t;
     ibm::DBuf<float> cap_inv32;
     ibm::DBuf<uint16_t> cap_mask[2];      // fluid, ghost
+    ibm::DBuf<uint8_t> cap_flag;          // flags with the zero ghost rows' cells as F_SOLID, if there are any
     std::vector<ibm::VGraph> vgraphs;     // captured V-cycles per (input, output)
     ibm::Krylov kry;
     ibm::GmresData gm;                    // SOLVER_GMRES / SOLVER_PCG / SOLVER_AMG scratch (pressure)

@@ -669,10 +669,18 @@ void ensure_mg(IBMSolver *s) {
     HIP_CHECK(hipStreamSynchronize(s->stream));
 }
 
+static void free_capacitance(IBMSolver *s) {
+    s->cap_on = false;
+    s->dev_bytes -= s->cap_inv64.n * sizeof(double) + s->cap_inv32.n * sizeof(float);
+    s->cap_inv64.free();
+    s->cap_inv32.free();
+}
+
 // The ghost rows of a body for the direct pressure solve: R A^-1 E column by
 // column (A^-1 of the unit vectors of the ghost cells), and its inverse. False
 // where the method does not apply: the box alone is singular, a fluid cell
-// borders a solid one that is no ghost cell, or there is no room.
+// borders a solid one that is no ghost cell, there is no room, or the inverse
+// is not finite.
 // Room: what the estimate of a solver's memory holds for the multigrid
 // hierarchy, which is then not built (and, for the inversion, for the fields
 // that are not there yet). The inverse is kept in FP64; in mixed-Krylov mode,
@@ -741,7 +749,7 @@ static bool build_capacitance(IBMSolver *s) {
     for (const auto &p : plane) src.insert(src.end(), p.begin(), p.end());
 
     size_t scratch_bytes = 0;
-    DBuf<int> dloc;
+    DBuf<int> dloc, bad;
     DBuf<int3> dsrc;
     DBuf<double> scratch, wide_inv;
     {
@@ -749,6 +757,7 @@ static bool build_capacitance(IBMSolver *s) {
         dloc.upload(loc);
         dsrc.upload(src);
         scratch.alloc(gauss_jordan_scratch(ng));
+        bad.alloc(1);
         if (!wide) wide_inv.alloc((size_t)ld * ld);
     }
     if (wide) s->cap_inv64.alloc((size_t)ld * ld);
@@ -769,8 +778,28 @@ static bool build_capacitance(IBMSolver *s) {
         s->cap_inv32.alloc((size_t)ld * ld);
         launch_d2f_flat(s->stream, inv, s->cap_inv32.p, (long)ld * ld);
     }
+    // without pivoting a pivot may vanish (bodies so far: growth below 50)
+    int lost = 0;
+    if (wide) launch_not_finite(s->stream, inv, (long)ld * ld, bad.p);
+    else launch_not_finite(s->stream, s->cap_inv32.p, (long)ld * ld, bad.p);
+    HIP_CHECK(hipMemcpyAsync(&lost, bad.p, sizeof lost, hipMemcpyDeviceToHost, s->stream));
     HIP_CHECK(hipStreamSynchronize(s->stream));  // the scratch is freed here
+    if (lost) {
+        free_capacitance(s);
+        return false;
+    }
     s->cap.flag = s->flag.p;
+    std::vector<uint8_t> flags = s->flag_dev_h;
+    bool zero = false;
+    for (const GhostCell &g : s->ghosts)
+        if (1 - g.wself == 0) {
+            flags[g.cell] = F_SOLID;
+            zero = true;
+        }
+    if (zero) {
+        s->cap_flag.upload(flags);
+        s->cap.flag = s->cap_flag.p;
+    }
     s->cap.G = s->gp.G64;
     s->cap.inv64 = wide ? s->cap_inv64.p : nullptr;
     s->cap.inv32 = wide ? nullptr : s->cap_inv32.p;

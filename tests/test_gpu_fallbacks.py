@@ -14,7 +14,8 @@ H = 0.125  # cell width of the uniform grids below: every face and centre is a b
 def setup_surface_body(s, I, cases, kind, shape=(32, 16, 16), tol=1e-12, precision=0):
     """Inlet, pressure outlet, free slip; a body whose surface runs through
     cell centres: a sphere of radius 3 h about a cell centre (30 of its 90 ghost
-    cells have phi = 0), or a box with its faces in planes of cell centres."""
+    cells have phi = 0), or a box (5 or, "wide", 30 cells) with its faces in
+    planes of cell centres (all 98 or 5048 have)."""
     f = [H * np.arange(n + 1) for n in shape]
     s.set_grid(*f)
     s.set_params(100.0, 0.01)
@@ -24,7 +25,9 @@ def setup_surface_body(s, I, cases, kind, shape=(32, 16, 16), tol=1e-12, precisi
     if kind == "sphere":
         s.set_obstacle_sphere(*[H * (n // 2 + 0.5) for n in shape], 3 * H)
     else:
-        lo, hi = [H * (n // 2 - 2.5) for n in shape], [H * (n // 2 + 1.5) for n in shape]
+        w = 4 if kind == "box" else 29
+        lo = [H * (n // 2 - w // 2 - 0.5) for n in shape]
+        hi = [a + H * w for a in lo]
         s.set_obstacle_stl_bytes(cases.blocks_stl([(lo[0], hi[0], lo[1], hi[1], hi[2])], base=lo[2]))
     s.set_linear_solver(I.SOLVER_BiCGSTAB, I.PRECOND_AMG, tol)
     s.set_precision(precision)
@@ -75,3 +78,30 @@ def test_body_surface_through_cell_centres(new_gpu, new_oracle, I, cases, kind, 
         s.iterate(3)
         assert (s.last_norms() <= tol).all()
         assert_close(fields(s), ref, 2 * tol * span_of(f))
+
+
+@pytest.mark.parametrize("kind,shape,precision,rounds", [
+    ("sphere", (32, 16, 16), 0, 2), ("sphere", (32, 16, 16), 2, 2),
+    ("box", (32, 16, 16), 0, 2), ("box", (32, 16, 16), 2, 2), ("wide", (96, 64, 64), 2, 4)])
+def test_zero_pressure_rows_are_solved_directly(new_gpu, I, cases, kind, shape, precision, rounds):
+    """Those bodies stay with the direct solve: at most two rounds, four where
+    the ghost rows' inverse is kept in FP32 (a box with 5048 such cells); p'
+    is exactly zero at the cells with phi = 0, and the fields are those of the
+    multigrid solve within the bound above."""
+    tol = 1e-12
+    out = []
+    for multigrid in (False, True):
+        s = new_gpu()
+        if multigrid:
+            s.set_mg_relaxation(1.3)
+        f = setup_surface_body(s, I, cases, kind, shape=shape, tol=tol, precision=precision)
+        s.iterate(2)
+        assert (s.last_norms() <= tol).all()
+        if not multigrid:
+            assert int(s.last_iters()[3]) <= rounds
+        g = s.ghost_cells()
+        on = s.get("LVSET")[tuple(g.T + 2)] == 0
+        assert on.sum() == {"sphere": 30, "box": 98, "wide": 5048}[kind]
+        assert (s.get("P_PRIME")[tuple(g[on].T + 2)] == 0).all()
+        out.append(fields(s))
+    assert_close(out[0], out[1], 2 * tol * span_of(f))
