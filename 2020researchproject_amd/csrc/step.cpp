@@ -669,6 +669,7 @@ void ensure_mg(IBMSolver *s) {
     HIP_CHECK(hipStreamSynchronize(s->stream));
 }
 
+// Gives the inverse back, and its bytes: serving admits by the solver's footprint
 static void free_capacitance(IBMSolver *s) {
     s->cap_on = false;
     s->dev_bytes -= s->cap_inv64.n * sizeof(double) + s->cap_inv32.n * sizeof(float);
@@ -1758,7 +1759,7 @@ static void momentum_concurrent(IBMSolver *s, F &&norms) {
 // until the FP64 residual meets the tolerance. One round reaches the rounding
 // level of the transforms (1e-12 .. 1e-10 of ||b||), a second one that of the
 // residual. A solve whose residual no longer halves is left to the iterative
-// path (false); its reason is the tolerance, not the method. separable_round
+// path (false): the tolerance lies below the rounding level. separable_round
 // enqueues a round, up to the partial sums of its residual's norms.
 static void separable_round(IBMSolver *s, const double *b, double *x, bool first) {
     const Dims &d = s->d;
@@ -1809,9 +1810,8 @@ static bool separable_finish(IBMSolver *s, const double *b, double *x, double bn
     // with a body the memory of the capacitance matrix is the hierarchy's: the
     // solver goes over to the iterative path for good
     if (s->cap_on) {
-        s->sep_on = s->cap_on = false;
-        s->cap_inv64.free();
-        s->cap_inv32.free();
+        s->sep_on = false;
+        free_capacitance(s);
     }
     return false;
 }
