@@ -1035,14 +1035,11 @@ extern "C" int IBMSolver_get_ghost_cells(IBMSolver *s, int *out) {
 }
 
 extern "C" int IBMSolver_get_mg_levels(IBMSolver *s, int *out, int max) {
-    if (s->assembled) ensure_mg(s);
-    const int n = (int)s->mg.size();
-    for (int l = 0; l < n && l < max && out; l++) {
-        out[3 * l] = s->mg[l].d.nx;
-        out[3 * l + 1] = s->mg[l].d.ny;
-        out[3 * l + 2] = s->mg[l].d.nz;
-    }
-    return n;
+    if (!s->assembled) return 0;
+    const auto levels = mg_shapes(s);
+    for (size_t l = 0; l < levels.size() && (int)l < max && out; l++)
+        std::copy(levels[l].begin(), levels[l].end(), out + 3 * l);
+    return (int)levels.size();
 }
 
 extern "C" double IBMSolver_max_div(IBMSolver *s) { return max_div_impl(s); }

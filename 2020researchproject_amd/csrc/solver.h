@@ -1,6 +1,7 @@
 // solver.h - host-side state of one IBMSolver instance (opaque to callers).
 #pragma once
 
+#include <array>
 #include <stdexcept>
 #include <string>
 #include <mutex>
@@ -376,6 +377,7 @@ void build_system(const IBMSolver *s, const std::vector<double> *D[3], const std
 void iterate_impl(IBMSolver *s, int steps, bool verbose);
 void build_mg(IBMSolver *s);
 void ensure_mg(IBMSolver *s);
+std::vector<std::array<int, 3>> mg_shapes(const IBMSolver *s);
 void build_separable(IBMSolver *s);
 void build_separable_momentum(IBMSolver *s);
 void build_momentum_tables(IBMSolver *s);

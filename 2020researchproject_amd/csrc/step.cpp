@@ -459,6 +459,68 @@ static void build_dense(IBMSolver *s, MGLevel &L) {
         if (!std::isfinite(v)) fatal("coarsest multigrid level: singular dense operator");
 }
 
+// Coarsening of one axis: parent of each finer cell, first finer cell of each
+// coarse one
+struct AxisMerge {
+    std::vector<int> parent, start;
+};
+
+// Faces f of level `level` -> those of the next one; false where it is the last.
+// Spacing-aware coarsening: along each axis, two neighbouring cells merge when
+// their combined width is at most 2 * gamma * h_l, where h_l = 2^l * (smallest
+// fine-grid width) is the target width of level l. Where one axis is much finer
+// than the others only that axis coarsens (semi-coarsening in the strongly
+// coupled direction), so the point smoother stays effective on stretched grids;
+// gamma <= 0 selects plain full coarsening of even-sized axes.
+static bool coarsen(const IBMSolver *s, int level, std::vector<double> (&f)[3], AxisMerge (&m)[3]) {
+    const int lo[3] = {3, 2, 4}, hi[3] = {1, 0, 5};
+    const long n[3] = {(long)f[0].size() - 1, (long)f[1].size() - 1, (long)f[2].size() - 1};
+    if (level > 0 && n[0] * n[1] * n[2] <= kDenseCells) return false;
+    double h0 = 1e300;
+    for (const std::vector<double> *x : {&s->xf, &s->yf, &s->zf})
+        for (size_t i = 0; i + 1 < x->size(); i++) h0 = std::min(h0, (*x)[i + 1] - (*x)[i]);
+    const double thr = 2 * s->mg_gamma * h0 * std::ldexp(1.0, level) * (1 + 1e-9);
+    bool merged = false;
+    for (int a = 0; a < 3; a++) {
+        const bool full = s->mg_gamma <= 0 && n[a] % 2 == 0 && n[a] >= 2;
+        // a periodic axis keeps an even cell count, so the two neighbours
+        // across the wrap have different red-black colours
+        const bool per = s->bc[lo[a]].type == BC_ALL_PERIODIC && s->bc[hi[a]].type == BC_ALL_PERIODIC;
+        for (int pass = 0; pass < 2; pass++) {
+            const bool allow = pass == 0;
+            std::vector<double> g{f[a][0]};
+            m[a].parent.assign(n[a], 0);
+            m[a].start.clear();
+            bool any = false;
+            for (int i = 0; i < n[a];) {
+                const bool pair = allow && i + 1 < n[a] &&
+                                  (full || (s->mg_gamma > 0 && f[a][i + 2] - f[a][i] <= thr));
+                m[a].start.push_back(i);
+                m[a].parent[i] = (int)m[a].start.size() - 1;
+                if (pair) { m[a].parent[i + 1] = m[a].parent[i]; any = true; }
+                i += pair ? 2 : 1;
+                g.push_back(f[a][i]);
+            }
+            m[a].start.push_back((int)n[a]);
+            if (pass == 0 && per && any && (g.size() - 1) % 2 == 1) continue;  // odd: leave this axis
+            merged = merged || any;
+            f[a] = g;
+            break;
+        }
+    }
+    return merged;
+}
+
+// Cells per axis of every level, built or not
+std::vector<std::array<int, 3>> mg_shapes(const IBMSolver *s) {
+    std::vector<double> f[3] = {s->xf, s->yf, s->zf};
+    AxisMerge m[3];
+    std::vector<std::array<int, 3>> out;
+    do out.push_back({(int)f[0].size() - 1, (int)f[1].size() - 1, (int)f[2].size() - 1});
+    while (coarsen(s, (int)out.size() - 1, f, m));
+    return out;
+}
+
 void build_mg(IBMSolver *s) {
     s->mg.clear();
     s->mg.emplace_back();
@@ -478,68 +540,27 @@ void build_mg(IBMSolver *s) {
         s->sys[3].S64.omega = s->mg_omega;
         s->sys[3].S32.omega = (float)s->mg_omega;
     }
-    std::vector<double> xf = s->xf, yf = s->yf, zf = s->zf;
+    std::vector<double> f[3] = {s->xf, s->yf, s->zf};
+    AxisMerge merge[3];
     const int lo[3] = {3, 2, 4}, hi[3] = {1, 0, 5};
-    double h0 = 1e300;
-    for (const std::vector<double> *f : {&xf, &yf, &zf})
-        for (size_t i = 0; i + 1 < f->size(); i++) h0 = std::min(h0, (*f)[i + 1] - (*f)[i]);
-    while (true) {
+    while (coarsen(s, (int)s->mg.size() - 1, f, merge)) {
         const MGLevel &P = s->mg.back();
         const int n[3] = {P.d.nx, P.d.ny, P.d.nz};
-        if (s->mg.size() > 1 && (long)n[0] * n[1] * n[2] <= kDenseCells) break;
-        // Spacing-aware coarsening: along each axis, two neighbouring cells
-        // merge when their combined width is at most 2 * gamma * h_l, where
-        // h_l = 2^l * (smallest fine-grid width) is the target width of level
-        // l. Where one axis is much finer than the others only that axis
-        // coarsens (semi-coarsening in the strongly coupled direction), so the
-        // point smoother stays effective on stretched grids; gamma <= 0
-        // selects plain full coarsening of even-sized axes.
-        std::vector<double> *F[3] = {&xf, &yf, &zf};
-        const double thr = 2 * s->mg_gamma * h0 * std::ldexp(1.0, (int)s->mg.size() - 1) * (1 + 1e-9);
-        std::vector<int> parent[3], start[3];
-        bool merged = false;
-        for (int a = 0; a < 3; a++) {
-            const std::vector<double> &f = *F[a];
-            const bool full = s->mg_gamma <= 0 && n[a] % 2 == 0 && n[a] >= 2;
-            // a periodic axis keeps an even cell count, so the two neighbours
-            // across the wrap have different red-black colours
-            const bool per = s->bc[lo[a]].type == BC_ALL_PERIODIC && s->bc[hi[a]].type == BC_ALL_PERIODIC;
-            for (int pass = 0; pass < 2; pass++) {
-                const bool allow = pass == 0;
-                std::vector<double> g{f[0]};
-                parent[a].assign(n[a], 0);
-                start[a].clear();
-                bool any = false;
-                for (int i = 0; i < n[a];) {
-                    const bool pair = allow && i + 1 < n[a] &&
-                                      (full || (s->mg_gamma > 0 && f[i + 2] - f[i] <= thr));
-                    start[a].push_back(i);
-                    parent[a][i] = (int)start[a].size() - 1;
-                    if (pair) { parent[a][i + 1] = parent[a][i]; any = true; }
-                    i += pair ? 2 : 1;
-                    g.push_back(f[i]);
-                }
-                start[a].push_back(n[a]);
-                if (pass == 0 && per && any && (g.size() - 1) % 2 == 1) continue;  // odd: leave this axis
-                merged = merged || any;
-                *F[a] = g;
-                break;
-            }
-        }
-        if (!merged) break;
+        const std::vector<int> *parent[3], *start[3];
+        for (int a = 0; a < 3; a++) parent[a] = &merge[a].parent, start[a] = &merge[a].start;
         MGLevel L;
-        const int m[3] = {(int)xf.size() - 1, (int)yf.size() - 1, (int)zf.size() - 1};
+        const int m[3] = {(int)f[0].size() - 1, (int)f[1].size() - 1, (int)f[2].size() - 1};
         L.d = make_dims(m[0], m[1], m[2]);
-        level_geometry(s, L, xf, yf, zf);
+        level_geometry(s, L, f[0], f[1], f[2]);
         // activity: any fluid child (outer layers active)
         L.hflag.assign(L.d.ncell, F_FLUID);
         for (int K = 0; K < m[2]; K++)
             for (int J = 0; J < m[1]; J++)
                 for (int I = 0; I < m[0]; I++) {
                     bool act = false;
-                    for (int k = start[2][K]; k < start[2][K + 1]; k++)
-                        for (int j = start[1][J]; j < start[1][J + 1]; j++)
-                            for (int i = start[0][I]; i < start[0][I + 1]; i++)
+                    for (int k = (*start[2])[K]; k < (*start[2])[K + 1]; k++)
+                        for (int j = (*start[1])[J]; j < (*start[1])[J + 1]; j++)
+                            for (int i = (*start[0])[I]; i < (*start[0])[I + 1]; i++)
                                 if (P.hflag[cidx(P.d, i, j, k)] == F_FLUID) act = true;
                     L.hflag[cidx(L.d, I, J, K)] = act ? F_FLUID : F_SOLID;
                 }
@@ -598,9 +619,9 @@ void build_mg(IBMSolver *s) {
             std::vector<double> w(n[a]);
             const bool per = s->bc[lo[a]].type == BC_ALL_PERIODIC && s->bc[hi[a]].type == BC_ALL_PERIODIC;
             for (int i = 0; i < n[a]; i++) {
-                const int I = parent[a][i];
+                const int I = (*parent[a])[i];
                 const double xf_ = H1((*cf[a]), i), Xn = H1((*cc[a]), I);
-                if (start[a][I + 1] - start[a][I] == 1) { far[i] = I; w[i] = 1; continue; }
+                if ((*start[a])[I + 1] - (*start[a])[I] == 1) { far[i] = I; w[i] = 1; continue; }
                 const int J = xf_ > Xn ? I + 1 : I - 1;
                 const double Xf = H1((*cc[a]), J);  // outer-layer centre beyond the ends
                 const double wn = (Xf - xf_) / (Xf - Xn);
@@ -621,8 +642,8 @@ void build_mg(IBMSolver *s) {
             }
             pidx[a]->upload(far);
             pw[a]->upload(w);
-            cpar[a]->upload(parent[a]);
-            cst[a]->upload(start[a]);
+            cpar[a]->upload(*parent[a]);
+            cst[a]->upload(*start[a]);
         }
         {
             // fine cells whose interpolation stencil touches an inactive coarse cell
@@ -630,8 +651,8 @@ void build_mg(IBMSolver *s) {
             for (int k = 0; k < n[2]; k++)
                 for (int j = 0; j < n[1]; j++)
                     for (int i = 0; i < n[0]; i++) {
-                        const int I2[2] = {parent[0][i], hfar[0][i]}, J2[2] = {parent[1][j], hfar[1][j]},
-                                  K2[2] = {parent[2][k], hfar[2][k]};
+                        const int I2[2] = {(*parent[0])[i], hfar[0][i]}, J2[2] = {(*parent[1])[j], hfar[1][j]},
+                                  K2[2] = {(*parent[2])[k], hfar[2][k]};
                         bool solid = false;
                         for (int c = 0; c < 8; c++)
                             solid |= L.hflag[cidx(L.d, I2[c & 1], J2[(c >> 1) & 1], K2[c >> 2])] == F_SOLID;

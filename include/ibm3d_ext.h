@@ -125,9 +125,11 @@ void IBMSolver_get_last_iters(IBMSolver *, int out[4]);
    fastest): writes 3*count ints when out != NULL, returns count. */
 int IBMSolver_get_ghost_cells(IBMSolver *, int *out);
 
-/* Shapes of the pressure multigrid levels built by IBMSolver_assemble, or by
-   this call where the pressure is solved directly (level 0 = the fine grid): writes nx, ny, nz of up to max levels into out
-   when out != NULL, returns the number of levels. */
+/* Shapes of the pressure multigrid levels (level 0 = the fine grid), which a
+   directly solved system has only once a solve leaves that path: the call
+   itself builds and allocates nothing. Writes nx, ny, nz of up to max levels
+   into out when out != NULL, returns the number of levels (0 before
+   IBMSolver_assemble). */
 int IBMSolver_get_mg_levels(IBMSolver *, int *out, int max);
 
 /* max |div U| over fluid cells, U the face velocity after projection. Where

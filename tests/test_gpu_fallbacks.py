@@ -147,3 +147,23 @@ def test_hand_over_from_the_direct_solves(new_gpu, gpu_lib, cases, kind, shape, 
         assert 8 * ld * ld > keep
         assert held[0] - held[1] <= keep
     assert held[0] <= gpu_lib.IBMSolver_estimate_device_bytes(*shape, precision, 0)
+
+
+@pytest.mark.parametrize("kind,shape", [("sphere", (66, 33, 35)), ("cavity", (45, 37, 29)), ("channel", (64, 48, 32))])
+def test_level_shapes_are_asked_for_without_building_them(new_gpu, cases, kind, shape):
+    """The query gives a directly solved system the levels of the iterative
+    solver and leaves the footprint as it was."""
+    levels = []
+    for direct in (True, False):
+        s = new_gpu()
+        assert s.mg_levels() == []
+        if not direct:
+            s.set_mg_relaxation(1.3)
+        if kind == "cavity":
+            cases.setup_cavity(s, shape=shape)
+        else:
+            {"sphere": cases.setup_sphere, "channel": cases.setup_channel}[kind](s, *shape)
+        held = s.device_bytes()
+        levels.append(s.mg_levels())
+        assert s.device_bytes() == held
+    assert levels[0] == levels[1] and levels[0][0] == shape and len(levels[0]) > 1
