@@ -642,18 +642,7 @@ static void alloc_fields(IBMSolver *s) {
         s->ref_e32.alloc(n);
         if (s->precision == IBM3D_PREC_MIXED_KRYLOV) s->ref_e32b.alloc(n);
     }
-    if (s->solver_type != SOLVER_BiCGSTAB) {
-        // pressure solver scratch: GMRES basis, or the PCG / stationary
-        // multigrid vectors (Krylov vectors above) and scalars
-        GmresData &G = s->gm;
-        if (s->solver_type == SOLVER_GMRES) {
-            for (int v = 0; v <= kGmresRestart; v++) G.V[v].alloc(n);
-            for (int v = 0; v < kGmresRestart; v++) G.Z[v].alloc(n);
-            G.t.alloc(n);
-        }
-        G.dev.alloc(64);
-        G.partial.alloc((size_t)krylov_blocks(s->d) * (kVecSetMax + 1));
-    }
+    ensure_solver_vectors(s);
     long nb = conv_rhs_blocks(s->d) + 64;
     nb = std::max(nb, apply_partials(s->d, s->ng) + 64);
     nb = std::max(nb, vec_partials(s->d) + 64);

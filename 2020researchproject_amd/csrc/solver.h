@@ -377,6 +377,7 @@ void build_system(const IBMSolver *s, const std::vector<double> *D[3], const std
 void iterate_impl(IBMSolver *s, int steps, bool verbose);
 void build_mg(IBMSolver *s);
 void ensure_mg(IBMSolver *s);
+void ensure_solver_vectors(IBMSolver *s);
 std::vector<std::array<int, 3>> mg_shapes(const IBMSolver *s);
 void build_separable(IBMSolver *s);
 void build_separable_momentum(IBMSolver *s);

@@ -844,6 +844,22 @@ static bool build_capacitance(IBMSolver *s) {
     return true;
 }
 
+// GMRES basis, or the scalars of the PCG and stationary multigrid solvers, where
+// such a pressure solver is set and has none yet
+void ensure_solver_vectors(IBMSolver *s) {
+    if (s->solver_type == SOLVER_BiCGSTAB) return;
+    GmresData &G = s->gm;
+    DevBytesScope account(&s->dev_bytes);
+    if (s->solver_type == SOLVER_GMRES && !G.t.p) {
+        for (auto &v : G.V) v.alloc(s->d.ncell);
+        for (auto &v : G.Z) v.alloc(s->d.ncell);
+        G.t.alloc(s->d.ncell);
+    }
+    if (G.dev.p) return;
+    G.dev.alloc(64);
+    G.partial.alloc((size_t)krylov_blocks(s->d) * (kVecSetMax + 1));
+}
+
 // Direct pressure solve (separable.hip) where the system allows it: every axis
 // symmetric in its cell widths (all but a periodic axis that is not uniform),
 // no body or one that build_capacitance takes, and the solver asked for is the
@@ -1844,7 +1860,15 @@ static void solve_system(IBMSolver *s, int sk, const double *b, double *x, doubl
     const int maxit = sk == 3 ? 1000 : 200;  // src/ibm3d_setup.c:1413, 1467
     double rel = 0;
     int it;
-    if (sk == 3) ensure_mg(s);
+    // (the solver and preconditioner types may have been set since the assembly)
+    if (sk == 3 && (s->precond_type == PRECOND_AMG || s->solver_type == SOLVER_AMG)) {
+        if (s->cap_on) {  // its memory is the hierarchy's
+            s->sep_on = false;
+            free_capacitance(s);
+        }
+        ensure_mg(s);
+    }
+    if (sk == 3) ensure_solver_vectors(s);
     if (sk == 3 && s->solver_type != SOLVER_BiCGSTAB && s->precision != IBM3D_PREC_MIXED) {
         // multigrid cycles in FP32 in the mixed-Krylov mode; SOLVER_AMG is the
         // cycle itself, with no separate preconditioner
@@ -2248,7 +2272,7 @@ static void do_step(IBMSolver *s) {
         TIMED("k3_update", cn * (15 * 8 + 1),
               launch_update(s->stream, s->geo, sp, s->flag.p, s->p.p, s->pp.p, us3, Fs, s->pn.p, un, Fn));
     };
-    const bool direct = s->sep_on;
+    const bool direct = s->sep_on && s->solver_type == SOLVER_BiCGSTAB && s->precond_type == PRECOND_AMG;
     double bnp = 0;
     for (;;) {
         // outer layers of the three solutions from their BC rows (the per-component
