@@ -199,8 +199,14 @@ void IBMSolver_set_bc(IBMSolver *s, IBMSolverDirection dir, IBMSolverBCType type
         fprintf(stderr, "error: invalid boundary condition value type\n");
     v.type = type;
     v.set = true;
+    bool retyped = false;
     for (int i = 0; i < 6; i++)
-        if (dir & (1 << i)) s->bc[i] = v;
+        if (dir & (1 << i)) {
+            retyped |= s->bc[i].type != v.type;
+            s->bc[i] = v;
+        }
+    // the outer layers follow the type as it is now
+    if (s->assembled && retyped) build_outer_rules(s);
 }
 
 void IBMSolver_set_obstacle(IBMSolver *s, Polyhedron *poly) {

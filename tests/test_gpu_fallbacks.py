@@ -207,3 +207,38 @@ def test_pressure_solver_set_after_assembly(new_gpu, gpu_lib, I, cases, solver, 
     assert its[0] == its[1] and its[0][0][3] > 2
     for n, a in out[0].items():
         assert np.array_equal(a, out[1][n], equal_nan=True), n
+
+
+@pytest.mark.parametrize("face,types", [
+    ("DIR_NORTH", ("wall", "slip")), ("DIR_UP", ("slip", "velocity")), ("DIR_EAST", ("pressure", "velocity")),
+    ("DIR_SOUTH", ("velocity", "pressure")), ("DIR_NORTH", ("velocity", "velocity2"))])
+def test_boundary_types_set_after_assembly(new_gpu, new_oracle, I, face, types):
+    """IBMSolver_set_bc after the assembly: the outer layers follow the type
+    and the values as they are now (the systems keep those they were assembled
+    with). A short sum of products: 1e-12 of the largest value."""
+    args = {"wall": (I.BC_STATIONARY_WALL,), "slip": (I.BC_FREE_SLIP_WALL,),
+            "pressure": (I.BC_PRESSURE, I.VAL_CONST, 0.75),
+            "velocity": (I.BC_VELOCITY_COMPONENT, I.VAL_CONST, 1.0, 0.25, -0.5),
+            "velocity2": (I.BC_VELOCITY_COMPONENT, I.VAL_CONST, -2.0, 0.5, 0.125)}
+    out = []
+    for new in (new_gpu, new_oracle):
+        s = new()
+        s.set_grid(*[np.linspace(0.0, 1.0 + a, n + 1) ** 1.5 for a, n in enumerate((18, 16, 14))])
+        s.set_params(100.0, 0.002)
+        s.set_bc(63, I.BC_STATIONARY_WALL)
+        s.set_bc(I.DIR_WEST, I.BC_PRESSURE, I.VAL_CONST, 0.0)
+        s.set_bc(getattr(I, face), *args[types[0]])
+        s.set_obstacle(None)
+        s.set_linear_solver(I.SOLVER_BiCGSTAB, I.PRECOND_AMG, 1e-10)
+        s.assemble()
+        s.init_flow_const(0, 0, 0, 0)
+        rng = np.random.default_rng(5)
+        for n in ("U1", "U2", "U3", "P"):
+            s.set(n, rng.standard_normal(s.shape))
+        s.iterate(0)
+        s.set_bc(getattr(I, face), *args[types[1]])
+        s.iterate(0)
+        out.append({n: s.get(n) for n in ("U1", "U2", "U3", "P")})
+    for n, a in out[0].items():
+        error, scale = np.abs(a - out[1][n]).max(), np.abs(out[1][n]).max()
+        assert error <= 1e-12 * scale, n
