@@ -1944,7 +1944,13 @@ static int momentum_sweeps(IBMSolver *s) {
     const double rate = s->ng > 0 ? std::max(rj * rj, kMomGhostRate) : rj * rj;
     s->mom_rate = rate;
     const double target = s->precision == IBM3D_PREC_FP64 ? 0.5 * s->tol : kMomRoundTarget;
-    s->mom_sweeps = (rate > 0 && rate <= kMomMaxRate)
+    // an odd periodic axis (accepted without the multigrid preconditioner): the two
+    // cells beside the wrap share a colour, and a colour launch would read a
+    // neighbour that it is writing
+    bool odd = false;
+    const int n[3] = {s->Nx, s->Ny, s->Nz};
+    for (int a = 0; a < 3; a++) odd |= s->sys[0].S64.ax[a].periodic && n[a] % 2;
+    s->mom_sweeps = (rate > 0 && rate <= kMomMaxRate && !odd)
                         ? std::max(2, (int)std::ceil(std::log(target) / std::log(rate))) : 0;
     return s->mom_sweeps;
 }

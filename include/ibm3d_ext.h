@@ -99,8 +99,8 @@ int IBMSolver_get_pressure_mg_bits(IBMSolver *);
    the tolerance, red-black Gauss-Seidel sweeps, in FP64 on the system itself
    or (mixed) in FP32 inside FP64 iterative refinement, where the operator is
    diagonally dominant enough (max over cells of sum K / (1 + sum K) squared
-   <= 0.5), BiCGSTAB elsewhere and for any component whose residual stops
-   falling; 1: always BiCGSTAB (FP64, Jacobi preconditioner; mixed: FP32 stored
+   <= 0.5) and periodic axes have even cell counts, BiCGSTAB elsewhere and for
+   any component whose residual stops falling; 1: always BiCGSTAB (FP64, Jacobi preconditioner; mixed: FP32 stored
    directions). All stop on the reference's test ||b - A x|| <= tol ||b|| in
    FP64; IBMSolver_get_last_iters counts sweeps or iterations (1: direct). */
 void IBMSolver_set_momentum_solver(IBMSolver *, int mode);
