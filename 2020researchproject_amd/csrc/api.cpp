@@ -12,8 +12,8 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <exception>
 #include <sched.h>
-#include <system_error>
 #include <thread>
 
 #include "solver.h"
@@ -871,11 +871,12 @@ static void download(IBMSolver *s, const void *dev, size_t bytes, void *out) {
     };
     std::vector<std::thread> threads;
     hipError_t err = hipSuccess;
-    threads.reserve(kStageThreads);
     try {
+        threads.reserve(kStageThreads);
         while (threads.size() < kStageThreads) threads.emplace_back(worker);
-    } catch (const std::system_error &) {
-        // with the threads there are; without any, the copies are made below
+    } catch (const std::exception &) {
+        // no thread or no memory for one: with the threads there are; without
+        // any, the copies are made below
     }
     long issued = 0;
     for (long c = 0; c < chunks && err == hipSuccess; c++) {

@@ -3,8 +3,14 @@ from the iterative ones: systems they cannot hold, tolerances they cannot
 reach, settings made after assembly."""
 from __future__ import annotations
 
+import subprocess
+import sys
+import textwrap
+
 import numpy as np
 import pytest
+
+from conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -272,3 +278,26 @@ def test_odd_periodic_axis_takes_no_red_black_sweeps(new_gpu, I, shape, precisio
     assert out[0][0] == out[1][0]
     for n, a in out[0][1].items():
         assert np.array_equal(a, out[1][1][n], equal_nan=True), n
+
+
+def test_large_field_without_copying_threads():
+    """A field that crosses through the ring of pinned chunks where no thread
+    can be made: the caller's own copies it, bit for bit. In a child process
+    whose limit is lowered once its first read has set the runtime up."""
+    code = textwrap.dedent(f"""
+        import sys, importlib, resource
+        import numpy as np
+        sys.path.insert(0, {ROOT!r})
+        pkg = importlib.import_module("2020researchproject_amd")
+        s = pkg.ibm3d.Solver()
+        pkg.cases.setup_cavity(s, shape=(128, 96, 96), tol=1e-8)
+        a = np.random.default_rng(2).standard_normal(s.shape)
+        s.set("P", a)
+        assert a.nbytes > 8 << 20 and np.array_equal(s.get("P"), a)
+        resource.setrlimit(resource.RLIMIT_NPROC, (1, resource.getrlimit(resource.RLIMIT_NPROC)[1]))
+        for _ in range(2):
+            assert np.array_equal(s.get("P"), a)
+        print("same")
+    """)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "same" in r.stdout, (r.returncode, r.stderr)
