@@ -5,8 +5,9 @@
 // Assembly differs by design: instead of building four Hypre ParCSR matrices
 // (src/ibm3d_setup.c:1566-2908) it folds the outer boundary rows into
 // separable per-axis stencil coefficients, precomputes the immersed-boundary
-// ghost stencils once (they only depend on the static level set), and builds
-// the geometric multigrid hierarchy of the pressure system.
+// ghost stencils once (they only depend on the static level set), and sets up
+// the pressure solve: eigenvectors of the axes and the ghost rows' inverse for
+// the direct one, else the geometric multigrid hierarchy.
 #include <algorithm>
 #include <atomic>
 #include <cmath>

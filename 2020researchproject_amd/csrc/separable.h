@@ -1,4 +1,5 @@
-// separable.h - direct solve of the pressure system of a box without a body.
+// separable.h - direct solves of separable systems: the pressure and momentum of
+// a box, the pressure with an immersed body.
 #pragma once
 
 #include <vector>

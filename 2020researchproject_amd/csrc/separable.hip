@@ -360,8 +360,10 @@ __global__ void __launch_bounds__(kSepThreads) k_sep_back(Dims d, SeparableBatch
 
 static int sep_pad16(int n) { return (n + 15) / 16 * 16; }
 
-// LDS of a workgroup: two fit a compute unit (with 64 KB the last kernel takes
-// 103 us at 256 x 128 x 128 instead of 71: two row tiles need 66 KB)
+// LDS tile of a workgroup, at most half a compute unit's: two workgroups share
+// one up to a few bytes less (k_sep_z's 64 static bytes leave one at exactly
+// half: 256 cells in z). With 64 KB the last kernel takes 103 us at 256 x 128 x
+// 128 instead of 71: two row tiles need 66 KB.
 constexpr size_t kSepLds = 80 * 1024;
 
 // Row pitch of a column-read tile of nb tiles of 16 beside a padded axis of np

@@ -289,9 +289,10 @@ double IBMSolver_estimate_device_bytes(int Nx, int Ny, int Nz, int precision, in
     // (+ a second FP32 correction in mode 2); mode 1: 8 FP32 Krylov vectors
     if (mixed) per += 8 + 4 + 4 + (precision == IBM3D_PREC_MIXED_KRYLOV ? 4 : 0);
     if (precision == IBM3D_PREC_MIXED) per += 4 * 8;
-    // the multigrid hierarchy, or the ghost rows' capacitance matrix of a
-    // direct pressure solve, which is limited to its size
-    // reduction partials, ghost lists, 1-D metrics and folded coefficients
+    // multigrid_bytes: the multigrid hierarchy, or the ghost rows' capacitance
+    // matrix of a direct pressure solve, which is limited to its size. 16 MiB:
+    // reduction partials, ghost lists, 1-D metrics, folded coefficients and
+    // eigenvectors of the axes.
     return cells * per + ibm::multigrid_bytes(d, precision) + 16.0 * (1 << 20);
 }
 

@@ -297,7 +297,7 @@ struct _ibm_solver {
     ibm::SysData sys[4];                  // u1, u2, u3, p
     long pin = -1;
     std::vector<ibm::MGLevel> mg;         // mg[0] = fine pressure level; empty until ensure_mg
-    // direct pressure solve of a box without a body (build_separable)
+    // direct pressure solve (build_separable)
     bool sep_on = false;
     ibm::SeparableSys sep{};
     ibm::DBuf<double> sep_mat[3][3];      // V, Vi, lam per axis

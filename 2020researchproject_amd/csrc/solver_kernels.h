@@ -271,9 +271,10 @@ template <typename T>
 void launch_coarse_solve(hipStream_t st, const Dims &d, const SysCoef<T> &S, const uint8_t *flag, const T *b, T *x,
                          int sweeps, int singular, const double *dxyz);
 
-// In-place Gauss-Jordan inversion without pivoting of
-// the n x n row-major matrix A of row pitch ld (diagonally dominant M-matrix
-// rows); scratch: gauss_jordan_scratch(n) doubles.
+// In-place Gauss-Jordan inversion without pivoting of the n x n row-major
+// matrix A of row pitch ld: for diagonally dominant M-matrix rows (coarsest
+// multigrid level); other matrices (ghost rows, growth below 50 on spheres) are
+// to be looked at afterwards. scratch: gauss_jordan_scratch(n) doubles.
 size_t gauss_jordan_scratch(int n);
 void gauss_jordan_invert(hipStream_t st, double *A, int n, long ld, double *scratch);
 void launch_d2f_flat(hipStream_t st, const double *a, float *b, long n);

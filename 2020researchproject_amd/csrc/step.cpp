@@ -1923,7 +1923,12 @@ static void solve_system(IBMSolver *s, int sk, const double *b, double *x, doubl
 // too few and a round more followed (sphere 133 x 67 x 61: 70 us against 22 for
 // a sweep more). What that third round gave beyond the tolerance a Jacobi step
 // gives as well (k_mom_residual<3>, 8 us); at larger rates there were two
-// rounds, and the step would gain less (256 x 128 x 128: 70 us).
+// rounds before as well, and the step would cost more (256 x 128 x 128: 70 us).
+// Error of the pressure against FP64 solves at 1e-14, ten steps with the
+// convective outlet: with the step 1.3e-13 (133 x 67 x 61; three rounds
+// 2.6e-12); without it 5.3e-10 (256 x 128 x 128, two rounds before 5.4e-10).
+// Spheres at rates 0.01 to 0.48, three steps: 1e-11 to 6e-11 without it, 6e-12 to
+// 1.2e-10 by the rounds and BiCGSTAB solves before.
 static const double kMomGhostRate = 3e-3;
 static const double kMomRoundTarget = 1e-6;  // residual reduction aimed at per FP32 round
 // Largest rho_J^2 for which sweeps are used, the largest measured: ms per step
@@ -1932,7 +1937,7 @@ static const double kMomRoundTarget = 1e-6;  // residual reduction aimed at per 
 // 96^3 at 0.337 4.26 : 5.26 / 3.86 : 5.04, 128^3 at 0.008 5.27 : 6.25 / 5.73 :
 // 6.51, at 0.246 6.18 : 8.27 / 6.29 : 8.34, at 0.505 7.52 : 10.41 / 7.28 : 10.10
 static const double kMomMaxRate = 0.5;
-static const int kMomMaxRounds = 8; 
+static const int kMomMaxRounds = 8;
 
 static int momentum_sweeps(IBMSolver *s) {
     if (s->mom_sweeps >= 0) return s->mom_sweeps;
